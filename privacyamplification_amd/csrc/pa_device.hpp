@@ -53,6 +53,18 @@ __device__ __forceinline__ float2 w32pow(float2 v, int r) {
     return make_float2(-t.x, -t.y);
 }
 
+// v * exp(-2 pi i r / 64) for a compile-time-foldable r in [0, 16).
+__device__ __forceinline__ float2 w64pow(float2 v, int r) {
+    if ((r & 1) == 0) return twc<32>(v, r / 2);
+    const float c = r == 1 ? 9.951847267e-01f : r == 3 ? 9.569403357e-01f : r == 5 ? 8.819212643e-01f
+                  : r == 7 ? 7.730104534e-01f : r == 9 ? 6.343932842e-01f : r == 11 ? 4.713967368e-01f
+                  : r == 13 ? 2.902846773e-01f : 9.801714033e-02f;
+    const float n = r == 1 ? 9.801714033e-02f : r == 3 ? 2.902846773e-01f : r == 5 ? 4.713967368e-01f
+                  : r == 7 ? 6.343932842e-01f : r == 9 ? 7.730104534e-01f : r == 11 ? 8.819212643e-01f
+                  : r == 13 ? 9.569403357e-01f : 9.951847267e-01f;
+    return cmul(v, make_float2(c, -n));
+}
+
 // tan(pi q / 16), q = 1, 2, 3, 4 (exact values rounded to float).
 __host__ __device__ constexpr float tan16(int q) {
     return q == 1 ? 1.989123674e-01f : q == 2 ? 4.142135624e-01f : q == 3 ? 6.681786379e-01f : 1.0f;
@@ -147,19 +159,58 @@ __device__ __forceinline__ void load_twl(float2* twl, const float2* __restrict__
         twl[i] = i < 128 ? tw14[i] : tw14[((i - 128) * 128) & (TW14 - 1)];
 }
 
-// tw[r] = exp(-2 pi i r x / 2^14) for r < R from log2(R) table reads (r = 2^b) and at most
-// log2(R)-1 products for the other r.
-template <int R>
-__device__ __forceinline__ void twiddle_powers(float2 (&tw)[R], const float2* twl, int x) {
-    tw[0] = make_float2(1.f, 0.f);
+// DFT of twiddled inputs, X[q] = sum_r x_r w^r exp(-2 pi i r q / R), with the twiddles merged into the
+// butterflies: the size-s level of the radix-2 decimation combines E[q] +- w^(R/s) w_s^q O[q], six
+// FMAs per butterfly (the second output as 2 E - first), where separate products cost 4 more per
+// input.  tw holds the R/2 distinct factors: size 2 at [0], size s >= 4 at [s/4 + q], q < s/4 (the
+// factor of q + s/4 is -i times that of q).
+__device__ __forceinline__ void bfly_tw(float2 e, float2 o, float2 w, float2& lo, float2& hi) {
+    lo = make_float2(fmaf(w.x, o.x, fmaf(-w.y, o.y, e.x)), fmaf(w.x, o.y, fmaf(w.y, o.x, e.y)));
+    hi = make_float2(fmaf(2.f, e.x, -lo.x), fmaf(2.f, e.y, -lo.y));
+}
+template <int R, int RT>
+__device__ __forceinline__ void dft_tw_level(float2 (&x)[R], const float2 (&tw)[RT / 2]) {
+    if constexpr (R == 2) {
+        const float2 e = x[0], o = x[1];
+        bfly_tw(e, o, tw[0], x[0], x[1]);
+    } else {
+        constexpr int Q = R / 2;
+        float2 e[Q], o[Q];
 #pragma unroll
-    for (int b = 1; b < R; b <<= 1) tw[b] = tw_lds(twl, (b * x) & (TW14 - 1));
+        for (int i = 0; i < Q; ++i) {
+            e[i] = x[2 * i];
+            o[i] = x[2 * i + 1];
+        }
+        dft_tw_level<Q, RT>(e, tw);
+        dft_tw_level<Q, RT>(o, tw);
 #pragma unroll
-    for (int r = 3; r < R; ++r) {
-        if ((r & (r - 1)) == 0) continue;
-        const int hb = 1 << (31 - __builtin_clz(r));
-        tw[r] = cmul(tw[hb], tw[r - hb]);
+        for (int k = 0; k < Q; ++k) {
+            const float2 w = tw[R / 4 + k % (R / 4)];
+            bfly_tw(e[k], o[k], k < R / 4 ? w : make_float2(w.y, -w.x), x[k], x[k + Q]);
+        }
     }
+}
+template <int R>
+__device__ __forceinline__ void dft_tw(float2 (&x)[R], const float2 (&tw)[R / 2]) {
+    dft_tw_level<R, R>(x, tw);
+}
+// The factors of dft_tw<R> from w^(R/2), w^(R/4), ..., w (pw[0], pw[1], ...).
+template <int R>
+__device__ __forceinline__ void twiddle_set(float2 (&tw)[R / 2], const float2* pw) {
+    tw[0] = pw[0];
+#pragma unroll
+    for (int s = 4, l = 1; s <= R; s *= 2, ++l) {
+#pragma unroll
+        for (int q = 0; q < s / 4; ++q) tw[s / 4 + q] = w32pow(pw[l], q * (32 / s));
+    }
+}
+// The same with w = exp(-2 pi i x / 2^14) from the LDS table: log2(R) table reads.
+template <int R>
+__device__ __forceinline__ void twiddle_set_lds(float2 (&tw)[R / 2], const float2* twl, int x) {
+    float2 pw[5];
+#pragma unroll
+    for (int m = R / 2, l = 0; m >= 1; m /= 2, ++l) pw[l] = tw_lds(twl, (m * x) & (TW14 - 1));
+    twiddle_set<R>(tw, pw);
 }
 
 // Hides an integer's value from the optimiser: per-lane address arithmetic repeated in two phases
@@ -169,13 +220,19 @@ __device__ __forceinline__ int opaque_int(int x) {
     return x;
 }
 
-// Twiddle table of one Stockham stage in LDS: row q < NS holds w^(q r / (NS R)) for r < R, rows
-// padded to R + 1 entries (bank spread).  Filled by all threads; the caller synchronises.
+// Factor table of one Stockham stage in LDS: row q < NS holds dft_tw<R>'s factors for
+// w = exp(-2 pi i q / (NS R)), rows padded to R/2 + 1 entries (bank spread).  Filled by all threads;
+// the caller synchronises.
+template <int R>
+__host__ __device__ constexpr int stage_row() { return R / 2 + 1; }
 template <int R, int NS>
 __device__ __forceinline__ void fill_stage_table(float2* tab, const float2* __restrict__ tw14, int nthreads) {
-    for (int e = threadIdx.x; e < NS * (R + 1); e += nthreads) {
-        const int q = e / (R + 1), r = e % (R + 1);
-        tab[e] = r < R ? tw14[(q * (TW14 / (NS * R)) * r) & (TW14 - 1)] : make_float2(0.f, 0.f);
+    for (int e = threadIdx.x; e < NS * (R / 2); e += nthreads) {
+        const int q = e / (R / 2), i = e % (R / 2);
+        int s = 2;  // the size of entry i and its index k at that size
+        while (s / 2 <= i && i > 0) s *= 2;
+        const int k = i ? i - s / 4 : 0;
+        tab[q * stage_row<R>() + i] = tw14[(q * (TW14 / (NS * s)) + k * (TW14 / s)) & (TW14 - 1)];
     }
 }
 
@@ -212,17 +269,19 @@ __device__ __forceinline__ void stockham_stage(float2* buf, const float2* twl) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) v[i][r] = base[padi(j + r * BPS)];
             }
-            if constexpr (NS > 1 && TAB) {
-                const float2* trow = twl + (j % NS) * (R + 1);
+            if constexpr (NS > 1) {
+                float2 tw[R / 2];
+                if constexpr (TAB) {
+                    const float2* trow = twl + (j % NS) * stage_row<R>();
 #pragma unroll
-                for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], trow[r]);
-            } else if constexpr (NS > 1) {
-                float2 tw[R];
-                twiddle_powers<R>(tw, twl, (j % NS) * (TW14 / (NS * R)));
-#pragma unroll
-                for (int r = 1; r < R; ++r) v[i][r] = cmul(v[i][r], tw[r]);
+                    for (int r = 0; r < R / 2; ++r) tw[r] = trow[r];
+                } else {
+                    twiddle_set_lds<R>(tw, twl, (j % NS) * (TW14 / (NS * R)));
+                }
+                dft_tw<R>(v[i], tw);
+            } else {
+                dft<R>(v[i]);
             }
-            dft<R>(v[i]);
         }
     }
     __syncthreads();
@@ -258,8 +317,7 @@ __device__ __forceinline__ void stage_first_to_lds(float2 (&v)[R], float2* seqbu
 // Last Stockham stage (span L/R) for one butterfly j, read from LDS; the outputs stay in
 // registers: v[r] = X[j + r L/R].
 template <int R, int L>
-__device__ __forceinline__ void stage_last_from_lds(float2 (&v)[R], const float2* seqbuf, int j,
-                                                    const float2* twl) {
+__device__ __forceinline__ void stage_last_read(float2 (&v)[R], const float2* seqbuf, int j) {
     constexpr int NS = L / R;
     if constexpr (NS % (1 << PAD_SHIFT) == 0) {
         const float2* rb = seqbuf + padi(j);
@@ -269,30 +327,25 @@ __device__ __forceinline__ void stage_last_from_lds(float2 (&v)[R], const float2
 #pragma unroll
         for (int r = 0; r < R; ++r) v[r] = seqbuf[padi(j + r * NS)];
     }
-    float2 tw[R];
-    twiddle_powers<R>(tw, twl, j * (TW14 / L));
-#pragma unroll
-    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], tw[r]);
-    dft<R>(v);
+}
+template <int R, int L>
+__device__ __forceinline__ void stage_last_from_lds(float2 (&v)[R], const float2* seqbuf, int j,
+                                                    const float2* twl) {
+    stage_last_read<R, L>(v, seqbuf, j);
+    float2 tw[R / 2];
+    twiddle_set_lds<R>(tw, twl, j * (TW14 / L));
+    dft_tw<R>(v, tw);
 }
 
-// stage_last_from_lds with the twiddles of butterfly j read from a stage table
-// (fill_stage_table<R, L / R>): trow = table + (j % (L / R)) * (R + 1).
+// stage_last_from_lds with butterfly j's factors read from a table row.
 template <int R, int L>
 __device__ __forceinline__ void stage_last_from_lds_tab(float2 (&v)[R], const float2* seqbuf, int j,
                                                         const float2* trow) {
-    constexpr int NS = L / R;
-    if constexpr (NS % (1 << PAD_SHIFT) == 0) {
-        const float2* rb = seqbuf + padi(j);
+    stage_last_read<R, L>(v, seqbuf, j);
+    float2 tw[R / 2];
 #pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = rb[r * padi(NS)];
-    } else {
-#pragma unroll
-        for (int r = 0; r < R; ++r) v[r] = seqbuf[padi(j + r * NS)];
-    }
-#pragma unroll
-    for (int r = 1; r < R; ++r) v[r] = cmul(v[r], trow[r]);
-    dft<R>(v);
+    for (int r = 0; r < R / 2; ++r) tw[r] = trow[r];
+    dft_tw<R>(v, tw);
 }
 
 // Radix-16 stages from span NS up to 2^LG; a final radix-32 stage absorbs a leftover factor 2.
@@ -325,7 +378,7 @@ __device__ __forceinline__ void lds_fft(float2* buf, const float2* twl) {
     }
 }
 
-// exp(-2 pi i x / L) from a two-level table: lo[x mod 2^14] * hi[x >> 14].
+// exp(-2 pi i x / (2L)) from a two-level table: lo[x mod 2^14] * hi[x >> 14].
 __device__ __forceinline__ float2 tw_two_level(const float2* __restrict__ lo,
                                                const float2* __restrict__ hi, uint32_t x) {
     return cmul(lo[x & (TW14 - 1)], hi[x >> TW14_LOG]);
@@ -351,24 +404,6 @@ __device__ __forceinline__ float2 c2r_split(float2 pk, float2 pp, float2 w) {
     const float2 t = cmul(conjf2(w), d);
     return make_float2(e.x - t.y, e.y + t.x);  // e + i*t
 }
-// Both splits of a partner pair k, N-k at once.  The partner's twiddle is
-// exp(-2 pi i (N-k)/(2N)) = -conj(w), so its sum, difference and twiddled difference are the
-// conjugate, the negated conjugate and the conjugate of the first one's: one complex product
-// serves both.  r2c_split_pair returns 2 X[k], 2 X[N-k]; c2r_split_pair returns 2 Q[k], 2 Q[N-k].
-__device__ __forceinline__ void r2c_split_pair(float2 zk, float2 zp, float2 w, float2& xk, float2& xp) {
-    const float2 zc = conjf2(zp);
-    const float2 e = cadd(zk, zc);
-    const float2 t = cmul(w, csub(zk, zc));
-    xk = make_float2(e.x + t.y, e.y - t.x);
-    xp = make_float2(e.x - t.y, -(e.y + t.x));
-}
-__device__ __forceinline__ void c2r_split_pair(float2 pk, float2 pp, float2 w, float2& qk, float2& qp) {
-    const float2 pc = conjf2(pp);
-    const float2 e = cadd(pk, pc);
-    const float2 t = cmul(conjf2(w), csub(pk, pc));
-    qk = make_float2(e.x - t.y, e.y + t.x);
-    qp = make_float2(e.x + t.y, t.x - e.y);
-}
 // 2 X[N] (Nyquist) of the length-2N real transform from Z[0], matching r2c_split's scale.
 __device__ __forceinline__ float2 r2c_nyquist(float2 z0) { return make_float2(2.f * (z0.x - z0.y), 0.f); }
 
@@ -389,6 +424,12 @@ __device__ __forceinline__ float correction(uint32_t wk, uint32_t ws, uint32_t L
     const uint64_t prod = (uint64_t)wk * (uint64_t)ws;
     const uint64_t r = prod & (2ull * L - 1ull);  // L is a power of two
     return (float)((double)r / (double)L);
+}
+
+// The half-integer part of the four-step path's conv values at a position q of column t2 (q = t2
+// mod 4; pops = both operands' popcounts): (pops + q + 1) / 2 mod 2, see pa_geom.hpp.
+__device__ __forceinline__ float mean_half(uint32_t pops, uint32_t t2) {
+    return 0.5f * (float)((pops + t2 + 1u) & 3u);
 }
 
 // The output bit of a pre-rounding value: round half to even, then the parity (ToBinaryArray,

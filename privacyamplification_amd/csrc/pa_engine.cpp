@@ -30,6 +30,7 @@
 namespace {
 
 using pa::Geom;
+using pa::mid_size;
 
 #define PA_HIP(expr)                                              \
     do {                                                          \
@@ -46,6 +47,7 @@ void set_error(hipError_t e, const char* what, const char* file, int line) {
     snprintf(g_last_error, sizeof(g_last_error), "%s: %s (%s:%d)", what, hipGetErrorString(e), file, line);
 }
 
+uint64_t align256(uint64_t x) { return (x + 255u) & ~uint64_t(255); }
 bool is_pow2(uint32_t x) { return x && !(x & (x - 1)); }
 uint32_t log2u(uint64_t x) {
     uint32_t r = 0;
@@ -79,15 +81,13 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
         x.lg2 = x.lgN;
         x.M = 1;
         x.D = 1;
-        x.W = 1;
     } else {
-        x.lg2 = pa::ROW_LOG;
-        x.N2 = 1u << x.lg2;
-        x.lg1 = x.lgN - x.lg2;
+        x.lg1 = x.lgN <= (uint32_t)pa::MID_MAX_LOG_N ? (uint32_t)pa::mid_lg1((int)x.lgN) : x.lgN - pa::ROW_LOG;
+        x.lg2 = x.lgN - x.lg1;
         x.N1 = 1u << x.lg1;
+        x.N2 = 1u << x.lg2;
         x.M = x.N1 <= 512 ? x.N1 : (x.N1 / 16 > 512 ? x.N1 / 16 : 512);  // D <= 16 bit classes
         x.D = x.N1 / x.M;
-        x.W = (uint32_t)pa::inv_cols_width((int)x.lg1);
     }
     x.out_bits = compress ? m : n / 2;
     x.out_off = pow2 ? 0 : x.h;
@@ -96,7 +96,13 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
     x.key_hw = x.h / 32;
     x.do_xor = (flags & PA_XOR_KEY_REST) ? 1u : 0u;
     x.reverse_endian = reverse_endian ? 1u : 0u;
-    x.inv_N = 1.0f / (8.0f * (float)x.N);  // exact: includes the factor 8 the real splits leave
+    if (x.N1 > 1) {
+        x.rho = pa::RHO;
+        x.scan = mid_size(x) ? 0 : 2;
+        x.inv_N = 1.0f / (float)x.N;
+    } else {
+        x.inv_N = 1.0f / (8.0f * (float)x.N);  // exact: includes the factor 8 the real splits leave
+    }
     *g = x;
     return PA_OK;
 }
@@ -121,6 +127,9 @@ uint64_t stage_out_bytes(const Geom& g) { return out_bytes_of(g) + 16; }
 uint64_t ws_key_bytes(uint32_t L) { return (uint64_t)(L / 32 + 2) * 4; }
 uint64_t ws_out_bytes(uint32_t L) { return (uint64_t)L / 8 + 16; }
 
+// one operand's bit masks (none below L = 2^23)
+uint64_t mask_bytes(const Geom& g) { return g.N1 == 1 || mid_size(g) ? 0 : (uint64_t)(g.N / g.D) * 4; }
+
 struct Extents {
     uint64_t touched[PA_BUF_COUNT] = {};
     uint64_t alloc[PA_BUF_COUNT] = {};
@@ -134,64 +143,60 @@ struct Extents {
 Extents block_extents(const Geom& g) {
     Extents x;
     const uint64_t N = g.N;
-    // key: k_transpose_bits / k_small read words [0, h/32] through key_word(); with the key-rest
-    // XOR, k_pack / k_small read key[h/32 + w + 1] for 32 w < m, i.e. up to word n/32
+    // key: pass A, the scan and k_small read words [0, h/32] through key_word(); with the key-rest
+    // XOR, the output stages read key[h/32 + w + 1] for 32 w < m, i.e. up to word n/32
     x.touched[PA_BUF_KEY] = (uint64_t)(g.do_xor ? g.n / 32 + 1 : g.key_hw + 1) * 4;
     x.touched[PA_BUF_SEED] = (uint64_t)g.seed_words * 4;  // seed_word(): words [0, n/32)
-    // k_pack (four-step) and k_small write output words [0, out_bits / 32)
+    // k_pack, k_mid_inv and k_small write output words [0, out_bits / 32)
     x.touched[PA_BUF_OUT] = (uint64_t)g.out_bits / 8;
     x.alloc[PA_BUF_KEY] = std::min(stage_key_bytes(g), ws_key_bytes(g.L));
     x.alloc[PA_BUF_SEED] = std::min(stage_seed_bytes(g), ws_key_bytes(g.L));
     // the device entry points' caller contract: m/8 bytes (compress) or n/16; staging is larger
     x.alloc[PA_BUF_OUT] = std::min({(uint64_t)out_bytes_of(g), stage_out_bytes(g), ws_out_bytes(g.L)});
-    x.alloc[PA_BUF_COUNTS] = 2 * pa::POP_SLOTS * 4;
     if (g.N1 == 1) return x;  // the one-workgroup path keeps everything else on chip
-    x.touched[PA_BUF_COUNTS] = 2 * pa::POP_SLOTS * 4;
-    // k_transpose_bits writes tb[u N2 + t2] for u < M, t2 < N2
-    x.touched[PA_BUF_BITS_KEY] = x.touched[PA_BUF_BITS_SEED] = (uint64_t)g.M * g.N2 * 4;
-    // pass A writes Y[k1 N2 + t2], k1 < N1; the seed-spectrum pass adds the Nyquist value S[N]
-    x.touched[PA_BUF_SPEC_KEY] = N * 8;
-    x.touched[PA_BUF_SPEC_SEED] = (N + 1) * 8;
-    // pass A' writes crumbs [0, N) (one column per workgroup) or nibbles [0, N/2); k_pack reads
-    // 4 bytes at (column or pair) * N1 + row for rows row < N1, row a multiple of 4
-    {
-        const uint64_t cols = g.W == 1 ? g.N2 : g.N2 / 2;
-        const uint64_t last_row = g.N1 >= 4 ? g.N1 - 4 : 0;
-        const uint64_t wr = cols * g.N1, rd = (cols - 1) * g.N1 + last_row + 4;
-        x.touched[PA_BUF_NIB] = std::max(wr, rd);
+    x.alloc[PA_BUF_COUNTS] = pa::info_bytes(g);
+    // the last parity byte, scan_parities(info)[chunks - 1]
+    x.touched[PA_BUF_COUNTS] = pa::INFO_HEAD * 4 + pa::scan_chunks(g) * 9ull;
+    if (!mid_size(g)) {
+        // k_transpose_bits writes tb[u N2 + t2] for u < M, t2 < N2
+        x.touched[PA_BUF_BITS_KEY] = x.touched[PA_BUF_BITS_SEED] = (uint64_t)g.M * g.N2 * 4;
+        x.alloc[PA_BUF_BITS_KEY] = x.alloc[PA_BUF_BITS_SEED] = mask_bytes(g);
     }
+    // pass A writes Y[k1 N2 + t2], k1 < N1
+    x.touched[PA_BUF_SPEC_KEY] = N * 8;
+    x.touched[PA_BUF_SPEC_SEED] = N * 8;
+    // pass A' writes pieces below N/4 bytes; the prefix words q[0 .. end of the window) follow
+    x.touched[PA_BUF_NIB] = N / 4 + ((uint64_t)g.out_off + g.out_bits) / 8;
     x.alloc[PA_BUF_SPEC_KEY] = N * 8;
     x.alloc[PA_BUF_SPEC_SEED] = (N + 1) * 8;
-    x.alloc[PA_BUF_BITS_KEY] = x.alloc[PA_BUF_BITS_SEED] = (uint64_t)(N / g.D) * 4;
-    x.alloc[PA_BUF_NIB] = pa::nib_bytes(g.N, g.W);
+    x.alloc[PA_BUF_NIB] = pa::nib_bytes(g.N);
     if (pa::rt_tiled(g.lg1)) {
-        // pass B writes tile ((t2 / RT_COLS) N1/2 + p) 2 RT_COLS + s RT_COLS + t2 mod RT_COLS for
-        // t2 < N2, p < N1/2, s < 2 (the last: N - 1); pass A' reads the same range
-        const uint64_t last = ((uint64_t)(g.N2 - 1) / pa::RT_COLS * (g.N1 / 2) + (g.N1 / 2 - 1)) * (2 * pa::RT_COLS) +
-                              pa::RT_COLS + (g.N2 - 1) % pa::RT_COLS;
+        // pass B writes ((t2 / RT_COLS) N1 + k1) RT_COLS + t2 mod RT_COLS for t2 < N2, k1 < N1 (the
+        // last: N - 1); pass A' reads the same range
+        const uint64_t last = ((uint64_t)(g.N2 - 1) / pa::RT_COLS * g.N1 + (g.N1 - 1)) * pa::RT_COLS +
+                              (g.N2 - 1) % pa::RT_COLS;
         x.touched[PA_BUF_TILES] = (last + 1) * 8;
         x.alloc[PA_BUF_TILES] = N * 8;
     }
     return x;
 }
 
-// Per transform length: w_L^x = lo[x mod 2^14] * hi[x >> 14].
+// Per transform length: exp(-2 pi i x / (2L)) = lo[x mod 2^14] * hi[x >> 14].
 struct Twiddles {
     float2* lo = nullptr;      // 2^14 entries
-    float2* hi = nullptr;      // max(1, L / 2^14) entries
+    float2* hi = nullptr;      // max(1, 2L / 2^14) entries
 };
 
 // Per transform length: the device scratch of one (unbatched) block.
 struct Workspace {
     uint32_t L = 0;
     float2* Yk = nullptr;      // N complex (key rows / R')
-    float2* Ys = nullptr;      // N+1 complex (seed rows / split seed spectrum)
+    float2* Ys = nullptr;      // N+1 complex (seed rows)
     float2* Rt = nullptr;      // N complex: pass B's output tiles (rt_tiled(lg1) only)
-    uint32_t* tbk = nullptr;   // N/D words
+    uint32_t* tbk = nullptr;   // N/D words (not below L = 2^23)
     uint32_t* tbs = nullptr;
-    uint8_t* nib = nullptr;    // L/4 bytes
-    uint32_t* counts = nullptr;  // POP_SLOTS key popcount partials, then POP_SLOTS seed partials
-    bool counts_zero = false;    // counts are known to be zero (the last block's pack cleared them)
+    uint8_t* nib = nullptr;    // rounded bits, then prefix words
+    uint32_t* info = nullptr;  // scan results (pa_geom.hpp)
     uint32_t* d_key = nullptr;   // staging for the host-buffer API
     uint32_t* d_seed = nullptr;
     uint32_t* d_out = nullptr;
@@ -205,8 +210,11 @@ struct Workspace {
 
 struct Seed {
     Geom g{};
-    float2* spec = nullptr;    // N+1 complex split spectrum
+    float2* spec = nullptr;    // spectrum: N complex (four-step path), N+1 split (small path)
     uint32_t* ws = nullptr;    // device popcount (POP_SLOTS partials)
+    uint32_t* sq = nullptr;    // prefix words (four-step path): L/8 bytes, 1/32 of the spectrum, not
+                               // charged to the budget, so that it holds as many seeds as it says
+                               // (spec, ws and sq are one allocation at spec)
     int32_t reuse = 0;
     uint64_t bytes = 0;
 };
@@ -294,8 +302,7 @@ struct pa_engine {
     uint32_t stage_count[16] = {};
     // batched launches
     BatchSlot batch;                         // pa_batch_device / pa_run_batch
-    struct Tuned { uint32_t grid_x, fwd_per; };
-    std::map<std::string, Tuned> tuned;      // launch shape per (L, seed mode, count)
+    std::map<std::string, uint32_t> tuned;   // pass A walk length per (L, seed mode, count)
     struct Server* server = nullptr;         // pa_serve_*
     struct PinRange { uint64_t bytes; uint8_t* dev; };
     std::map<uintptr_t, PinRange> pinned;    // pa_host_alloc ranges: base -> size, mapped address
@@ -399,8 +406,8 @@ std::vector<float2> twiddles(uint64_t L, uint64_t count, uint64_t stride) {
     return t;
 }
 
-// Pass A's class tables (layout in pa_kernels.hpp): sums of D-th roots of unity over the set bits
-// of a byte, in double precision, rounded once.
+// Pass A's class tables (layout in pa_kernels.hpp): sums of the quarter-shifted D-th roots of unity
+// times the +-1/2-encoded bits of a byte, in double precision, rounded once.
 std::vector<float2> class_tables() {
     std::vector<float2> t(pa::CLS_TABLE_TOTAL);
     for (int D = 1; D <= 16; D *= 2) {
@@ -409,12 +416,12 @@ std::vector<float2> class_tables() {
             for (int q = 0; q < NB; ++q)
                 for (int byte = 0; byte < (1 << BW); ++byte) {
                     double re = 0.0, im = 0.0;
-                    for (int b = 0; b < BW; ++b)
-                        if ((byte >> b) & 1) {
-                            const double a = -2.0 * M_PI * (double)(((BW * q + b) * c) % D) / (double)D;
-                            re += std::cos(a);
-                            im += std::sin(a);
-                        }
+                    for (int b = 0; b < BW; ++b) {
+                        const double a = -2.0 * M_PI * (double)(((BW * q + b) * (4 * c + 1)) % (4 * D)) / (4.0 * D);
+                        const double h = ((byte >> b) & 1) ? 0.5 : -0.5;
+                        re += h * std::cos(a);
+                        im += h * std::sin(a);
+                    }
                     t[pa::cls_table_offset(D) + (c * NB + q) * (1 << BW) + byte] = make_float2((float)re, (float)im);
                 }
     }
@@ -423,13 +430,13 @@ std::vector<float2> class_tables() {
 
 uint64_t workspace_bytes(const Geom& g) {
     const uint64_t N = g.N;
-    uint64_t b = (16384 + (N > 8192 ? g.L / 16384 : 1)) * sizeof(float2);
+    uint64_t b = (16384 + (N > 8192 ? g.L / 8192 : 1)) * sizeof(float2);
     if (g.N1 > 1) {
         b += N * sizeof(float2) + (N + 1) * sizeof(float2);
-        b += 2 * (N / g.D) * 4 + pa::nib_bytes(g.N, g.W) + 192;
+        b += 2 * mask_bytes(g) + pa::nib_bytes(g.N) + pa::info_bytes(g);
         if (pa::rt_tiled(g.lg1)) b += N * sizeof(float2);
     }
-    b += 256 + ws_key_bytes(g.L) * 2 + ws_out_bytes(g.L);  // key/seed and output staging
+    b += ws_key_bytes(g.L) * 2 + ws_out_bytes(g.L);  // key/seed and output staging
     return b;
 }
 
@@ -440,7 +447,7 @@ int get_twiddles(pa_engine* e, uint32_t L, Twiddles** out) {
         return PA_OK;
     }
     Twiddles t;
-    const uint64_t hi_n = L > 16384 ? L / 16384 : 1;
+    const uint64_t hi_n = L > 8192 ? L / 8192 : 1;
     int rc = dev_alloc(e, (void**)&t.lo, 16384 * sizeof(float2));
     if (rc != PA_OK) return rc;
     rc = dev_alloc(e, (void**)&t.hi, hi_n * sizeof(float2));
@@ -448,8 +455,8 @@ int get_twiddles(pa_engine* e, uint32_t L, Twiddles** out) {
         dev_free(e, t.lo, 16384 * sizeof(float2));
         return rc;
     }
-    auto lo = twiddles(L, 16384, 1);
-    auto hi = twiddles(L, hi_n, 16384);
+    auto lo = twiddles(2ull * L, 16384, 1);
+    auto hi = twiddles(2ull * L, hi_n, 16384);
     PA_HIP(hipMemcpy(t.lo, lo.data(), lo.size() * sizeof(float2), hipMemcpyHostToDevice));
     PA_HIP(hipMemcpy(t.hi, hi.data(), hi.size() * sizeof(float2), hipMemcpyHostToDevice));
     *out = &e->tw.emplace(L, t).first->second;
@@ -470,7 +477,6 @@ int get_workspace(pa_engine* e, const Geom& g, Workspace** out) {
     const size_t key_bytes = ws_key_bytes(g.L), out_bytes = ws_out_bytes(g.L);
     struct A { void** p; size_t b; };
     std::vector<A> allocs = {
-        {(void**)&w->counts, 2 * pa::POP_SLOTS * sizeof(uint32_t)},
         {(void**)&w->d_key, key_bytes},
         {(void**)&w->d_seed, key_bytes},
         {(void**)&w->d_out, out_bytes},
@@ -478,9 +484,12 @@ int get_workspace(pa_engine* e, const Geom& g, Workspace** out) {
     if (g.N1 > 1) {
         allocs.push_back({(void**)&w->Yk, (size_t)g.N * sizeof(float2)});
         allocs.push_back({(void**)&w->Ys, (size_t)(g.N + 1) * sizeof(float2)});
-        allocs.push_back({(void**)&w->tbk, (size_t)(g.N / g.D) * 4});
-        allocs.push_back({(void**)&w->tbs, (size_t)(g.N / g.D) * 4});
-        allocs.push_back({(void**)&w->nib, (size_t)pa::nib_bytes(g.N, g.W)});
+        if (!mid_size(g)) {
+            allocs.push_back({(void**)&w->tbk, (size_t)mask_bytes(g)});
+            allocs.push_back({(void**)&w->tbs, (size_t)mask_bytes(g)});
+        }
+        allocs.push_back({(void**)&w->nib, (size_t)pa::nib_bytes(g.N)});
+        allocs.push_back({(void**)&w->info, (size_t)pa::info_bytes(g)});
         if (pa::rt_tiled(g.lg1)) allocs.push_back({(void**)&w->Rt, (size_t)g.N * sizeof(float2)});
     }
     for (auto& a : allocs) {
@@ -506,10 +515,10 @@ pa::Tables tables(pa_engine* e, uint32_t L) {
 
 hipStream_t stream_of(pa_engine* e, void* s) { return s ? (hipStream_t)s : e->stream; }
 
-enum Stage { ST_SMALL, ST_ZERO, ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, ST_TRANSPOSE_BOTH, ST_FWD_COLS_BOTH,
+enum Stage { ST_SMALL, ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, ST_TRANSPOSE_BOTH, ST_FWD_COLS_BOTH,
              ST_ROWS_SEEDPREP, ST_ROWS, ST_INV_COLS, ST_PACK, ST_TRANSPOSE_SEED, ST_FWD_COLS_SEED, ST_COUNT };
 const char* const kStageNames[ST_COUNT] = {
-    "k_small", "k_zero_u32", "k_transpose_bits(key)", "k_fwd_cols(key)", "k_transpose_bits(key+seed)",
+    "k_small", "k_transpose_bits(key)", "k_fwd_cols(key)", "k_transpose_bits(key+seed)",
     "k_fwd_cols(key+seed)", "k_rows(seedprep)", "k_rows", "k_inv_cols", "k_pack", "k_transpose_bits(seed)",
     "k_fwd_cols(seed)"};
 static_assert(ST_COUNT <= 16, "stage tables hold 16 entries");
@@ -551,22 +560,20 @@ hipError_t timed(pa_engine* e, int stage, hipStream_t s, F&& launch) {
     return r;
 }
 
-// The hot path on device buffers.  sspec/ws_dev != null selects the resident seed; su != null
-// brings a fresh seed up from host memory during the key's passes (seed = su->dev).
+// The hot path on device buffers.  sd != null selects the resident seed; su != null brings a fresh
+// seed up from host memory during the key's passes (seed = su->dev).
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
-                    const float2* sspec, const uint32_t* ws_dev, uint32_t* out, hipStream_t s, float* margin,
-                    const SeedUpload* su);
+                    const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su);
 
 // Orders the workspace's uses across streams (not while s is being captured into a graph: a
 // capture only records work, and the caller owns the ordering of its replays).
 int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
-               const float2* sspec, const uint32_t* ws_dev, uint32_t* out, hipStream_t s, float* margin,
-               const SeedUpload* su = nullptr) {
+               const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su = nullptr) {
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     PA_HIP(hipStreamIsCapturing(s, &cap));
     const bool guard = cap == hipStreamCaptureStatusNone;
     if (guard && w->last_stream && w->last_stream != s) PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
-    const int rc = run_device_body(e, g, w, key, seed, sspec, ws_dev, out, s, margin, su);
+    const int rc = run_device_body(e, g, w, key, seed, sd, out, s, margin, su);
     if (rc != PA_OK) return rc;
     if (guard) {
         PA_HIP(hipEventRecord(w->last_done, s));
@@ -576,48 +583,58 @@ int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, c
 }
 
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
-                    const float2* sspec, const uint32_t* ws_dev, uint32_t* out, hipStream_t s, float* margin,
-                    const SeedUpload* su) {
+                    const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su) {
     const pa::Tables t = tables(e, g.L);
     if (g.N1 == 1) {
         PA_HIP(timed(e, ST_SMALL, s, [&] {
-            return pa::launch_small(key, seed, sspec, ws_dev, out, g, t, margin, nullptr, nullptr, s);
+            return pa::launch_small(key, seed, sd ? sd->spec : nullptr, sd ? sd->ws : nullptr, out, g, t, margin, nullptr,
+                                    nullptr, s);
         }));
         return PA_OK;
     }
-    uint32_t* key_cnt = w->counts;
-    uint32_t* seed_cnt = w->counts + pa::POP_SLOTS;
-    if (!w->counts_zero)
-        PA_HIP(timed(e, ST_ZERO, s, [&] { return pa::launch_zero_u32(w->counts, 2 * pa::POP_SLOTS, s); }));
-    w->counts_zero = false;  // until this block's pack stage is enqueued
-    if (!sspec && su) {  // key passes first, the seed's after its upload
-        PA_HIP(timed(e, ST_TRANSPOSE_KEY, s, [&] { return pa::launch_transpose(key, w->tbk, key_cnt, g, 0, s); }));
-        PA_HIP(timed(e, ST_FWD_COLS_KEY, s, [&] { return pa::launch_fwd_cols(w->tbk, w->Yk, g, t, s); }));
+    uint32_t* q = pa::prefix_words(w->nib, g.N);
+    pa::ScanArgs scan{key, su ? su->dev : seed, nullptr, q, w->info};
+    float2* S = w->Ys;
+    const bool mid = mid_size(g);
+    // pass A reads the bit masks, or for a mid-size transform the words themselves
+    const uint32_t* kin = mid ? key : w->tbk;
+    const uint32_t* sin = mid ? scan.seed : w->tbs;
+    // `ops` operands from `first` on through the bit transpose and pass A; sc: with the input scan
+    auto fwd = [&](int tstage, int fstage, uint32_t first, uint32_t ops, const pa::ScanArgs* sc) {
+        hipError_t r = hipSuccess;
+        if (!mid)
+            r = timed(e, tstage, s, [&] {
+                return pa::launch_transpose(key, scan.seed, w->tbk, w->tbs, first, ops, g, sc, s);
+            });
+        if (r != hipSuccess) return r;
+        return timed(e, fstage, s, [&] { return pa::launch_fwd_cols(kin, sin, w->Yk, w->Ys, first, ops, g, t, sc, s); });
+    };
+    if (!sd && su) {  // key passes first, the seed's (and the scan of both) after its upload
+        PA_HIP(fwd(ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, 0, 1, nullptr));
         PA_HIP(hipStreamWaitEvent(su->up, su->key_up, 0));
         PA_HIP(hipMemcpyAsync(su->dev, su->host, su->bytes, hipMemcpyHostToDevice, su->up));
         PA_HIP(hipEventRecord(su->done, su->up));
         PA_HIP(hipStreamWaitEvent(s, su->done, 0));
-        PA_HIP(timed(e, ST_TRANSPOSE_SEED, s, [&] { return pa::launch_transpose(su->dev, w->tbs, seed_cnt, g, 1, s); }));
-        PA_HIP(timed(e, ST_FWD_COLS_SEED, s, [&] { return pa::launch_fwd_cols(w->tbs, w->Ys, g, t, s); }));
-        PA_HIP(timed(e, ST_ROWS, s, [&] { return pa::launch_rows(pa::ROWS_DYN, w->Yk, w->Ys, w->Rt, g, t, e->cus, s); }));
-        ws_dev = seed_cnt;
-    } else if (!sspec) {  // key and seed share each launch of the bit transpose and of pass A
-        PA_HIP(timed(e, ST_TRANSPOSE_BOTH, s, [&] {
-            return pa::launch_transpose(key, w->tbk, key_cnt, g, 0, s, seed, w->tbs);
-        }));
-        PA_HIP(timed(e, ST_FWD_COLS_BOTH, s, [&] { return pa::launch_fwd_cols(w->tbk, w->Yk, g, t, s, w->tbs, w->Ys); }));
-        PA_HIP(timed(e, ST_ROWS, s, [&] { return pa::launch_rows(pa::ROWS_DYN, w->Yk, w->Ys, w->Rt, g, t, e->cus, s); }));
-        ws_dev = seed_cnt;
+        PA_HIP(fwd(ST_TRANSPOSE_SEED, ST_FWD_COLS_SEED, 1, 1, &scan));
+    } else if (!sd) {  // key and seed share each launch of the bit transpose and of pass A
+        PA_HIP(fwd(ST_TRANSPOSE_BOTH, ST_FWD_COLS_BOTH, 0, 2, &scan));
     } else {
-        float2* S = const_cast<float2*>(sspec);
-        PA_HIP(timed(e, ST_TRANSPOSE_KEY, s, [&] { return pa::launch_transpose(key, w->tbk, key_cnt, g, 0, s); }));
-        PA_HIP(timed(e, ST_FWD_COLS_KEY, s, [&] { return pa::launch_fwd_cols(w->tbk, w->Yk, g, t, s); }));
-        PA_HIP(timed(e, ST_ROWS, s, [&] { return pa::launch_rows(pa::ROWS_STATIC, w->Yk, S, w->Rt, g, t, e->cus, s); }));
+        S = sd->spec;
+        scan.seed = nullptr;
+        scan.sq = sd->sq;
+        PA_HIP(fwd(ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, 0, 1, &scan));
+    }
+    PA_HIP(timed(e, ST_ROWS, s, [&] {
+        return pa::launch_rows(sd ? pa::ROWS_STATIC : pa::ROWS_DYN, w->Yk, S, w->Rt, g, t, w->info, sd ? sd->ws : nullptr,
+                               nullptr, s);
+    }));
+    if (mid) {
+        PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_mid_inv(w->Yk, key, out, g, w->info, q, t, margin, s); }));
+        return PA_OK;
     }
     const float2* R = pa::rt_tiled(g.lg1) ? w->Rt : w->Yk;
-    PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_inv_cols(R, w->nib, g, key_cnt, ws_dev, t, margin, s); }));
-    PA_HIP(timed(e, ST_PACK, s, [&] { return pa::launch_pack(w->nib, key, out, g, s, w->counts); }));
-    w->counts_zero = true;  // the pack stage clears the partials for the next block on the stream
+    PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_inv_cols(R, w->nib, g, w->info, t, margin, s); }));
+    PA_HIP(timed(e, ST_PACK, s, [&] { return pa::launch_pack(w->nib, key, out, g, w->info, q, s); }));
     return PA_OK;
 }
 
@@ -698,11 +715,10 @@ int pa_destroy(pa_engine* e) {
     }
     for (auto& kv : e->seeds) {
         (void)hipFree(kv.second.spec);
-        (void)hipFree(kv.second.ws);
     }
     for (auto& kv : e->ws) {
         Workspace* w = kv.second.get();
-        void* ps[] = {w->Yk, w->Ys, w->Rt, w->tbk, w->tbs, w->nib, w->counts, w->d_key, w->d_seed, w->d_out};
+        void* ps[] = {w->Yk, w->Ys, w->Rt, w->tbk, w->tbs, w->nib, w->info, w->d_key, w->d_seed, w->d_out};
         for (void* p : ps) (void)hipFree(p);
         if (w->last_done) (void)hipEventDestroy(w->last_done);
     }
@@ -750,6 +766,26 @@ int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform
     return PA_OK;
 }
 
+static int seed_alloc(pa_engine* e, Seed* sd) {
+    const Geom& g = sd->g;
+    const uint64_t spec = align256((uint64_t)(g.N + 1) * sizeof(float2)), ws = align256(pa::POP_SLOTS * 4);
+    sd->bytes = (uint64_t)(g.N + 1) * sizeof(float2) + pa::POP_SLOTS * sizeof(uint32_t);
+    if (e->cfg.hbm_budget_bytes && e->used_bytes + sd->bytes > e->cfg.hbm_budget_bytes) return PA_ERR_NOMEM;
+    uint8_t* p = nullptr;
+    const hipError_t r = hipMalloc((void**)&p, spec + ws + (g.N1 > 1 ? (uint64_t)g.L / 8 : 0));
+    if (r != hipSuccess) {
+        set_error(r, "hipMalloc", __FILE__, __LINE__);
+        (void)hipGetLastError();
+        return PA_ERR_NOMEM;
+    }
+    e->used_bytes += sd->bytes;
+    sd->spec = reinterpret_cast<float2*>(p);
+    sd->ws = reinterpret_cast<uint32_t*>(p + spec);
+    if (g.N1 > 1) sd->sq = reinterpret_cast<uint32_t*>(p + spec + ws);
+    return PA_OK;
+}
+static void seed_free(pa_engine* e, const Seed& sd) { dev_free(e, sd.spec, sd.bytes); }
+
 int pa_seed_put(pa_engine* e, const uint32_t* seed, uint32_t n, uint32_t m, int32_t reuse, pa_seed_id* id) {
     if (!e || !seed || !id) return PA_ERR_ARG;
     std::lock_guard<std::mutex> lk(e->mu);
@@ -760,26 +796,34 @@ int pa_seed_put(pa_engine* e, const uint32_t* seed, uint32_t n, uint32_t m, int3
     Seed sd;
     sd.g = g;
     sd.reuse = reuse;
-    sd.bytes = (uint64_t)(g.N + 1) * sizeof(float2) + pa::POP_SLOTS * sizeof(uint32_t);
-    rc = dev_alloc(e, (void**)&sd.spec, (size_t)(g.N + 1) * sizeof(float2));
+    auto launch = [&]() -> int {
+        hipStream_t s = e->stream;
+        // the workspace's masks and info words are scratch here: after a block on another stream
+        if (w->last_stream && w->last_stream != s) PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
+        PA_HIP(hipMemcpyAsync(w->d_seed, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
+        const pa::Tables t = tables(e, g.L);
+        if (g.N1 == 1) {
+            PA_HIP(pa::launch_small(nullptr, w->d_seed, nullptr, nullptr, nullptr, g, t, nullptr, sd.spec, sd.ws, s));
+        } else {
+            Geom gs = g;  // every word's prefix, whatever window a block will read
+            gs.out_off = 0;
+            gs.out_bits = g.L;
+            const pa::ScanArgs scan{nullptr, w->d_seed, nullptr, sd.sq, w->info};
+            if (!mid_size(g)) PA_HIP(pa::launch_transpose(nullptr, w->d_seed, nullptr, w->tbs, 1, 1, gs, &scan, s));
+            PA_HIP(pa::launch_fwd_cols(nullptr, mid_size(g) ? w->d_seed : w->tbs, nullptr, sd.spec, 1, 1, gs, t, &scan, s));
+            PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, sd.spec, nullptr, g, t, w->info, nullptr, sd.ws, s));
+            PA_HIP(pa::launch_prefix_apply(sd.sq, w->info, g, s));
+        }
+        PA_HIP(hipStreamSynchronize(s));
+        return PA_OK;
+    };
+    rc = seed_alloc(e, &sd);
     if (rc != PA_OK) return rc;
-    rc = dev_alloc(e, (void**)&sd.ws, pa::POP_SLOTS * sizeof(uint32_t));
+    rc = launch();
     if (rc != PA_OK) {
-        dev_free(e, sd.spec, (size_t)(g.N + 1) * sizeof(float2));
+        seed_free(e, sd);
         return rc;
     }
-    hipStream_t s = e->stream;
-    PA_HIP(hipMemcpyAsync(w->d_seed, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
-    const pa::Tables t = tables(e, g.L);
-    if (g.N1 == 1) {
-        PA_HIP(pa::launch_small(nullptr, w->d_seed, nullptr, nullptr, nullptr, g, t, nullptr, sd.spec, sd.ws, s));
-    } else {
-        PA_HIP(pa::launch_zero_u32(sd.ws, pa::POP_SLOTS, s));
-        PA_HIP(pa::launch_transpose(w->d_seed, w->tbs, sd.ws, g, 1, s));
-        PA_HIP(pa::launch_fwd_cols(w->tbs, sd.spec, g, t, s));
-        PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, sd.spec, nullptr, g, t, e->cus, s));
-    }
-    PA_HIP(hipStreamSynchronize(s));
     *id = e->next_seed++;
     e->seeds[*id] = sd;
     return PA_OK;
@@ -791,8 +835,7 @@ int pa_seed_drop(pa_engine* e, pa_seed_id id) {
     auto it = e->seeds.find(id);
     if (it == e->seeds.end()) return PA_ERR_NOT_FOUND;
     (void)hipStreamSynchronize(e->stream);
-    dev_free(e, it->second.spec, (size_t)(it->second.g.N + 1) * sizeof(float2));
-    dev_free(e, it->second.ws, pa::POP_SLOTS * sizeof(uint32_t));
+    seed_free(e, it->second);
     e->seeds.erase(it);
     return PA_OK;
 }
@@ -814,7 +857,7 @@ int pa_block_device(pa_engine* e, const uint32_t* d_key, const uint32_t* d_seed,
     Workspace* w;
     int rc = prepare(e, n, m, flags, &g, &w);
     if (rc != PA_OK) return rc;
-    return run_device(e, g, w, d_key, d_seed, nullptr, nullptr, (uint32_t*)d_out, stream_of(e, stream), d_margin);
+    return run_device(e, g, w, d_key, d_seed, nullptr, (uint32_t*)d_out, stream_of(e, stream), d_margin);
 }
 
 int pa_block_device_seeded(pa_engine* e, const uint32_t* d_key, pa_seed_id id, uint32_t n, uint32_t m,
@@ -828,7 +871,7 @@ int pa_block_device_seeded(pa_engine* e, const uint32_t* d_key, pa_seed_id id, u
     const Seed* sd;
     rc = seed_lookup(e, id, g, &sd);
     if (rc != PA_OK) return rc;
-    return run_device(e, g, w, d_key, nullptr, sd->spec, sd->ws, (uint32_t*)d_out, stream_of(e, stream), d_margin);
+    return run_device(e, g, w, d_key, nullptr, sd, (uint32_t*)d_out, stream_of(e, stream), d_margin);
 }
 
 int pa_block_device_noalloc(pa_engine* e, const uint32_t* d_key, const uint32_t* d_seed, uint32_t n, uint32_t m,
@@ -846,8 +889,7 @@ int pa_block_device_noalloc(pa_engine* e, const uint32_t* d_key, const uint32_t*
     }
     if (!block_extents(g).ok()) return PA_ERR_UNSUPPORTED;
     if (!e->noalloc || e->tw.find(g.L) == e->tw.end()) return PA_ERR_UNSUPPORTED;
-    // the workspace of this block, carved from the scratch array (no allocation); the popcount
-    // partials are cleared by a kernel at the start of the block (counts_zero = false)
+    // the workspace of this block, carved from the scratch array (no allocation)
     Workspace w;
     w.L = g.L;
     if (g.N1 > 1) {
@@ -859,17 +901,17 @@ int pa_block_device_noalloc(pa_engine* e, const uint32_t* d_key, const uint32_t*
         };
         w.Yk = reinterpret_cast<float2*>(take((uint64_t)g.N * 8));
         w.Ys = reinterpret_cast<float2*>(take((uint64_t)(g.N + 1) * 8));
-        w.tbk = reinterpret_cast<uint32_t*>(take((uint64_t)(g.N / g.D) * 4));
-        w.tbs = reinterpret_cast<uint32_t*>(take((uint64_t)(g.N / g.D) * 4));
-        w.nib = take(pa::nib_bytes(g.N, g.W));
-        w.counts = reinterpret_cast<uint32_t*>(take(2 * pa::POP_SLOTS * 4));
+        w.tbk = reinterpret_cast<uint32_t*>(take(mask_bytes(g)));
+        w.tbs = reinterpret_cast<uint32_t*>(take(mask_bytes(g)));
+        w.nib = take(pa::nib_bytes(g.N));
+        w.info = reinterpret_cast<uint32_t*>(take(pa::info_bytes(g)));
         if (pa::rt_tiled(g.lg1)) w.Rt = reinterpret_cast<float2*>(take((uint64_t)g.N * 8));
         if (off > NOALLOC_SCRATCH_BYTES) return PA_ERR_UNSUPPORTED;
     }
     const bool timing = e->timing;  // stage timing creates events: not on this path
     e->timing = false;
-    rc = run_device_body(e, g, &w, d_key, d_seed, nullptr, nullptr, reinterpret_cast<uint32_t*>(d_out),
-                         stream_of(e, stream), d_margin, nullptr);
+    rc = run_device_body(e, g, &w, d_key, d_seed, nullptr, reinterpret_cast<uint32_t*>(d_out), stream_of(e, stream),
+                         d_margin, nullptr);
     e->timing = timing;
     return rc;
 }
@@ -898,8 +940,7 @@ static int run_host(pa_engine* e, const uint32_t* key, const uint32_t* seed, pa_
     const bool overlap = seed && g.N1 > 1;
     if (overlap) PA_HIP(hipEventRecord(e->key_up, s));
     if (seed && !overlap) PA_HIP(hipMemcpyAsync(w->d_seed, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
-    rc = run_device(e, g, w, w->d_key, seed ? w->d_seed : nullptr, sd ? sd->spec : nullptr,
-                    sd ? sd->ws : nullptr, w->d_out, s, nullptr, overlap ? &su : nullptr);
+    rc = run_device(e, g, w, w->d_key, seed ? w->d_seed : nullptr, sd, w->d_out, s, nullptr, overlap ? &su : nullptr);
     if (rc != PA_OK) return rc;
     PA_HIP(hipMemcpyAsync(out, w->d_out, out_bytes_of(g), hipMemcpyDeviceToHost, s));
     PA_HIP(hipStreamSynchronize(s));
@@ -942,8 +983,7 @@ int pa_submit(pa_engine* e, const uint32_t* key, const uint32_t* seed, pa_seed_i
     PA_HIP(hipMemsetAsync(t.dev_key, 0, kbytes, s));
     PA_HIP(hipMemcpyAsync(t.dev_key, key, (size_t)key_words_for(g) * 4, hipMemcpyHostToDevice, s));
     if (seed) PA_HIP(hipMemcpyAsync(t.dev_seed, seed, stage_seed_bytes(g), hipMemcpyHostToDevice, s));
-    rc = run_device(e, g, w, t.dev_key, t.dev_seed, sd ? sd->spec : nullptr, sd ? sd->ws : nullptr,
-                    t.dev_out, s, nullptr);
+    rc = run_device(e, g, w, t.dev_key, t.dev_seed, sd, t.dev_out, s, nullptr);
     if (rc != PA_OK) return rc;
     PA_HIP(hipMemcpyAsync(out, t.dev_out, t.out_bytes, hipMemcpyDeviceToHost, s));
     PA_HIP(hipEventCreateWithFlags(&t.done, hipEventDisableTiming));
@@ -1001,8 +1041,6 @@ int pa_wait(pa_engine* e, pa_ticket ticket, int64_t timeout_ns) {
 // ------------------------------------------------------------------ batched launches ----
 namespace {
 
-uint64_t align256(uint64_t x) { return (x + 255u) & ~uint64_t(255); }
-
 struct BatchItem {
     Geom g{};
     const Seed* sd = nullptr;  // resident seed (static mode)
@@ -1014,8 +1052,7 @@ struct BatchGroup {
     bool dyn = true, small = false;
     std::vector<uint32_t> idx;  // blocks of the group (caller order)
     uint32_t tab0 = 0;          // first table row of the group
-    uint32_t tiles_y = 1;       // pack grid.y: the largest window of the group
-    uint32_t grid_x = 0;        // row-pass workgroups per block
+    uint32_t halves = 1;        // halves of the conv positions to pack: the most of the group
     uint32_t fwd_per = 0;       // pass A walk length (0: the launcher's default)
     double cost = 0.0;
 };
@@ -1029,9 +1066,9 @@ struct BatchPlan {
 // Device scratch of one block of a batch (the four-step path's intermediate buffers).
 uint64_t batch_scratch_bytes(const Geom& g, bool dyn) {
     if (g.N1 == 1) return 0;
-    uint64_t b = align256((uint64_t)g.N * 8) + align256((uint64_t)(g.N / g.D) * 4);  // Yk, tbk
-    if (dyn) b += align256((uint64_t)(g.N + 1) * 8) + align256((uint64_t)(g.N / g.D) * 4);  // Ys, tbs
-    b += align256(pa::nib_bytes(g.N, g.W)) + align256(2 * pa::POP_SLOTS * 4);  // nib, counts
+    uint64_t b = align256((uint64_t)g.N * 8) + align256(mask_bytes(g));            // Yk, tbk
+    if (dyn) b += align256((uint64_t)(g.N + 1) * 8) + align256(mask_bytes(g));     // Ys, tbs
+    b += align256(pa::nib_bytes(g.N)) + align256(pa::info_bytes(g));               // nib, info
     if (pa::rt_tiled(g.lg1)) b += align256((uint64_t)g.N * 8);     // R' tiles
     return b;
 }
@@ -1067,7 +1104,7 @@ int batch_plan(pa_engine* e, const pa_block* blocks, uint32_t count, BatchPlan* 
         BatchGroup& gr = p->groups[f->second];
         gr.idx.push_back(i);
         gr.cost += (double)it.g.L * (it.dyn ? 1.5 : 1.0);
-        if (!gr.small) gr.tiles_y = std::max(gr.tiles_y, pa::pack_tiles(it.g));
+        if (!gr.small) gr.halves = std::max(gr.halves, pa::pack_halves(it.g));
         p->scratch_bytes += batch_scratch_bytes(it.g, it.dyn);
     }
     uint32_t row = 0;
@@ -1106,7 +1143,7 @@ int ensure_arena(pa_engine* e, BatchSlot& sl, uint64_t bytes, uint64_t limit = 0
 
 // All launches of one group on stream s.
 int batch_group_launch(pa_engine* e, const BatchPlan& p, const BatchGroup& gr, const pa::BlockArgs* tab,
-                       uint32_t grid_x, uint32_t fwd_per, hipStream_t s) {
+                       uint32_t fwd_per, hipStream_t s) {
     const pa::BlockArgs* bt = tab + gr.tab0;
     const uint32_t cnt = (uint32_t)gr.idx.size();
     const Geom& g0 = p.items[gr.idx[0]].g;
@@ -1115,23 +1152,24 @@ int batch_group_launch(pa_engine* e, const BatchPlan& p, const BatchGroup& gr, c
         PA_HIP(pa::launch_batch_small(bt, cnt, g0, t, s));
         return PA_OK;
     }
-    PA_HIP(pa::launch_batch_zero(bt, cnt, s));
-    PA_HIP(pa::launch_batch_transpose(bt, cnt, g0, 0, s));
-    PA_HIP(pa::launch_batch_fwd_cols(bt, cnt, g0, t, 0, fwd_per, s));
-    if (gr.dyn) {
-        PA_HIP(pa::launch_batch_transpose(bt, cnt, g0, 1, s));
-        PA_HIP(pa::launch_batch_fwd_cols(bt, cnt, g0, t, 1, fwd_per, s));
+    const uint32_t ops = gr.dyn ? 2u : 1u;
+    const bool mid = mid_size(g0);
+    if (!mid) PA_HIP(pa::launch_batch_transpose(bt, cnt, g0, ops, s));
+    PA_HIP(pa::launch_batch_fwd_cols(bt, cnt, g0, t, ops, fwd_per, s));
+    PA_HIP(pa::launch_batch_rows(gr.dyn ? pa::ROWS_DYN : pa::ROWS_STATIC, bt, cnt, g0, t, s));
+    if (mid) {
+        PA_HIP(pa::launch_batch_mid_inv(bt, cnt, g0, t, s));
+        return PA_OK;
     }
-    PA_HIP(pa::launch_batch_rows(gr.dyn ? pa::ROWS_DYN : pa::ROWS_STATIC, bt, cnt, g0, t, grid_x, s));
     PA_HIP(pa::launch_batch_inv_cols(bt, cnt, g0, t, s));
-    PA_HIP(pa::launch_batch_pack(bt, cnt, g0, gr.tiles_y, s));
+    PA_HIP(pa::launch_batch_pack(bt, cnt, g0, gr.halves, s));
     return PA_OK;
 }
 
 // Groups on the fork streams (largest first onto the least-loaded stream), joined back into s.
 int batch_launch_all(pa_engine* e, BatchSlot& sl, const BatchPlan& p, const pa::BlockArgs* tab, hipStream_t s) {
     const size_t ng = p.groups.size();
-    if (ng == 1) return batch_group_launch(e, p, p.groups[0], tab, p.groups[0].grid_x, p.groups[0].fwd_per, s);
+    if (ng == 1) return batch_group_launch(e, p, p.groups[0], tab, p.groups[0].fwd_per, s);
     std::vector<size_t> order(ng);
     for (size_t i = 0; i < ng; ++i) order[i] = i;
     std::sort(order.begin(), order.end(), [&](size_t a, size_t b) { return p.groups[a].cost > p.groups[b].cost; });
@@ -1147,7 +1185,7 @@ int batch_launch_all(pa_engine* e, BatchSlot& sl, const BatchPlan& p, const pa::
             used[k] = true;
         }
         load[k] += p.groups[gi].cost;
-        int rc = batch_group_launch(e, p, p.groups[gi], tab, p.groups[gi].grid_x, p.groups[gi].fwd_per, sl.fork[k]);
+        int rc = batch_group_launch(e, p, p.groups[gi], tab, p.groups[gi].fwd_per, sl.fork[k]);
         if (rc != PA_OK) return rc;
     }
     for (int k = 0; k < BatchSlot::FORKS; ++k) {
@@ -1163,21 +1201,18 @@ std::string tune_key(const BatchGroup& gr) {
 }
 
 // The autotuner: times a group's whole launch sequence (the outputs are rewritten by the real run
-// that follows) over its launch-shape knobs and records the fastest shape per (L, seed mode,
-// count).  Knobs, tuned one after the other: the pass A walk length (column groups per persistent
-// workgroup, for N1 = 2^9 .. 2^13), then the row-pass grid (workgroups per block).
+// that follows) over the pass A walk length (column groups per persistent workgroup, for L = 2^23 ..
+// 2^27) and records the fastest per (L, seed mode, count).
 int batch_tune_group(pa_engine* e, const BatchPlan& p, BatchGroup& gr, const pa::BlockArgs* tab, hipStream_t s) {
     const Geom& g0 = p.items[gr.idx[0]].g;
-    const uint32_t items = g0.N1 / 2u;
     const uint32_t cnt = (uint32_t)gr.idx.size();
-    const uint32_t base = std::max<uint32_t>(1u, ((uint32_t)e->cus + cnt - 1u) / cnt);
     hipEvent_t a, b;
     PA_HIP(hipEventCreate(&a));
     PA_HIP(hipEventCreate(&b));
-    auto time_shape = [&](uint32_t x, uint32_t per, float* ms) -> int {
+    auto time_shape = [&](uint32_t per, float* ms) -> int {
         for (int rep = 0; rep < 2; ++rep) {  // the first run warms up
             PA_HIP(hipEventRecord(a, s));
-            int rc = batch_group_launch(e, p, gr, tab, x, per, s);
+            int rc = batch_group_launch(e, p, gr, tab, per, s);
             if (rc != PA_OK) return rc;
             PA_HIP(hipEventRecord(b, s));
             PA_HIP(hipEventSynchronize(b));
@@ -1186,36 +1221,25 @@ int batch_tune_group(pa_engine* e, const BatchPlan& p, BatchGroup& gr, const pa:
         return PA_OK;
     };
     int rc = PA_OK;
-    uint32_t best_x = std::min(base, items), best_per = 0;
-    if (g0.lg1 >= 9 && g0.lg1 <= 13) {
+    uint32_t best_per = 0;
+    if (!mid_size(g0) && g0.lg1 <= 13) {
         // walk lengths that leave at least one workgroup per compute unit (and the default)
         const uint32_t wgs = (g0.N2 / 16u) * g0.D * cnt;
         float best = 1e30f;
         for (uint32_t per = 1; per <= pa::FWD_PER_MAX && rc == PA_OK; per *= 2) {
             if (per > 1u && wgs / per < (uint32_t)e->cus) break;
             float ms = 0.f;
-            rc = time_shape(best_x, per, &ms);
+            rc = time_shape(per, &ms);
             if (rc == PA_OK && ms < best) {
                 best = ms;
                 best_per = per;
             }
         }
     }
-    float best = 1e30f;
-    for (uint32_t x = 1; x <= items && rc == PA_OK; x *= 2) {
-        if (x * 4u < base || x > base * 8u) continue;
-        float ms = 0.f;
-        rc = time_shape(x, best_per, &ms);
-        if (rc == PA_OK && ms < best) {
-            best = ms;
-            best_x = x;
-        }
-    }
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     if (rc != PA_OK) return rc;
-    e->tuned[tune_key(gr)] = {best_x, best_per};
-    gr.grid_x = best_x;
+    e->tuned[tune_key(gr)] = best_per;
     gr.fwd_per = best_per;
     return PA_OK;
 }
@@ -1255,6 +1279,7 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
             a.seed = it.dyn ? dev[i].seed : nullptr;
             a.sspec = it.sd ? it.sd->spec : nullptr;
             a.ws = it.sd ? it.sd->ws : nullptr;
+            a.sq = it.sd ? it.sd->sq : nullptr;
             a.out = reinterpret_cast<uint32_t*>(dev[i].out);
             a.margin = dev[i].margin;
             if (!gr.small) {
@@ -1265,24 +1290,21 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
                     return q;
                 };
                 a.Yk = reinterpret_cast<float2*>(take((uint64_t)g.N * 8));
-                a.tbk = reinterpret_cast<uint32_t*>(take((uint64_t)(g.N / g.D) * 4));
+                a.tbk = reinterpret_cast<uint32_t*>(take(mask_bytes(g)));
                 if (it.dyn) {
                     a.Ys = reinterpret_cast<float2*>(take((uint64_t)(g.N + 1) * 8));
-                    a.tbs = reinterpret_cast<uint32_t*>(take((uint64_t)(g.N / g.D) * 4));
+                    a.tbs = reinterpret_cast<uint32_t*>(take(mask_bytes(g)));
                 }
-                a.nib = take(pa::nib_bytes(g.N, g.W));
-                a.counts = reinterpret_cast<uint32_t*>(take(2 * pa::POP_SLOTS * 4));
+                a.nib = take(pa::nib_bytes(g.N));
+                a.q = pa::prefix_words(a.nib, g.N);
+                a.info = reinterpret_cast<uint32_t*>(take(pa::info_bytes(g)));
                 if (pa::rt_tiled(g.lg1)) a.Rt = reinterpret_cast<float2*>(take((uint64_t)g.N * 8));
             }
             sl.htab[gr.tab0 + j] = a;
         }
         if (!gr.small) {
             auto t = e->tuned.find(tune_key(gr));
-            const uint32_t items = p.items[gr.idx[0]].g.N1 / 2u;
-            const uint32_t cnt = (uint32_t)gr.idx.size();
-            gr.grid_x = t != e->tuned.end() ? t->second.grid_x
-                                            : std::min(items, std::max<uint32_t>(1u, ((uint32_t)e->cus + cnt - 1u) / cnt));
-            gr.fwd_per = t != e->tuned.end() ? t->second.fwd_per : 0u;
+            gr.fwd_per = t != e->tuned.end() ? t->second : 0u;
         }
     }
     // the table and the input ranges in one copy launch (read from mapped host memory)
@@ -1327,8 +1349,7 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
     auto replay = [&]() -> int {
         std::string key = std::to_string((uintptr_t)sl.arena) + ":";
         for (auto& gr : p.groups)
-            key += tune_key(gr) + "x" + std::to_string(gr.grid_x) + "p" + std::to_string(gr.fwd_per) + "y" +
-                   std::to_string(gr.tiles_y) + ";";
+            key += tune_key(gr) + "p" + std::to_string(gr.fwd_per) + "y" + std::to_string(gr.halves) + ";";
         auto f = sl.graphs.find(key);
         if (f == sl.graphs.end()) {
             hipGraph_t graph = nullptr;
@@ -2111,26 +2132,30 @@ int st_correction(pa_engine* e, Report& rp) {
     return rp.done("CalculateCorrectionFloat");
 }
 
-// The seed's split spectrum through the production pass A and row pass (pa_seed_put's launches).
-int st_seed_spectrum(pa_engine* e, const uint32_t* h_seed, uint32_t n, std::vector<float2>& S, uint32_t& ws) {
-    Geom g;
+// The seed's spectrum through the production pass A and row pass (pa_seed_put's launches), the seed
+// whitened by rho.
+int st_seed_spectrum(pa_engine* e, const uint32_t* h_seed, uint32_t n, uint32_t rho, std::vector<float2>& S, Geom& g,
+                     uint32_t& ws) {
     Workspace* w;
     int rc = prepare(e, n, 3 * n / 8, PA_DEFAULT_FLAGS, &g, &w);
     if (rc != PA_OK) return rc;
+    g.rho = rho;
     DevMem dS, dws, dseed;
-    ST_ALLOC(dS, (size_t)(g.N + 1) * 8);
+    const bool mid = mid_size(g);
+    ST_ALLOC(dS, (size_t)g.N * 8);
     ST_ALLOC(dws, pa::POP_SLOTS * 4);
     ST_ALLOC(dseed, (size_t)n / 8);
     hipStream_t s = e->stream;
     PA_HIP(hipMemcpyAsync(dseed.p, h_seed, n / 8, hipMemcpyHostToDevice, s));
     const pa::Tables t = tables(e, g.L);
-    PA_HIP(pa::launch_zero_u32(dws.as<uint32_t>(), pa::POP_SLOTS, s));
-    PA_HIP(pa::launch_transpose(dseed.as<uint32_t>(), w->tbs, dws.as<uint32_t>(), g, 1, s));
-    PA_HIP(pa::launch_fwd_cols(w->tbs, dS.as<float2>(), g, t, s));
-    PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, dS.as<float2>(), nullptr, g, t, e->cus, s));
-    S.resize(g.N + 1);
+    const pa::ScanArgs scan{nullptr, dseed.as<uint32_t>(), nullptr, pa::prefix_words(w->nib, g.N), w->info};
+    if (!mid) PA_HIP(pa::launch_transpose(nullptr, dseed.as<uint32_t>(), nullptr, w->tbs, 1, 1, g, &scan, s));
+    PA_HIP(pa::launch_fwd_cols(nullptr, mid ? dseed.as<uint32_t>() : w->tbs, nullptr, dS.as<float2>(), 1, 1, g, t, &scan, s));
+    PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, dS.as<float2>(), nullptr, g, t, w->info, nullptr,
+                           dws.as<uint32_t>(), s));
+    S.resize(g.N);
     std::vector<uint32_t> part(pa::POP_SLOTS);
-    PA_HIP(hipMemcpyAsync(S.data(), dS.p, (size_t)(g.N + 1) * 8, hipMemcpyDeviceToHost, s));
+    PA_HIP(hipMemcpyAsync(S.data(), dS.p, (size_t)g.N * 8, hipMemcpyDeviceToHost, s));
     PA_HIP(hipMemcpyAsync(part.data(), dws.p, pa::POP_SLOTS * 4, hipMemcpyDeviceToHost, s));
     PA_HIP(hipStreamSynchronize(s));
     ws = 0;
@@ -2139,25 +2164,42 @@ int st_seed_spectrum(pa_engine* e, const uint32_t* h_seed, uint32_t n, std::vect
 }
 
 int st_dc_zero(pa_engine* e, Report& rp) {
-    // setFirstElementToZero (:377-418): the DC bin of the seed spectrum leaves the row pass as an
-    // exact zero; an all-ones seed (a constant sequence, spectrum at DC only) leaves nothing else
+    // setFirstElementToZero (:377-418) removes the mean's contribution; here the +-1/2 encoding and
+    // the whitening do.  Unwhitened, an all-ones seed (a constant sequence) has the closed form
+    // S[k] = 1 / (1 - exp(-2 pi i (k + 1/4) / N)); whitened, nothing of its mean is left near k = 0;
+    // a random seed keeps a spectrum
     const uint32_t n = 1u << 20;
     std::vector<uint32_t> ones(n / 32, 0xFFFFFFFFu), rnd(n / 32);
     pa_synth_bits(0x5E1F, 0.5, n, rnd.data());
-    for (int which = 0; which < 2 && rp.ok; ++which) {
+    for (int which = 0; which < 3 && rp.ok; ++which) {
         std::vector<float2> S;
+        Geom g;
         uint32_t ws = 0;
-        int rc = st_seed_spectrum(e, which ? rnd.data() : ones.data(), n, S, ws);
+        const uint32_t rho = which == 0 ? 0u : pa::RHO;
+        const std::vector<uint32_t>& seed = which == 2 ? rnd : ones;
+        int rc = st_seed_spectrum(e, seed.data(), n, rho, S, g, ws);
         if (rc != PA_OK) return rc;
         uint32_t want_ws = 0;
-        for (uint32_t v : (which ? rnd : ones)) want_ws += (uint32_t)__builtin_popcount(v);
-        if (S[0].x != 0.f || S[0].y != 0.f) rp.fail("SetFirstElementToZero: DC bin (%g, %g), want 0", S[0].x, S[0].y);
-        else if (ws != want_ws) rp.fail("SetFirstElementToZero: seed popcount %u, want %u", ws, want_ws);
+        for (uint32_t v : seed) want_ws += (uint32_t)__builtin_popcount(v ^ rho);
+        if (ws != want_ws) rp.fail("SetFirstElementToZero: seed popcount %u, want %u", ws, want_ws);
+        auto at = [&](uint32_t k) { return S[(size_t)(k % g.N1) * g.N2 + k / g.N1]; };
         double mx = 0.0;
-        for (size_t k = 1; k < S.size(); ++k) mx = std::max(mx, (double)std::hypot(S[k].x, S[k].y));
-        if (rp.ok && which == 0 && mx > 1e-4 * n)
-            rp.fail("SetFirstElementToZero: constant seed leaves |S| %.3g outside DC", mx);
-        if (rp.ok && which == 1 && mx < 1.0) rp.fail("SetFirstElementToZero: random seed spectrum vanished");
+        for (uint32_t k = 0; k < g.N && rp.ok; ++k) {
+            const float2 v = at(k);
+            if (which == 0) {
+                const double a = 2.0 * M_PI * (k + 0.25) / g.N, d = 2.0 - 2.0 * std::cos(a);
+                const double re = (1.0 - std::cos(a)) / d, im = -std::sin(a) / d;
+                if (std::hypot(v.x - re, v.y - im) > 1e-6 * n)
+                    rp.fail("SetFirstElementToZero: constant seed, bin %u (%g, %g), want (%g, %g)", k, v.x, v.y, re, im);
+            } else {
+                mx = std::max(mx, k < g.N / 64 || which == 2 ? (double)std::hypot(v.x, v.y) : 0.0);
+            }
+        }
+        // a 32-periodic balanced sequence sums to at most 16 ones; the bins below N / 64 lie far
+        // from the first line of its spectrum (N / 16)
+        if (rp.ok && which == 1 && mx > 64.0)
+            rp.fail("SetFirstElementToZero: whitened constant seed leaves |S| %.3g near DC", mx);
+        if (rp.ok && which == 2 && mx < 1.0) rp.fail("SetFirstElementToZero: random seed spectrum vanished");
     }
     return rp.done("SetFirstElementToZero");
 }
@@ -2201,14 +2243,15 @@ int st_product(pa_engine* e, Report& rp) {
 inline uint32_t refbit(const uint32_t* w, uint64_t p) { return (w[p >> 5] >> (31u - (p & 31u))) & 1u; }
 
 int st_unpack(pa_engine* e, Report& rp) {
-    // binInt2float (:484-602): binIn[i] = i; the popcount of n bits is A000788(n/32 - 1); here the
-    // production bit transpose of pass A also lays the bits out for the class tables, checked too
+    // binInt2float (:484-602): binIn[i] = i; the popcount of n bits is A000788(n/32 - 1).  The
+    // production input scan counts them here; its prefix parities, and from 2^23 bits on the layout
+    // that the bit transpose gives pass A's class tables, are checked too
     const uint32_t nmax = 1u << 27;
     std::vector<uint32_t> bin(nmax / 32);
     for (uint32_t i = 0; i < nmax / 32; ++i) bin[i] = i;
-    DevMem dbin, dcnt;
+    DevMem dbin, dws;
     ST_ALLOC(dbin, nmax / 8);
-    ST_ALLOC(dcnt, pa::POP_SLOTS * 4);
+    ST_ALLOC(dws, pa::POP_SLOTS * 4);
     PA_HIP(hipMemcpy(dbin.p, bin.data(), nmax / 8, hipMemcpyHostToDevice));
     uint64_t lcg = 12345;
     for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
@@ -2217,33 +2260,46 @@ int st_unpack(pa_engine* e, Report& rp) {
         Workspace* w;
         int rc = prepare(e, n, 3 * n / 8, PA_DEFAULT_FLAGS, &g, &w);
         if (rc != PA_OK) return rc;
-        PA_HIP(pa::launch_zero_u32(dcnt.as<uint32_t>(), pa::POP_SLOTS, e->stream));
-        PA_HIP(pa::launch_transpose(dbin.as<uint32_t>(), w->tbs, dcnt.as<uint32_t>(), g, 1, e->stream));
-        std::vector<uint32_t> part(pa::POP_SLOTS), tb(g.N / g.D);
-        PA_HIP(hipMemcpyAsync(part.data(), dcnt.p, pa::POP_SLOTS * 4, hipMemcpyDeviceToHost, e->stream));
-        PA_HIP(hipMemcpyAsync(tb.data(), w->tbs, tb.size() * 4, hipMemcpyDeviceToHost, e->stream));
+        g.rho = 0;         // the plain bits
+        g.out_bits = g.L;  // every word's prefix
+        const bool mid = mid_size(g);
+        uint32_t* bits = dbin.as<uint32_t>();
+        uint32_t* q = pa::prefix_words(w->nib, g.N);
+        const pa::ScanArgs scan{nullptr, bits, nullptr, q, w->info};
+        const pa::Tables t = tables(e, g.L);
+        if (!mid) PA_HIP(pa::launch_transpose(nullptr, bits, nullptr, w->tbs, 1, 1, g, &scan, e->stream));
+        PA_HIP(pa::launch_fwd_cols(nullptr, mid ? bits : w->tbs, nullptr, w->Ys, 1, 1, g, t, &scan, e->stream));
+        PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, w->Ys, nullptr, g, t, w->info, nullptr, dws.as<uint32_t>(),
+                               e->stream));
+        PA_HIP(pa::launch_prefix_apply(q, w->info, g, e->stream));
+        std::vector<uint32_t> info(1), pre(g.L / 32), tb(mid ? 0 : g.N / g.D);
+        PA_HIP(hipMemcpyAsync(info.data(), w->info + pa::INFO_POPS, 4, hipMemcpyDeviceToHost, e->stream));
+        PA_HIP(hipMemcpyAsync(pre.data(), q, pre.size() * 4, hipMemcpyDeviceToHost, e->stream));
+        if (!mid) PA_HIP(hipMemcpyAsync(tb.data(), w->tbs, tb.size() * 4, hipMemcpyDeviceToHost, e->stream));
         PA_HIP(hipStreamSynchronize(e->stream));
-        uint64_t cnt = 0;
-        for (uint32_t v : part) cnt += v;
-        if (cnt != ones_upto(n / 32 - 1)) {
-            rp.fail("BinInt2float: n = 2^%u popcount %llu, want %llu", lg, (unsigned long long)cnt,
-                    (unsigned long long)ones_upto(n / 32 - 1));
+        if (info[0] != (uint32_t)ones_upto(n / 32 - 1)) {
+            rp.fail("BinInt2float: n = 2^%u popcount %u, want %llu", lg, info[0], (unsigned long long)ones_upto(n / 32 - 1));
             break;
         }
-        // tb[u N2 + t2] = E | O << 16: bit v of E / O = seed bit 2(t2 + N2 (u + M v)) / that + 1
-        const uint64_t words = tb.size(), checks = lg <= 21 ? words : 65536;
+        uint32_t par = 0;
+        for (uint32_t i = 0; i < g.L / 32 && rp.ok; ++i) {
+            uint32_t want = bin[i];
+            for (int sh = 1; sh < 32; sh *= 2) want ^= want >> sh;
+            if (par) want = ~want;
+            par = want & 1u;
+            if (pre[i] != want) rp.fail("BinInt2float: n = 2^%u prefix word %u = %08x, want %08x", lg, i, pre[i], want);
+        }
+        // tb[u N2 + t2] = E | O << 16: bit v of E / O = seed bit t2 + N2 (u + M v) / that + N
+        const uint64_t words = tb.size(), checks = std::min<uint64_t>(words, 65536);
         for (uint64_t c = 0; c < checks && rp.ok; ++c) {
-            uint64_t idx = c;
-            if (checks != words) {
-                lcg = lcg * 6364136223846793005ull + 1442695040888963407ull;
-                idx = (lcg >> 20) % words;
-            }
+            lcg = lcg * 6364136223846793005ull + 1442695040888963407ull;
+            const uint64_t idx = (lcg >> 20) % words;
             const uint64_t u = idx / g.N2, t2 = idx % g.N2;
             uint32_t want = 0;
             for (uint32_t v = 0; v < g.D; ++v) {
-                const uint64_t p = 2 * (t2 + (uint64_t)g.N2 * (u + (uint64_t)g.M * v));
+                const uint64_t p = t2 + (uint64_t)g.N2 * (u + (uint64_t)g.M * v);
                 want |= refbit(bin.data(), p) << v;
-                want |= refbit(bin.data(), p + 1) << (16 + v);
+                want |= refbit(bin.data(), p + g.N) << (16 + v);
             }
             if (tb[idx] != want) rp.fail("BinInt2float: n = 2^%u bit word %llu = %08x, want %08x", lg,
                                          (unsigned long long)idx, tb[idx], want);
@@ -2254,11 +2310,17 @@ int st_unpack(pa_engine* e, Report& rp) {
 
 int st_epilogue(pa_engine* e, Report& rp) {
     // ToBinaryArray (:605-737): v[p] = bit 31 - p % 32 of p / 32, corr = 1.9, norm = 1, key rest
-    // 0xAAAAAAAA words; output bit p = v[p] ^ key-rest bit p (NoXOR: v[p]), n = 2^10 .. 2^27,
-    // m = n/4 + n/8.  Pass A''s rounding (round_bit) writes the nibbles, the production pack stage
-    // assembles, XORs and orders the words.
+    // 0xAAAAAAAA words; output bit p = v[p] ^ key-rest bit p (NoXOR: v[p]), m = n/4 + n/8, for the
+    // lengths whose output stage is a kernel of its own, n = 2^23 .. 2^27 (shorter ones round and
+    // write in pass A').  round_bit writes the pieces, the production pack stage assembles, XORs and
+    // orders the words.
     const uint32_t nmax = 1u << 27;
-    DevMem dkey, dnib, dout;
+    DevMem dkey, dnib, dout, dinfo, dq;  // zero prefix parities: the rounded bits come out as they are
+    const size_t info_cap = 1u << 20;
+    ST_ALLOC(dinfo, info_cap);
+    ST_ALLOC(dq, nmax / 8);
+    PA_HIP(hipMemset(dinfo.p, 0, info_cap));
+    PA_HIP(hipMemset(dq.p, 0, nmax / 8));
     ST_ALLOC(dkey, (nmax / 32 + 2) * 4);
     ST_ALLOC(dout, nmax / 8 + 64);
     ST_ALLOC(dnib, (size_t)nmax / 2 + 64);
@@ -2267,15 +2329,17 @@ int st_epilogue(pa_engine* e, Report& rp) {
         std::vector<uint32_t> key(nmax / 32 + 2, 0x55555555u);
         PA_HIP(hipMemcpy(dkey.p, key.data(), key.size() * 4, hipMemcpyHostToDevice));
     }
-    for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
+    for (uint32_t lg = pa::MID_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
         const uint32_t n = 1u << lg, m = n / 4 + n / 8;
         for (int do_xor = 1; do_xor >= 0 && rp.ok; --do_xor) {
             Geom g;
             int rc = make_geom(n, m, PA_COMPRESS | (do_xor ? PA_XOR_KEY_REST : 0u), e->cfg.out_reverse_endian,
                                e->cfg.max_n_log2, &g);
             if (rc != PA_OK) return rc;
-            PA_HIP(pa::launch_st_nibbles(dnib.as<uint8_t>(), g, 1.9f, 1.0f, e->stream));
-            PA_HIP(pa::launch_pack(dnib.as<uint8_t>(), dkey.as<uint32_t>(), dout.as<uint32_t>(), g, e->stream));
+            if (pa::info_bytes(g) > info_cap) return PA_ERR_UNSUPPORTED;
+            PA_HIP(pa::launch_st_pieces(dnib.as<uint8_t>(), g, 1.9f, 1.0f, e->stream));
+            PA_HIP(pa::launch_pack(dnib.as<uint8_t>(), dkey.as<uint32_t>(), dout.as<uint32_t>(), g, dinfo.as<uint32_t>(),
+                                   dq.as<uint32_t>(), e->stream));
             std::vector<uint8_t> out(m / 8);
             PA_HIP(hipMemcpyAsync(out.data(), dout.p, m / 8, hipMemcpyDeviceToHost, e->stream));
             PA_HIP(hipStreamSynchronize(e->stream));

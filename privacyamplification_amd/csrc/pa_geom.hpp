@@ -5,14 +5,28 @@
 // read at conv indices [out_off, out_off + out_bits).  For power-of-two n, L = n and out_off = 0,
 // which is the reference's own circular form y[p] = XOR_j x[j] s[(p-j) mod n].
 //
-// The length-L real transform is a length-N complex transform (N = L/2, z[t] = x[2t] + i x[2t+1])
-// evaluated as a four-step FFT with N = N1 * N2 (t = t2 + N2*t1, k = k1 + N1*k2):
-//   pass A  (fwd_cols)  column FFTs of length N1, decimated by D classes of k1 (M = N1/D per class),
-//                       16 columns per workgroup, input from the bit-transposed key/seed;
-//   pass B  (rows)      row FFTs of length N2 on rows k1 and N1-k1, real split, DC zeroing, complex
-//                       product, inverse split, inverse row FFTs;
-//   pass A' (inv_cols)  inverse column FFTs of length N1, W columns per workgroup, round-mod-2 epilogue
-//                       (N1 = 2^15: one column per workgroup, 2-bit crumbs instead of nibbles).
+// The four-step path (L > 2^14) evaluates the NEGACYCLIC convolution of length L instead, c[q] =
+// sum_j sgn a[j] b[(q - j) mod L], sgn = -1 for j > q: wrapped terms change sign, which no parity
+// sees.  The polynomial product mod z^L + 1 is one complex transform of length N = L/2 per operand,
+// z[t] = a[t] - i a[t + N], at the quarter-shifted frequencies k + 1/4, whose values are multiplied
+// point by point: no real-FFT split, and so no frequency needs a partner from another row.
+//   Mean.  a, b are the bits minus 1/2.  With PX(q), PT(q) the inclusive prefix sums of both bit
+// sequences up to q and W the sum of both popcounts, sum_j sgn x[j] t[(q-j) mod L] = c[q] + PX(q) +
+// PT(q) - (W + q + 1)/2 + L/4.  So round(c[q] - ((W + q + 1) mod 4)/2), plus the parities of PX and PT,
+// is the bit; the parities are a bit scan over the inputs (prefix_chunk).
+//   Whitening.  Where both means are far from 1/2 the values of c would grow like n/4, past FP32's
+// resolution for long blocks.  The seed is therefore XORed with a balanced word RHO of flat
+// spectrum, repeated; conv(x, RHO repeated) mod 2 has period 32 and follows from the XOR of the
+// key's words, one correction word for the whole output.
+//   N = N1 * N2 (t = t2 + N2*t1, k = k1 + N1*k2):
+//   pass A  column FFTs of length N1, 16 columns per workgroup.  L >= 2^23: decimated by D classes of
+//           k1 (M = N1/D per class), input from the bit-transposed key/seed; below, straight from
+//           the words (k_mid_fwd);
+//   pass B  row FFTs of length N2, complex product, inverse row FFTs;
+//   pass A' inverse column FFTs of length N1, rounding; below L = 2^23 the output words too.
+// L >= 2^23 has N2 = 8192.  Below, N1 is 2^6 .. 2^9 and N2 = N / N1 is 2^8 .. 2^12 (mid_lg1): as many row
+// and column workgroups as the length allows, because there the time is one workgroup's latency --
+// at N2 = 8192 a row's three transforms alone take 20 us on one compute unit.
 // N <= 8192 (L <= 2^14) runs fully on chip in one workgroup (small path).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -20,17 +34,18 @@
 
 namespace pa {
 
-constexpr int ROW_LOG = 13;            // N2 = 8192 for the four-step path
+constexpr int ROW_LOG = 13;            // N2 = 8192 from L = 2^23 on
 constexpr int SMALL_MAX_LOG_N = 13;    // N <= 8192 -> single-workgroup path
 constexpr int MAX_L_LOG = 29;          // largest transform served (L = 2^29; the reference stops at 2^27)
 
-// Pass B's output R'[k1][t2] when 2^RT_LG1_MIN <= N1 <= 2^RT_LG1_MAX (transforms of 2^24 to 2^29
-// bits) goes to its own buffer in tiles: row pair p (rows p and N1-p, or 0 and N1/2 for p = 0), side
-// s (0: row p, 1: its partner) at Rt[((t2 / RT_COLS) N1/2 + p) 2 RT_COLS + s RT_COLS + t2 mod RT_COLS].
-// A tile holds both rows' RT_COLS columns (2 x 128 bytes): pass B writes whole 128-byte lines, and a
-// workgroup of pass A' (1 to 8 columns) reads its columns from consecutive lines along p instead of
-// from rows 8 N2 bytes apart.  At N1 = 2^RT_LG1 pass A' runs two 256-thread workgroups per CU.
-constexpr int RT_LG1_MIN = 10;
+constexpr uint32_t RHO = 0x8F205B9Bu;   // 16 ones; |DFT_32| <= 3.57 away from DC, 0 there
+
+// Pass B's output R'[k1][t2] when 2^RT_LG1_MIN <= N1 <= 2^RT_LG1_MAX (transforms of 2^25 to 2^29
+// bits) goes to its own buffer in tiles, Rt[((t2 / RT_COLS) N1 + k1) RT_COLS + t2 mod RT_COLS]: pass
+// B writes whole 128-byte lines, and a workgroup of pass A' (1 to 8 columns) reads its columns from
+// consecutive lines along k1 instead of from rows 8 N2 bytes apart.  At N1 = 2^RT_LG1 pass A' runs
+// two 256-thread workgroups per CU.
+constexpr int RT_LG1_MIN = 11;
 constexpr int RT_LG1 = 13;
 constexpr int RT_LG1_MAX = 15;
 constexpr int RT_COLS = 16;
@@ -38,18 +53,56 @@ __host__ __device__ constexpr bool rt_tiled(uint32_t lg1) {
     return lg1 >= (uint32_t)RT_LG1_MIN && lg1 <= (uint32_t)RT_LG1_MAX;
 }
 
+// log2(N1) of a transform of 2^14 <= N <= 2^MID_MAX_LOG_N complex points.
+__host__ __device__ constexpr int mid_lg1(int lgN) {
+    return lgN >= 23 ? 10 : lgN >= 21 ? 9 : lgN >= 16 ? 8 : lgN - 8;
+}
+constexpr int MID_MAX_LOG_N = 23;
+
 struct Geom {
     uint32_t n, m, h, kbits;           // block shape; kbits = h + 1
     uint32_t L, N, lgN;                // transform length, half length, log2(N)
     uint32_t N1, N2, lg1, lg2;         // four-step split (N1 = 1 on the small path)
-    uint32_t M, D, W;                  // pass A class length / classes, pass A' columns per workgroup
+    uint32_t M, D;                     // pass A class length / classes
     uint32_t out_bits, out_off;        // output window in conv indices
     uint32_t seed_words, seed_rot;     // n/32, rotation of the seed in words (m/32 when L > n); the
                                        // rotated seed repeats with period n up to L
     uint32_t key_hw;                   // h/32: index of the key word masked to its MSB
     uint32_t do_xor, reverse_endian;
-    float inv_N;                       // 1/(8N): output normalisation (r2c_split / c2r_split scale)
+    uint32_t rho;                      // whitening word of the seed (0 on the small path)
+    uint32_t scan;                     // words per scan chunk: 1024 << scan
+    float inv_N;                       // output normalisation: 1/N; on the small path 1/(8N), with the
+                                       // factor of r2c_split / c2r_split
 };
+
+// A four-step transform of the mid sizes: no bit masks, no separate output stage.
+__host__ __device__ inline bool mid_size(const Geom& g) { return g.N1 > 1u && g.lgN <= (uint32_t)MID_MAX_LOG_N; }
+
+// Inputs and outputs of the input scan: conv words of the key and the fresh seed (or the resident
+// seed's finished prefix words sq); prefix words q, and the block's info words.
+struct ScanArgs {
+    const uint32_t* key;
+    const uint32_t* seed;
+    const uint32_t* sq;
+    uint32_t* q;
+    uint32_t* info;
+};
+// A block's info buffer: what scan_finish writes, then per chunk its popcount and the XOR of its key
+// words (uint2), then per chunk one byte, its parity.
+constexpr int INFO_POPS = 0;    // both popcounts
+constexpr int INFO_WHITE = 1;   // the whitening's word
+constexpr int INFO_HEAD = 64;   // words before the chunk entries
+__host__ __device__ inline uint32_t scan_chunks(const Geom& g) { return g.L >> (15u + g.scan); }
+__host__ __device__ inline uint2* scan_entries(uint32_t* info) { return reinterpret_cast<uint2*>(info + INFO_HEAD); }
+__host__ __device__ inline uint8_t* scan_parities(uint32_t* info, const Geom& g) {
+    return reinterpret_cast<uint8_t*>(scan_entries(info) + scan_chunks(g));
+}
+__host__ __device__ inline const uint8_t* scan_parities(const uint32_t* info, const Geom& g) {
+    return scan_parities(const_cast<uint32_t*>(info), g);
+}
+inline uint64_t info_bytes(const Geom& g) {
+    return (uint64_t)INFO_HEAD * 4 + scan_chunks(g) * 8ull + (scan_chunks(g) + 255u) / 256u * 256u;
+}
 
 // One block of a batched launch: its geometry and device buffers.  The blocks of one launch share
 // the transform length L (and so N1, N2, M, D, W); n, m, flags and the buffers are per block.
@@ -57,15 +110,17 @@ struct BlockArgs {
     Geom g;
     const uint32_t* key;
     const uint32_t* seed;   // dynamic seed, or nullptr for a resident one
-    const float2* sspec;    // resident split spectrum (N+1 values) when seed == nullptr
+    const float2* sspec;    // resident spectrum when seed == nullptr
     const uint32_t* ws;     // resident seed popcount partials when seed == nullptr
+    const uint32_t* sq;     // resident seed prefix words when seed == nullptr (four-step path only)
     float2* Yk;             // N values (four-step path only)
     float2* Ys;             // N+1 values (dynamic seed, four-step path only)
-    uint32_t* tbk;
+    uint32_t* tbk;          // bit masks (N1 > 2^9 or N2 = 8192 only)
     uint32_t* tbs;
     float2* Rt;             // R' tiles (rt_tiled(lg1)), else nullptr
     uint8_t* nib;
-    uint32_t* counts;       // key partial popcounts, then seed partial popcounts
+    uint32_t* info;         // info words (above)
+    uint32_t* q;            // prefix words, L / 32 (in nib's upper half)
     uint32_t* out;
     float* margin;          // may be nullptr
 };

@@ -6,16 +6,19 @@
 // (FP32 FFT convolution, DC-zeroed spectra, round-mod-2 with the popcount correction) is fused
 // into a few HBM passes:
 //
-//   k_transpose_bits  key/seed RefBits -> per-(class,column) bit masks for pass A, plus popcounts
-//                     (binInt2float's popcount, PrivacyAmplification.cu:570-602)
+//   k_transpose_bits  key/seed RefBits -> per-(class,column) bit masks for pass A
 //   k_fwd_cols        pass A: decimated column FFTs of the +-1/2-encoded bits (R2C forward part);
-//   k_fwd_cols9p      its persistent form for 512-point classes (the 2^27-bit block's shape)
-//   k_rows            pass B: row FFTs, real split, DC zeroing (setFirstElementToZero, :408-418),
-//                     complex product (ElementWiseProduct, :465-481), inverse split, inverse row FFTs
-//   k_inv_cols        pass A': inverse column FFTs + round-mod-2 with the correction term
-//                     (calculateCorrectionFloat :363-373, ToBinaryArray :739-783)
-//   k_pack            output word assembly with the key-rest XOR and byte order
-//                     (key2StartRest's key_rest :873-878, ToBinaryArray's bswap XOR :757-762)
+//   k_fwd_cols9p      its persistent form for 512-point classes (the 2^27-bit block's shape);
+//   k_mid_fwd         its form for L <= 2^22, straight from the key's and the seed's words.
+//                     Their launches also scan the inputs' popcounts (binInt2float's popcount,
+//                     PrivacyAmplification.cu:570-602) and prefix parities
+//   k_rows            pass B: row FFTs, complex product (ElementWiseProduct, :465-481), inverse row FFTs
+//   k_inv_cols        pass A': inverse column FFTs + round-mod-2 (ToBinaryArray :739-783)
+//   k_pack            output word assembly with the mean's correction (calculateCorrectionFloat
+//                     :363-373 and setFirstElementToZero :408-418 remove it spectrally), the key-rest
+//                     XOR and byte order (key2StartRest's key_rest :873-878, ToBinaryArray's bswap
+//                     XOR :757-762)
+//   k_mid_inv         pass A' and the output in one for L <= 2^22
 //   k_small           the whole block in one workgroup for L <= 2^14
 #include <hip/hip_runtime.h>
 
@@ -37,20 +40,20 @@ __device__ __forceinline__ uint32_t key_word(const uint32_t* __restrict__ key, c
     return 0u;
 }
 // Word widx (< L/32) of the seed sequence t: the n seed bits rotated left by seed_rot words and
-// repeated with period n up to the transform length L.  The output window only reads t[0, n),
-// where the repetition changes nothing; beyond n it keeps the +-1/2-encoded sequence free of a
-// constant block.  A zero pad there would become a -1/2 block whose convolution with the key's
-// pad swings by about h/4 across positions after the mean is removed, far beyond FP32's
+// repeated with period n up to the transform length L, XORed with the whitening word g.rho.  The
+// output window only reads t[0, n), where the repetition changes nothing; beyond n it keeps the
+// +-1/2-encoded sequence free of a constant block.  A zero pad there would become a -1/2 block
+// whose convolution with the key's pad swings by about h/4 across positions, far beyond FP32's
 // resolution at L = 2^24; the repeated seed leaves every position a random-walk sum of the same
-// statistics, and every sum in the correction stays constant (ws counts all L positions).
+// statistics.
 __device__ __forceinline__ uint32_t seed_word(const uint32_t* __restrict__ seed, const Geom& g, uint32_t widx) {
     uint32_t s = widx + g.seed_rot;  // < 3 seed_words: L < 2n when L > n
     if (s >= g.seed_words) s -= g.seed_words;
     if (s >= g.seed_words) s -= g.seed_words;
-    return seed[s];
+    return seed[s] ^ g.rho;
 }
 
-// Popcounts are accumulated in POP_SLOTS partial counters (spread atomics); readers sum them.
+// A resident seed's popcount, kept as POP_SLOTS partials.
 __device__ __forceinline__ uint32_t pop_total(const uint32_t* __restrict__ c) {
     uint32_t t = 0;
 #pragma unroll 8
@@ -58,13 +61,6 @@ __device__ __forceinline__ uint32_t pop_total(const uint32_t* __restrict__ c) {
     return t;
 }
 
-
-// Batched launches (BATCH = true) take each block's geometry and buffers from bt[blockIdx.z].
-template <bool BATCH>
-__global__ __launch_bounds__(256) void k_zero_u32(uint32_t* p, uint32_t count, const BlockArgs* __restrict__ bt) {
-    if constexpr (BATCH) p = bt[blockIdx.z].counts;
-    for (uint32_t i = threadIdx.x; i < count; i += 256) p[i] = 0u;
-}
 
 // ------------------------------------------------------------------ staging copies ----
 // One launch moves every staging range of a batch: workgroup (i, y) copies chunks y, y + grid.y,
@@ -108,6 +104,148 @@ __global__ __launch_bounds__(COPY_NT) void k_copies(const CopyDesc* __restrict__
     }
 }
 
+// ------------------------------------------------------------------ mean correction ----
+// The conv value of the +-1/2-encoded sequences differs from the integer it stands for by the
+// prefix sums of both bit sequences (see pa_geom.hpp); mod 2 only their parities matter.  A scan
+// workgroup takes one chunk of 1024 << g.scan words: inclusive prefix parities of x ^ t inside the
+// chunk go to q (bit p of word w: the parity of the chunk's bits up to there; only words up to the
+// end of the output window), the chunk's parity to its byte of cp, its popcount (key + seed) and
+// the XOR of its key words to its entry.  A resident seed brings its own finished prefix words sq;
+// x alone is scanned then.  The scan workgroups ride in the bit transpose's launch (in pass A's below
+// L = 2^23); scan_finish, in pass B's, turns the entries into what pass A' and the output stage read.
+// (In pass A's launch at 2^27 they cost 15 us: with its 74 KB of LDS only two fit a compute unit.)
+__device__ __forceinline__ uint32_t prefix_bits(uint32_t w) {  // bit p: parity of bits 0..p, MSB first
+    w ^= w >> 1;
+    w ^= w >> 2;
+    w ^= w >> 4;
+    w ^= w >> 8;
+    return w ^ (w >> 16);
+}
+// NT threads; lds: 3 NT / 64 words.  key == nullptr scans the seed alone.  Per 1024 words a wave takes 64 PER
+// consecutive ones, 64 at a time: coalesced, the carry between lanes from a ballot.
+template <int NT>
+__device__ __forceinline__ void scan_chunk(uint32_t chunk, const ScanArgs& a, const Geom& g, uint32_t* lds) {
+    constexpr uint32_t PER = 1024 / NT;
+    static_assert(PER * NT == 1024 && NT % 64 == 0, "a thread takes whole words");
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const uint64_t before = (1ull << lane) - 1ull;
+    const uint32_t w_end = (g.out_off + g.out_bits) >> 5;
+    uint32_t pops = 0, kx = 0, chunk_par = 0;
+    for (uint32_t sub = 0; sub < (1u << g.scan); ++sub) {
+        const uint32_t w0 = ((chunk << g.scan) + sub) * 1024u + 64u * PER * wave + lane;
+        uint32_t w[PER], run = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            const uint32_t kw = a.key ? key_word(a.key, g, w0 + 64u * i) : 0u;
+            const uint32_t sw = a.seed ? seed_word(a.seed, g, w0 + 64u * i) : 0u;
+            pops += (uint32_t)(__popc(kw) + __popc(sw));
+            kx ^= kw;
+            w[i] = kw ^ sw;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            w[i] = prefix_bits(w[i]);
+            const uint64_t b = __ballot((w[i] & 1u) != 0u);
+            w[i] ^= 0u - ((run + (uint32_t)__popcll(b & before)) & 1u);
+            run += (uint32_t)__popcll(b);
+        }
+        uint32_t carry = chunk_par;
+        if (sub) __syncthreads();  // the previous round's reads of lds are done
+        if (lane == 0) lds[wave] = run;
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < NT / 64; ++k) {
+            const uint32_t t = lds[k];
+            if (k < wave) carry += t;
+            chunk_par += t;
+        }
+        chunk_par &= 1u;
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            const uint32_t wi = w0 + 64u * i;
+            if (wi < w_end) a.q[wi] = w[i] ^ (0u - (carry & 1u)) ^ (a.sq ? a.sq[wi] : 0u);
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        pops += __shfl_xor(pops, off);
+        kx ^= __shfl_xor(kx, off);
+    }
+    if (lane == 0) {
+        lds[NT / 64 + wave] = pops;
+        lds[2 * (NT / 64) + wave] = kx;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        pops = kx = 0;
+        for (int k = 0; k < NT / 64; ++k) {
+            pops += lds[NT / 64 + k];
+            kx ^= lds[2 * (NT / 64) + k];
+        }
+        scan_entries(a.info)[chunk] = make_uint2(pops, kx);
+        scan_parities(a.info, g)[chunk] = (uint8_t)chunk_par;
+    }
+}
+// One workgroup of NT threads: info[INFO_POPS] = both popcounts (ws: a resident seed's partials),
+// info[INFO_WHITE] = conv(x, rho) mod 2 at conv bits 32 w .. 32 w + 31, the same word for every w
+// (the seed was whitened by rho, period 32, so that product depends on x only through K, the XOR of
+// its words), and the chunks' parities become their exclusive prefix.  lds: 3 NT / 64 words.
+// seed_ws != nullptr (resident seed being prepared): it receives the popcount as partials.
+template <int NT>
+__device__ __forceinline__ void scan_finish(uint32_t* info, const Geom& g, const uint32_t* ws, uint32_t* seed_ws,
+                                            uint32_t* lds) {
+    const uint32_t count = scan_chunks(g), per = (count + NT - 1) / NT, i0 = threadIdx.x * per;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    uint8_t* cp = scan_parities(info, g);
+    uint32_t par = 0, pops = 0, k = 0;
+#pragma unroll 4
+    for (uint32_t i = i0; i < i0 + per && i < count; ++i) {
+        par ^= cp[i];
+        const uint2 e = scan_entries(info)[i];
+        pops += e.x;
+        k ^= e.y;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        pops += __shfl_xor(pops, off);
+        k ^= __shfl_xor(k, off);
+    }
+    const uint64_t b = __ballot(par != 0u);
+    uint32_t carry = (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
+    if (lane == 0) {
+        lds[wave] = (uint32_t)__popcll(b);
+        lds[NT / 64 + wave] = pops;
+        lds[2 * (NT / 64) + wave] = k;
+    }
+    __syncthreads();
+    for (uint32_t i = 0; i < wave; ++i) carry += lds[i];
+    carry &= 1u;
+    for (uint32_t i = i0; i < i0 + per && i < count; ++i) {
+        const uint32_t c = cp[i];
+        cp[i] = (uint8_t)carry;
+        carry ^= c;
+    }
+    if (wave == 0) {
+        pops = k = 0;
+        for (int i = 0; i < NT / 64; ++i) {
+            pops += lds[NT / 64 + i];
+            k ^= lds[2 * (NT / 64) + i];
+        }
+        const uint32_t sh = lane & 31u;  // bit sh of K moves rho sh places on
+        uint32_t e = (lane < 32u && ((k >> (31u - sh)) & 1u)) ? ((g.rho >> sh) | (g.rho << ((32u - sh) & 31u))) : 0u;
+        for (int off = 32; off > 0; off >>= 1) e ^= __shfl_xor(e, off);
+        if (lane == 0) {
+            info[INFO_POPS] = pops + (ws ? pop_total(ws) : 0u);
+            info[INFO_WHITE] = e;
+        }
+        if (seed_ws) seed_ws[lane] = lane == 0 ? pops : 0u;
+    }
+}
+// A resident seed's prefix words once their chunks' exclusive parities are known (pa_seed_put).
+__global__ __launch_bounds__(256) void k_prefix_apply(uint32_t* __restrict__ q, const uint32_t* __restrict__ info,
+                                                      Geom g) {
+    const uint32_t w = blockIdx.x * 256u + threadIdx.x;
+    if (scan_parities(info, g)[w >> (10u + g.scan)]) q[w] = ~q[w];
+}
+
 // ------------------------------------------------------------------ bit transpose ----
 // One round of the recursive 32 x 32 bit-matrix transpose (rows A[k], column 0 = the MSB): swap
 // the off-diagonal J x J blocks of every 2J x 2J block.  Five rounds J = 16, 8, 4, 2, 1 transpose.
@@ -125,163 +263,168 @@ __device__ __forceinline__ void bit_transpose_round(uint32_t (&A)[32]) {
         }
 }
 
-// tb[u*N2 + t2] = E | O << 16 with E bit v = x[2(t2 + N2(u + M v))], O bit v = the odd bit.
+__device__ __forceinline__ void bit_transpose(uint32_t (&A)[32]) {
+    bit_transpose_round<16>(A);
+    bit_transpose_round<8>(A);
+    bit_transpose_round<4>(A);
+    bit_transpose_round<2>(A);
+    bit_transpose_round<1>(A);
+}
+
+// tb[u*N2 + t2] = E | O << 16 with E bit v = x[t2 + N2(u + M v)], O bit v = x[N + t2 + N2(u + M v)].
 // Workgroup (u, part): thread k covers t2 in [part*TB_SPAN + 32k, +32): for each class v it reads
-// the two words holding those 64 bits (coalesced across the workgroup), transposes the D x 32
-// bit-pairs in registers, and the workgroup writes its TB_SPAN outputs through LDS.  Popcounts
-// are reduced per workgroup into one of POP_SLOTS counters.
+// the two words holding those bits (coalesced across the workgroup), transposes the 2 D x 32 bits
+// in registers, and the workgroup writes its TB_SPAN outputs through LDS.  The launch's first
+// `scan_wgs` workgroups scan the inputs, the next ones are operand `first` (0 key, 1 seed), then the
+// next operand.
+// Batched launches (BATCH = true) take each block's geometry and buffers from bt[blockIdx.z].
 template <int D, bool BATCH>
-__global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __restrict__ bits,
-                                                          uint32_t* __restrict__ tb,
-                                                          uint32_t* __restrict__ count, Geom g,
-                                                          int is_seed, const BlockArgs* __restrict__ bt,
-                                                          const uint32_t* __restrict__ bits2,
-                                                          uint32_t* __restrict__ tb2) {
+__global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __restrict__ key,
+                                                          const uint32_t* __restrict__ seed,
+                                                          uint32_t* __restrict__ tbk, uint32_t* __restrict__ tbs,
+                                                          uint32_t first, Geom g, ScanArgs scan, uint32_t scan_wgs,
+                                                          const BlockArgs* __restrict__ bt) {
     __shared__ uint32_t stage[TB_NT * 33];
-    __shared__ uint32_t red[TB_NT / 64];
-    if (!BATCH && blockIdx.y == 1) {  // key and seed in one launch: grid.y selects the seed
-        bits = bits2;
-        tb = tb2;
-        count += POP_SLOTS;
-        is_seed = 1;
-    }
     if constexpr (BATCH) {
         const BlockArgs& a = bt[blockIdx.z];
-        if (is_seed && a.seed == nullptr) return;  // resident seed: nothing to transpose
         g = a.g;
-        bits = is_seed ? a.seed : a.key;
-        tb = is_seed ? a.tbs : a.tbk;
-        count = a.counts + (is_seed ? POP_SLOTS : 0);
+        key = a.key;
+        seed = a.seed;
+        tbk = a.tbk;
+        tbs = a.tbs;
+        scan = ScanArgs{a.key, a.seed, a.sq, a.q, a.info};
+    }
+    if (blockIdx.x < scan_wgs) {
+        scan_chunk<TB_NT>(blockIdx.x, scan, g, stage);
+        return;
     }
     constexpr int PARTS_LOG = ROW_LOG - TB_SPAN_LOG;
-    const uint32_t u = blockIdx.x >> PARTS_LOG, part = blockIdx.x & ((1u << PARTS_LOG) - 1u);
+    uint32_t b = blockIdx.x - scan_wgs;
+    const uint32_t nA = g.M << PARTS_LOG;
+    const bool is_seed = first + b / nA == 1u;
+    const uint32_t* __restrict__ bits = is_seed ? seed : key;
+    uint32_t* __restrict__ tb = is_seed ? tbs : tbk;
+    if (BATCH && bits == nullptr) return;  // resident seed: nothing to transpose
+    b %= nA;
+    const uint32_t u = b >> PARTS_LOG, part = b & ((1u << PARTS_LOG) - 1u);
     const uint32_t t0 = (part << TB_SPAN_LOG) + 32u * threadIdx.x;
     uint32_t w0[D], w1[D];
-    uint32_t pc = 0;
 #pragma unroll
     for (int v = 0; v < D; ++v) {
-        const uint32_t widx = (2u * (t0 + g.N2 * (u + g.M * (uint32_t)v))) >> 5;  // even
+        const uint32_t widx = (t0 + g.N2 * (u + g.M * (uint32_t)v)) >> 5;
         w0[v] = is_seed ? seed_word(bits, g, widx) : key_word(bits, g, widx);
-        w1[v] = is_seed ? seed_word(bits, g, widx + 1u) : key_word(bits, g, widx + 1u);
-        pc += (uint32_t)(__popc(w0[v]) + __popc(w1[v]));
+        w1[v] = is_seed ? seed_word(bits, g, widx + (g.N >> 5)) : key_word(bits, g, widx + (g.N >> 5));
     }
     uint32_t* srow = stage + threadIdx.x * 33;
     if constexpr (D >= 8) {
         // Rows A[15 - v] = w1[v], A[31 - v] = w0[v] (zero for v >= D), transposed: A[c] then holds
-        // bit 31 - c of w0[v] at bit v and of w1[v] at bit v + 16, so output i (E bits from the
-        // pair's even bit 2i, MSB first, O bits from the odd one) is two half-words.
+        // bit 31 - c (column t0 + c) of w0[v] at bit v and of w1[v] at bit v + 16: output c.
         uint32_t A[32];
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
             A[15 - v] = v < D ? w1[v < D ? v : 0] : 0u;
             A[31 - v] = v < D ? w0[v < D ? v : 0] : 0u;
         }
-        bit_transpose_round<16>(A);
-        bit_transpose_round<8>(A);
-        bit_transpose_round<4>(A);
-        bit_transpose_round<2>(A);
-        bit_transpose_round<1>(A);
+        bit_transpose(A);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            srow[i] = (A[2 * i] & 0xFFFFu) | (A[2 * i + 1] << 16);
-            srow[16 + i] = (A[2 * i] >> 16) | (A[2 * i + 1] & 0xFFFF0000u);
-        }
+        for (int i = 0; i < 32; ++i) srow[i] = A[i];
     } else {
 #pragma unroll
         for (int i = 0; i < 32; ++i) {
-            const int sh = 31 - 2 * (i & 15);  // even bit 2i of the 64-bit pair, MSB first
             uint32_t E = 0, O = 0;
 #pragma unroll
             for (int v = 0; v < D; ++v) {
-                const uint32_t w = i < 16 ? w0[v] : w1[v];
-                E |= ((w >> sh) & 1u) << v;
-                O |= ((w >> (sh - 1)) & 1u) << v;
+                E |= ((w0[v] >> (31 - i)) & 1u) << v;
+                O |= ((w1[v] >> (31 - i)) & 1u) << v;
             }
             srow[i] = E | (O << 16);
         }
     }
-    for (int off = 32; off > 0; off >>= 1) pc += __shfl_xor(pc, off);
-    if ((threadIdx.x & 63u) == 0u) red[threadIdx.x >> 6] = pc;
     __syncthreads();
     uint32_t* out = tb + (size_t)u * g.N2 + (part << TB_SPAN_LOG);
     for (int e = threadIdx.x; e < (1 << TB_SPAN_LOG); e += TB_NT) out[e] = stage[(e >> 5) * 33 + (e & 31)];
-    if (threadIdx.x == 0) {
-        uint32_t t = 0;
-#pragma unroll
-        for (int k = 0; k < TB_NT / 64; ++k) t += red[k];
-        if (t) atomicAdd(count + (blockIdx.x % POP_SLOTS), t);
-    }
 }
 
 // ------------------------------------------------------------------ pass A ----
+// One launch serves `ops` operands from `first` on (0 key, 1 seed), nA workgroups each (k_mid_fwd: and
+// then the scan workgroups).  Where a block is one of a batch, its arguments come from the table.
+struct FwdArgs {
+    const uint32_t* in[2];  // bit masks (k_mid_fwd: the words themselves) of key and seed
+    float2* Y[2];
+    uint32_t first, ops, nA;
+    ScanArgs scan;
+};
+template <bool BATCH, bool WORDS>
+__device__ __forceinline__ void fwd_batch_args(FwdArgs& a, Geom& g, const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) {
+        const BlockArgs& b = bt[blockIdx.z];
+        g = b.g;
+        a.in[0] = WORDS ? b.key : b.tbk;
+        a.in[1] = WORDS ? b.seed : b.tbs;
+        a.Y[0] = b.Yk;
+        a.Y[1] = b.Ys;
+        a.scan = ScanArgs{b.key, b.seed, b.sq, b.q, b.info};
+    }
+}
+// w_4N1^x from the 2^14 table while 4 N1 <= 2^14, else from the two-level table of w_2L (2L = 4 N1 N2).
+__device__ __forceinline__ float2 w_4n1(const Geom& g, const float2* __restrict__ tw14, const float2* __restrict__ twlo,
+                                        const float2* __restrict__ twhi, uint32_t x) {
+    if (4u * g.N1 <= (uint32_t)TW14) return tw14[x * (TW14 / (4u * g.N1))];
+    return tw_two_level(twlo, twhi, x * g.N2);
+}
+__device__ __forceinline__ float2 uniform_f2(float2 v) {
+    return make_float2(__uint_as_float(__builtin_amdgcn_readfirstlane((int)__float_as_uint(v.x))),
+                       __uint_as_float(__builtin_amdgcn_readfirstlane((int)__float_as_uint(v.y))));
+}
+
 // Workgroup (column group grp of CPW columns, class c): computes Y[k1][t2] for k1 = c + D*k1',
-// t2 in the group:  Y = w_N^{t2 k1} * FFT_M( w_N1^{u c} * sum_v z[t2 + N2(u + M v)] w_D^{v c} ).
-// The class sum over v is one or two 256-entry table lookups per operand half (bits of tb).  The
-// class values go to LDS and the M-point FFT runs there.  M = 512 (N1 = 512 D, the 2^27-bit
-// block's shape) runs in k_fwd_cols9p instead.
+// t2 in the group, at the quarter-shifted frequencies k1 + 1/4 (c' = c + 1/4):
+//   Y = w_N^{t2 (k1 + 1/4)} * FFT_M( w_N1^{u c'} * sum_v z[t2 + N2(u + M v)] w_D^{v c'} ),
+// z[t] = a[t] - i a[t + N], a = bit - 1/2.  The class sum over v is one or two 256-entry table
+// lookups per operand half (bits of tb), the -1/2 included in the tables.  The class values go to
+// LDS and the M-point FFT runs there: M = 1024, 2048 (N1 = 2^14, 2^15).  M = 512 runs in
+// k_fwd_cols9p instead.
 template <int LGM, int D, bool BATCH, int CPW = fwd_cols_width(LGM)>
-__global__ __launch_bounds__(fwd_cols_threads(LGM)) void k_fwd_cols(const uint32_t* __restrict__ tb,
-                                                     float2* __restrict__ Y, Geom g,
+__global__ __launch_bounds__(fwd_cols_threads(LGM)) void k_fwd_cols(FwdArgs a, Geom g,
                                                      const float2* __restrict__ tw14,
                                                      const float2* __restrict__ twlo,
                                                      const float2* __restrict__ twhi,
                                                      const float2* __restrict__ cls,
-                                                     const BlockArgs* __restrict__ bt, int is_seed,
-                                                     const uint32_t* __restrict__ tb2,
-                                                     float2* __restrict__ Y2) {
-    if (!BATCH && blockIdx.y == 1) {  // key and seed in one launch: grid.y selects the seed
-        tb = tb2;
-        Y = Y2;
-    }
-    if constexpr (BATCH) {
-        const BlockArgs& a = bt[blockIdx.z];
-        if (is_seed && a.seed == nullptr) return;
-        g = a.g;
-        tb = is_seed ? a.tbs : a.tbk;
-        Y = is_seed ? a.Ys : a.Yk;
-    }
+                                                     const BlockArgs* __restrict__ bt) {
+    fwd_batch_args<BATCH, false>(a, g, bt);
     constexpr int M = 1 << LGM;
     constexpr int NT = fwd_cols_threads(LGM);
     constexpr int SEQS = seq_stride(M);
-    static_assert(LGM != 9, "512-point classes run in k_fwd_cols9p");
+    static_assert(LGM >= 10, "512-point classes run in k_fwd_cols9p");
     __shared__ float2 buf[CPW * SEQS];
     __shared__ float2 twl[TWL_SIZE];
     constexpr int BW = cls_bits(D);         // bits per table: v in [BW q, BW q + BW)
     constexpr int NB = cls_tables(D);       // tables per 16-bit half
     constexpr uint32_t MASK = (1u << BW) - 1u;
-    __shared__ float2 TB[NB][1 << BW];      // TB[q][byte] = sum_b bit_b(byte) w_D^{(BW q + b) c}
-    __shared__ float2 TU[M];                // w_N1^{u c}
-    const uint32_t logical = xcd_logical(blockIdx.x, gridDim.x);
+    __shared__ float2 TB[NB][1 << BW];      // TB[q][byte] = sum_b (bit_b(byte) - 1/2) w_D^{(BW q + b) c'}
+    __shared__ float2 TU[M];                // w_N1^{u c'} = w_4N1^{u (4c + 1)}
+    const uint32_t op = blockIdx.x / a.nA;
+    const bool is_seed = a.first + op == 1u;
+    const uint32_t* __restrict__ tb = is_seed ? a.in[1] : a.in[0];
+    float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
+    if (BATCH && tb == nullptr) return;
+    const uint32_t logical = xcd_logical(blockIdx.x - op * a.nA, a.nA);
     const uint32_t c = logical % D, grp = logical / D;  // columns [CPW grp, CPW grp + CPW)
     load_twl(twl, tw14, NT);
     {
         const float2* src = cls + cls_table_offset(D) + (size_t)c * (NB << BW);
         for (int e = threadIdx.x; e < NB << BW; e += NT) TB[e >> BW][e & (int)MASK] = src[e];
     }
-    // w_N1^{u c}: from the 2^14 table while N1 <= 2^14, else from the length-L two-level table
-    if (g.N1 <= (uint32_t)TW14) {
-        const uint32_t step_n1 = TW14 / g.N1;
-        for (int u = threadIdx.x; u < M; u += NT) TU[u] = tw14[((uint32_t)u * c) * step_n1];
-    } else {
-        const uint32_t step_l = g.L / g.N1;
-        for (int u = threadIdx.x; u < M; u += NT) TU[u] = tw_two_level(twlo, twhi, ((uint32_t)u * c) * step_l);
-    }
-    // the element z(col, u) of this class (both halves of tb: even and odd bits)
-    auto zval = [&](uint32_t t, int u, auto is_c0) {
+    for (uint32_t u = threadIdx.x; u < (uint32_t)M; u += NT) TU[u] = w_4n1(g, tw14, twlo, twhi, u * (4u * c + 1u));
+    // the element z(col, u) of this class (both halves of tb: positions t and t + N)
+    auto zval = [&](uint32_t t, int u) {
         float2 sE = TB[0][t & MASK], sO = TB[0][(t >> 16) & MASK];
 #pragma unroll
         for (int q = 1; q < NB; ++q) {
             sE = cadd(sE, TB[q][(t >> (BW * q)) & MASK]);
             sO = cadd(sO, TB[q][(t >> (16 + BW * q)) & MASK]);
         }
-        float2 z = make_float2(sE.x - sO.y, sE.y + sO.x);
-        if constexpr (decltype(is_c0)::value) {
-            z.x -= 0.5f * (float)D;
-            z.y -= 0.5f * (float)D;
-        } else {
-            z = cmul(z, TU[u]);
-        }
-        return z;
+        return cmul(make_float2(sE.x + sO.y, sE.y - sO.x), TU[u]);
     };
     constexpr int IPT = (CPW * M + NT - 1) / NT;
     uint32_t tbv[IPT];
@@ -294,28 +437,25 @@ __global__ __launch_bounds__(fwd_cols_threads(LGM)) void k_fwd_cols(const uint32
 #pragma unroll
     for (int i = 0; i < IPT; ++i) {
         const int e = threadIdx.x + i * NT;
-        if (e < CPW * M)
-            buf[(e % CPW) * SEQS + padi(e / CPW)] =
-                c == 0 ? zval(tbv[i], e / CPW, std::true_type{}) : zval(tbv[i], e / CPW, std::false_type{});
+        if (e < CPW * M) buf[(e % CPW) * SEQS + padi(e / CPW)] = zval(tbv[i], e / CPW);
     }
     __syncthreads();
     lds_fft<LGM, CPW, SEQS, NT>(buf, twl);
     // Output e = tid + NT i is column tid mod CPW, k1' = tid / CPW + RPI i: its twiddle
-    // w_L^{2 t2 k1} is base step^i, re-anchored from the table every 8 steps (a gather per point
-    // cost more than the transform at N1 >= 2^14)
+    // w_2L^{t2 (4 k1 + 1)} is base step^i, re-anchored from the table every 8 steps (a gather per
+    // point cost more than the transform at N1 >= 2^14)
     static_assert(NT % CPW == 0, "a thread keeps one column");
     constexpr int RPI = NT / CPW;
     const int col = threadIdx.x % CPW, jt = threadIdx.x / CPW;
     const uint32_t t2 = grp * CPW + (uint32_t)col;
-    const uint64_t L1m = g.L - 1u;
+    const uint32_t L2m = 2u * g.L - 1u;
     auto tw_at = [&](uint32_t k1p) {
-        return tw_two_level(twlo, twhi, (uint32_t)((2ull * t2 * (c + (uint64_t)D * k1p)) & L1m));
+        return tw_two_level(twlo, twhi, (t2 * (4u * (c + (uint32_t)D * k1p) + 1u)) & L2m);
     };
-    const float2 step = tw_two_level(twlo, twhi, (uint32_t)((2ull * t2 * (uint64_t)D * RPI) & L1m));
+    const float2 step = tw_two_level(twlo, twhi, (t2 * (4u * (uint32_t)D * RPI)) & L2m);
     float2 tw = make_float2(1.f, 0.f);
-    for (int i = 0; i < (CPW * M + NT - 1) / NT; ++i) {
+    for (int i = 0; i < (CPW * M) / NT; ++i) {
         const uint32_t k1p = (uint32_t)jt + (uint32_t)RPI * (uint32_t)i;
-        if (k1p >= (uint32_t)M) break;  // CPW M < NT: the upper threads have no output
         tw = (i & 7) == 0 ? tw_at(k1p) : cmul(tw, step);
         const uint32_t k1 = c + (uint32_t)D * k1p;
         st_nt(&Y[(size_t)k1 * g.N2 + t2], cmul(buf[col * SEQS + padi((int)k1p)], tw));
@@ -351,28 +491,30 @@ __device__ __forceinline__ void fwd9_load_tv(uint32_t (&tv)[2][16], __amdgpu_buf
         for (int r = 0; r < 16; ++r) tv[i][r] = buf_load_u32(rtb, voff, (uint32_t)(32 * r) * N2 * 4u);
     }
 }
-// Table entries of the output twiddles w_N^{t2 k1}, k1 = c + D (jt + 16 r) = base step^r, with
+// Table entries of the output twiddles w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + 16 r) = base step^r, with
 // anchors w_N^{t2 16 D 8 (a+1)}: (lo, hi) pairs of base, step, anchor 0..2.  The products are
 // formed where they are used, so that gathering them never waits on other loads.
 template <int D>
 __device__ __forceinline__ void fwd9_load_tw(float2 (&tw)[10], const float2* __restrict__ lo,
                                              const float2* __restrict__ hi, uint32_t L, uint32_t c, uint32_t t2,
                                              int jt) {
-    const uint64_t T = t2;
+    const uint32_t L2m = 2u * L - 1u;
     uint32_t x[5];
-    x[0] = (uint32_t)((2ull * T * (c + (uint64_t)D * (uint32_t)jt)) & (L - 1u));
-    x[1] = (uint32_t)((2ull * T * 16ull * D) & (L - 1u));
+    x[0] = (t2 * (4u * (c + (uint32_t)D * (uint32_t)jt) + 1u)) & L2m;
+    x[1] = (t2 * (64u * (uint32_t)D)) & L2m;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) x[2 + a] = (uint32_t)((2ull * T * 16ull * D * (8 * (a + 1))) & (L - 1u));
+    for (int a = 0; a < 3; ++a) x[2 + a] = (t2 * (64u * (uint32_t)D * 8u * (uint32_t)(a + 1))) & L2m;
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
         tw[2 * e] = lo[x[e] & (TW14 - 1)];
         tw[2 * e + 1] = hi[x[e] >> TW14_LOG];
     }
 }
-template <int D, bool C0>
+// tw1: the first stage's factors for w_N1^{32 c'} (one class per workgroup: uniform).
+template <int D>
 __device__ __forceinline__ void fwd9_stage1(const uint32_t (&tv)[2][16], float2* buf,
-                                            const float2 (*TB)[1 << cls_bits(D)], const float2* TU, int col, int jt) {
+                                            const float2 (*TB)[1 << cls_bits(D)], const float2 (&tw1)[8], int col,
+                                            int jt) {
     constexpr int SEQS = seq_stride(512);
     constexpr int BW = cls_bits(D);
     constexpr int NB = cls_tables(D);
@@ -390,26 +532,22 @@ __device__ __forceinline__ void fwd9_stage1(const uint32_t (&tv)[2][16], float2*
                 sE = cadd(sE, TB[q][(t >> (BW * q)) & MASK]);
                 sO = cadd(sO, TB[q][(t >> (16 + BW * q)) & MASK]);
             }
-            float2 z = make_float2(sE.x - sO.y, sE.y + sO.x);
-            if constexpr (C0) {
-                z.x -= 0.5f * (float)D;
-                z.y -= 0.5f * (float)D;
-            } else {
-                z = cmul(z, TU[j + 32 * r]);
-            }
-            v[r] = z;
+            v[r] = make_float2(sE.x + sO.y, sE.y - sO.x);
         }
-        stage_first_to_lds<16>(v, buf + col * SEQS, j);
+        dft_tw<16>(v, tw1);
+        float2* seqbuf = buf + col * SEQS;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) seqbuf[padi(j * 16 + r)] = v[r];
     }
 }
-// tw2: the radix-32 stage's twiddle table, w_512^(jt r) at tw2[jt * 33 + r] (fill_stage_table<32, 16>).
+// tw2: the radix-32 stage's factors, row jt for w_512^jt w_N1^c' (the class twiddle of input j).
 template <int D>
 __device__ __forceinline__ void fwd9_stage2(const float2* buf, const float2* tw2, const float2 (&tw)[10],
                                             __amdgpu_buffer_rsrc_t ry, uint32_t N2, uint32_t c, uint32_t t2,
                                             int col, int jt) {
     constexpr int SEQS = seq_stride(512);
     float2 F[32];
-    stage_last_from_lds_tab<32, 512>(F, buf + col * SEQS, jt, tw2 + jt * 33);
+    stage_last_from_lds_tab<32, 512>(F, buf + col * SEQS, jt, tw2 + jt * stage_row<32>());
     const float2 base = cmul(tw[0], tw[1]), step = cmul(tw[2], tw[3]);
     const uint32_t voff = ((c + (uint32_t)D * (uint32_t)jt) * N2 + t2) * 8u;
     float2 w = base;
@@ -420,11 +558,11 @@ __device__ __forceinline__ void fwd9_stage2(const float2* buf, const float2* tw2
         w = cmul(w, step);
     }
 }
-template <int D, bool C0>
+template <int D>
 __device__ __forceinline__ void fwd9_walk(__amdgpu_buffer_rsrc_t rtb, __amdgpu_buffer_rsrc_t ry, const Geom& g,
                                           const float2* __restrict__ twlo, const float2* __restrict__ twhi,
                                           float2* buf, const float2* tw2, const float2 (*TB)[1 << cls_bits(D)],
-                                          const float2* TU, uint32_t c, uint32_t grp0, uint32_t per) {
+                                          const float2 (&tw1)[8], uint32_t c, uint32_t grp0, uint32_t per) {
     const int col = threadIdx.x & 15;
     const int jt = threadIdx.x >> 4;
     const uint32_t N2 = g.N2;
@@ -436,7 +574,7 @@ __device__ __forceinline__ void fwd9_walk(__amdgpu_buffer_rsrc_t rtb, __amdgpu_b
     fwd9_load_tv(tv, rtb, N2, grp0 * 16u + (uint32_t)col, jt);
     fwd9_load_tw<D>(tw, twlo, twhi, g.L, c, grp0 * 16u + (uint32_t)col, jt);
     __syncthreads();  // tables
-    fwd9_stage1<D, C0>(tv, buf, TB, TU, col, jt);
+    fwd9_stage1<D>(tv, buf, TB, tw1, col, jt);
     __syncthreads();
     if (per > 1) {
         fwd9_load_tv(tv, rtb, N2, (grp0 + 1u) * 16u + (uint32_t)col, jt);
@@ -448,7 +586,7 @@ __device__ __forceinline__ void fwd9_walk(__amdgpu_buffer_rsrc_t rtb, __amdgpu_b
 #pragma unroll
         for (int e = 0; e < 10; ++e) tw[e] = twn[e];
         __syncthreads();  // stage-2 reads of the previous group are done
-        fwd9_stage1<D, C0>(tv, buf, TB, TU, col, jt);
+        fwd9_stage1<D>(tv, buf, TB, tw1, col, jt);
         __syncthreads();
         if (it + 1 < per) {
             fwd9_load_tv(tv, rtb, N2, (grp + 1u) * 16u + (uint32_t)col, jt);
@@ -458,346 +596,344 @@ __device__ __forceinline__ void fwd9_walk(__amdgpu_buffer_rsrc_t rtb, __amdgpu_b
     }
 }
 
-// Persistent pass A for M = 512 (the fused 16 x 32 plan of k_fwd_cols): workgroup L of G keeps one
-// class c = L mod D and walks the column groups [k per, k per + per), k = L / D, so its class
-// tables are loaded once, and each group's stores drain while the next group is transformed (its
-// loads were issued before those stores).  The D workgroups of one k sit on one XCD and walk the
-// same groups in step, so each bit word is fetched into L2 once.
+// Persistent pass A for M = 512 (plan 16 x 32): workgroup L of G keeps one class c = L mod D and
+// walks the column groups [k per, k per + per), k = L / D, so its class tables are loaded once, and
+// each group's stores drain while the next group is transformed (its loads were issued before those
+// stores).  The D workgroups of one k sit on one XCD and walk the same groups in step, so each bit
+// word is fetched into L2 once.  The class twiddles w_N1^{u c'}, u = j + 32 r, cost nothing: their
+// r part is in the first stage's factors, their j part in the second's.
 template <int D, bool BATCH>
-__global__ __launch_bounds__(FWD_NT, 2) void k_fwd_cols9p(const uint32_t* __restrict__ tb,
-                                                          float2* __restrict__ Y, Geom g,
-                                                          const float2* __restrict__ tw14,
+__global__ __launch_bounds__(FWD_NT, 2) void k_fwd_cols9p(FwdArgs a, Geom g, const float2* __restrict__ tw14,
                                                           const float2* __restrict__ twlo,
                                                           const float2* __restrict__ twhi,
-                                                          const float2* __restrict__ cls,
-                                                          const uint32_t* __restrict__ tb2,
-                                                          float2* __restrict__ Y2, uint32_t per,
-                                                          const BlockArgs* __restrict__ bt, int is_seed) {
-    if constexpr (BATCH) {  // grid.z = block of a batch group (one transform length)
-        const BlockArgs& a = bt[blockIdx.z];
-        if (is_seed && a.seed == nullptr) return;  // resident seed: nothing to transform
-        g = a.g;
-        tb = is_seed ? a.tbs : a.tbk;
-        Y = is_seed ? a.Ys : a.Yk;
-    } else if (blockIdx.y == 1) {  // key and seed in one launch: grid.y selects the seed
-        tb = tb2;
-        Y = Y2;
-    }
+                                                          const float2* __restrict__ cls, uint32_t per,
+                                                          const BlockArgs* __restrict__ bt) {
+    fwd_batch_args<BATCH, false>(a, g, bt);
     constexpr int M = 512;
     constexpr int NT = FWD_NT;
     constexpr int SEQS = seq_stride(M);
     static_assert(NT == 256, "fused pass A expects 256 threads");
     __shared__ float2 buf[16 * SEQS];
-    __shared__ float2 tw2[16 * 33];  // radix-32 stage twiddles w_512^(jt r), rows padded to 33
+    __shared__ float2 tw2[16 * stage_row<32>()];
     constexpr int BW = cls_bits(D);
     constexpr int NB = cls_tables(D);
     constexpr uint32_t MASK = (1u << BW) - 1u;
     __shared__ float2 TB[NB][1 << BW];
-    __shared__ float2 TU[M];
-    const uint32_t logical = xcd_logical(blockIdx.x, gridDim.x);
+    const uint32_t op = blockIdx.x / a.nA;
+    const bool is_seed = a.first + op == 1u;
+    const uint32_t* __restrict__ tb = is_seed ? a.in[1] : a.in[0];
+    float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
+    if (BATCH && tb == nullptr) return;  // resident seed: nothing to transform
+    const uint32_t logical = xcd_logical(blockIdx.x - op * a.nA, a.nA);
     const uint32_t c = logical % D, grp0 = (logical / D) * per;
     const __amdgpu_buffer_rsrc_t rtb = make_rsrc(tb, (uint32_t)M * g.N2 * 4u);
     const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * g.N2 * 8u);
-    fill_stage_table<32, 16>(tw2, tw14, NT);
     {
         const float2* src = cls + cls_table_offset(D) + (size_t)c * (NB << BW);
         for (int e = threadIdx.x; e < NB << BW; e += NT) TB[e >> BW][e & (int)MASK] = src[e];
     }
-    if (g.N1 <= (uint32_t)TW14) {
-        const uint32_t step_n1 = TW14 / g.N1;
-        for (int u = threadIdx.x; u < M; u += NT) TU[u] = tw14[((uint32_t)u * c) * step_n1];
-    } else {
-        const uint32_t step_l = g.L / g.N1;
-        for (int u = threadIdx.x; u < M; u += NT) TU[u] = tw_two_level(twlo, twhi, ((uint32_t)u * c) * step_l);
+    const uint32_t m4 = 4u * g.N1 - 1u, f = 4u * c + 1u;  // exponents of w_4N1
+    {
+        const uint32_t q = threadIdx.x >> 4, i = threadIdx.x & 15u;
+        uint32_t s = 2;  // the size of factor i and its index k at that size (dft_tw's order)
+        while (s / 2u <= i && i > 0u) s *= 2u;
+        const uint32_t k = i ? i - s / 4u : 0u;
+        tw2[q * stage_row<32>() + i] =
+            w_4n1(g, tw14, twlo, twhi, ((32u / s) * (4u * (uint32_t)D * q + f) + k * (4u * g.N1 / s)) & m4);
     }
-    if (c == 0) fwd9_walk<D, true>(rtb, ry, g, twlo, twhi, buf, tw2, TB, TU, c, grp0, per);
-    else fwd9_walk<D, false>(rtb, ry, g, twlo, twhi, buf, tw2, TB, TU, c, grp0, per);
+    float2 tw1[8];
+#pragma unroll
+    for (uint32_t i = 0; i < 8; ++i) {
+        const uint32_t s = i == 0 ? 2u : i == 1 ? 4u : i < 4 ? 8u : 16u, k = i ? i - s / 4u : 0u;
+        tw1[i] = uniform_f2(w_4n1(g, tw14, twlo, twhi, ((16u / s) * 32u * f + k * (4u * g.N1 / s)) & m4));
+    }
+    fwd9_walk<D>(rtb, ry, g, twlo, twhi, buf, tw2, TB, tw1, c, grp0, per);
+}
+
+// Pass A for L <= 2^24 (N1 = 2^6 .. 2^10), straight from the key's and the seed's words: 16 adjacent
+// columns of one row are half a word, so no bit transpose is needed.  Plan R1 x 16 (R1 x 32 from
+// 512 on): the quarter shift sits in the stages' factors.
+template <int LG1, bool BATCH>
+__global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g, const float2* __restrict__ tw14,
+                                                              const float2* __restrict__ twlo,
+                                                              const float2* __restrict__ twhi,
+                                                              const BlockArgs* __restrict__ bt) {
+    fwd_batch_args<BATCH, true>(a, g, bt);
+    constexpr int N1 = 1 << LG1, NT = mid_threads(LG1), R1 = mid_r1(LG1), R2 = N1 / R1, S1 = N1 / R1;
+    constexpr int K1 = 16 * S1 / NT, SEQS = seq_stride(N1);
+    static_assert(16 * R1 == NT && K1 * R1 == R2, "one second-stage butterfly per thread");
+    __shared__ float2 buf[16 * SEQS];
+    __shared__ float2 tab[R1 * stage_row<R2>()];
+    __shared__ uint32_t bw[N1];  // the group's 16 bits of row u, and of row u + N1 above them
+    const uint32_t op = blockIdx.x / a.nA;
+    if (op >= a.ops) {
+        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, bw);
+        return;
+    }
+    const bool is_seed = a.first + op == 1u;
+    const uint32_t* __restrict__ in = is_seed ? a.in[1] : a.in[0];
+    float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
+    if (BATCH && in == nullptr) return;
+    const uint32_t grp = blockIdx.x - op * a.nA, sh = (grp & 1u) ? 0u : 16u;
+    for (uint32_t u = threadIdx.x; u < (uint32_t)N1; u += NT) {
+        const uint32_t w = (16u * grp + g.N2 * u) >> 5, wh = w + (g.N >> 5);
+        const uint32_t lo = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
+        const uint32_t hi = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
+        bw[u] = ((lo >> sh) & 0xFFFFu) | ((hi >> sh) << 16);
+    }
+    // second stage's factors: row q for w_N1^(q + 1/4)
+    for (int e = threadIdx.x; e < R1 * (R2 / 2); e += NT) {
+        const int q = e / (R2 / 2), i = e % (R2 / 2);
+        int s = 2;
+        while (s / 2 <= i && i > 0) s *= 2;
+        const int k = i ? i - s / 4 : 0;
+        tab[q * stage_row<R2>() + i] = tw14[((4 * q + 1) * (TW14 / (4 * R1 * s)) + k * (TW14 / s)) & (TW14 - 1)];
+    }
+    float2 tw1[R1 / 2];  // first stage: w = exp(-2 pi i / (4 R1)), size s, k: exp(-2 pi i (4k + 1) / (4s))
+#pragma unroll
+    for (int i = 0; i < R1 / 2; ++i) {
+        const int s = i == 0 ? 2 : i == 1 ? 4 : i < 4 ? 8 : i < 8 ? 16 : 32, k = i ? i - s / 4 : 0;
+        tw1[i] = uniform_f2(tw14[(4 * k + 1) * (TW14 / (4 * s))]);
+    }
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    const uint32_t t2 = 16u * grp + (uint32_t)col;
+    const uint32_t L2m = 2u * g.L - 1u;
+    const float2 step = tw_two_level(twlo, twhi, (t2 * 4u * R1) & L2m);
+    __syncthreads();
+    float2* seqbuf = buf + col * SEQS;
+#pragma unroll
+    for (int i = 0; i < K1; ++i) {
+        const int j = jt + (NT / 16) * i;
+        float2 v[R1];
+#pragma unroll
+        for (int r = 0; r < R1; ++r) {  // z = (bit - 1/2) - i (bit' - 1/2)
+            const uint32_t b = bw[j + S1 * r] << (16 + col);
+            const uint32_t bh = bw[j + S1 * r] << col;
+            v[r] = make_float2((int)b < 0 ? 0.5f : -0.5f, (int)bh < 0 ? -0.5f : 0.5f);
+        }
+        dft_tw<R1>(v, tw1);
+#pragma unroll
+        for (int r = 0; r < R1; ++r) seqbuf[padi(j * R1 + r)] = v[r];
+    }
+    __syncthreads();
+    float2 F[R2];
+    stage_last_from_lds_tab<R2, N1>(F, seqbuf, jt, tab + jt * stage_row<R2>());
+    // k1 = jt + R1 r: w_2L^{t2 (4 k1 + 1)} = base step^r, re-anchored from the table every 8 steps
+    float2 tw = make_float2(1.f, 0.f);
+#pragma unroll
+    for (int r = 0; r < R2; ++r) {
+        const uint32_t k1 = (uint32_t)jt + (uint32_t)(R1 * r);
+        tw = (r & 7) == 0 ? tw_two_level(twlo, twhi, (t2 * (4u * k1 + 1u)) & L2m) : cmul(tw, step);
+        Y[(size_t)k1 * g.N2 + t2] = cmul(F[r], tw);
+    }
 }
 
 // ------------------------------------------------------------------ pass B ----
-// Item w (one row pair) owns rows (w, N1-w), or (0, N1/2) for w = 0: the rows whose frequencies
-// pair k <-> N-k in the real split (k = row + N1*k2).  Row transforms have N2 = 8192 points:
-//   forward plan 32 x 16 x 16: stage 1 straight from global memory, stage 3 into registers;
-//   inverse plan 16 x 16 x 32: stage 1 from registers, stage 3 straight to global memory.
-// After forward stage 3 a thread holds Z at k2 = jA + 512 r (row sA) and k2 = jB + 512 r (row sB)
-// for r < 16, chosen so that the partners of the first are the second read backwards:
-//   w != 0:                     (row0, t)      and (row1, 511-t)        pairs (A r, B 15-r)
-//   w == 0, 0 < t < 256:        (row0, t)      and (row0, 512-t)        pairs (A r, B 15-r)
-//   w == 0, t >= 256:           (row1, t-256)  and (row1, 767-t)        pairs (A r, B 15-r)
-//   w == 0, t == 0:             (row0, 0)      and (row0, 256)          pairs (A r, A 16-r) with
-//                               k = 0 (DC zeroed, Nyquist carried) and k = N/2 self-paired,
-//                               and (B r, B 15-r)
-// so the real split, product and inverse split need no data exchange, and their results are
-// exactly the inputs of inverse stage 1.
-//   ROWS_SEEDPREP: seed rows (pass-A output) -> split seed spectrum S, in place (+ S[N] at index N).
-//   ROWS_STATIC:   key rows + resident S -> R'[k1][t2] = w_N^{t2 k1} FFT_N2(conj Q)[t2], in place,
-//                  or into pass A''s tiles (Rt) when rt_tiled(lg1).
+// Rows of N2 = 2^LG2 points.  The frequencies k1 + N1 k2 + 1/4 of a row have no partners in other
+// rows, so rows are independent:
+//   forward plan R1 x 16 x 16 (16 x 16 at N2 = 256): stage 1 straight from global memory, stage 3
+//   into registers, where thread j of a row holds k2 = j + NTR h + (N2/16) r (r < 16);
+//   the product there;
+//   inverse plan 16 x 16 x R1: stage 1 from those registers, stage 3 straight to global memory.
+//   ROWS_SEEDPREP: seed rows (pass-A output) -> the seed spectrum S[k1 N2 + k2], in place.
+//   ROWS_STATIC:   key rows + resident S -> R'[k1][t2] = w_N^{t2 (k1 + 1/4)} FFT_N2(conj P)[t2], in
+//                  place, or into pass A''s tiles (Rt) when rt_tiled(lg1).
 //   ROWS_DYN:      key rows + seed rows; S is formed first and held in registers.
-// Persistent: each workgroup walks the items blockIdx.x, +gridDim.x, ...; the global inputs of
-// the next transform are requested while the current one runs (register prefetch).
-struct RowMap {
-    uint32_t row0, row1, rowA, rowB;
-    int sA, jA, sB, jB;
-    bool special;
-};
-__device__ __forceinline__ RowMap row_map(uint32_t w, uint32_t N1, int tid) {
-    RowMap m;
-    const bool w0 = (w == 0);
-    m.row0 = w;
-    m.row1 = w0 ? (N1 >> 1) : (N1 - w);
-    m.special = w0 && tid == 0;
-    if (!w0) { m.sA = 0; m.jA = tid; m.sB = 1; m.jB = 511 - tid; }
-    else if (tid == 0) { m.sA = 0; m.jA = 0; m.sB = 0; m.jB = 256; }
-    else if (tid < 256) { m.sA = 0; m.jA = tid; m.sB = 0; m.jB = 512 - tid; }
-    else { m.sA = 1; m.jA = tid - 256; m.sB = 1; m.jB = 767 - tid; }
-    m.rowA = m.sA ? m.row1 : m.row0;
-    m.rowB = m.sB ? m.row1 : m.row0;
-    return m;
-}
-
-template <int MODE, bool BATCH>
-__global__ __launch_bounds__(ROWS_NT) void k_rows(float2* __restrict__ Yk, float2* __restrict__ Sst,
-                                                  float2* __restrict__ Rt, Geom g, const float2* __restrict__ tw14,
-                                                  const float2* __restrict__ twlo,
-                                                  const float2* __restrict__ twhi,
-                                                  const BlockArgs* __restrict__ bt) {
+// N2 = 8192 runs one row per 256-thread workgroup, 32 points per thread, 74 KB of LDS, so two share
+// a compute unit and one's memory requests overlap the other's transforms.  Shorter rows take 16
+// points per thread and at least one wave per workgroup (rows_per_wg rows).
+// The launch's first workgroup finishes the scan (scan_finish).
+template <int LG2, int MODE, bool BATCH>
+__global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
+    float2* __restrict__ Yk, float2* __restrict__ Sst, float2* __restrict__ Rt, Geom g,
+    const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
+    uint32_t* __restrict__ info, const uint32_t* __restrict__ ws, uint32_t* __restrict__ seed_ws,
+    const BlockArgs* __restrict__ bt) {
     if constexpr (BATCH) {
         const BlockArgs& a = bt[blockIdx.z];
         g = a.g;
         Yk = a.Yk;
         Sst = (MODE == ROWS_STATIC) ? const_cast<float2*>(a.sspec) : a.Ys;
         Rt = a.Rt;
+        info = a.info;
+        ws = a.seed ? nullptr : a.ws;
     }
-    constexpr int N2 = 1 << ROW_LOG, NT = ROWS_NT, SEQS = seq_stride(N2);
-    static_assert(N2 == 8192 && NT == 512, "row pass is written for 8192-point rows, 512 threads");
-    static_assert(2 * N2 == TW14, "row split twiddle assumes N2 = 2^13");
-    __shared__ float2 buf[2 * SEQS];
+    constexpr int N2 = 1 << LG2, NT = rows_threads(LG2), RPW = rows_per_wg(LG2), NTR = NT / RPW;
+    constexpr int PPT = N2 / NTR, KL = PPT / 16;          // points and radix-16 butterflies per thread
+    constexpr int R1 = LG2 == 8 ? 16 : N2 / 256, K1 = PPT / R1;
+    constexpr int SEQS = seq_stride(N2);
+    __shared__ float2 buf[RPW * SEQS];
     __shared__ float2 twl[TWL_SIZE];
-    __shared__ float2 ttf[32 * 17];  // forward middle stage (radix 16, span 32)
-    __shared__ float2 tti[16 * 17];  // inverse middle stage (radix 16, span 16)
-    load_twl(twl, tw14, NT);
-    fill_stage_table<16, 32>(ttf, tw14, NT);
-    fill_stage_table<16, 16>(tti, tw14, NT);
-    const uint32_t N1 = g.N1, items = N1 >> 1;
-    const int tid = threadIdx.x;
-    // stage-1 butterfly of this thread: row (t >> 8), j = t & 255, inputs j + 256 r
-    const int s1seq = tid >> 8, s1j = tid & 255;
-
-    // Buffer loads: one 32-bit offset register per thread.  A 64-bit row pointer here was kept
-    // spilled, and its reload before the next item's request waited for the output stores.
-    auto s1_load = [&](const float2* __restrict__ src, uint32_t w, float2 (&v)[32]) {
-        const uint32_t row = s1seq ? ((w == 0) ? (N1 >> 1) : (N1 - w)) : w;
+    __shared__ float2 ttf[LG2 == 8 ? 1 : R1 * stage_row<16>()];  // forward middle stage (radix 16, span R1)
+    __shared__ float2 tti[LG2 == 8 ? 1 : 16 * stage_row<16>()];  // inverse middle stage (radix 16, span 16)
+    const uint32_t N1 = g.N1;
+    if (blockIdx.x == 0) {
+        scan_finish<NT>(info, g, ws, seed_ws, reinterpret_cast<uint32_t*>(buf));
+        return;
+    }
+    const uint32_t row = (blockIdx.x - 1u) * RPW + threadIdx.x / NTR;
+    const int j = threadIdx.x % NTR;
+    float2* seqbuf = buf + (threadIdx.x / NTR) * SEQS;
+    // buffer loads: one 32-bit offset register per thread
+    const uint32_t vrow = (row * N2 + (uint32_t)j) * 8u;
+    auto load = [&](const float2* __restrict__ src, float2 (&v)[PPT]) {
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, N1 * N2 * 8u);
-        const uint32_t vo = (row * N2 + (uint32_t)s1j) * 8u;
 #pragma unroll
-        for (int r = 0; r < 32; ++r) v[r] = buf_load_f2(rs, vo, 2048u * r);
+        for (int e = 0; e < PPT; ++e) v[e] = buf_load_f2(rs, vrow, (uint32_t)(8 * NTR * e));
     };
-    // forward stages 1 (inputs in v) .. 3; after stage 1 has consumed v, refill(v) requests the
-    // next transform's inputs into the same registers; ends with this thread's stage-3 outputs
-    auto forward = [&](float2 (&v)[32], const RowMap& m, float2 (&zA)[16], float2 (&zB)[16],
-                       auto&& refill) {
-        stage_first_to_lds<32>(v, buf + s1seq * SEQS, s1j);
-        refill(v);
+    float2 v[PPT];
+    load(MODE == ROWS_STATIC ? Yk : Sst, v);
+    load_twl(twl, tw14, NT);
+    if constexpr (LG2 != 8) {
+        fill_stage_table<16, R1>(ttf, tw14, NT);
+        fill_stage_table<16, 16>(tti, tw14, NT);
+    }
+    __syncthreads();  // tables
+    // forward stages 1 (inputs in v) .. 3; request() runs once stage 1 has consumed v
+    auto forward = [&](float2 (&z)[KL][16], auto&& request) {
+#pragma unroll
+        for (int i = 0; i < K1; ++i) {
+            float2 x[R1];
+#pragma unroll
+            for (int r = 0; r < R1; ++r) x[r] = v[i + K1 * r];
+            stage_first_to_lds<R1>(x, seqbuf, j + NTR * i);
+        }
+        request();
         __syncthreads();
-        stockham_stage<16, 32, ROW_LOG, 2, SEQS, NT, true>(buf, ttf);
-        stage_last_from_lds<16, N2>(zA, buf + m.sA * SEQS, m.jA, twl);
-        stage_last_from_lds<16, N2>(zB, buf + m.sB * SEQS, m.jB, twl);
+        if constexpr (LG2 != 8) stockham_stage<16, R1, LG2, RPW, SEQS, NT, true>(buf, ttf);
+#pragma unroll
+        for (int h = 0; h < KL; ++h) stage_last_from_lds<16, N2>(z[h], seqbuf, j + NTR * h, twl);
+        __syncthreads();  // stage-3 reads are done before LDS is overwritten
     };
-
-    uint32_t w = blockIdx.x;
-    if (w >= items) return;
-    // vmcnt retires in issue order, so a prefetch only overlaps work if no later-issued global
-    // load is waited on before the prefetched data is used: the small gathers of the next item
-    // (row twiddles) are issued and consumed before its prefetch.
-    RowMap m = row_map(w, N1, tid);
-    float2 wrA = tw_two_level(twlo, twhi, m.rowA), wrB = tw_two_level(twlo, twhi, m.rowB);
-    float2 pre[32];  // prefetched stage-1 inputs of the next transform
-    s1_load(MODE == ROWS_STATIC ? Yk : Sst, w, pre);
-    __syncthreads();  // twl
-
-    while (true) {
-        // split twiddles w_L^k at k = row + N1 (j + 512 r): w_L^row w_2^14^j w_32^r
-        const float2 baseA = cmul(wrA, tw_lds(twl, m.jA)), baseB = cmul(wrB, tw_lds(twl, m.jB));
-        auto wkA = [&](int r) { return w32pow(opaque_f2(baseA), r); };
-        auto wkB = [&](int r) { return w32pow(opaque_f2(baseB), r); };
-        const uint32_t wn = w + gridDim.x;
-        const bool more = wn < items;
-        RowMap mn = m;
-        float2 wrAn = wrA, wrBn = wrB;
-
-        float2 SA[16], SB[16];
-        float2 Sn = make_float2(0.f, 0.f);
-        if constexpr (MODE == ROWS_SEEDPREP || MODE == ROWS_DYN) {
-            float2 zA[16], zB[16];
-            // next request: the key rows of this item (DYN) or the seed rows of the next item
-            forward(pre, m, zA, zB, [&](float2 (&v)[32]) {
-                if (MODE == ROWS_DYN) s1_load(Yk, w, v);
-                else if (more) s1_load(Sst, wn, v);
-            });
-            if (!m.special) {
+    float2 S[KL][16];
+    if constexpr (MODE == ROWS_SEEDPREP || MODE == ROWS_DYN) {
+        forward(S, [&] {
+            if constexpr (MODE == ROWS_DYN) load(Yk, v);  // the key row, while the seed row is transformed
+        });
+        if constexpr (MODE == ROWS_SEEDPREP) {
+            // in place: every thread of the workgroup has consumed this row
 #pragma unroll
-                for (int r = 0; r < 16; ++r) r2c_split_pair(zA[r], zB[15 - r], wkA(r), SA[r], SB[15 - r]);
-            } else {
-                Sn = r2c_nyquist(zA[0]);
-                SA[0] = make_float2(0.f, 0.f);
-                SA[8] = r2c_split(zA[8], zA[8], wkA(8));
+            for (int h = 0; h < KL; ++h)
 #pragma unroll
-                for (int r = 1; r < 8; ++r) {
-                    SA[r] = r2c_split(zA[r], zA[16 - r], wkA(r));
-                    SA[16 - r] = r2c_split(zA[16 - r], zA[r], wkA(16 - r));
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) SB[r] = r2c_split(zB[r], zB[15 - r], wkB(r));
-            }
-            __syncthreads();  // stage-3 reads done before LDS is reused
-            if constexpr (MODE == ROWS_SEEDPREP) {
-                // in place: every thread of the workgroup has consumed these rows
-                if (more) {
-                    mn = row_map(wn, N1, tid);
-                    wrAn = tw_two_level(twlo, twhi, mn.rowA);
-                    wrBn = tw_two_level(twlo, twhi, mn.rowB);
-                }
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    st_nt(&Sst[(size_t)m.rowA * N2 + m.jA + 512 * r], SA[r]);
-                    st_nt(&Sst[(size_t)m.rowB * N2 + m.jB + 512 * r], SB[r]);
-                }
-                if (m.special) Sst[(size_t)N1 * N2] = Sn;
-                if (!more) break;
-                w = wn;
-                m = mn;
-                wrA = wrAn;
-                wrB = wrBn;
-                continue;
-            }
+                for (int r = 0; r < 16; ++r) st_nt(&Sst[(size_t)row * N2 + j + NTR * h + (N2 / 16) * r], S[h][r]);
+            return;
         }
-
-        // key rows: forward, split, product, inverse split -> conj(Q) at the same positions
-        float2 qA[16], qB[16];
-        {
-            float2 zA[16], zB[16];
-            forward(pre, m, zA, zB, [&](float2 (&)[32]) {
-                if constexpr (MODE == ROWS_STATIC) {
-                    // the resident spectrum of this item is requested now, used after the FFT
+    }
+    float2 z[KL][16];
+    forward(z, [&] {
+        if constexpr (MODE == ROWS_STATIC) {
+            // the resident spectrum is requested now, used after the FFT
+            const __amdgpu_buffer_rsrc_t rs = make_rsrc(Sst, N1 * N2 * 8u);
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        SA[r] = Sst[(size_t)m.rowA * N2 + m.jA + 512 * r];
-                        SB[r] = Sst[(size_t)m.rowB * N2 + m.jB + 512 * r];
-                    }
-                    if (m.special) Sn = Sst[(size_t)N1 * N2];
-                }
-            });
-            auto unit = [&](float2 za, float2 zb, float2 sa, float2 sb, float2 wa, float2 wb, float2& qa,
-                            float2& qb) {
-                const float2 pa = cmul(r2c_split(za, zb, wa), sa);
-                const float2 pb = cmul(r2c_split(zb, za, wb), sb);
-                qa = conjf2(c2r_split(pa, pb, wa));
-                qb = conjf2(c2r_split(pb, pa, wb));
-            };
-            if (!m.special) {
-                // partner pairs (A r, B 15-r): k and N-k, one twiddle for both
+            for (int h = 0; h < KL; ++h)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float2 w = wkA(r);
-                    float2 xa, xb, ua, ub;
-                    r2c_split_pair(zA[r], zB[15 - r], w, xa, xb);
-                    c2r_split_pair(cmul(xa, SA[r]), cmul(xb, SB[15 - r]), w, ua, ub);
-                    qA[r] = conjf2(ua);
-                    qB[15 - r] = conjf2(ub);
-                }
-            } else {
-                const float2 pn = cmul(r2c_nyquist(zA[0]), Sn);
-                qA[0] = conjf2(c2r_split(make_float2(0.f, 0.f), pn, make_float2(1.f, 0.f)));
-                {
-                    const float2 w8 = wkA(8);
-                    const float2 p8 = cmul(r2c_split(zA[8], zA[8], w8), SA[8]);
-                    qA[8] = conjf2(c2r_split(p8, p8, w8));
-                }
-#pragma unroll
-                for (int r = 1; r < 8; ++r)
-                    unit(zA[r], zA[16 - r], SA[r], SA[16 - r], wkA(r), wkA(16 - r), qA[r], qA[16 - r]);
-#pragma unroll
-                for (int r = 0; r < 8; ++r)
-                    unit(zB[r], zB[15 - r], SB[r], SB[15 - r], wkB(r), wkB(15 - r), qB[r], qB[15 - r]);
-            }
+                for (int r = 0; r < 16; ++r) S[h][r] = buf_load_f2(rs, vrow, (uint32_t)(8 * NTR * h + (N2 / 2) * r));
         }
-        __syncthreads();  // all forward stage-3 reads are done before LDS is overwritten
-        stage_first_to_lds<16>(qA, buf + m.sA * SEQS, m.jA);
-        stage_first_to_lds<16>(qB, buf + m.sB * SEQS, m.jB);
-        __syncthreads();
-        stockham_stage<16, 16, ROW_LOG, 2, SEQS, NT, true>(buf, tti);
-        {
-            float2 F[32];
-            stage_last_from_lds<32, N2>(F, buf + s1seq * SEQS, s1j, twl);
-            // R'[row][t2] = F[t2] w_N^{t2 row}, t2 = j + 256 r:  w_L^{2 row j} * w_L^{512 row r}
-            const uint32_t row = s1seq ? m.row1 : m.row0;
-            const float2 base = tw_two_level(twlo, twhi, (2u * row * (uint32_t)s1j) & (g.L - 1u));
-            const float2 step = tw_two_level(twlo, twhi, (512u * row) & (g.L - 1u));
-            float2 anchor[3];
+    });
 #pragma unroll
-            for (int a = 0; a < 3; ++a)
-                anchor[a] = tw_two_level(twlo, twhi, (512u * row * (uint32_t)(8 * (a + 1))) & (g.L - 1u));
-            if (more) {
-                mn = row_map(wn, N1, tid);
-                wrAn = tw_two_level(twlo, twhi, mn.rowA);
-                wrBn = tw_two_level(twlo, twhi, mn.rowB);
-            }
-            float2 tw = base;
-            if (rt_tiled(g.lg1)) {
-                // tiles: pair w, side s1seq, t2 = s1j + 256 r -> tile row t2 / RT_COLS = s1j / RT_COLS
-                // + (256 / RT_COLS) r, one scalar offset per r
-                const __amdgpu_buffer_rsrc_t ro = make_rsrc(Rt, N1 * N2 * 8u);
-                const uint32_t vo = ((((uint32_t)s1j / RT_COLS) * (N1 >> 1) + w) * (2u * RT_COLS) +
-                                     (uint32_t)s1seq * RT_COLS + ((uint32_t)s1j % RT_COLS)) * 8u;
-                const uint32_t rstep = (256u / RT_COLS) * (N1 >> 1) * (2u * RT_COLS) * 8u;  // t2 -> t2 + 256
+    for (int h = 0; h < KL; ++h) {
 #pragma unroll
-                for (int r = 0; r < 32; ++r) {
-                    if ((r & 7) == 0 && r) tw = cmul(base, anchor[r / 8 - 1]);
-                    buf_store_nt(cmul(F[r], tw), ro, vo, (uint32_t)r * rstep);
-                    tw = cmul(tw, step);
-                }
-            } else {
-                float2* op = Yk + (size_t)row * N2 + s1j;
+        for (int r = 0; r < 16; ++r) z[h][r] = conjf2(cmul(z[h][r], S[h][r]));
+        stage_first_to_lds<16>(z[h], seqbuf, j + NTR * h);
+    }
+    __syncthreads();
+    if constexpr (LG2 != 8) stockham_stage<16, 16, LG2, RPW, SEQS, NT, true>(buf, tti);
+    float2 F[PPT];
 #pragma unroll
-                for (int r = 0; r < 32; ++r) {
-                    if ((r & 7) == 0 && r)  // re-anchor every 8 steps to bound the recurrence error
-                        tw = cmul(base, anchor[r / 8 - 1]);
-                    st_nt(&op[256 * r], cmul(F[r], tw));
-                    tw = cmul(tw, step);
-                }
-            }
-        }
-        __syncthreads();  // stage-3 reads done before the next item writes LDS
-        if (!more) break;
-        // next request: the first operand of the next item (issued here rather than during the
-        // inverse transform, whose registers are full)
-        s1_load(MODE == ROWS_STATIC ? Yk : Sst, wn, pre);
-        w = wn;
-        m = mn;
-        wrA = wrAn;
-        wrB = wrBn;
+    for (int i = 0; i < K1; ++i) {
+        float2 x[R1];
+        stage_last_from_lds<R1, N2>(x, seqbuf, j + NTR * i, twl);
+#pragma unroll
+        for (int r = 0; r < R1; ++r) F[i + K1 * r] = x[r];
+    }
+    // R'[row][t2] = F[t2] w_2L^{t2 (4 row + 1)}, t2 = j + NTR e: base step^e, re-anchored every 8
+    // steps to bound the recurrence error
+    const uint32_t L2m = 2u * g.L - 1u, f = 4u * row + 1u;
+    const float2 base = tw_two_level(twlo, twhi, (f * (uint32_t)j) & L2m);
+    const float2 step = tw_two_level(twlo, twhi, (f * (uint32_t)NTR) & L2m);
+    float2 anchor[PPT / 8 - 1];
+#pragma unroll
+    for (int a = 0; a < PPT / 8 - 1; ++a)
+        anchor[a] = tw_two_level(twlo, twhi, (f * (uint32_t)(NTR * 8 * (a + 1))) & L2m);
+    // tiled (N2 = 8192): t2 = j + 256 e -> tile row t2 / RT_COLS = j / RT_COLS + (256 / RT_COLS) e, one
+    // scalar offset per e; row-major: in place
+    const bool tiled = LG2 == 13 && rt_tiled(g.lg1);
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(tiled ? Rt : Yk, N1 * N2 * 8u);
+    const uint32_t vo = tiled ? ((((uint32_t)j / RT_COLS) * N1 + row) * RT_COLS + ((uint32_t)j % RT_COLS)) * 8u : vrow;
+    const uint32_t estep = tiled ? (256u / RT_COLS) * N1 * RT_COLS * 8u : (uint32_t)(8 * NTR);  // e -> e + 1
+    float2 tw = base;
+#pragma unroll
+    for (int e = 0; e < PPT; ++e) {
+        if ((e & 7) == 0 && e) tw = cmul(base, anchor[e / 8 - 1]);
+        buf_store_nt(cmul(F[e], tw), ro, vo, (uint32_t)e * estep);
+        tw = cmul(tw, step);
     }
 }
 
 // ------------------------------------------------------------------ pass A' ----
-// Workgroup grp owns columns [W*grp, W*grp + W): G[t1] = FFT_N1(R'[.][t2])[t1] = conj of the
-// unnormalised inverse, so c[2t] = Re G / N and c[2t+1] = -Im G / N at t = t2 + N2*t1.  R' is
-// row-major, or pass B's tiles when rt_tiled(LG1).
-// Writes one nibble (4 conv bits, MSB first) per (column pair, t1) inside the output window, in
-// column-pair-major order nibT[pair * N1 + t1] so that each workgroup's writes are contiguous.
+// Workgroup grp owns columns [W*grp, W*grp + W): G[t1] = FFT_N1(R'[.][t2])[t1] w_4N1^{t1}, so that the
+// conv values of positions t = t2 + N2 t1 and t + N are Re G / N and Im G / N.  R' is row-major, or pass
+// B's tiles when rt_tiled(LG1).
+// Rounding: conv - mean_half(column) is an integer; its parity, corrected by the prefix parities (in
+// the output stage), is the product's bit.
+// A thread holds the outputs t1 = j + (N1/16) e, e < 16, of a column, so their bits are one 16-bit
+// piece, bit e: piece[(half N2 + t2) N1/16 + j], half 0 for the positions t and 1 for t + N, each half
+// only where the output window touches it.
+struct InvOut {
+    uint32_t lo, len;        // output window in conv positions
+    uint32_t N, N2, S;       // S = N1 / 16
+    uint16_t* piece;
+    float* margin;
+    __device__ __forceinline__ InvOut(const Geom& g, uint8_t* nib, uint32_t S_, float* margin_)
+        : lo(g.out_off), len(g.out_bits), N(g.N), N2(g.N2), S(S_), piece(reinterpret_cast<uint16_t*>(nib)),
+          margin(margin_) {}
+    __device__ __forceinline__ bool low() const { return lo < N; }
+    __device__ __forceinline__ bool high() const { return lo + len > N; }
+};
+// The 16-bit piece of half h from X[e] w_64^e (times the caller's scale: conv + i conv'): rounding by the
+// 1.5 2^23 trick, whose last mantissa bit is the parity.  dist: max |v - rint v| inside the window.
+template <bool HIGH, bool DIST>
+__device__ __forceinline__ uint32_t inv_piece(const float2 (&X)[16], float mean, const InvOut& o, uint32_t t2, uint32_t j,
+                                              float& dist) {
+    constexpr float MAGIC = 12582912.f;
+    const uint32_t i0 = t2 + o.N2 * j + (HIGH ? o.N : 0u) - o.lo;
+    uint32_t acc = 0;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const float2 w = w64pow(make_float2(1.f, 0.f), e);  // cos, -sin: constants
+        const float v = HIGH ? fmaf(X[e].y, w.x, fmaf(X[e].x, w.y, -mean)) : fmaf(X[e].x, w.x, fmaf(X[e].y, -w.y, -mean));
+        const float t = v + MAGIC;
+        acc = __builtin_amdgcn_alignbit(__float_as_uint(t), acc, 1);
+        if constexpr (DIST) {
+            const float d = fabsf(v - (t - MAGIC));
+            dist = fmaxf(dist, i0 + o.N2 * o.S * (uint32_t)e < o.len ? d : 0.f);
+        }
+    }
+    return acc >> 16;
+}
+__device__ __forceinline__ void inv_store(const float2 (&X)[16], float mean, const InvOut& o, uint32_t t2, uint32_t j,
+                                          float& dist) {
+    uint16_t* p = o.piece + (size_t)t2 * o.S + j;
+    const size_t plane = (size_t)o.N2 * o.S;
+    if (o.margin) {
+        if (o.low()) p[0] = (uint16_t)inv_piece<false, true>(X, mean, o, t2, j, dist);
+        if (o.high()) p[plane] = (uint16_t)inv_piece<true, true>(X, mean, o, t2, j, dist);
+    } else {
+        if (o.low()) p[0] = (uint16_t)inv_piece<false, false>(X, mean, o, t2, j, dist);
+        if (o.high()) p[plane] = (uint16_t)inv_piece<true, false>(X, mean, o, t2, j, dist);
+    }
+}
 template <int LG1, bool BATCH>
 __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_LG1 ? 2 : 1) void k_inv_cols(
-    const float2* __restrict__ Rp, uint8_t* __restrict__ nibT, Geom g,
-    const uint32_t* __restrict__ wk_cnt, const uint32_t* __restrict__ ws_cnt,
+    const float2* __restrict__ Rp, uint8_t* __restrict__ nib, Geom g, const uint32_t* __restrict__ info,
     const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
     float* __restrict__ margin, const BlockArgs* __restrict__ bt) {
     if constexpr (BATCH) {
         const BlockArgs& a = bt[blockIdx.z];
         g = a.g;
         Rp = rt_tiled(LG1) ? a.Rt : a.Yk;
-        nibT = a.nib;
-        wk_cnt = a.counts;
-        ws_cnt = a.seed ? a.counts + POP_SLOTS : a.ws;
+        nib = a.nib;
+        info = a.info;
         margin = a.margin;
     }
     constexpr int N1 = 1 << LG1;
@@ -806,101 +942,69 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
     constexpr int LGL = LG1 < 14 ? LG1 : 14;  // LDS transform length (N1 = 2^15: two halves)
     constexpr int SEQS = seq_stride(1 << LGL);
     constexpr int WL = (LG1 == RT_LG1 || LG1 >= 14) ? 1 : W;  // columns held in LDS at once
+    constexpr int S = N1 / 16;
     __shared__ float2 buf[WL * SEQS];
     __shared__ float2 twl[TWL_SIZE];
     load_twl(twl, tw14, NT);
     const uint32_t grp = xcd_logical(blockIdx.x, gridDim.x);
+    const InvOut out(g, nib, S, margin);
+    float dist = 0.f;
+    // w_4N1^{j} / N from the length-2L table (2L = 4 N1 N2)
+    auto out_tw = [&](uint32_t j) { return cscale(tw_two_level(twlo, twhi, j * g.N2), g.inv_N); };
     if constexpr (LG1 == 14) {
         // Column pair t2 = 2 grp, 2 grp + 1 per 1024-thread workgroup, one column in LDS at a time
         // (one workgroup per CU).  Thread j loads both columns of row k1 = j + 1024 r from pass B's
-        // tiles with one 16-byte load (side 0 of pair k1 for k1 < N1/2, side 1 of pair N1 - k1
-        // after).  The first column's bits wait packed in a register (2 per t1 = j + 1024 q) for the
-        // second's; the output is one nibble per (column pair, t1).
-        static_assert(W == 2 && NT == 1024 && rt_tiled(LG1), "paired column pass expects 2 columns, 1024 threads");
-        constexpr int PT = N1 / NT;
+        // tiles with one 16-byte load.
+        static_assert(W == 2 && NT == 1024 && rt_tiled(LG1) && S == NT, "paired column pass expects 2 columns, 1024 threads");
         const int j = threadIdx.x;
-        float2 v0[PT], v1[PT];
+        float2 v0[16], v1[16];
         const uint32_t c0 = grp * W;
         {
-            const float2* tp = Rp + (size_t)(c0 / RT_COLS) * (N1 / 2) * (2 * RT_COLS) + (c0 % RT_COLS);
+            const float2* tp = Rp + (size_t)(c0 / RT_COLS) * N1 * RT_COLS + (c0 % RT_COLS);
 #pragma unroll
-            for (int r = 0; r < PT; ++r) {
-                const uint32_t k1 = (uint32_t)j + (uint32_t)NT * r;
-                const uint32_t pr = r < PT / 2 ? k1 : (((uint32_t)N1 - k1) & ((uint32_t)N1 / 2 - 1));
-                const float4 x = *reinterpret_cast<const float4*>(tp + (size_t)pr * (2 * RT_COLS) + (r < PT / 2 ? 0 : RT_COLS));
+            for (int r = 0; r < 16; ++r) {
+                const float4 x = *reinterpret_cast<const float4*>(tp + (size_t)(j + NT * r) * RT_COLS);
                 v0[r] = make_float2(x.x, x.y);
                 v1[r] = make_float2(x.z, x.w);
             }
         }
-        const float corr = correction(pop_total(wk_cnt), pop_total(ws_cnt), g.L);
-        const float invN = g.inv_N;
-        float dist = 0.f;
-        auto inwin = [&](uint32_t t1) {
-            const uint32_t i0 = 2u * (c0 + g.N2 * t1);
-            return !(i0 + 4u <= g.out_off || i0 >= g.out_off + g.out_bits);
-        };
+        const uint32_t pops = info[INFO_POPS];
+        const float2 wb = out_tw((uint32_t)j);
         __syncthreads();  // twl
 #pragma unroll
-        for (int r = 0; r < PT; ++r) buf[padi(j + NT * r)] = v0[r];
+        for (int r = 0; r < 16; ++r) buf[padi(j + NT * r)] = v0[r];
         __syncthreads();
         lds_fft<LG1, 1, SEQS, NT>(buf, twl);
-        uint32_t lo = 0u;
 #pragma unroll
-        for (int q = 0; q < PT; ++q) {
-            const uint32_t t1 = (uint32_t)j + (uint32_t)NT * q;
-            if (!inwin(t1)) continue;
-            const float2 G = buf[padi((int)t1)];
-            const uint32_t b0 = round_bit(G.x * invN + corr, dist);
-            const uint32_t b1 = round_bit(-G.y * invN + corr, dist);
-            lo |= ((b0 << 1) | b1) << (2 * q);
-        }
+        for (int e = 0; e < 16; ++e) v0[e] = cmul(buf[padi(j + S * e)], wb);
+        inv_store(v0, mean_half(pops, c0), out, c0, (uint32_t)j, dist);
         __syncthreads();  // the first column's reads are done
 #pragma unroll
-        for (int r = 0; r < PT; ++r) buf[padi(j + NT * r)] = v1[r];
+        for (int r = 0; r < 16; ++r) buf[padi(j + NT * r)] = v1[r];
         __syncthreads();
         lds_fft<LG1, 1, SEQS, NT>(buf, twl);
 #pragma unroll
-        for (int q = 0; q < PT; ++q) {
-            const uint32_t t1 = (uint32_t)j + (uint32_t)NT * q;
-            if (!inwin(t1)) continue;
-            const float2 G = buf[padi((int)t1)];
-            const uint32_t b2 = round_bit(G.x * invN + corr, dist);
-            const uint32_t b3 = round_bit(-G.y * invN + corr, dist);
-            st_nt_u8(&nibT[(size_t)grp * N1 + t1], (uint8_t)((((lo >> (2 * q)) & 3u) << 2) | (b2 << 1) | b3));
-        }
-        if (margin) margin_publish(dist, margin);
-        return;
+        for (int e = 0; e < 16; ++e) v1[e] = cmul(buf[padi(j + S * e)], wb);
+        inv_store(v1, mean_half(pops, c0 + 1u), out, c0 + 1u, (uint32_t)j, dist);
     } else if constexpr (LG1 >= 14) {
-        // One column t2 = grp per workgroup; output one 2-bit crumb per t1 at nibT[t2 * N1 + t1]
-        // (bits c[2t], c[2t+1] of t = t2 + N2 t1).  N1 = 2^15 splits the column first by one
-        // radix-2 step in registers (X[2k] = FFT(a)[k], X[2k+1] = FFT(b)[k] with a = x[j] + x[j+N1/2],
+        // One column t2 = grp per workgroup.  N1 = 2^15 splits the column first by one radix-2 step in
+        // registers (X[2k] = FFT(a)[k], X[2k+1] = FFT(b)[k] with a = x[j] + x[j+N1/2],
         // b = (x[j] - x[j+N1/2]) w_N1^j), then transforms the two 2^14-point halves in turn.
-        static_assert(W == 1 && NT == 1024, "single-column pass expects 1024 threads");
+        static_assert(W == 1 && NT == 1024 && rt_tiled(LG1), "single-column pass expects 1024 threads");
         constexpr int H = 1 << LGL;       // points per LDS transform
-        constexpr int PT = N1 / NT;       // values per thread (16 or 32)
+        constexpr int PT = N1 / NT;       // values per thread (32)
+        static_assert(N1 == 2 * H && S == 2 * NT, "two halves");
         const uint32_t t2 = grp;
-        const float corr = correction(pop_total(wk_cnt), pop_total(ws_cnt), g.L);
-        const float invN = g.inv_N;
-        float dist = 0.f;
+        const float mean = mean_half(info[INFO_POPS], t2);
         float2 v[PT];
-        if constexpr (rt_tiled(LG1)) {
-            // pass B's tiles: rows k1 < N1/2 are side 0 of pair k1, the others side 1 of pair
-            // (N1 - k1) mod N1/2, so consecutive threads read consecutive tile lines
-            const float2* tp = Rp + (size_t)(t2 / RT_COLS) * (N1 / 2) * (2 * RT_COLS) + (t2 % RT_COLS);
+        {
+            const float2* tp = Rp + (size_t)(t2 / RT_COLS) * N1 * RT_COLS + (t2 % RT_COLS);
 #pragma unroll
-            for (int r = 0; r < PT; ++r) {
-                const uint32_t k1 = threadIdx.x + (uint32_t)NT * r;
-                const uint32_t pr = r < PT / 2 ? k1 : (((uint32_t)N1 - k1) & ((uint32_t)N1 / 2 - 1));
-                v[r] = tp[(size_t)pr * (2 * RT_COLS) + (r < PT / 2 ? 0 : RT_COLS)];
-            }
-        } else {
-#pragma unroll
-            for (int r = 0; r < PT; ++r) v[r] = Rp[(size_t)(threadIdx.x + NT * r) * g.N2 + t2];
+            for (int r = 0; r < PT; ++r) v[r] = tp[(size_t)(threadIdx.x + NT * r) * RT_COLS];
         }
         __syncthreads();  // twl
-        constexpr int HALVES = N1 / H;
-        if constexpr (HALVES == 2) {
-            const uint32_t step = g.L / (uint32_t)N1;
+        {
+            const uint32_t step = 2u * g.L / (uint32_t)N1;
 #pragma unroll
             for (int r = 0; r < PT / 2; ++r) {
                 const float2 x0 = v[r], x1 = v[r + PT / 2];
@@ -909,204 +1013,263 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
             }
         }
 #pragma unroll
-        for (int hv = 0; hv < HALVES; ++hv) {
+        for (int hv = 0; hv < 2; ++hv) {
 #pragma unroll
             for (int r = 0; r < H / NT; ++r) buf[padi(threadIdx.x + NT * r)] = v[hv * (H / NT) + r];
             __syncthreads();
             lds_fft<LGL, 1, SEQS, NT>(buf, twl);
-            for (int k = threadIdx.x; k < H; k += NT) {
-                const uint32_t t1 = (uint32_t)(k * HALVES + hv);
-                const uint32_t i0 = 2u * (t2 + g.N2 * t1);
-                if (i0 + 2u <= g.out_off || i0 >= g.out_off + g.out_bits) continue;
-                const float2 G = buf[padi(k)];
-                const uint32_t b0 = round_bit(G.x * invN + corr, dist);
-                const uint32_t b1 = round_bit(-G.y * invN + corr, dist);
-                st_nt_u8(&nibT[(size_t)t2 * N1 + t1], (uint8_t)((b0 << 1) | b1));
-            }
+            // t1 = 2 (tid + 1024 e) + hv
+            const uint32_t j = 2u * threadIdx.x + (uint32_t)hv;
+            const float2 wb = out_tw(j);
+            float2 X[16];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) X[e] = cmul(buf[padi((int)threadIdx.x + NT * e)], wb);
+            inv_store(X, mean, out, t2, j, dist);
             __syncthreads();  // reads done before the next half is written
         }
-        if (margin) margin_publish(dist, margin);
-        return;
-    } else {
-    if constexpr (LG1 == RT_LG1) {
+    } else if constexpr (LG1 == RT_LG1) {
         // One column pair t2 = 2 grp, 2 grp + 1 from pass B's tiles per 256-thread workgroup, one
-        // column in LDS at a time (74 KB), so that two workgroups share a compute unit and one's
+        // column in LDS at a time (72 KB), so that two workgroups share a compute unit and one's
         // reads overlap the other's transforms.  Thread j loads both columns of row k1 = j + 256 r
-        // with one 16-byte load: rows k1 < N1/2 are side 0 of pair k1, the others side 1 of pair
-        // (N1 - k1) mod N1/2, so a workgroup walks consecutive lines.  Plan 32 x 16 x 16 per
+        // with one 16-byte load, so a workgroup walks consecutive lines.  Plan 32 x 16 x 16 per
         // column: stage 1 from the loaded registers, stage 2 in LDS, stage 3 into registers for
-        // butterflies b = j and j + 256 (t1 = b + 512 r).  The first column's bits wait packed in
-        // registers (2 per t1) for the second's.
+        // butterflies b = j and j + 256 (t1 = b + 512 r), w_4N1^b / N in its first level.
+        // What bounds it is the L1 refill: 16 of each line's 128 bytes per workgroup, 8 times the
+        // data in lines; the loads alone take 0.205 ms at 2^27, the transforms alone 0.14.
         static_assert(W == 2 && NT == 256, "tiled column pass expects 2 columns, 256 threads");
         static_assert(RT_COLS % W == 0, "a workgroup's columns lie in one tile");
-        __shared__ float2 ttf[32 * 17];
+        __shared__ float2 ttf[32 * stage_row<16>()];
         fill_stage_table<16, 32>(ttf, tw14, NT);
         const int j = threadIdx.x;
+        const uint32_t t2 = grp * W;
         float2 v0[32], v1[32];
         {
-            const uint32_t c0 = grp * W;
-            const float2* tp = Rp + (size_t)(c0 / RT_COLS) * (N1 / 2) * (2 * RT_COLS) + (c0 % RT_COLS);
+            const float2* tp = Rp + (size_t)(t2 / RT_COLS) * N1 * RT_COLS + (t2 % RT_COLS);
 #pragma unroll
             for (int r = 0; r < 32; ++r) {
-                const uint32_t k1 = (uint32_t)j + 256u * r;
-                const uint32_t pr = r < 16 ? k1 : ((N1 - k1) & (N1 / 2 - 1));
-                const float4 x = *reinterpret_cast<const float4*>(tp + (size_t)pr * (2 * RT_COLS) + (r < 16 ? 0 : RT_COLS));
+                const float4 x = *reinterpret_cast<const float4*>(tp + (size_t)(j + 256 * r) * RT_COLS);
                 v0[r] = make_float2(x.x, x.y);
                 v1[r] = make_float2(x.z, x.w);
             }
         }
-        const float corr = correction(pop_total(wk_cnt), pop_total(ws_cnt), g.L);
-        const float invN = g.inv_N;
-        float dist = 0.f;
-        const uint32_t t2 = grp * W;
-        auto inwin = [&](uint32_t t1) {
-            const uint32_t i0 = 2u * (t2 + g.N2 * t1);
-            return !(i0 + 4u <= g.out_off || i0 >= g.out_off + g.out_bits);
+        const uint32_t pops = info[INFO_POPS];
+        const float2 wb[2] = {out_tw((uint32_t)j), out_tw((uint32_t)j + 256u)};
+        auto column = [&](float2 (&v)[32], uint32_t col) {
+            stage_first_to_lds<32>(v, buf, j);
+            __syncthreads();
+            stockham_stage<16, 32, LG1, 1, SEQS, NT, true>(buf, ttf);
+            const float mean = mean_half(pops, col);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float2 G[16], tw[8];
+                const int b = j + 256 * h;
+                stage_last_read<16, N1>(G, buf, b);
+                twiddle_set_lds<16>(tw, twl, b * (TW14 / N1));
+                tw[0] = cmul(tw[0], wb[h]);
+#pragma unroll
+                for (int r = 0; r < 8; ++r) G[r] = cmul(G[r], wb[h]);
+                dft_tw<16>(G, tw);
+                inv_store(G, mean, out, col, (uint32_t)b, dist);
+            }
         };
         __syncthreads();  // twl, ttf
-        stage_first_to_lds<32>(v0, buf, j);
-        __syncthreads();
-        stockham_stage<16, 32, LG1, 1, SEQS, NT, true>(buf, ttf);
-        uint32_t lo[2] = {0u, 0u};
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float2 G[16];
-            const int bf = j + 256 * h;
-            stage_last_from_lds<16, N1>(G, buf, bf, twl);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                if (!inwin((uint32_t)bf + 512u * r)) continue;
-                const uint32_t b0 = round_bit(G[r].x * invN + corr, dist);
-                const uint32_t b1 = round_bit(-G[r].y * invN + corr, dist);
-                lo[h] |= ((b0 << 1) | b1) << (2 * r);
-            }
-        }
+        column(v0, t2);
         __syncthreads();  // the first column's stage-3 reads are done
-        stage_first_to_lds<32>(v1, buf, j);
-        __syncthreads();
-        stockham_stage<16, 32, LG1, 1, SEQS, NT, true>(buf, ttf);
+        column(v1, t2 + 1u);
+    } else {
+        constexpr int LPT = (W * N1 + NT - 1) / NT;
+        static_assert(W * S == NT, "one piece per thread");
+        float2 v[LPT];
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            float2 G[16];
-            const int bf = j + 256 * h;
-            stage_last_from_lds<16, N1>(G, buf, bf, twl);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const uint32_t t1 = (uint32_t)bf + 512u * r;
-                if (!inwin(t1)) continue;
-                const uint32_t b2 = round_bit(G[r].x * invN + corr, dist);
-                const uint32_t b3 = round_bit(-G[r].y * invN + corr, dist);
-                st_nt_u8(&nibT[(size_t)grp * N1 + t1], (uint8_t)((((lo[h] >> (2 * r)) & 3u) << 2) | (b2 << 1) | b3));
-            }
-        }
-        if (margin) margin_publish(dist, margin);
-        return;
-    }
-    constexpr int LPT = (W * N1 + NT - 1) / NT;
-    float2 v[LPT];
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-        const int e = threadIdx.x + i * NT;
-        if (e < W * N1) {
+        for (int i = 0; i < LPT; ++i) {
+            const int e = threadIdx.x + i * NT;
             const uint32_t k1 = (uint32_t)(e / W), t2 = grp * W + (uint32_t)(e % W);
-            if constexpr (rt_tiled(LG1)) {  // pass B's tiles: side 0 of pair k1, or side 1 of N1 - k1
-                const uint32_t pr = k1 < (uint32_t)N1 / 2 ? k1 : (((uint32_t)N1 - k1) & ((uint32_t)N1 / 2 - 1));
-                const uint32_t sd = k1 < (uint32_t)N1 / 2 ? 0u : 1u;
-                v[i] = Rp[((size_t)(t2 / RT_COLS) * (N1 / 2) + pr) * (2 * RT_COLS) + sd * RT_COLS + t2 % RT_COLS];
+            if constexpr (rt_tiled(LG1)) {  // pass B's tiles
+                v[i] = Rp[((size_t)(t2 / RT_COLS) * N1 + k1) * RT_COLS + t2 % RT_COLS];
             } else {
                 v[i] = Rp[(size_t)k1 * g.N2 + t2];
             }
         }
-    }
 #pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-        const int e = threadIdx.x + i * NT;
-        if (e < W * N1) buf[(e % W) * SEQS + padi(e / W)] = v[i];
-    }
-    __syncthreads();
-    lds_fft<LG1, W, SEQS, NT>(buf, twl);
-    const float corr = correction(pop_total(wk_cnt), pop_total(ws_cnt), g.L);
-    const float invN = g.inv_N;
-    float dist = 0.f;
-    constexpr int P = W / 2;
-    // the output window [out_off, out_off + out_bits) as a t1 range for this pair of columns
-    for (int e = threadIdx.x; e < P * N1; e += NT) {
-        const int p = e / N1, t1 = e % N1;
-        const uint32_t t2 = grp * W + 2u * (uint32_t)p;
-        const uint32_t i0 = 2u * (t2 + g.N2 * (uint32_t)t1);
-        if (i0 + 4u <= g.out_off || i0 >= g.out_off + g.out_bits) continue;
-        const float2 G0 = buf[(2 * p) * SEQS + padi(t1)];
-        const float2 G1 = buf[(2 * p + 1) * SEQS + padi(t1)];
-        const uint32_t b0 = round_bit(G0.x * invN + corr, dist);
-        const uint32_t b1 = round_bit(-G0.y * invN + corr, dist);
-        const uint32_t b2 = round_bit(G1.x * invN + corr, dist);
-        const uint32_t b3 = round_bit(-G1.y * invN + corr, dist);
-        nibT[(size_t)(grp * P + (uint32_t)p) * N1 + (uint32_t)t1] = (uint8_t)((b0 << 3) | (b1 << 2) | (b2 << 1) | b3);
+        for (int i = 0; i < LPT; ++i) {
+            const int e = threadIdx.x + i * NT;
+            buf[(e % W) * SEQS + padi(e / W)] = v[i];
+        }
+        __syncthreads();
+        lds_fft<LG1, W, SEQS, NT>(buf, twl);
+        const int col = threadIdx.x / S, j = threadIdx.x % S;
+        const float2 wb = out_tw((uint32_t)j);
+        float2 X[16];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) X[e] = cmul(buf[col * SEQS + padi(j + S * e)], wb);
+        const uint32_t t2 = grp * W + (uint32_t)col;
+        inv_store(X, mean_half(info[INFO_POPS], t2), out, t2, (uint32_t)j, dist);
     }
     if (margin) margin_publish(dist, margin);
-    }
 }
 
 // ------------------------------------------------------------------ output ----
-// The conv bit stream in nibbles: nibble q (bits 4q..4q+3) is nibT[(q mod P2) * N1 + q / P2] with
-// P2 = N2/2 column pairs.  A workgroup transposes a tile of PACK_T1 rows x PACK_G pairs through
-// LDS and writes the output words whose 8 nibbles lie in the tile: conv bits
-// [out_off + 32w, +32), XOR key_rest word w ((key[h/32+w] << 1) | (key[h/32+w+1] >> 31),
-// key2StartRest PrivacyAmplification.cu:873-878), byte-swapped for the OutBytes layout
-// (ToBinaryArray, PrivacyAmplification.cu:757-762).
-// CRUMB: pass A' wrote one 2-bit crumb per column, crumb[t2 * N1 + t1]; the nibble of pair p is
-// crumb[2p] << 2 | crumb[2p + 1].
-// zero_counts (single-block form): the popcount partials, which no later stage of this block
-// reads, are cleared for the next block on the stream.
-template <bool BATCH, bool CRUMB>
-__global__ __launch_bounds__(256) void k_pack(const uint8_t* __restrict__ nibT,
-                                              const uint32_t* __restrict__ key,
-                                              uint32_t* __restrict__ out, Geom g,
-                                              const BlockArgs* __restrict__ bt,
-                                              uint32_t* __restrict__ zero_counts) {
-    if (!BATCH && zero_counts && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x < 2 * POP_SLOTS)
-        zero_counts[threadIdx.x] = 0u;
-    __shared__ uint8_t tile[PACK_T1][PACK_G + 4];
-    if constexpr (BATCH) {  // grid.y covers the largest window of the launch; rows past this
-        const BlockArgs& a = bt[blockIdx.z];  // block's window load nothing and store nothing
+// The correction of conv word w, MSB first: the prefix parities (q and its chunk's cp), the
+// whitening's word and key_rest word wo = w - out_off / 32 ((key[h/32+wo] << 1) | (key[h/32+wo+1] >> 31),
+// key2StartRest PrivacyAmplification.cu:873-878).  No load is conditional on a lane, so that a thread
+// with several words has all their operands in flight.
+__device__ __forceinline__ uint32_t out_correction(uint32_t w, uint32_t wo, const Geom& g, const uint32_t* __restrict__ q,
+                                                   const uint32_t* __restrict__ info, uint32_t white,
+                                                   const uint32_t* __restrict__ key) {
+    uint32_t c = q[w] ^ (0u - (uint32_t)scan_parities(info, g)[w >> (10u + g.scan)]) ^ white;
+    if (g.do_xor) {
+        const bool in = 32u * wo < g.m;
+        const uint32_t k = g.key_hw + (in ? wo : 0u);
+        const uint32_t r = (key[k] << 1) | (key[k + 1] >> 31);
+        c ^= in ? r : 0u;
+    }
+    return c;
+}
+// Pieces (pass A') to output words.  Thread (cw, jp) of a tile of 16 column words x 8 piece pairs takes
+// the 32 columns of word cw at rows t1 = j + (N1/16) e, j = 2 jp and 2 jp + 1: a 32 x 32 bit matrix, one
+// word per column, transposed in registers to one word per row; through LDS the tile's 256 rows are
+// then written as whole 64-byte runs, corrected and byte-swapped for the OutBytes layout
+// (ToBinaryArray, PrivacyAmplification.cu:757-762), eight rows' operands in flight per thread.
+template <bool BATCH>
+__global__ __launch_bounds__(PACK_NT) void k_pack(const uint8_t* __restrict__ nib, const uint32_t* __restrict__ key,
+                                                  uint32_t* __restrict__ out, Geom g, const uint32_t* __restrict__ info,
+                                                  const uint32_t* __restrict__ q, const BlockArgs* __restrict__ bt) {
+    static_assert(PACK_CW * 8 == PACK_NT, "a thread per word column and piece pair");
+    __shared__ uint32_t tile[256 * (PACK_CW + 1)];
+    if constexpr (BATCH) {  // grid.y covers the most halves of the launch
+        const BlockArgs& a = bt[blockIdx.z];
         g = a.g;
-        nibT = a.nib;
+        nib = a.nib;
         key = a.key;
         out = a.out;
+        info = a.info;
+        q = a.q;
     }
-    const uint32_t P2 = g.N2 >> 1;
-    const uint32_t q_lo = g.out_off >> 2, q_hi = (g.out_off + g.out_bits) >> 2;
-    const uint32_t row0 = ((q_lo / P2) & ~3u) + blockIdx.y * PACK_T1;  // 4-aligned for 32-bit reads
-    const uint32_t g0 = blockIdx.x * PACK_G;
-    // load: PACK_G pairs x PACK_T1 rows, 4 rows per 32-bit read
-    for (uint32_t e = threadIdx.x; e < PACK_G * (PACK_T1 / 4); e += 256) {
-        const uint32_t gp = e / (PACK_T1 / 4), r4 = (e % (PACK_T1 / 4)) * 4;
-        const uint32_t row = row0 + r4;
-        uint32_t v = 0;
-        if constexpr (CRUMB) {
-            if (row < g.N1) {
-                const uint32_t ve = *reinterpret_cast<const uint32_t*>(nibT + (size_t)(2u * (g0 + gp)) * g.N1 + row);
-                const uint32_t vo = *reinterpret_cast<const uint32_t*>(nibT + (size_t)(2u * (g0 + gp) + 1u) * g.N1 + row);
-                v = ((ve & 0x03030303u) << 2) | (vo & 0x03030303u);
+    const uint32_t S = g.N1 >> 4, per_half = S / 16u;
+    const uint32_t w_lo = g.out_off >> 5, w_hi = (g.out_off + g.out_bits) >> 5;
+    const uint32_t half = blockIdx.y / per_half + (g.out_off < g.N ? 0u : 1u);
+    if (half > 1u || (half == 1u && 32u * w_hi <= g.N)) return;
+    const uint32_t jl = threadIdx.x & 7u, cl = threadIdx.x >> 3;
+    const uint32_t jp0 = (blockIdx.y % per_half) * 8u, c0 = blockIdx.x * PACK_CW;
+    {
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(nib) +
+                            ((size_t)half * g.N2 + 32u * (c0 + cl)) * (S / 2u) + jp0 + jl;
+        uint32_t A[32];
+#pragma unroll
+        for (int k = 0; k < 32; ++k) A[k] = p[(size_t)k * (S / 2u)];
+        bit_transpose(A);  // A[31 - b]: bit b of every column, first column in the MSB
+#pragma unroll
+        for (int b = 0; b < 32; ++b) tile[(b * 8 + jl) * (PACK_CW + 1) + cl] = A[31 - b];
+    }
+    const uint32_t white = info[INFO_WHITE];
+    __syncthreads();
+    const uint32_t lane = threadIdx.x % PACK_CW;
+    const uint8_t* cp = scan_parities(info, g);
+    for (uint32_t r0 = threadIdx.x / PACK_CW; r0 < 256u; r0 += 64u) {
+        // the operands of out_correction for eight words, requested together
+        uint32_t w[8], c[8], flip[8], k0[8], k1[8];
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t r = r0 + 8u * k, b = r >> 3, t1 = 2u * (jp0 + (r & 7u)) + (b >> 4) + S * (b & 15u);
+            w[k] = (half * g.N1 + t1) * (g.N2 >> 5) + c0 + lane;  // conv word
+            const uint32_t wc = w[k] >= w_lo && w[k] < w_hi ? w[k] : w_lo;
+            c[k] = q[wc];
+            flip[k] = cp[wc >> (10u + g.scan)];
+        }
+        if (g.do_xor) {
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k) {
+                const uint32_t wo = w[k] - w_lo, i = g.key_hw + (32u * wo < g.m && w[k] >= w_lo ? wo : 0u);
+                k0[k] = key[i];
+                k1[k] = key[i + 1];
             }
-        } else {
-            if (row < g.N1) v = *reinterpret_cast<const uint32_t*>(nibT + (size_t)(g0 + gp) * g.N1 + row);
         }
 #pragma unroll
-        for (int k = 0; k < 4; ++k) tile[r4 + k][gp] = (uint8_t)(v >> (8 * k));
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t wo = w[k] - w_lo;
+            uint32_t cw = tile[(r0 + 8u * k) * (PACK_CW + 1) + lane] ^ c[k] ^ (0u - flip[k]) ^ white;
+            if (g.do_xor && 32u * wo < g.m) cw ^= (k0[k] << 1) | (k1[k] >> 31);
+            if (w[k] >= w_lo && w[k] < w_hi) out[wo] = g.reverse_endian ? __builtin_bswap32(cw) : cw;
+        }
     }
-    __syncthreads();
-    for (uint32_t e = threadIdx.x; e < PACK_T1 * (PACK_G / 8); e += 256) {
-        const uint32_t r = e / (PACK_G / 8), gw = (e % (PACK_G / 8)) * 8;
-        const uint32_t q = (row0 + r) * P2 + g0 + gw;
-        if (q < q_lo || q >= q_hi) continue;
-        const uint32_t w = (q - q_lo) >> 3;
-        uint32_t cw = 0;
+}
+
+// Pass A' and the output in one for L <= 2^22: 16 columns per workgroup, plan R1 x 16 (R1 x 32 at 512).
+// A wave's 64 lanes are 16 columns x 4 rows, so a ballot is 4 rows' 16 bits: half an output word
+// each, corrected and written as 16 bits.
+template <int LG1, bool BATCH>
+__global__ __launch_bounds__(mid_threads(LG1)) void k_mid_inv(const float2* __restrict__ Rp, const uint32_t* __restrict__ key,
+                                                              uint32_t* __restrict__ out, Geom g,
+                                                              const uint32_t* __restrict__ info,
+                                                              const uint32_t* __restrict__ q,
+                                                              const float2* __restrict__ tw14,
+                                                              float* __restrict__ margin,
+                                                              const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) {
+        const BlockArgs& a = bt[blockIdx.z];
+        g = a.g;
+        Rp = a.Yk;
+        key = a.key;
+        out = a.out;
+        info = a.info;
+        q = a.q;
+        margin = a.margin;
+    }
+    constexpr int N1 = 1 << LG1, NT = mid_threads(LG1), R1 = mid_r1(LG1), R2 = N1 / R1, S1 = N1 / R1;
+    constexpr int K1 = 16 * S1 / NT, SEQS = seq_stride(N1);
+    __shared__ float2 buf[16 * SEQS];
+    __shared__ float2 tab[R1 * stage_row<R2>()];
+    __shared__ float2 tq[N1];  // w_4N1^{t1} / N
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    const uint32_t grp = blockIdx.x, t2 = 16u * grp + (uint32_t)col;
+    float2 v[K1][R1];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) cw |= ((uint32_t)tile[r][gw + j] & 0xFu) << (28 - 4 * j);
-        if (g.do_xor && 32u * w < g.m) cw ^= (key[g.key_hw + w] << 1) | (key[g.key_hw + w + 1] >> 31);
-        out[w] = g.reverse_endian ? __builtin_bswap32(cw) : cw;
+    for (int i = 0; i < K1; ++i)
+#pragma unroll
+        for (int r = 0; r < R1; ++r) v[i][r] = Rp[(size_t)(jt + (NT / 16) * i + S1 * r) * g.N2 + t2];
+    fill_stage_table<R2, R1>(tab, tw14, NT);
+    for (int e = threadIdx.x; e < N1; e += NT) tq[e] = cscale(tw14[e * (TW14 / (4 * N1))], g.inv_N);
+    const uint32_t pops = info[INFO_POPS], white = info[INFO_WHITE];
+#pragma unroll
+    for (int i = 0; i < K1; ++i) stage_first_to_lds<R1>(v[i], buf + col * SEQS, jt + (NT / 16) * i);
+    __syncthreads();
+    float2 G[R2];
+    stage_last_from_lds_tab<R2, N1>(G, buf + col * SEQS, jt, tab + jt * stage_row<R2>());
+    const float mean = mean_half(pops, t2);
+    const uint32_t RW = g.N2 >> 5, w_lo = g.out_off >> 5, w_hi = (g.out_off + g.out_bits) >> 5;
+    const uint32_t lane = threadIdx.x & 63u, sh = (grp & 1u) ? 0u : 16u;
+    float dist = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        if (half == 0 ? g.out_off >= g.N : 32u * w_hi <= g.N) continue;
+#pragma unroll
+        for (int p = 0; p < R2 / 16; ++p) {
+            uint32_t mine = 0;  // the 16 bits of row jt + R1 (16 p + col)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t t1 = (uint32_t)jt + (uint32_t)(R1 * (16 * p + e));
+                const float2 X = G[16 * p + e], w = tq[t1];
+                const float val = half == 0 ? fmaf(X.x, w.x, fmaf(-X.y, w.y, -mean)) : fmaf(X.x, w.y, fmaf(X.y, w.x, -mean));
+                float d = 0.f;
+                const uint64_t b = __ballot(round_bit(val, d) != 0u);
+                const uint32_t pos = t2 + g.N2 * t1 + (half ? g.N : 0u) - g.out_off;
+                dist = fmaxf(dist, pos < g.out_bits ? d : 0.f);
+                const uint32_t word = (lane & 32u) ? (uint32_t)(b >> 32) : (uint32_t)b;
+                mine = col == e ? word >> (lane & 16u) : mine;
+            }
+            const uint32_t R = (uint32_t)(half * N1 + jt + R1 * (16 * p + col));
+            const uint32_t w = R * RW + (grp >> 1);
+            if (w >= w_lo && w < w_hi) {
+                const uint32_t wo = w - w_lo;
+                // bit i of `mine` is column i: MSB first after the reversal
+                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, white, key) >> sh) & 0xFFFFu);
+                uint16_t* o = reinterpret_cast<uint16_t*>(out + wo);
+                if (g.reverse_endian) o[grp & 1u] = (uint16_t)((c16 >> 8) | (c16 << 8));
+                else o[(grp & 1u) ^ 1u] = (uint16_t)c16;
+            }
+        }
     }
+    if (margin) margin_publish(dist, margin);
 }
 
 // ------------------------------------------------------------------ small path ----
@@ -1325,39 +1488,105 @@ hipError_t launch_split_finish(const uint32_t* acc, const uint32_t* key, uint32_
 
 // ================================================================== launchers ====
 namespace {
-template <int LGM, int D>
-hipError_t launch_fwd_cols_t(const uint32_t* tb, float2* Y, const Geom& g, const Tables& t, hipStream_t s,
-                             const uint32_t* tb2, float2* Y2) {
-    if constexpr (LGM == 9) {
-        // Each workgroup holds one class of one operand and walks `per` column groups: 16 (8 for a
-        // single operand), fewer while that would leave under 256 (512) workgroups per operand.
-        // 1024 workgroups at 2^27, two waves of two per CU: as fast as one persistent wave, and a
-        // CU that cannot take its second workgroup at once delays a short walk, not a long one.
-        const uint32_t groups = g.N2 / 16u, target = Y2 ? 256u : 512u;
-        uint32_t per = Y2 ? 16u : 8u;
-        while (per > 1u && groups * (uint32_t)D / per < target) per >>= 1;
-        const uint32_t G = groups * (uint32_t)D / per;  // groups = 512 and per divides it
-        k_fwd_cols9p<D, false><<<dim3(G, Y2 ? 2 : 1), FWD_NT, 0, s>>>(tb, Y, g, t.tw14, t.lo, t.hi, t.cls, tb2, Y2,
-                                                                     per, nullptr, 0);
-    } else {
-        const uint32_t grid = (g.N2 / (uint32_t)fwd_cols_width(LGM)) * (uint32_t)D;
-        k_fwd_cols<LGM, D, false><<<dim3(grid, Y2 ? 2 : 1), fwd_cols_threads(LGM), 0, s>>>(tb, Y, g, t.tw14, t.lo, t.hi, t.cls,
-                                                                        nullptr, 0, tb2, Y2);
+// f(std::integral_constant<int, lg>) for the mid-size column lengths, row lengths and the others.
+template <typename F>
+hipError_t by_mid_lg1(uint32_t lg1, F&& f) {
+    switch (lg1) {
+    case 6: return f(std::integral_constant<int, 6>());
+    case 7: return f(std::integral_constant<int, 7>());
+    case 8: return f(std::integral_constant<int, 8>());
+    case 9: return f(std::integral_constant<int, 9>());
+    case 10: return f(std::integral_constant<int, 10>());
+    default: return hipErrorInvalidValue;
     }
-    return hipGetLastError();
 }
-template <int LG1>
-hipError_t launch_inv_cols_t(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* wk,
-                             const uint32_t* ws, const Tables& t, float* margin, hipStream_t s) {
-    const uint32_t grid = g.N2 / (uint32_t)inv_cols_width(LG1);
-    k_inv_cols<LG1, false><<<grid, inv_cols_threads(LG1), 0, s>>>(R, nib, g, wk, ws, t.tw14, t.lo, t.hi, margin, nullptr);
-    return hipGetLastError();
+template <typename F>
+hipError_t by_lg2(uint32_t lg2, F&& f) {
+    switch (lg2) {
+    case 8: return f(std::integral_constant<int, 8>());
+    case 9: return f(std::integral_constant<int, 9>());
+    case 10: return f(std::integral_constant<int, 10>());
+    case 11: return f(std::integral_constant<int, 11>());
+    case 12: return f(std::integral_constant<int, 12>());
+    case 13: return f(std::integral_constant<int, 13>());
+    default: return hipErrorInvalidValue;
+    }
 }
-template <int D>
-hipError_t launch_transpose_t(const uint32_t* bits, uint32_t* tb, uint32_t* count, const Geom& g,
-                              int is_seed, hipStream_t s, const uint32_t* bits2, uint32_t* tb2) {
-    const dim3 grid(g.M << (ROW_LOG - TB_SPAN_LOG), bits2 ? 2 : 1);
-    k_transpose_bits<D, false><<<grid, TB_NT, 0, s>>>(bits, tb, count, g, is_seed, nullptr, bits2, tb2);
+template <typename F>
+hipError_t by_lg1(uint32_t lg1, F&& f) {
+    switch (lg1) {
+    case 11: return f(std::integral_constant<int, 11>());
+    case 12: return f(std::integral_constant<int, 12>());
+    case 13: return f(std::integral_constant<int, 13>());
+    case 14: return f(std::integral_constant<int, 14>());
+    case 15: return f(std::integral_constant<int, 15>());
+    default: return hipErrorInvalidValue;
+    }
+}
+
+// Pass A of `count` blocks (bt, BATCH) or one (a); per: see launch_batch_fwd_cols.
+template <bool BATCH>
+hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uint32_t scan_wgs, const BlockArgs* bt,
+                    uint32_t count, hipStream_t s) {
+    if (mid_size(g))
+        return by_mid_lg1(g.lg1, [&](auto lg) {
+            constexpr int LG1 = decltype(lg)::value;
+            a.nA = g.N2 / 16u;
+            k_mid_fwd<LG1, BATCH><<<dim3(a.nA * a.ops + scan_wgs, 1, count), mid_threads(LG1), 0, s>>>(
+                a, g, t.tw14, t.lo, t.hi, bt);
+            return hipGetLastError();
+        });
+    return by_lg1(g.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value, D = LG1 >= 13 ? 16 : 1 << (LG1 - 9);
+        if constexpr (LG1 <= 13) {
+            a.nA = g.N2 / 16u * (uint32_t)D / per;  // N2 / 16 = 512 groups and per divides it
+            k_fwd_cols9p<D, BATCH><<<dim3(a.nA * a.ops, 1, count), FWD_NT, 0, s>>>(a, g, t.tw14, t.lo, t.hi,
+                                                                                            t.cls, per, bt);
+        } else {
+            constexpr int LGM = LG1 - 4;
+            a.nA = g.N2 / (uint32_t)fwd_cols_width(LGM) * (uint32_t)D;
+            k_fwd_cols<LGM, D, BATCH><<<dim3(a.nA * a.ops, 1, count), fwd_cols_threads(LGM), 0, s>>>(
+                a, g, t.tw14, t.lo, t.hi, t.cls, bt);
+        }
+        return hipGetLastError();
+    });
+}
+template <bool BATCH>
+hipError_t rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, uint32_t* info,
+                const uint32_t* ws, uint32_t* seed_ws, const BlockArgs* bt, uint32_t count, hipStream_t s) {
+    return by_lg2(g.lg2, [&](auto lg) {
+        constexpr int LG2 = decltype(lg)::value, NT = rows_threads(LG2);
+        const dim3 grid(g.N1 / (uint32_t)rows_per_wg(LG2) + 1u, 1, count);  // + scan_finish
+        switch (mode) {
+        case ROWS_STATIC:
+            k_rows<LG2, ROWS_STATIC, BATCH><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+            break;
+        case ROWS_DYN:
+            k_rows<LG2, ROWS_DYN, BATCH><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+            break;
+        case ROWS_SEEDPREP:
+            if constexpr (!BATCH) {
+                k_rows<LG2, ROWS_SEEDPREP, false><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+                break;
+            }
+            [[fallthrough]];
+        default: return hipErrorInvalidValue;
+        }
+        return hipGetLastError();
+    });
+}
+template <bool BATCH>
+hipError_t transpose(const uint32_t* key, const uint32_t* seed, uint32_t* tbk, uint32_t* tbs, uint32_t first, uint32_t ops,
+                     const Geom& g, const ScanArgs* scan, uint32_t scan_wgs, const BlockArgs* bt, uint32_t count,
+                     hipStream_t s) {
+    const dim3 grid(scan_wgs + ops * (g.M << (ROW_LOG - TB_SPAN_LOG)), 1, count);
+    const ScanArgs sc = scan ? *scan : ScanArgs{};
+    switch (g.D) {
+    case 4: k_transpose_bits<4, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
+    case 8: k_transpose_bits<8, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
+    case 16: k_transpose_bits<16, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
+    default: return hipErrorInvalidValue;
+    }
     return hipGetLastError();
 }
 template <int LGN>
@@ -1372,6 +1601,12 @@ hipError_t launch_small_t(const uint32_t* key, const uint32_t* seed, const float
                                                                    margin, sspec_out, ws_out, nullptr);
     return hipGetLastError();
 }
+template <int LGN>
+hipError_t batch_small_t(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
+    k_small<LGN, false, true><<<dim3(1, 1, count), small_threads(LGN), 0, s>>>(
+        nullptr, nullptr, nullptr, nullptr, nullptr, g0, t.tw14, nullptr, nullptr, nullptr, bt);
+    return hipGetLastError();
+}
 }  // namespace
 
 hipError_t launch_copies(const CopyDesc* d, uint32_t count, uint64_t max_bytes, hipStream_t s) {
@@ -1382,89 +1617,59 @@ hipError_t launch_copies(const CopyDesc* d, uint32_t count, uint64_t max_bytes, 
     return hipGetLastError();
 }
 
-hipError_t launch_zero_u32(uint32_t* p, uint32_t count, hipStream_t s) {
-    k_zero_u32<false><<<1, 256, 0, s>>>(p, count, nullptr);
+hipError_t launch_transpose(const uint32_t* key, const uint32_t* seed, uint32_t* tbk, uint32_t* tbs, uint32_t first,
+                            uint32_t ops, const Geom& g, const ScanArgs* scan, hipStream_t s) {
+    return transpose<false>(key, seed, tbk, tbs, first, ops, g, scan, scan ? scan_chunks(g) : 0u, nullptr, 1, s);
+}
+
+hipError_t launch_fwd_cols(const uint32_t* key_in, const uint32_t* seed_in, float2* Yk, float2* Ys, uint32_t first,
+                           uint32_t ops, const Geom& g, const Tables& t, const ScanArgs* scan, hipStream_t s) {
+    // The persistent form: each workgroup holds one class of one operand and walks `per` column
+    // groups: 16 (8 for a single operand), fewer while that would leave under 256 (512) workgroups
+    // per operand.  1024 workgroups at 2^27, two waves of two per CU: as fast as one persistent
+    // wave, and a CU that cannot take its second workgroup at once delays a short walk, not a long one.
+    const uint32_t target = ops == 2u ? 256u : 512u;
+    uint32_t per = ops == 2u ? 16u : 8u;
+    while (per > 1u && g.N2 / 16u * g.D / per < target) per >>= 1;
+    FwdArgs a{{key_in, seed_in}, {Yk, Ys}, first, ops, 0u, scan ? *scan : ScanArgs{}};
+    return fwd_cols<false>(a, g, t, per, scan ? scan_chunks(g) : 0u, nullptr, 1, s);
+}
+
+hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, uint32_t* info,
+                       const uint32_t* ws, uint32_t* seed_ws, hipStream_t s) {
+    return rows<false>(mode, Yk, S, Rt, g, t, info, ws, seed_ws, nullptr, 1, s);
+}
+
+hipError_t launch_prefix_apply(uint32_t* q, const uint32_t* info, const Geom& g, hipStream_t s) {
+    k_prefix_apply<<<g.L / 32u / 256u, 256, 0, s>>>(q, info, g);
     return hipGetLastError();
 }
 
-hipError_t launch_transpose(const uint32_t* bits, uint32_t* tb, uint32_t* count, const Geom& g,
-                            int is_seed, hipStream_t s, const uint32_t* bits2, uint32_t* tb2) {
-    switch (g.D) {
-    case 1: return launch_transpose_t<1>(bits, tb, count, g, is_seed, s, bits2, tb2);
-    case 2: return launch_transpose_t<2>(bits, tb, count, g, is_seed, s, bits2, tb2);
-    case 4: return launch_transpose_t<4>(bits, tb, count, g, is_seed, s, bits2, tb2);
-    case 8: return launch_transpose_t<8>(bits, tb, count, g, is_seed, s, bits2, tb2);
-    case 16: return launch_transpose_t<16>(bits, tb, count, g, is_seed, s, bits2, tb2);
-    default: return hipErrorInvalidValue;
-    }
+hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
+                           float* margin, hipStream_t s) {
+    return by_lg1(g.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value;
+        k_inv_cols<LG1, false><<<g.N2 / (uint32_t)inv_cols_width(LG1), inv_cols_threads(LG1), 0, s>>>(
+            R, nib, g, info, t.tw14, t.lo, t.hi, margin, nullptr);
+        return hipGetLastError();
+    });
 }
 
-hipError_t launch_fwd_cols(const uint32_t* tb, float2* Y, const Geom& g, const Tables& t, hipStream_t s,
-                           const uint32_t* tb2, float2* Y2) {
-    switch (g.lg1) {
-    case 1: return launch_fwd_cols_t<1, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 2: return launch_fwd_cols_t<2, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 3: return launch_fwd_cols_t<3, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 4: return launch_fwd_cols_t<4, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 5: return launch_fwd_cols_t<5, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 6: return launch_fwd_cols_t<6, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 7: return launch_fwd_cols_t<7, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 8: return launch_fwd_cols_t<8, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 9: return launch_fwd_cols_t<9, 1>(tb, Y, g, t, s, tb2, Y2);
-    case 10: return launch_fwd_cols_t<9, 2>(tb, Y, g, t, s, tb2, Y2);
-    case 11: return launch_fwd_cols_t<9, 4>(tb, Y, g, t, s, tb2, Y2);
-    case 12: return launch_fwd_cols_t<9, 8>(tb, Y, g, t, s, tb2, Y2);
-    case 13: return launch_fwd_cols_t<9, 16>(tb, Y, g, t, s, tb2, Y2);
-    case 14: return launch_fwd_cols_t<10, 16>(tb, Y, g, t, s, tb2, Y2);
-    case 15: return launch_fwd_cols_t<11, 16>(tb, Y, g, t, s, tb2, Y2);
-    default: return hipErrorInvalidValue;
-    }
-}
+uint32_t pack_halves(const Geom& g) { return (g.out_off < g.N ? 1u : 0u) + (g.out_off + g.out_bits > g.N ? 1u : 0u); }
 
-hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, int cus,
-                       hipStream_t s) {
-    const uint32_t items = g.N1 / 2u;
-    const uint32_t grid = items < (uint32_t)cus ? items : (uint32_t)cus;  // one workgroup per CU
-    switch (mode) {
-    case ROWS_STATIC: k_rows<ROWS_STATIC, false><<<grid, ROWS_NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, nullptr); break;
-    case ROWS_DYN: k_rows<ROWS_DYN, false><<<grid, ROWS_NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, nullptr); break;
-    case ROWS_SEEDPREP: k_rows<ROWS_SEEDPREP, false><<<grid, ROWS_NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, nullptr); break;
-    default: return hipErrorInvalidValue;
-    }
+hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
+                       const uint32_t* q, hipStream_t s) {
+    k_pack<false><<<dim3(g.N2 / 32u / PACK_CW, g.N1 / 256u * pack_halves(g)), PACK_NT, 0, s>>>(nib, key, out, g, info, q, nullptr);
     return hipGetLastError();
 }
 
-hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* wk,
-                           const uint32_t* ws, const Tables& t, float* margin, hipStream_t s) {
-    switch (g.lg1) {
-    case 1: return launch_inv_cols_t<1>(R, nib, g, wk, ws, t, margin, s);
-    case 2: return launch_inv_cols_t<2>(R, nib, g, wk, ws, t, margin, s);
-    case 3: return launch_inv_cols_t<3>(R, nib, g, wk, ws, t, margin, s);
-    case 4: return launch_inv_cols_t<4>(R, nib, g, wk, ws, t, margin, s);
-    case 5: return launch_inv_cols_t<5>(R, nib, g, wk, ws, t, margin, s);
-    case 6: return launch_inv_cols_t<6>(R, nib, g, wk, ws, t, margin, s);
-    case 7: return launch_inv_cols_t<7>(R, nib, g, wk, ws, t, margin, s);
-    case 8: return launch_inv_cols_t<8>(R, nib, g, wk, ws, t, margin, s);
-    case 9: return launch_inv_cols_t<9>(R, nib, g, wk, ws, t, margin, s);
-    case 10: return launch_inv_cols_t<10>(R, nib, g, wk, ws, t, margin, s);
-    case 11: return launch_inv_cols_t<11>(R, nib, g, wk, ws, t, margin, s);
-    case 12: return launch_inv_cols_t<12>(R, nib, g, wk, ws, t, margin, s);
-    case 13: return launch_inv_cols_t<13>(R, nib, g, wk, ws, t, margin, s);
-    case 14: return launch_inv_cols_t<14>(R, nib, g, wk, ws, t, margin, s);
-    case 15: return launch_inv_cols_t<15>(R, nib, g, wk, ws, t, margin, s);
-    default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_pack(const uint8_t* nibT, const uint32_t* key, uint32_t* out, const Geom& g, hipStream_t s,
-                       uint32_t* zero_counts) {
-    const uint32_t P2 = g.N2 >> 1;
-    const uint32_t q_lo = g.out_off >> 2, q_hi = (g.out_off + g.out_bits) >> 2;
-    const uint32_t rows = (q_hi - 1u) / P2 - ((q_lo / P2) & ~3u) + 1u;
-    dim3 grid(P2 / PACK_G, (rows + PACK_T1 - 1u) / PACK_T1);
-    if (g.W == 1) k_pack<false, true><<<grid, 256, 0, s>>>(nibT, key, out, g, nullptr, zero_counts);
-    else k_pack<false, false><<<grid, 256, 0, s>>>(nibT, key, out, g, nullptr, zero_counts);
-    return hipGetLastError();
+hipError_t launch_mid_inv(const float2* R, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
+                          const uint32_t* q, const Tables& t, float* margin, hipStream_t s) {
+    return by_mid_lg1(g.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value;
+        k_mid_inv<LG1, false><<<g.N2 / 16u, mid_threads(LG1), 0, s>>>(R, key, out, g, info, q, t.tw14, margin, nullptr);
+        return hipGetLastError();
+    });
 }
 
 hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2* sspec,
@@ -1487,133 +1692,50 @@ hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2*
 // ---------------------------------------------------------------- batched launchers ----
 // `count` blocks of one transform length; block b's geometry and buffers are bt[b] (device
 // memory) and g0 is any block's geometry (only its L-derived fields are used here).
-uint32_t pack_tiles(const Geom& g) {
-    const uint32_t P2 = g.N2 >> 1;
-    const uint32_t q_lo = g.out_off >> 2, q_hi = (g.out_off + g.out_bits) >> 2;
-    const uint32_t rows = (q_hi - 1u) / P2 - ((q_lo / P2) & ~3u) + 1u;
-    return (rows + PACK_T1 - 1u) / PACK_T1;
+hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t ops, hipStream_t s) {
+    return transpose<true>(nullptr, nullptr, nullptr, nullptr, 0u, ops, g0, nullptr, scan_chunks(g0), bt, count, s);
 }
 
-hipError_t launch_batch_zero(const BlockArgs* bt, uint32_t count, hipStream_t s) {
-    k_zero_u32<true><<<dim3(1, 1, count), 256, 0, s>>>(nullptr, 2 * POP_SLOTS, bt);
-    return hipGetLastError();
-}
-
-namespace {
-template <int D>
-hipError_t batch_transpose_t(const BlockArgs* bt, uint32_t count, const Geom& g0, int is_seed, hipStream_t s) {
-    k_transpose_bits<D, true><<<dim3(g0.M << (ROW_LOG - TB_SPAN_LOG), 1, count), TB_NT, 0, s>>>(
-        nullptr, nullptr, nullptr, g0, is_seed, bt, nullptr, nullptr);
-    return hipGetLastError();
-}
-template <int LGM, int D>
-hipError_t batch_fwd_cols_t(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, int is_seed,
-                            uint32_t per, hipStream_t s) {
-    if constexpr (LGM == 9) {
-        // one class per workgroup walking `per` column groups (a power of two dividing the N2 / 16
-        // groups); by default 16, fewer while the launch would have under 512 workgroups
-        const uint32_t groups = g0.N2 / 16u;
-        if (per == 0u) {
-            per = 16u;
-            while (per > 1u && groups * (uint32_t)D / per * count < 512u) per >>= 1;
-        }
-        if (per > FWD_PER_MAX || (per & (per - 1u)) != 0u || groups % per != 0u) return hipErrorInvalidValue;
-        const uint32_t G = groups * (uint32_t)D / per;
-        k_fwd_cols9p<D, true><<<dim3(G, 1, count), FWD_NT, 0, s>>>(nullptr, nullptr, g0, t.tw14, t.lo, t.hi, t.cls,
-                                                                  nullptr, nullptr, per, bt, is_seed);
-    } else {
-        k_fwd_cols<LGM, D, true><<<dim3((g0.N2 / (uint32_t)fwd_cols_width(LGM)) * (uint32_t)D, 1, count),
-                                   fwd_cols_threads(LGM), 0,
-                                   s>>>(nullptr, nullptr, g0, t.tw14, t.lo, t.hi, t.cls, bt, is_seed, nullptr, nullptr);
-    }
-    return hipGetLastError();
-}
-template <int LG1>
-hipError_t batch_inv_cols_t(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
-    k_inv_cols<LG1, true><<<dim3(g0.N2 / (uint32_t)inv_cols_width(LG1), 1, count), inv_cols_threads(LG1), 0, s>>>(
-        nullptr, nullptr, g0, nullptr, nullptr, t.tw14, t.lo, t.hi, nullptr, bt);
-    return hipGetLastError();
-}
-template <int LGN>
-hipError_t batch_small_t(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
-    k_small<LGN, false, true><<<dim3(1, 1, count), small_threads(LGN), 0, s>>>(
-        nullptr, nullptr, nullptr, nullptr, nullptr, g0, t.tw14, nullptr, nullptr, nullptr, bt);
-    return hipGetLastError();
-}
-}  // namespace
-
-hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geom& g0, int is_seed, hipStream_t s) {
-    switch (g0.D) {
-    case 1: return batch_transpose_t<1>(bt, count, g0, is_seed, s);
-    case 2: return batch_transpose_t<2>(bt, count, g0, is_seed, s);
-    case 4: return batch_transpose_t<4>(bt, count, g0, is_seed, s);
-    case 8: return batch_transpose_t<8>(bt, count, g0, is_seed, s);
-    case 16: return batch_transpose_t<16>(bt, count, g0, is_seed, s);
-    default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, int is_seed,
+hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, uint32_t ops,
                                  uint32_t per, hipStream_t s) {
-    switch (g0.lg1) {
-    case 1: return batch_fwd_cols_t<1, 1>(bt, count, g0, t, is_seed, per, s);
-    case 2: return batch_fwd_cols_t<2, 1>(bt, count, g0, t, is_seed, per, s);
-    case 3: return batch_fwd_cols_t<3, 1>(bt, count, g0, t, is_seed, per, s);
-    case 4: return batch_fwd_cols_t<4, 1>(bt, count, g0, t, is_seed, per, s);
-    case 5: return batch_fwd_cols_t<5, 1>(bt, count, g0, t, is_seed, per, s);
-    case 6: return batch_fwd_cols_t<6, 1>(bt, count, g0, t, is_seed, per, s);
-    case 7: return batch_fwd_cols_t<7, 1>(bt, count, g0, t, is_seed, per, s);
-    case 8: return batch_fwd_cols_t<8, 1>(bt, count, g0, t, is_seed, per, s);
-    case 9: return batch_fwd_cols_t<9, 1>(bt, count, g0, t, is_seed, per, s);
-    case 10: return batch_fwd_cols_t<9, 2>(bt, count, g0, t, is_seed, per, s);
-    case 11: return batch_fwd_cols_t<9, 4>(bt, count, g0, t, is_seed, per, s);
-    case 12: return batch_fwd_cols_t<9, 8>(bt, count, g0, t, is_seed, per, s);
-    case 13: return batch_fwd_cols_t<9, 16>(bt, count, g0, t, is_seed, per, s);
-    case 14: return batch_fwd_cols_t<10, 16>(bt, count, g0, t, is_seed, per, s);
-    case 15: return batch_fwd_cols_t<11, 16>(bt, count, g0, t, is_seed, per, s);
-    default: return hipErrorInvalidValue;
+    const uint32_t groups = g0.N2 / 16u;
+    if (per == 0u) {
+        per = 16u;
+        while (per > 1u && groups * g0.D / per * count * ops < 512u) per >>= 1;
     }
+    if (per > FWD_PER_MAX || (per & (per - 1u)) != 0u || (!mid_size(g0) && groups % per != 0u)) return hipErrorInvalidValue;
+    FwdArgs a{};
+    a.ops = ops;
+    return fwd_cols<true>(a, g0, t, per, scan_chunks(g0), bt, count, s);
 }
 
 hipError_t launch_batch_rows(int mode, const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t,
-                             uint32_t grid_x, hipStream_t s) {
-    const uint32_t items = g0.N1 / 2u;
-    if (grid_x == 0 || grid_x > items) grid_x = items;
-    const dim3 grid(grid_x, 1, count);
-    switch (mode) {
-    case ROWS_STATIC: k_rows<ROWS_STATIC, true><<<grid, ROWS_NT, 0, s>>>(nullptr, nullptr, nullptr, g0, t.tw14, t.lo, t.hi, bt); break;
-    case ROWS_DYN: k_rows<ROWS_DYN, true><<<grid, ROWS_NT, 0, s>>>(nullptr, nullptr, nullptr, g0, t.tw14, t.lo, t.hi, bt); break;
-    default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+                             hipStream_t s) {
+    return rows<true>(mode, nullptr, nullptr, nullptr, g0, t, nullptr, nullptr, nullptr, bt, count, s);
 }
 
 hipError_t launch_batch_inv_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
-    switch (g0.lg1) {
-    case 1: return batch_inv_cols_t<1>(bt, count, g0, t, s);
-    case 2: return batch_inv_cols_t<2>(bt, count, g0, t, s);
-    case 3: return batch_inv_cols_t<3>(bt, count, g0, t, s);
-    case 4: return batch_inv_cols_t<4>(bt, count, g0, t, s);
-    case 5: return batch_inv_cols_t<5>(bt, count, g0, t, s);
-    case 6: return batch_inv_cols_t<6>(bt, count, g0, t, s);
-    case 7: return batch_inv_cols_t<7>(bt, count, g0, t, s);
-    case 8: return batch_inv_cols_t<8>(bt, count, g0, t, s);
-    case 9: return batch_inv_cols_t<9>(bt, count, g0, t, s);
-    case 10: return batch_inv_cols_t<10>(bt, count, g0, t, s);
-    case 11: return batch_inv_cols_t<11>(bt, count, g0, t, s);
-    case 12: return batch_inv_cols_t<12>(bt, count, g0, t, s);
-    case 13: return batch_inv_cols_t<13>(bt, count, g0, t, s);
-    case 14: return batch_inv_cols_t<14>(bt, count, g0, t, s);
-    case 15: return batch_inv_cols_t<15>(bt, count, g0, t, s);
-    default: return hipErrorInvalidValue;
-    }
+    return by_lg1(g0.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value;
+        k_inv_cols<LG1, true><<<dim3(g0.N2 / (uint32_t)inv_cols_width(LG1), 1, count), inv_cols_threads(LG1), 0, s>>>(
+            nullptr, nullptr, g0, nullptr, t.tw14, t.lo, t.hi, nullptr, bt);
+        return hipGetLastError();
+    });
 }
 
-hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t tiles_y, hipStream_t s) {
-    const dim3 grid((g0.N2 >> 1) / PACK_G, tiles_y, count);
-    if (g0.W == 1) k_pack<true, true><<<grid, 256, 0, s>>>(nullptr, nullptr, nullptr, g0, bt, nullptr);
-    else k_pack<true, false><<<grid, 256, 0, s>>>(nullptr, nullptr, nullptr, g0, bt, nullptr);
+hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t halves, hipStream_t s) {
+    k_pack<true><<<dim3(g0.N2 / 32u / PACK_CW, g0.N1 / 256u * halves, count), PACK_NT, 0, s>>>(nullptr, nullptr, nullptr, g0, nullptr,
+                                                                                  nullptr, bt);
     return hipGetLastError();
+}
+
+hipError_t launch_batch_mid_inv(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
+    return by_mid_lg1(g0.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value;
+        k_mid_inv<LG1, true><<<dim3(g0.N2 / 16u, 1, count), mid_threads(LG1), 0, s>>>(nullptr, nullptr, nullptr, g0, nullptr,
+                                                                                     nullptr, t.tw14, nullptr, bt);
+        return hipGetLastError();
+    });
 }
 
 hipError_t launch_batch_small(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {

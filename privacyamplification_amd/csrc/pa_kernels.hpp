@@ -8,18 +8,23 @@
 namespace pa {
 
 enum { ROWS_DYN = 0, ROWS_STATIC = 1, ROWS_SEEDPREP = 2 };
-constexpr int ROWS_NT = 512;  // threads of the row pass (256-VGPR budget per lane)
+// Row pass: threads per workgroup and rows per workgroup (a row takes N2 / 16 threads, N2 / 32 at 8192).
+__host__ __device__ constexpr int rows_per_wg(int lg2) { return lg2 == 8 ? 4 : lg2 == 9 ? 2 : 1; }
+__host__ __device__ constexpr int rows_threads(int lg2) { return lg2 == 13 ? 256 : rows_per_wg(lg2) * (1 << lg2) / 16; }
+// Column passes for L <= 2^22: threads and first radix (16 columns, one second-stage butterfly each).
+__host__ __device__ constexpr int mid_threads(int lg1) { return lg1 >= 10 ? 512 : lg1 >= 8 ? 256 : 1 << lg1; }
+__host__ __device__ constexpr int mid_r1(int lg1) { return lg1 >= 10 ? 32 : lg1 >= 8 ? 16 : 1 << (lg1 - 4); }
 constexpr int FWD_NT = 256;   // threads of the forward column pass
 constexpr int TB_NT = 128;        // bit-transpose threads: 32 outputs each
 constexpr int TB_SPAN_LOG = 12;   // bit-transpose outputs per workgroup (2^12 of a row of N2 = 2^13)
-constexpr int POP_SLOTS = 64; // partial popcount counters per operand
-constexpr int PACK_T1 = 32;   // output packer tile: rows x column pairs
-constexpr int PACK_G = 256;
+constexpr int POP_SLOTS = 64; // partial popcounts of a resident seed
+constexpr int PACK_NT = 128;  // output stage: threads and word columns of a tile
+constexpr int PACK_CW = 16;
 
-// Device twiddle tables: tw14[x] = exp(-2 pi i x / 2^14); lo/hi: exp(-2 pi i x / L) split as
+// Device twiddle tables: tw14[x] = exp(-2 pi i x / 2^14); lo/hi: exp(-2 pi i x / (2L)) split as
 // lo[x mod 2^14] * hi[x >> 14].
 // cls: pass A's class tables, cls_table_offset(D) onwards: entry [(c NB + q) 2^BW + byte] =
-// sum over the set bits b of byte of exp(-2 pi i ((BW q + b) c mod D) / D), BW = min(D, 8),
+// sum over the bits b of byte of (bit - 1/2) exp(-2 pi i (BW q + b)(c + 1/4) / D), BW = min(D, 8),
 // NB = D / BW; computed in double precision and rounded once.
 struct Tables {
     const float2* tw14;
@@ -36,24 +41,21 @@ __host__ __device__ constexpr int cls_table_offset(int D) {
 constexpr int CLS_TABLE_TOTAL = cls_table_offset(32);  // D = 1 .. 16
 
 // Columns per workgroup in pass A' (tile of W x N1 complex <= 16384 values in LDS) and its threads.
-// N1 = 2^10 .. 2^12 take 8192 / N1 columns (about 68 KB of LDS) and N1 = 8192 takes 2 columns one at
-// a time, so that two workgroups share a compute unit.  N1 = 2^14 takes 2 columns one at a time
-// (one workgroup per CU), N1 = 2^15 one column in two LDS halves.
-__host__ __device__ constexpr int inv_cols_width(int lg1) {
-    return lg1 >= 15 ? 1 : (lg1 >= 13 ? 2 : (lg1 >= 10 ? (1 << (13 - lg1)) : ((14 - lg1) >= 4 ? 16 : (1 << (14 - lg1)))));
-}
+// N1 = 2^9 takes 16 columns, 2^10 .. 2^12 take 8192 / N1 (about 68 KB of LDS) and N1 = 8192 takes 2
+// columns one at a time, so that two workgroups share a compute unit.  N1 = 2^14 takes 2 columns one
+// at a time (one workgroup per CU), N1 = 2^15 one column in two LDS halves.
+__host__ __device__ constexpr int inv_cols_width(int lg1) { return lg1 >= 15 ? 1 : (lg1 >= 13 ? 2 : 1 << (13 - lg1)); }
 __host__ __device__ constexpr int clamp_threads(int t) { return t < 64 ? 64 : (t > 1024 ? 1024 : t); }
-__host__ __device__ constexpr int inv_cols_threads(int lg1) {
-    return lg1 == 13 ? 256 : (lg1 >= 14 ? 1024 : clamp_threads(inv_cols_width(lg1) * (1 << lg1) / 16));
-}
+__host__ __device__ constexpr int inv_cols_threads(int lg1) { return lg1 == 13 ? 256 : (lg1 >= 14 ? 1024 : 512); }
 // Columns per workgroup in pass A (16; 8 when the class length M = 2048 would overflow LDS).
 __host__ __device__ constexpr int fwd_cols_width(int lgm) { return lgm >= 11 ? 8 : 16; }
 // Threads of the generic pass A: 1024 for classes of 1024 and 2048 points, whose 128 KB of columns
 // leave room for one workgroup per CU, so that it brings 16 waves instead of 4.
 __host__ __device__ constexpr int fwd_cols_threads(int lgm) { return lgm >= 10 ? 1024 : FWD_NT; }
-// Bytes of the pass-A' output: nibbles per column pair (N/2), or 2-bit crumbs per column (N) when
-// a workgroup holds a single column.
-__host__ __device__ constexpr uint64_t nib_bytes(uint32_t N, uint32_t W) { return (W == 1 ? (uint64_t)N : N / 2) + 64; }
+// Bytes of the nib buffer: pass A''s pieces (one bit per conv value, N/4 bytes), then the prefix
+// words (L/8 bytes).
+__host__ __device__ constexpr uint64_t nib_bytes(uint32_t N) { return N / 2 + 64; }
+inline uint32_t* prefix_words(uint8_t* nib, uint32_t N) { return reinterpret_cast<uint32_t*>(nib + N / 4); }
 __host__ __device__ constexpr int small_threads(int lgn) { return clamp_threads(2 * (1 << lgn) / 16); }
 
 // A staging range: `bytes` from src to dst, either side device memory or pinned, device-mapped
@@ -65,45 +67,51 @@ struct CopyDesc {
 };
 // Copies every range of d[0 .. count) in one launch; max_bytes = the longest range.
 hipError_t launch_copies(const CopyDesc* d, uint32_t count, uint64_t max_bytes, hipStream_t s);
-hipError_t launch_zero_u32(uint32_t* p, uint32_t count, hipStream_t s);
-// bits2/tb2 (and tb2/Y2) non-null: the seed is transformed in the same launch (grid.y = 2),
-// its popcount into count + POP_SLOTS.
-hipError_t launch_transpose(const uint32_t* bits, uint32_t* tb, uint32_t* count, const Geom& g,
-                            int is_seed, hipStream_t s, const uint32_t* bits2 = nullptr, uint32_t* tb2 = nullptr);
-hipError_t launch_fwd_cols(const uint32_t* tb, float2* Y, const Geom& g, const Tables& t, hipStream_t s,
-                           const uint32_t* tb2 = nullptr, float2* Y2 = nullptr);
-// ROWS_SEEDPREP: S <- split spectrum of the seed rows held in S (in place, N+1 values).
-// ROWS_STATIC:   R' from the key rows in Yk and the split seed spectrum S.
+// Bit masks of `ops` operands from `first` on (0 key, 1 seed); scan != 0: the launch also scans the
+// inputs (ScanArgs), which takes every operand of the block.
+hipError_t launch_transpose(const uint32_t* key, const uint32_t* seed, uint32_t* tbk, uint32_t* tbs, uint32_t first,
+                            uint32_t ops, const Geom& g, const ScanArgs* scan, hipStream_t s);
+// Pass A of `ops` operands from `first` on; in: the masks, or for a mid-size transform the words, and
+// there the scan as above.
+hipError_t launch_fwd_cols(const uint32_t* key_in, const uint32_t* seed_in, float2* Yk, float2* Ys, uint32_t first,
+                           uint32_t ops, const Geom& g, const Tables& t, const ScanArgs* scan, hipStream_t s);
+// ROWS_SEEDPREP: S <- spectrum of the seed rows held in S (in place, N values).
+// ROWS_STATIC:   R' from the key rows in Yk and the seed spectrum S.
 // ROWS_DYN:      R' from the key rows in Yk and the seed rows (pass-A output) in S.
 // R' goes to Rt in tiles when rt_tiled(g.lg1) (N complex values), else to Yk in place.
-// Persistent: at most `cus` workgroups (one per compute unit) walk the row pairs.
-hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, int cus,
-                       hipStream_t s);
+// info: finished by the launch (ws: a resident seed's popcount partials; seed_ws: receives them).
+hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, uint32_t* info,
+                       const uint32_t* ws, uint32_t* seed_ws, hipStream_t s);
+// A resident seed's chunk-wise prefix words q[0 .. L/32) finished with its chunks' parities.
+hipError_t launch_prefix_apply(uint32_t* q, const uint32_t* info, const Geom& g, hipStream_t s);
 // R: pass B's output (the tile buffer when rt_tiled(g.lg1)).
-hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* wk,
-                           const uint32_t* ws, const Tables& t, float* margin, hipStream_t s);
-// zero_counts != null: the launch also clears those 2 * POP_SLOTS popcount partials.
-hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, const Geom& g, hipStream_t s,
-                       uint32_t* zero_counts = nullptr);
+hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
+                           float* margin, hipStream_t s);
+hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
+                       const uint32_t* q, hipStream_t s);
+// Pass A' and the output of a mid-size transform.
+hipError_t launch_mid_inv(const float2* R, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
+                          const uint32_t* q, const Tables& t, float* margin, hipStream_t s);
 hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2* sspec,
                         const uint32_t* ws_ptr, uint32_t* out, const Geom& g, const Tables& t,
                         float* margin, float2* sspec_out, uint32_t* ws_out, hipStream_t s);
 
 // Batched forms: `count` blocks of one transform length in one launch each (grid z = block),
 // block b's geometry and buffers in bt[b] (device memory); g0 is any block's geometry.
-uint32_t pack_tiles(const Geom& g);  // grid.y the pack stage needs for this block's window
-hipError_t launch_batch_zero(const BlockArgs* bt, uint32_t count, hipStream_t s);
-hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geom& g0, int is_seed, hipStream_t s);
-// per: column groups each workgroup of the persistent pass A (N1 = 2^9 .. 2^13) walks, a power of
-// two up to 32; 0 picks 16, halved while the launch would have under 512 workgroups.
-hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, int is_seed,
+uint32_t pack_halves(const Geom& g);  // halves of the conv positions (t, t + N) the window touches
+// ops: 1 (key) or 2 (key and seed).
+hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t ops, hipStream_t s);
+// per: column groups each workgroup of the persistent pass A (N1 = 2^9 .. 2^13, N2 = 8192) walks, a
+// power of two up to 32; 0 picks 16, halved while the launch would have under 512 workgroups.
+hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, uint32_t ops,
                                  uint32_t per, hipStream_t s);
 constexpr uint32_t FWD_PER_MAX = 32;
-// grid_x workgroups per block walk that block's row pairs (0 = one per row pair).
 hipError_t launch_batch_rows(int mode, const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t,
-                             uint32_t grid_x, hipStream_t s);
+                             hipStream_t s);
 hipError_t launch_batch_inv_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s);
-hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t tiles_y, hipStream_t s);
+// halves: the most of a block of the launch.
+hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t halves, hipStream_t s);
+hipError_t launch_batch_mid_inv(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s);
 hipError_t launch_batch_small(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s);
 
 // Sub-block split (tiles of b x b through the batched engine, XOR-accumulated per band).
@@ -120,6 +128,6 @@ hipError_t launch_st_correction(const uint32_t* wk, const uint32_t* ws, uint32_t
                                 hipStream_t s);
 hipError_t launch_st_product(const float2* a, const float2* b, float r, float2* prod, const float2* z, float2* zz,
                              uint32_t N, hipStream_t s);
-hipError_t launch_st_nibbles(uint8_t* nib, const Geom& g, float corr, float invN, hipStream_t s);
+hipError_t launch_st_pieces(uint8_t* nib, const Geom& g, float corr, float invN, hipStream_t s);
 
 }  // namespace pa
