@@ -86,7 +86,7 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
         x.lg2 = x.lgN - x.lg1;
         x.N1 = 1u << x.lg1;
         x.N2 = 1u << x.lg2;
-        x.M = x.N1 <= 512 ? x.N1 : (x.N1 / 16 > 512 ? x.N1 / 16 : 512);  // D <= 16 bit classes
+        x.M = x.N1 <= 512 ? x.N1 : x.N1 <= 8192 ? 512 : 1024;  // up to 16 classes of 512, 32 of 1024
         x.D = x.N1 / x.M;
     }
     x.out_bits = compress ? m : n / 2;
@@ -128,7 +128,9 @@ uint64_t ws_key_bytes(uint32_t L) { return (uint64_t)(L / 32 + 2) * 4; }
 uint64_t ws_out_bytes(uint32_t L) { return (uint64_t)L / 8 + 16; }
 
 // one operand's bit masks (none below L = 2^23)
-uint64_t mask_bytes(const Geom& g) { return g.N1 == 1 || mid_size(g) ? 0 : (uint64_t)(g.N / g.D) * 4; }
+uint64_t mask_bytes(const Geom& g) {
+    return g.N1 == 1 || mid_size(g) ? 0 : (uint64_t)(g.N / g.D) * (g.D == 32 ? 8 : 4);
+}
 
 struct Extents {
     uint64_t touched[PA_BUF_COUNT] = {};
@@ -158,8 +160,8 @@ Extents block_extents(const Geom& g) {
     // the last parity byte, scan_parities(info)[chunks - 1]
     x.touched[PA_BUF_COUNTS] = pa::INFO_HEAD * 4 + pa::scan_chunks(g) * 9ull;
     if (!mid_size(g)) {
-        // k_transpose_bits writes tb[u N2 + t2] for u < M, t2 < N2
-        x.touched[PA_BUF_BITS_KEY] = x.touched[PA_BUF_BITS_SEED] = (uint64_t)g.M * g.N2 * 4;
+        // k_transpose_bits writes tb[u N2 + t2] for u < M, t2 < N2 (D = 32: u < 2 M)
+        x.touched[PA_BUF_BITS_KEY] = x.touched[PA_BUF_BITS_SEED] = (uint64_t)g.M * g.N2 * (g.D == 32 ? 8 : 4);
         x.alloc[PA_BUF_BITS_KEY] = x.alloc[PA_BUF_BITS_SEED] = mask_bytes(g);
     }
     // pass A writes Y[k1 N2 + t2], k1 < N1
@@ -410,19 +412,23 @@ std::vector<float2> twiddles(uint64_t L, uint64_t count, uint64_t stride) {
 // times the +-1/2-encoded bits of a byte, in double precision, rounded once.
 std::vector<float2> class_tables() {
     std::vector<float2> t(pa::CLS_TABLE_TOTAL);
-    for (int D = 1; D <= 16; D *= 2) {
+    for (int D = 1; D <= 32; D *= 2) {
         const int BW = pa::cls_bits(D), NB = pa::cls_tables(D);
+        std::vector<double> re(4 * D), im(4 * D);  // half the 4D-th roots of unity
+        for (int k = 0; k < 4 * D; ++k) {
+            re[k] = 0.5 * std::cos(-2.0 * M_PI * k / (4.0 * D));
+            im[k] = 0.5 * std::sin(-2.0 * M_PI * k / (4.0 * D));
+        }
         for (int c = 0; c < D; ++c)
             for (int q = 0; q < NB; ++q)
                 for (int byte = 0; byte < (1 << BW); ++byte) {
-                    double re = 0.0, im = 0.0;
+                    double x = 0.0, y = 0.0;
                     for (int b = 0; b < BW; ++b) {
-                        const double a = -2.0 * M_PI * (double)(((BW * q + b) * (4 * c + 1)) % (4 * D)) / (4.0 * D);
-                        const double h = ((byte >> b) & 1) ? 0.5 : -0.5;
-                        re += h * std::cos(a);
-                        im += h * std::sin(a);
+                        const int k = ((BW * q + b) * (4 * c + 1)) % (4 * D);
+                        x += ((byte >> b) & 1) ? re[k] : -re[k];
+                        y += ((byte >> b) & 1) ? im[k] : -im[k];
                     }
-                    t[pa::cls_table_offset(D) + (c * NB + q) * (1 << BW) + byte] = make_float2((float)re, (float)im);
+                    t[pa::cls_table_offset(D) + (c * NB + q) * (1 << BW) + byte] = make_float2((float)x, (float)y);
                 }
     }
     return t;
@@ -632,8 +638,7 @@ int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* k
         PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_mid_inv(w->Yk, key, out, g, w->info, q, t, margin, s); }));
         return PA_OK;
     }
-    const float2* R = pa::rt_tiled(g.lg1) ? w->Rt : w->Yk;
-    PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_inv_cols(R, w->nib, g, w->info, t, margin, s); }));
+    PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_inv_cols(w->Rt, w->nib, g, w->info, t, margin, s); }));
     PA_HIP(timed(e, ST_PACK, s, [&] { return pa::launch_pack(w->nib, key, out, g, w->info, q, s); }));
     return PA_OK;
 }

@@ -8,8 +8,7 @@
 //
 //   k_transpose_bits  key/seed RefBits -> per-(class,column) bit masks for pass A
 //   k_fwd_cols        pass A: decimated column FFTs of the +-1/2-encoded bits (R2C forward part);
-//   k_fwd_cols9p      its persistent form for 512-point classes (the 2^27-bit block's shape);
-//   k_mid_fwd         its form for L <= 2^22, straight from the key's and the seed's words.
+//   k_mid_fwd         its form for L <= 2^24, straight from the key's and the seed's words.
 //                     Their launches also scan the inputs' popcounts (binInt2float's popcount,
 //                     PrivacyAmplification.cu:570-602) and prefix parities
 //   k_rows            pass B: row FFTs, complex product (ElementWiseProduct, :465-481), inverse row FFTs
@@ -18,7 +17,8 @@
 //                     :363-373 and setFirstElementToZero :408-418 remove it spectrally), the key-rest
 //                     XOR and byte order (key2StartRest's key_rest :873-878, ToBinaryArray's bswap
 //                     XOR :757-762)
-//   k_mid_inv         pass A' and the output in one for L <= 2^22
+//   k_inv_big1, 2     pass A' for L >= 2^28
+//   k_mid_inv         pass A' and the output in one for L <= 2^24
 //   k_small           the whole block in one workgroup for L <= 2^14
 #include <hip/hip_runtime.h>
 
@@ -271,7 +271,8 @@ __device__ __forceinline__ void bit_transpose(uint32_t (&A)[32]) {
     bit_transpose_round<1>(A);
 }
 
-// tb[u*N2 + t2] = E | O << 16 with E bit v = x[t2 + N2(u + M v)], O bit v = x[N + t2 + N2(u + M v)].
+// tb[u*N2 + t2] = E | O << 16 with E bit v = x[t2 + N2(u + M v)], O bit v = x[N + t2 + N2(u + M v)]
+// (D = 32: E at tb[u*N2 + t2] and O at tb[(M + u) N2 + t2]).
 // Workgroup (u, part): thread k covers t2 in [part*TB_SPAN + 32k, +32): for each class v it reads
 // the two words holding those bits (coalesced across the workgroup), transposes the 2 D x 32 bits
 // in registers, and the workgroup writes its TB_SPAN outputs through LDS.  The launch's first
@@ -316,7 +317,26 @@ __global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __rest
         w1[v] = is_seed ? seed_word(bits, g, widx + (g.N >> 5)) : key_word(bits, g, widx + (g.N >> 5));
     }
     uint32_t* srow = stage + threadIdx.x * 33;
-    if constexpr (D >= 8) {
+    uint32_t* out = tb + (size_t)u * g.N2 + (part << TB_SPAN_LOG);
+    auto write = [&] {
+        __syncthreads();
+        for (int e = threadIdx.x; e < (1 << TB_SPAN_LOG); e += TB_NT) out[e] = stage[(e >> 5) * 33 + (e & 31)];
+    };
+    if constexpr (D == 32) {  // a word per half: E in the first M N2 words, O in the next
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            uint32_t A[32];
+#pragma unroll
+            for (int v = 0; v < 32; ++v) A[31 - v] = h ? w1[v] : w0[v];
+            bit_transpose(A);
+            if (h) __syncthreads();  // the first half has been written out
+#pragma unroll
+            for (int i = 0; i < 32; ++i) srow[i] = A[i];
+            write();
+            out += (size_t)g.M * g.N2;
+        }
+        return;
+    } else if constexpr (D >= 8) {
         // Rows A[15 - v] = w1[v], A[31 - v] = w0[v] (zero for v >= D), transposed: A[c] then holds
         // bit 31 - c (column t0 + c) of w0[v] at bit v and of w1[v] at bit v + 16: output c.
         uint32_t A[32];
@@ -340,9 +360,7 @@ __global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __rest
             srow[i] = E | (O << 16);
         }
     }
-    __syncthreads();
-    uint32_t* out = tb + (size_t)u * g.N2 + (part << TB_SPAN_LOG);
-    for (int e = threadIdx.x; e < (1 << TB_SPAN_LOG); e += TB_NT) out[e] = stage[(e >> 5) * 33 + (e & 31)];
+    write();
 }
 
 // ------------------------------------------------------------------ pass A ----
@@ -377,91 +395,6 @@ __device__ __forceinline__ float2 uniform_f2(float2 v) {
                        __uint_as_float(__builtin_amdgcn_readfirstlane((int)__float_as_uint(v.y))));
 }
 
-// Workgroup (column group grp of CPW columns, class c): computes Y[k1][t2] for k1 = c + D*k1',
-// t2 in the group, at the quarter-shifted frequencies k1 + 1/4 (c' = c + 1/4):
-//   Y = w_N^{t2 (k1 + 1/4)} * FFT_M( w_N1^{u c'} * sum_v z[t2 + N2(u + M v)] w_D^{v c'} ),
-// z[t] = a[t] - i a[t + N], a = bit - 1/2.  The class sum over v is one or two 256-entry table
-// lookups per operand half (bits of tb), the -1/2 included in the tables.  The class values go to
-// LDS and the M-point FFT runs there: M = 1024, 2048 (N1 = 2^14, 2^15).  M = 512 runs in
-// k_fwd_cols9p instead.
-template <int LGM, int D, bool BATCH, int CPW = fwd_cols_width(LGM)>
-__global__ __launch_bounds__(fwd_cols_threads(LGM)) void k_fwd_cols(FwdArgs a, Geom g,
-                                                     const float2* __restrict__ tw14,
-                                                     const float2* __restrict__ twlo,
-                                                     const float2* __restrict__ twhi,
-                                                     const float2* __restrict__ cls,
-                                                     const BlockArgs* __restrict__ bt) {
-    fwd_batch_args<BATCH, false>(a, g, bt);
-    constexpr int M = 1 << LGM;
-    constexpr int NT = fwd_cols_threads(LGM);
-    constexpr int SEQS = seq_stride(M);
-    static_assert(LGM >= 10, "512-point classes run in k_fwd_cols9p");
-    __shared__ float2 buf[CPW * SEQS];
-    __shared__ float2 twl[TWL_SIZE];
-    constexpr int BW = cls_bits(D);         // bits per table: v in [BW q, BW q + BW)
-    constexpr int NB = cls_tables(D);       // tables per 16-bit half
-    constexpr uint32_t MASK = (1u << BW) - 1u;
-    __shared__ float2 TB[NB][1 << BW];      // TB[q][byte] = sum_b (bit_b(byte) - 1/2) w_D^{(BW q + b) c'}
-    __shared__ float2 TU[M];                // w_N1^{u c'} = w_4N1^{u (4c + 1)}
-    const uint32_t op = blockIdx.x / a.nA;
-    const bool is_seed = a.first + op == 1u;
-    const uint32_t* __restrict__ tb = is_seed ? a.in[1] : a.in[0];
-    float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
-    if (BATCH && tb == nullptr) return;
-    const uint32_t logical = xcd_logical(blockIdx.x - op * a.nA, a.nA);
-    const uint32_t c = logical % D, grp = logical / D;  // columns [CPW grp, CPW grp + CPW)
-    load_twl(twl, tw14, NT);
-    {
-        const float2* src = cls + cls_table_offset(D) + (size_t)c * (NB << BW);
-        for (int e = threadIdx.x; e < NB << BW; e += NT) TB[e >> BW][e & (int)MASK] = src[e];
-    }
-    for (uint32_t u = threadIdx.x; u < (uint32_t)M; u += NT) TU[u] = w_4n1(g, tw14, twlo, twhi, u * (4u * c + 1u));
-    // the element z(col, u) of this class (both halves of tb: positions t and t + N)
-    auto zval = [&](uint32_t t, int u) {
-        float2 sE = TB[0][t & MASK], sO = TB[0][(t >> 16) & MASK];
-#pragma unroll
-        for (int q = 1; q < NB; ++q) {
-            sE = cadd(sE, TB[q][(t >> (BW * q)) & MASK]);
-            sO = cadd(sO, TB[q][(t >> (16 + BW * q)) & MASK]);
-        }
-        return cmul(make_float2(sE.x + sO.y, sE.y - sO.x), TU[u]);
-    };
-    constexpr int IPT = (CPW * M + NT - 1) / NT;
-    uint32_t tbv[IPT];
-#pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int e = threadIdx.x + i * NT;
-        tbv[i] = (e < CPW * M) ? tb[(uint32_t)(e / CPW) * g.N2 + grp * CPW + (uint32_t)(e % CPW)] : 0u;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int e = threadIdx.x + i * NT;
-        if (e < CPW * M) buf[(e % CPW) * SEQS + padi(e / CPW)] = zval(tbv[i], e / CPW);
-    }
-    __syncthreads();
-    lds_fft<LGM, CPW, SEQS, NT>(buf, twl);
-    // Output e = tid + NT i is column tid mod CPW, k1' = tid / CPW + RPI i: its twiddle
-    // w_2L^{t2 (4 k1 + 1)} is base step^i, re-anchored from the table every 8 steps (a gather per
-    // point cost more than the transform at N1 >= 2^14)
-    static_assert(NT % CPW == 0, "a thread keeps one column");
-    constexpr int RPI = NT / CPW;
-    const int col = threadIdx.x % CPW, jt = threadIdx.x / CPW;
-    const uint32_t t2 = grp * CPW + (uint32_t)col;
-    const uint32_t L2m = 2u * g.L - 1u;
-    auto tw_at = [&](uint32_t k1p) {
-        return tw_two_level(twlo, twhi, (t2 * (4u * (c + (uint32_t)D * k1p) + 1u)) & L2m);
-    };
-    const float2 step = tw_two_level(twlo, twhi, (t2 * (4u * (uint32_t)D * RPI)) & L2m);
-    float2 tw = make_float2(1.f, 0.f);
-    for (int i = 0; i < (CPW * M) / NT; ++i) {
-        const uint32_t k1p = (uint32_t)jt + (uint32_t)RPI * (uint32_t)i;
-        tw = (i & 7) == 0 ? tw_at(k1p) : cmul(tw, step);
-        const uint32_t k1 = c + (uint32_t)D * k1p;
-        st_nt(&Y[(size_t)k1 * g.N2 + t2], cmul(buf[col * SEQS + padi((int)k1p)], tw));
-    }
-}
-
 // Raw buffer access (vector memory instructions): one per-lane byte offset plus a uniform
 // scalar offset, so a run of accesses at fixed strides keeps a single address register.
 typedef unsigned int pa_u2v __attribute__((ext_vector_type(2)));
@@ -480,30 +413,52 @@ __device__ __forceinline__ uint32_t buf_load_u32(__amdgpu_buffer_rsrc_t rs, uint
     return __builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, (int)soff, 0);
 }
 
-// Pieces of the persistent pass A (k_fwd_cols9p).  Thread (col = t mod 16, jt = t / 16).
-// Bit words of column group grp: stage-1 butterflies j = jt + 16 i, inputs u = j + 32 r.
-__device__ __forceinline__ void fwd9_load_tv(uint32_t (&tv)[2][16], __amdgpu_buffer_rsrc_t rtb, uint32_t N2,
-                                             uint32_t t2, int jt) {
+// Pass A for L >= 2^25: a workgroup has 16 columns (group grp) and one class c of D, and computes
+// Y[k1][t2] for k1 = c + D k1', at the quarter-shifted frequencies k1 + 1/4 (c' = c + 1/4):
+//   Y = w_N^{t2 (k1 + 1/4)} * FFT_M( w_N1^{u c'} * sum_v z[t2 + N2(u + M v)] w_D^{v c'} ),
+// z[t] = a[t] - i a[t + N], a = bit - 1/2.  The class sum over v is one 256-entry table lookup per byte
+// of the bit masks, the -1/2 included in the tables.
+// Plan R1 x 32 with M = 32 R1: M = 512 for N1 <= 2^13 (256 threads, two workgroups per compute unit),
+// M = 1024 for 2^14 and 2^15 (512 threads, one: its 16 columns take 135 KB of LDS).
+template <int LGM, int D>
+struct FwdPlan {
+    static constexpr int M = 1 << LGM, R1 = M / 32, NT = fwd_cols_threads(LGM), JT = NT / 16, K1 = 32 / JT;
+    static constexpr int NW = D == 32 ? 2 : 1;   // mask words per position (both halves in one up to D = 16)
+    static constexpr int BW = cls_bits(D), NB = cls_tables(D);  // bits per table, tables per half
+    static constexpr int SEQS = seq_stride(M);
+    static_assert(JT == R1, "one second-stage butterfly per thread");
+    using Bits = uint32_t[K1][R1][NW];
+    using Tables = float2[NB][1 << BW];
+};
+// Pieces of the persistent walk.  Thread (col = t mod 16, jt = t / 16).
+// Bit words of column group grp: stage-1 butterflies j = jt + JT i, inputs u = j + 32 r.
+template <int LGM, int D>
+__device__ __forceinline__ void fwd_load_bits(typename FwdPlan<LGM, D>::Bits& tv, __amdgpu_buffer_rsrc_t rtb, uint32_t N2,
+                                              uint32_t t2, int jt) {
+    using P = FwdPlan<LGM, D>;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const uint32_t voff = ((uint32_t)(jt + 16 * i) * N2 + t2) * 4u;
+    for (int i = 0; i < P::K1; ++i) {
+        const uint32_t voff = ((uint32_t)(jt + P::JT * i) * N2 + t2) * 4u;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tv[i][r] = buf_load_u32(rtb, voff, (uint32_t)(32 * r) * N2 * 4u);
+        for (int r = 0; r < P::R1; ++r)
+#pragma unroll
+            for (int h = 0; h < P::NW; ++h)
+                tv[i][r][h] = buf_load_u32(rtb, voff, (uint32_t)(32 * r + P::M * h) * N2 * 4u);
     }
 }
-// Table entries of the output twiddles w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + 16 r) = base step^r, with
-// anchors w_N^{t2 16 D 8 (a+1)}: (lo, hi) pairs of base, step, anchor 0..2.  The products are
+// Table entries of the output twiddles w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + R1 r) = base step^r, with
+// anchors w_N^{t2 R1 D 8 (a+1)}: (lo, hi) pairs of base, step, anchor 0..2.  The products are
 // formed where they are used, so that gathering them never waits on other loads.
-template <int D>
-__device__ __forceinline__ void fwd9_load_tw(float2 (&tw)[10], const float2* __restrict__ lo,
-                                             const float2* __restrict__ hi, uint32_t L, uint32_t c, uint32_t t2,
-                                             int jt) {
+template <int LGM, int D>
+__device__ __forceinline__ void fwd_load_tw(float2 (&tw)[10], const float2* __restrict__ lo,
+                                            const float2* __restrict__ hi, uint32_t L, uint32_t c, uint32_t t2, int jt) {
+    constexpr uint32_t R1 = FwdPlan<LGM, D>::R1;
     const uint32_t L2m = 2u * L - 1u;
     uint32_t x[5];
     x[0] = (t2 * (4u * (c + (uint32_t)D * (uint32_t)jt) + 1u)) & L2m;
-    x[1] = (t2 * (64u * (uint32_t)D)) & L2m;
+    x[1] = (t2 * (4u * R1 * (uint32_t)D)) & L2m;
 #pragma unroll
-    for (int a = 0; a < 3; ++a) x[2 + a] = (t2 * (64u * (uint32_t)D * 8u * (uint32_t)(a + 1))) & L2m;
+    for (int a = 0; a < 3; ++a) x[2 + a] = (t2 * (4u * R1 * (uint32_t)D * 8u * (uint32_t)(a + 1))) & L2m;
 #pragma unroll
     for (int e = 0; e < 5; ++e) {
         tw[2 * e] = lo[x[e] & (TW14 - 1)];
@@ -511,129 +466,83 @@ __device__ __forceinline__ void fwd9_load_tw(float2 (&tw)[10], const float2* __r
     }
 }
 // tw1: the first stage's factors for w_N1^{32 c'} (one class per workgroup: uniform).
-template <int D>
-__device__ __forceinline__ void fwd9_stage1(const uint32_t (&tv)[2][16], float2* buf,
-                                            const float2 (*TB)[1 << cls_bits(D)], const float2 (&tw1)[8], int col,
-                                            int jt) {
-    constexpr int SEQS = seq_stride(512);
-    constexpr int BW = cls_bits(D);
-    constexpr int NB = cls_tables(D);
-    constexpr uint32_t MASK = (1u << BW) - 1u;
+template <int LGM, int D>
+__device__ __forceinline__ void fwd_stage1(const typename FwdPlan<LGM, D>::Bits& tv, float2* seqbuf,
+                                           const typename FwdPlan<LGM, D>::Tables& TB,
+                                           const float2 (&tw1)[FwdPlan<LGM, D>::R1 / 2], int jt) {
+    using P = FwdPlan<LGM, D>;
+    constexpr uint32_t MASK = (1u << P::BW) - 1u;
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int j = jt + 16 * i;
-        float2 v[16];
+    for (int i = 0; i < P::K1; ++i) {
+        const int j = jt + P::JT * i;
+        float2 v[P::R1];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const uint32_t t = tv[i][r];
-            float2 sE = TB[0][t & MASK], sO = TB[0][(t >> 16) & MASK];
+        for (int r = 0; r < P::R1; ++r) {
+            const uint32_t tE = tv[i][r][0], tO = P::NW == 2 ? tv[i][r][P::NW - 1] : tE >> 16;
+            float2 sE = TB[0][tE & MASK], sO = TB[0][tO & MASK];
 #pragma unroll
-            for (int q = 1; q < NB; ++q) {
-                sE = cadd(sE, TB[q][(t >> (BW * q)) & MASK]);
-                sO = cadd(sO, TB[q][(t >> (16 + BW * q)) & MASK]);
+            for (int q = 1; q < P::NB; ++q) {
+                sE = cadd(sE, TB[q][(tE >> (P::BW * q)) & MASK]);
+                sO = cadd(sO, TB[q][(tO >> (P::BW * q)) & MASK]);
             }
             v[r] = make_float2(sE.x + sO.y, sE.y - sO.x);
         }
-        dft_tw<16>(v, tw1);
-        float2* seqbuf = buf + col * SEQS;
+        dft_tw<P::R1>(v, tw1);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) seqbuf[padi(j * 16 + r)] = v[r];
+        for (int r = 0; r < P::R1; ++r) seqbuf[padi(j * P::R1 + r)] = v[r];
     }
 }
-// tw2: the radix-32 stage's factors, row jt for w_512^jt w_N1^c' (the class twiddle of input j).
-template <int D>
-__device__ __forceinline__ void fwd9_stage2(const float2* buf, const float2* tw2, const float2 (&tw)[10],
-                                            __amdgpu_buffer_rsrc_t ry, uint32_t N2, uint32_t c, uint32_t t2,
-                                            int col, int jt) {
-    constexpr int SEQS = seq_stride(512);
+// tw2: the second stage's factors, row jt for w_M^jt w_N1^c' (the class twiddle of input j).
+template <int LGM, int D>
+__device__ __forceinline__ void fwd_stage2(const float2* seqbuf, const float2* tw2, const float2 (&tw)[10],
+                                           __amdgpu_buffer_rsrc_t ry, uint32_t N2, uint32_t c, uint32_t t2, int jt) {
+    using P = FwdPlan<LGM, D>;
     float2 F[32];
-    stage_last_from_lds_tab<32, 512>(F, buf + col * SEQS, jt, tw2 + jt * stage_row<32>());
+    stage_last_from_lds_tab<32, P::M>(F, seqbuf, jt, tw2 + jt * stage_row<32>());
     const float2 base = cmul(tw[0], tw[1]), step = cmul(tw[2], tw[3]);
     const uint32_t voff = ((c + (uint32_t)D * (uint32_t)jt) * N2 + t2) * 8u;
     float2 w = base;
 #pragma unroll
     for (int r = 0; r < 32; ++r) {
         if ((r & 7) == 0 && r) w = cmul(base, cmul(tw[2 * (1 + r / 8)], tw[2 * (1 + r / 8) + 1]));
-        buf_store_nt(cmul(F[r], w), ry, voff, (uint32_t)(16 * D * r) * N2 * 8u);
+        buf_store_nt(cmul(F[r], w), ry, voff, (uint32_t)(P::R1 * D * r) * N2 * 8u);
         w = cmul(w, step);
     }
 }
-template <int D>
-__device__ __forceinline__ void fwd9_walk(__amdgpu_buffer_rsrc_t rtb, __amdgpu_buffer_rsrc_t ry, const Geom& g,
-                                          const float2* __restrict__ twlo, const float2* __restrict__ twhi,
-                                          float2* buf, const float2* tw2, const float2 (*TB)[1 << cls_bits(D)],
-                                          const float2 (&tw1)[8], uint32_t c, uint32_t grp0, uint32_t per) {
-    const int col = threadIdx.x & 15;
-    const int jt = threadIdx.x >> 4;
-    const uint32_t N2 = g.N2;
-    uint32_t tv[2][16];
-    float2 tw[10], twn[10];
-    // group grp0, peeled: every entry into the loop below then has the same memory-operation
-    // history (next group's loads, then this group's stores), so the compiler's waits on the
-    // prefetched registers count past the stores instead of draining them
-    fwd9_load_tv(tv, rtb, N2, grp0 * 16u + (uint32_t)col, jt);
-    fwd9_load_tw<D>(tw, twlo, twhi, g.L, c, grp0 * 16u + (uint32_t)col, jt);
-    __syncthreads();  // tables
-    fwd9_stage1<D>(tv, buf, TB, tw1, col, jt);
-    __syncthreads();
-    if (per > 1) {
-        fwd9_load_tv(tv, rtb, N2, (grp0 + 1u) * 16u + (uint32_t)col, jt);
-        fwd9_load_tw<D>(twn, twlo, twhi, g.L, c, (grp0 + 1u) * 16u + (uint32_t)col, jt);
-    }
-    fwd9_stage2<D>(buf, tw2, tw, ry, N2, c, grp0 * 16u + (uint32_t)col, col, jt);
-    for (uint32_t it = 1; it < per; ++it) {
-        const uint32_t grp = grp0 + it;
-#pragma unroll
-        for (int e = 0; e < 10; ++e) tw[e] = twn[e];
-        __syncthreads();  // stage-2 reads of the previous group are done
-        fwd9_stage1<D>(tv, buf, TB, tw1, col, jt);
-        __syncthreads();
-        if (it + 1 < per) {
-            fwd9_load_tv(tv, rtb, N2, (grp + 1u) * 16u + (uint32_t)col, jt);
-            fwd9_load_tw<D>(twn, twlo, twhi, g.L, c, (grp + 1u) * 16u + (uint32_t)col, jt);
-        }
-        fwd9_stage2<D>(buf, tw2, tw, ry, N2, c, grp * 16u + (uint32_t)col, col, jt);
-    }
-}
 
-// Persistent pass A for M = 512 (plan 16 x 32): workgroup L of G keeps one class c = L mod D and
-// walks the column groups [k per, k per + per), k = L / D, so its class tables are loaded once, and
-// each group's stores drain while the next group is transformed (its loads were issued before those
-// stores).  The D workgroups of one k sit on one XCD and walk the same groups in step, so each bit
-// word is fetched into L2 once.  The class twiddles w_N1^{u c'}, u = j + 32 r, cost nothing: their
-// r part is in the first stage's factors, their j part in the second's.
-template <int D, bool BATCH>
-__global__ __launch_bounds__(FWD_NT, 2) void k_fwd_cols9p(FwdArgs a, Geom g, const float2* __restrict__ tw14,
-                                                          const float2* __restrict__ twlo,
-                                                          const float2* __restrict__ twhi,
-                                                          const float2* __restrict__ cls, uint32_t per,
-                                                          const BlockArgs* __restrict__ bt) {
+// Persistent: workgroup L of G keeps one class c = L mod D and walks the column groups
+// [k per, k per + per), k = L / D, so its class tables are loaded once, and each group's stores drain
+// while the next group is transformed (its loads were issued before those stores).  The D workgroups
+// of one k sit on one XCD and walk the same groups in step, so each bit word is fetched into L2 once.
+// The class twiddles w_N1^{u c'}, u = j + 32 r, cost nothing: their r part is in the first stage's
+// factors, their j part in the second's.
+template <int LGM, int D, bool BATCH>
+__global__ __launch_bounds__(fwd_cols_threads(LGM), LGM == 9 ? 2 : 1) void k_fwd_cols(
+    FwdArgs a, Geom g, const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
+    const float2* __restrict__ cls, uint32_t per, const BlockArgs* __restrict__ bt) {
     fwd_batch_args<BATCH, false>(a, g, bt);
-    constexpr int M = 512;
-    constexpr int NT = FWD_NT;
-    constexpr int SEQS = seq_stride(M);
-    static_assert(NT == 256, "fused pass A expects 256 threads");
-    __shared__ float2 buf[16 * SEQS];
-    __shared__ float2 tw2[16 * stage_row<32>()];
-    constexpr int BW = cls_bits(D);
-    constexpr int NB = cls_tables(D);
-    constexpr uint32_t MASK = (1u << BW) - 1u;
-    __shared__ float2 TB[NB][1 << BW];
+    using P = FwdPlan<LGM, D>;
+    constexpr int NT = P::NT;
+    constexpr uint32_t MASK = (1u << P::BW) - 1u;
+    __shared__ float2 buf[16 * P::SEQS];
+    __shared__ float2 tw2[P::R1 * stage_row<32>()];
+    __shared__ typename P::Tables TB;
     const uint32_t op = blockIdx.x / a.nA;
     const bool is_seed = a.first + op == 1u;
     const uint32_t* __restrict__ tb = is_seed ? a.in[1] : a.in[0];
     float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
     if (BATCH && tb == nullptr) return;  // resident seed: nothing to transform
     const uint32_t logical = xcd_logical(blockIdx.x - op * a.nA, a.nA);
-    const uint32_t c = logical % D, grp0 = (logical / D) * per;
-    const __amdgpu_buffer_rsrc_t rtb = make_rsrc(tb, (uint32_t)M * g.N2 * 4u);
-    const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * g.N2 * 8u);
+    const uint32_t c = logical % D, grp0 = (logical / D) * per, N2 = g.N2;
+    const __amdgpu_buffer_rsrc_t rtb = make_rsrc(tb, (uint32_t)(P::M * P::NW) * N2 * 4u);
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * N2 * 8u);
     {
-        const float2* src = cls + cls_table_offset(D) + (size_t)c * (NB << BW);
-        for (int e = threadIdx.x; e < NB << BW; e += NT) TB[e >> BW][e & (int)MASK] = src[e];
+        const float2* src = cls + cls_table_offset(D) + (size_t)c * (P::NB << P::BW);
+        for (int e = threadIdx.x; e < P::NB << P::BW; e += NT) TB[e >> P::BW][e & (int)MASK] = src[e];
     }
     const uint32_t m4 = 4u * g.N1 - 1u, f = 4u * c + 1u;  // exponents of w_4N1
     {
+        static_assert(P::R1 * 16 == NT, "one factor per thread");
         const uint32_t q = threadIdx.x >> 4, i = threadIdx.x & 15u;
         uint32_t s = 2;  // the size of factor i and its index k at that size (dft_tw's order)
         while (s / 2u <= i && i > 0u) s *= 2u;
@@ -641,13 +550,43 @@ __global__ __launch_bounds__(FWD_NT, 2) void k_fwd_cols9p(FwdArgs a, Geom g, con
         tw2[q * stage_row<32>() + i] =
             w_4n1(g, tw14, twlo, twhi, ((32u / s) * (4u * (uint32_t)D * q + f) + k * (4u * g.N1 / s)) & m4);
     }
-    float2 tw1[8];
+    float2 tw1[P::R1 / 2];
 #pragma unroll
-    for (uint32_t i = 0; i < 8; ++i) {
-        const uint32_t s = i == 0 ? 2u : i == 1 ? 4u : i < 4 ? 8u : 16u, k = i ? i - s / 4u : 0u;
-        tw1[i] = uniform_f2(w_4n1(g, tw14, twlo, twhi, ((16u / s) * 32u * f + k * (4u * g.N1 / s)) & m4));
+    for (uint32_t i = 0; i < P::R1 / 2; ++i) {
+        const uint32_t s = i == 0 ? 2u : i == 1 ? 4u : i < 4 ? 8u : i < 8 ? 16u : 32u, k = i ? i - s / 4u : 0u;
+        tw1[i] = uniform_f2(w_4n1(g, tw14, twlo, twhi, ((P::R1 / s) * 32u * f + k * (4u * g.N1 / s)) & m4));
     }
-    fwd9_walk<D>(rtb, ry, g, twlo, twhi, buf, tw2, TB, tw1, c, grp0, per);
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    float2* seqbuf = buf + col * P::SEQS;
+    typename P::Bits tv;
+    float2 tw[10], twn[10];
+    // group grp0, peeled: every entry into the loop below then has the same memory-operation
+    // history (next group's loads, then this group's stores), so the compiler's waits on the
+    // prefetched registers count past the stores instead of draining them
+    uint32_t t2 = grp0 * 16u + (uint32_t)col;
+    fwd_load_bits<LGM, D>(tv, rtb, N2, t2, jt);
+    fwd_load_tw<LGM, D>(tw, twlo, twhi, g.L, c, t2, jt);
+    __syncthreads();  // tables
+    fwd_stage1<LGM, D>(tv, seqbuf, TB, tw1, jt);
+    __syncthreads();
+    if (per > 1) {
+        fwd_load_bits<LGM, D>(tv, rtb, N2, t2 + 16u, jt);
+        fwd_load_tw<LGM, D>(twn, twlo, twhi, g.L, c, t2 + 16u, jt);
+    }
+    fwd_stage2<LGM, D>(seqbuf, tw2, tw, ry, N2, c, t2, jt);
+    for (uint32_t it = 1; it < per; ++it) {
+        t2 += 16u;
+#pragma unroll
+        for (int e = 0; e < 10; ++e) tw[e] = twn[e];
+        __syncthreads();  // stage-2 reads of the previous group are done
+        fwd_stage1<LGM, D>(tv, seqbuf, TB, tw1, jt);
+        __syncthreads();
+        if (it + 1 < per) {
+            fwd_load_bits<LGM, D>(tv, rtb, N2, t2 + 16u, jt);
+            fwd_load_tw<LGM, D>(twn, twlo, twhi, g.L, c, t2 + 16u, jt);
+        }
+        fwd_stage2<LGM, D>(seqbuf, tw2, tw, ry, N2, c, t2, jt);
+    }
 }
 
 // Pass A for L <= 2^24 (N1 = 2^6 .. 2^10), straight from the key's and the seed's words: 16 adjacent
@@ -872,8 +811,7 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
 
 // ------------------------------------------------------------------ pass A' ----
 // Workgroup grp owns columns [W*grp, W*grp + W): G[t1] = FFT_N1(R'[.][t2])[t1] w_4N1^{t1}, so that the
-// conv values of positions t = t2 + N2 t1 and t + N are Re G / N and Im G / N.  R' is row-major, or pass
-// B's tiles when rt_tiled(LG1).
+// conv values of positions t = t2 + N2 t1 and t + N are Re G / N and Im G / N.  R' is in pass B's tiles.
 // Rounding: conv - mean_half(column) is an integer; its parity, corrected by the prefix parities (in
 // the output stage), is the product's bit.
 // A thread holds the outputs t1 = j + (N1/16) e, e < 16, of a column, so their bits are one 16-bit
@@ -924,14 +862,14 @@ __device__ __forceinline__ void inv_store(const float2 (&X)[16], float mean, con
     }
 }
 template <int LG1, bool BATCH>
-__global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_LG1 ? 2 : 1) void k_inv_cols(
+__global__ __launch_bounds__(inv_cols_threads(LG1), 2) void k_inv_cols(
     const float2* __restrict__ Rp, uint8_t* __restrict__ nib, Geom g, const uint32_t* __restrict__ info,
     const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
     float* __restrict__ margin, const BlockArgs* __restrict__ bt) {
     if constexpr (BATCH) {
         const BlockArgs& a = bt[blockIdx.z];
         g = a.g;
-        Rp = rt_tiled(LG1) ? a.Rt : a.Yk;
+        Rp = a.Rt;
         nib = a.nib;
         info = a.info;
         margin = a.margin;
@@ -939,9 +877,8 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
     constexpr int N1 = 1 << LG1;
     constexpr int W = inv_cols_width(LG1);
     constexpr int NT = inv_cols_threads(LG1);
-    constexpr int LGL = LG1 < 14 ? LG1 : 14;  // LDS transform length (N1 = 2^15: two halves)
-    constexpr int SEQS = seq_stride(1 << LGL);
-    constexpr int WL = (LG1 == RT_LG1 || LG1 >= 14) ? 1 : W;  // columns held in LDS at once
+    constexpr int SEQS = seq_stride(N1);
+    constexpr int WL = LG1 == RT_LG1 ? 1 : W;  // columns held in LDS at once
     constexpr int S = N1 / 16;
     __shared__ float2 buf[WL * SEQS];
     __shared__ float2 twl[TWL_SIZE];
@@ -951,83 +888,7 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
     float dist = 0.f;
     // w_4N1^{j} / N from the length-2L table (2L = 4 N1 N2)
     auto out_tw = [&](uint32_t j) { return cscale(tw_two_level(twlo, twhi, j * g.N2), g.inv_N); };
-    if constexpr (LG1 == 14) {
-        // Column pair t2 = 2 grp, 2 grp + 1 per 1024-thread workgroup, one column in LDS at a time
-        // (one workgroup per CU).  Thread j loads both columns of row k1 = j + 1024 r from pass B's
-        // tiles with one 16-byte load.
-        static_assert(W == 2 && NT == 1024 && rt_tiled(LG1) && S == NT, "paired column pass expects 2 columns, 1024 threads");
-        const int j = threadIdx.x;
-        float2 v0[16], v1[16];
-        const uint32_t c0 = grp * W;
-        {
-            const float2* tp = Rp + (size_t)(c0 / RT_COLS) * N1 * RT_COLS + (c0 % RT_COLS);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const float4 x = *reinterpret_cast<const float4*>(tp + (size_t)(j + NT * r) * RT_COLS);
-                v0[r] = make_float2(x.x, x.y);
-                v1[r] = make_float2(x.z, x.w);
-            }
-        }
-        const uint32_t pops = info[INFO_POPS];
-        const float2 wb = out_tw((uint32_t)j);
-        __syncthreads();  // twl
-#pragma unroll
-        for (int r = 0; r < 16; ++r) buf[padi(j + NT * r)] = v0[r];
-        __syncthreads();
-        lds_fft<LG1, 1, SEQS, NT>(buf, twl);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v0[e] = cmul(buf[padi(j + S * e)], wb);
-        inv_store(v0, mean_half(pops, c0), out, c0, (uint32_t)j, dist);
-        __syncthreads();  // the first column's reads are done
-#pragma unroll
-        for (int r = 0; r < 16; ++r) buf[padi(j + NT * r)] = v1[r];
-        __syncthreads();
-        lds_fft<LG1, 1, SEQS, NT>(buf, twl);
-#pragma unroll
-        for (int e = 0; e < 16; ++e) v1[e] = cmul(buf[padi(j + S * e)], wb);
-        inv_store(v1, mean_half(pops, c0 + 1u), out, c0 + 1u, (uint32_t)j, dist);
-    } else if constexpr (LG1 >= 14) {
-        // One column t2 = grp per workgroup.  N1 = 2^15 splits the column first by one radix-2 step in
-        // registers (X[2k] = FFT(a)[k], X[2k+1] = FFT(b)[k] with a = x[j] + x[j+N1/2],
-        // b = (x[j] - x[j+N1/2]) w_N1^j), then transforms the two 2^14-point halves in turn.
-        static_assert(W == 1 && NT == 1024 && rt_tiled(LG1), "single-column pass expects 1024 threads");
-        constexpr int H = 1 << LGL;       // points per LDS transform
-        constexpr int PT = N1 / NT;       // values per thread (32)
-        static_assert(N1 == 2 * H && S == 2 * NT, "two halves");
-        const uint32_t t2 = grp;
-        const float mean = mean_half(info[INFO_POPS], t2);
-        float2 v[PT];
-        {
-            const float2* tp = Rp + (size_t)(t2 / RT_COLS) * N1 * RT_COLS + (t2 % RT_COLS);
-#pragma unroll
-            for (int r = 0; r < PT; ++r) v[r] = tp[(size_t)(threadIdx.x + NT * r) * RT_COLS];
-        }
-        __syncthreads();  // twl
-        {
-            const uint32_t step = 2u * g.L / (uint32_t)N1;
-#pragma unroll
-            for (int r = 0; r < PT / 2; ++r) {
-                const float2 x0 = v[r], x1 = v[r + PT / 2];
-                v[r] = cadd(x0, x1);
-                v[r + PT / 2] = cmul(csub(x0, x1), tw_two_level(twlo, twhi, (threadIdx.x + NT * r) * step));
-            }
-        }
-#pragma unroll
-        for (int hv = 0; hv < 2; ++hv) {
-#pragma unroll
-            for (int r = 0; r < H / NT; ++r) buf[padi(threadIdx.x + NT * r)] = v[hv * (H / NT) + r];
-            __syncthreads();
-            lds_fft<LGL, 1, SEQS, NT>(buf, twl);
-            // t1 = 2 (tid + 1024 e) + hv
-            const uint32_t j = 2u * threadIdx.x + (uint32_t)hv;
-            const float2 wb = out_tw(j);
-            float2 X[16];
-#pragma unroll
-            for (int e = 0; e < 16; ++e) X[e] = cmul(buf[padi((int)threadIdx.x + NT * e)], wb);
-            inv_store(X, mean, out, t2, j, dist);
-            __syncthreads();  // reads done before the next half is written
-        }
-    } else if constexpr (LG1 == RT_LG1) {
+    if constexpr (LG1 == RT_LG1) {
         // One column pair t2 = 2 grp, 2 grp + 1 from pass B's tiles per 256-thread workgroup, one
         // column in LDS at a time (72 KB), so that two workgroups share a compute unit and one's
         // reads overlap the other's transforms.  Thread j loads both columns of row k1 = j + 256 r
@@ -1084,11 +945,7 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
         for (int i = 0; i < LPT; ++i) {
             const int e = threadIdx.x + i * NT;
             const uint32_t k1 = (uint32_t)(e / W), t2 = grp * W + (uint32_t)(e % W);
-            if constexpr (rt_tiled(LG1)) {  // pass B's tiles
-                v[i] = Rp[((size_t)(t2 / RT_COLS) * N1 + k1) * RT_COLS + t2 % RT_COLS];
-            } else {
-                v[i] = Rp[(size_t)k1 * g.N2 + t2];
-            }
+            v[i] = Rp[((size_t)(t2 / RT_COLS) * N1 + k1) * RT_COLS + t2 % RT_COLS];  // pass B's tiles
         }
 #pragma unroll
         for (int i = 0; i < LPT; ++i) {
@@ -1104,6 +961,87 @@ __global__ __launch_bounds__(inv_cols_threads(LG1), rt_tiled(LG1) && LG1 <= RT_L
         for (int e = 0; e < 16; ++e) X[e] = cmul(buf[col * SEQS + padi(j + S * e)], wb);
         const uint32_t t2 = grp * W + (uint32_t)col;
         inv_store(X, mean_half(info[INFO_POPS], t2), out, t2, (uint32_t)j, dist);
+    }
+    if (margin) margin_publish(dist, margin);
+}
+
+// N1 = 2^14, 2^15: a column of 128 or 256 KB leaves a single-pass kernel one or two columns per
+// workgroup, which refill L1 with 16 or 8 times the data (0.8 and 3.0 ms at 2^28 and 2^29).  Two
+// passes over whole 128-byte lines instead, k1 = j + J i with J = N1 / 1024:
+//   k_inv_big1: 1024-point FFTs over i, in place: Z_j[s] = sum_i R'[j + J i] w_1024^{i s} at row j + J s;
+//   k_inv_big2: G[s + 1024 b] = sum_j Z_j[s] w_N1^{(j + 1/4)(s + 1024 b)}, J points from J adjacent rows,
+//               in registers, then the rounding.
+// At 2^29: 0.79 ms (4.3 GB, the card's copy rate) + 0.43 ms (2.1 GB), from 3.02.
+template <int LG1, bool BATCH>
+__global__ __launch_bounds__(512) void k_inv_big1(float2* __restrict__ Rp, Geom g, const float2* __restrict__ tw14,
+                                                  const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) Rp = bt[blockIdx.z].Rt;
+    constexpr int N1 = 1 << LG1, J = N1 / 1024, NT = 512, SEQS = seq_stride(1024);
+    static_assert(RT_COLS == 16, "a workgroup has the columns of a tile");
+    __shared__ float2 buf[16 * SEQS];
+    __shared__ float2 tab[32 * stage_row<32>()];
+    const uint32_t logical = xcd_logical(blockIdx.x, gridDim.x), grp = logical / J, j = logical % J;
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(Rp, g.N1 * g.N2 * 8u);
+    // row j + J i, i = jt + 32 r
+    const uint32_t vo = ((grp * (uint32_t)N1 + j + (uint32_t)(J * jt)) * 16u + (uint32_t)col) * 8u;
+    float2 v[32];
+#pragma unroll
+    for (int r = 0; r < 32; ++r) v[r] = buf_load_f2(rs, vo, (uint32_t)(32 * J * r) * 128u);
+    fill_stage_table<32, 32>(tab, tw14, NT);
+    float2* seqbuf = buf + col * SEQS;
+    stage_first_to_lds<32>(v, seqbuf, jt);
+    __syncthreads();
+    stage_last_from_lds_tab<32, 1024>(v, seqbuf, jt, tab + jt * stage_row<32>());
+#pragma unroll
+    for (int r = 0; r < 32; ++r) buf_store_nt(v[r], rs, vo, (uint32_t)(32 * J * r) * 128u);
+}
+template <int LG1, bool BATCH>
+__global__ __launch_bounds__(256) void k_inv_big2(const float2* __restrict__ Rp, uint8_t* __restrict__ nib, Geom g,
+                                                  const uint32_t* __restrict__ info, const float2* __restrict__ twlo,
+                                                  const float2* __restrict__ twhi, float* __restrict__ margin,
+                                                  const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) {
+        const BlockArgs& a = bt[blockIdx.z];
+        g = a.g;
+        Rp = a.Rt;
+        nib = a.nib;
+        info = a.info;
+        margin = a.margin;
+    }
+    constexpr int N1 = 1 << LG1, J = N1 / 1024;
+    // 16 columns x 16 values of s per workgroup
+    const uint32_t logical = xcd_logical(blockIdx.x, gridDim.x);
+    const uint32_t grp = logical / 64u, s = (logical % 64u) * 16u + (threadIdx.x >> 4);
+    const uint32_t t2 = grp * 16u + (threadIdx.x & 15u);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(Rp, g.N1 * g.N2 * 8u);
+    const uint32_t vo = ((grp * (uint32_t)N1 + (uint32_t)J * s) * 16u + (threadIdx.x & 15u)) * 8u;
+    float2 v[J];
+#pragma unroll
+    for (int j = 0; j < J; ++j) v[j] = buf_load_f2(rs, vo, (uint32_t)(128 * j));
+    // w_N1^{j s} in the butterflies, K = w_4N1^s / N on the result; the output factor w_4J^b of b = e
+    // (J = 16) is inv_store's w_64^e, of b = 2e and 2e + 1 (J = 32) that and w_128 times it
+    const uint32_t u = s * g.N2;  // w_4N1^s = w_2L^u
+    const float2 K = cscale(tw_two_level(twlo, twhi, u), g.inv_N);
+    float2 pw[5], tw[J / 2];
+#pragma unroll
+    for (int m = J / 2, l = 0; m >= 1; m /= 2, ++l) pw[l] = tw_two_level(twlo, twhi, (4u * u * (uint32_t)m) & (2u * g.L - 1u));
+    twiddle_set<J>(tw, pw);
+    tw[0] = cmul(tw[0], K);
+#pragma unroll
+    for (int j = 0; j < J / 2; ++j) v[j] = cmul(v[j], K);
+    dft_tw<J>(v, tw);
+    const InvOut out(g, nib, N1 / 16, margin);
+    const float mean = mean_half(info[INFO_POPS], t2);
+    float dist = 0.f;
+    float2 X[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) X[e] = v[J / 16 * e];
+    inv_store(X, mean, out, t2, s, dist);
+    if constexpr (J == 32) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) X[e] = cmul(v[2 * e + 1], make_float2(9.987954562e-01f, -4.906767433e-02f));  // w_128
+        inv_store(X, mean, out, t2, s + 1024u, dist);
     }
     if (margin) margin_publish(dist, margin);
 }
@@ -1537,16 +1475,25 @@ hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uin
             return hipGetLastError();
         });
     return by_lg1(g.lg1, [&](auto lg) {
-        constexpr int LG1 = decltype(lg)::value, D = LG1 >= 13 ? 16 : 1 << (LG1 - 9);
-        if constexpr (LG1 <= 13) {
-            a.nA = g.N2 / 16u * (uint32_t)D / per;  // N2 / 16 = 512 groups and per divides it
-            k_fwd_cols9p<D, BATCH><<<dim3(a.nA * a.ops, 1, count), FWD_NT, 0, s>>>(a, g, t.tw14, t.lo, t.hi,
-                                                                                            t.cls, per, bt);
+        constexpr int LG1 = decltype(lg)::value, LGM = LG1 <= 13 ? 9 : 10, D = 1 << (LG1 - LGM);
+        a.nA = g.N2 / 16u * (uint32_t)D / per;  // N2 / 16 = 512 groups and per divides it
+        k_fwd_cols<LGM, D, BATCH><<<dim3(a.nA * a.ops, 1, count), fwd_cols_threads(LGM), 0, s>>>(a, g, t.tw14, t.lo, t.hi,
+                                                                                               t.cls, per, bt);
+        return hipGetLastError();
+    });
+}
+// Pass A' of `count` blocks (bt, BATCH) or one.
+template <bool BATCH>
+hipError_t inv_cols(float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t, float* margin,
+                    const BlockArgs* bt, uint32_t count, hipStream_t s) {
+    return by_lg1(g.lg1, [&](auto lg) {
+        constexpr int LG1 = decltype(lg)::value;
+        if constexpr (LG1 <= RT_LG1) {
+            k_inv_cols<LG1, BATCH><<<dim3(g.N2 / (uint32_t)inv_cols_width(LG1), 1, count), inv_cols_threads(LG1), 0, s>>>(
+                R, nib, g, info, t.tw14, t.lo, t.hi, margin, bt);
         } else {
-            constexpr int LGM = LG1 - 4;
-            a.nA = g.N2 / (uint32_t)fwd_cols_width(LGM) * (uint32_t)D;
-            k_fwd_cols<LGM, D, BATCH><<<dim3(a.nA * a.ops, 1, count), fwd_cols_threads(LGM), 0, s>>>(
-                a, g, t.tw14, t.lo, t.hi, t.cls, bt);
+            k_inv_big1<LG1, BATCH><<<dim3(g.N2 / 16u * (g.N1 / 1024u), 1, count), 512, 0, s>>>(R, g, t.tw14, bt);
+            k_inv_big2<LG1, BATCH><<<dim3(g.N2 / 16u * 64u, 1, count), 256, 0, s>>>(R, nib, g, info, t.lo, t.hi, margin, bt);
         }
         return hipGetLastError();
     });
@@ -1585,6 +1532,7 @@ hipError_t transpose(const uint32_t* key, const uint32_t* seed, uint32_t* tbk, u
     case 4: k_transpose_bits<4, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
     case 8: k_transpose_bits<8, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
     case 16: k_transpose_bits<16, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
+    case 32: k_transpose_bits<32, BATCH><<<grid, TB_NT, 0, s>>>(key, seed, tbk, tbs, first, g, sc, scan_wgs, bt); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
@@ -1645,14 +1593,9 @@ hipError_t launch_prefix_apply(uint32_t* q, const uint32_t* info, const Geom& g,
     return hipGetLastError();
 }
 
-hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
+hipError_t launch_inv_cols(float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
                            float* margin, hipStream_t s) {
-    return by_lg1(g.lg1, [&](auto lg) {
-        constexpr int LG1 = decltype(lg)::value;
-        k_inv_cols<LG1, false><<<g.N2 / (uint32_t)inv_cols_width(LG1), inv_cols_threads(LG1), 0, s>>>(
-            R, nib, g, info, t.tw14, t.lo, t.hi, margin, nullptr);
-        return hipGetLastError();
-    });
+    return inv_cols<false>(R, nib, g, info, t, margin, nullptr, 1, s);
 }
 
 uint32_t pack_halves(const Geom& g) { return (g.out_off < g.N ? 1u : 0u) + (g.out_off + g.out_bits > g.N ? 1u : 0u); }
@@ -1715,12 +1658,7 @@ hipError_t launch_batch_rows(int mode, const BlockArgs* bt, uint32_t count, cons
 }
 
 hipError_t launch_batch_inv_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
-    return by_lg1(g0.lg1, [&](auto lg) {
-        constexpr int LG1 = decltype(lg)::value;
-        k_inv_cols<LG1, true><<<dim3(g0.N2 / (uint32_t)inv_cols_width(LG1), 1, count), inv_cols_threads(LG1), 0, s>>>(
-            nullptr, nullptr, g0, nullptr, t.tw14, t.lo, t.hi, nullptr, bt);
-        return hipGetLastError();
-    });
+    return inv_cols<true>(nullptr, nullptr, g0, nullptr, t, nullptr, bt, count, s);
 }
 
 hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t halves, hipStream_t s) {

@@ -14,7 +14,6 @@ __host__ __device__ constexpr int rows_threads(int lg2) { return lg2 == 13 ? 256
 // Column passes for L <= 2^22: threads and first radix (16 columns, one second-stage butterfly each).
 __host__ __device__ constexpr int mid_threads(int lg1) { return lg1 >= 10 ? 512 : lg1 >= 8 ? 256 : 1 << lg1; }
 __host__ __device__ constexpr int mid_r1(int lg1) { return lg1 >= 10 ? 32 : lg1 >= 8 ? 16 : 1 << (lg1 - 4); }
-constexpr int FWD_NT = 256;   // threads of the forward column pass
 constexpr int TB_NT = 128;        // bit-transpose threads: 32 outputs each
 constexpr int TB_SPAN_LOG = 12;   // bit-transpose outputs per workgroup (2^12 of a row of N2 = 2^13)
 constexpr int POP_SLOTS = 64; // partial popcounts of a resident seed
@@ -38,20 +37,15 @@ __host__ __device__ constexpr int cls_table_size(int D) { return D * cls_tables(
 __host__ __device__ constexpr int cls_table_offset(int D) {
     return D <= 1 ? 0 : cls_table_offset(D / 2) + cls_table_size(D / 2);
 }
-constexpr int CLS_TABLE_TOTAL = cls_table_offset(32);  // D = 1 .. 16
+constexpr int CLS_TABLE_TOTAL = cls_table_offset(64);  // D = 1 .. 32
 
-// Columns per workgroup in pass A' (tile of W x N1 complex <= 16384 values in LDS) and its threads.
-// N1 = 2^9 takes 16 columns, 2^10 .. 2^12 take 8192 / N1 (about 68 KB of LDS) and N1 = 8192 takes 2
-// columns one at a time, so that two workgroups share a compute unit.  N1 = 2^14 takes 2 columns one
-// at a time (one workgroup per CU), N1 = 2^15 one column in two LDS halves.
-__host__ __device__ constexpr int inv_cols_width(int lg1) { return lg1 >= 15 ? 1 : (lg1 >= 13 ? 2 : 1 << (13 - lg1)); }
+// Columns per workgroup in pass A' and its threads: N1 = 2^11, 2^12 take 8192 / N1 (about 68 KB of LDS)
+// and N1 = 8192 takes 2 columns one at a time, so that two workgroups share a compute unit.
+__host__ __device__ constexpr int inv_cols_width(int lg1) { return lg1 >= 13 ? 2 : 1 << (13 - lg1); }
 __host__ __device__ constexpr int clamp_threads(int t) { return t < 64 ? 64 : (t > 1024 ? 1024 : t); }
-__host__ __device__ constexpr int inv_cols_threads(int lg1) { return lg1 == 13 ? 256 : (lg1 >= 14 ? 1024 : 512); }
-// Columns per workgroup in pass A (16; 8 when the class length M = 2048 would overflow LDS).
-__host__ __device__ constexpr int fwd_cols_width(int lgm) { return lgm >= 11 ? 8 : 16; }
-// Threads of the generic pass A: 1024 for classes of 1024 and 2048 points, whose 128 KB of columns
-// leave room for one workgroup per CU, so that it brings 16 waves instead of 4.
-__host__ __device__ constexpr int fwd_cols_threads(int lgm) { return lgm >= 10 ? 1024 : FWD_NT; }
+__host__ __device__ constexpr int inv_cols_threads(int lg1) { return lg1 == 13 ? 256 : 512; }
+// Threads of pass A: 16 columns, one second-stage butterfly each.
+__host__ __device__ constexpr int fwd_cols_threads(int lgm) { return 16 << (lgm - 5); }
 // Bytes of the nib buffer: pass A''s pieces (one bit per conv value, N/4 bytes), then the prefix
 // words (L/8 bytes).
 __host__ __device__ constexpr uint64_t nib_bytes(uint32_t N) { return N / 2 + 64; }
@@ -84,8 +78,8 @@ hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& 
                        const uint32_t* ws, uint32_t* seed_ws, hipStream_t s);
 // A resident seed's chunk-wise prefix words q[0 .. L/32) finished with its chunks' parities.
 hipError_t launch_prefix_apply(uint32_t* q, const uint32_t* info, const Geom& g, hipStream_t s);
-// R: pass B's output (the tile buffer when rt_tiled(g.lg1)).
-hipError_t launch_inv_cols(const float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
+// R: pass B's tiles (transformed in place from L = 2^28 on).
+hipError_t launch_inv_cols(float2* R, uint8_t* nib, const Geom& g, const uint32_t* info, const Tables& t,
                            float* margin, hipStream_t s);
 hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
                        const uint32_t* q, hipStream_t s);
