@@ -412,23 +412,23 @@ std::vector<float2> twiddles(uint64_t L, uint64_t count, uint64_t stride) {
 // times the +-1/2-encoded bits of a byte, in double precision, rounded once.
 std::vector<float2> class_tables() {
     std::vector<float2> t(pa::CLS_TABLE_TOTAL);
-    for (int D = 1; D <= 32; D *= 2) {
+    for (int D = 4; D <= 32; D *= 2) {
         const int BW = pa::cls_bits(D), NB = pa::cls_tables(D);
-        std::vector<double> re(4 * D), im(4 * D);  // half the 4D-th roots of unity
-        for (int k = 0; k < 4 * D; ++k) {
-            re[k] = 0.5 * std::cos(-2.0 * M_PI * k / (4.0 * D));
-            im[k] = 0.5 * std::sin(-2.0 * M_PI * k / (4.0 * D));
-        }
-        for (int c = 0; c < D; ++c)
+        for (int c = 0; c < D / 2; ++c)
             for (int q = 0; q < NB; ++q)
-                for (int byte = 0; byte < (1 << BW); ++byte) {
+                for (int index = 0; index < (1 << BW); ++index) {
                     double x = 0.0, y = 0.0;
-                    for (int b = 0; b < BW; ++b) {
-                        const int k = ((BW * q + b) * (4 * c + 1)) % (4 * D);
-                        x += ((byte >> b) & 1) ? re[k] : -re[k];
-                        y += ((byte >> b) & 1) ? im[k] : -im[k];
-                    }
-                    t[pa::cls_table_offset(D) + (c * NB + q) * (1 << BW) + byte] = make_float2((float)x, (float)y);
+                    for (int h = 0; h < (D <= 8 ? 2 : 1); ++h)
+                        for (int v = 0; v < D; ++v) {
+                            const int b = pa::mask_bit(D, h, v) - BW * q;
+                            if (b < 0 || b >= BW) continue;
+                            // -i of the second half: a quarter turn more
+                            const double w = -2.0 * M_PI * ((v * (4 * c + 1) + h * D) % (4 * D)) / (4.0 * D);
+                            const double sign = ((index >> b) & 1) ? 0.5 : -0.5;
+                            x += sign * std::cos(w);
+                            y += sign * std::sin(w);
+                        }
+                    t[pa::cls_table_offset(D) + ((c * NB + q) << BW) + index] = make_float2((float)x, (float)y);
                 }
     }
     return t;
@@ -1229,7 +1229,7 @@ int batch_tune_group(pa_engine* e, const BatchPlan& p, BatchGroup& gr, const pa:
     uint32_t best_per = 0;
     if (!mid_size(g0) && g0.lg1 <= 13) {
         // walk lengths that leave at least one workgroup per compute unit (and the default)
-        const uint32_t wgs = (g0.N2 / 16u) * g0.D * cnt;
+        const uint32_t wgs = (g0.N2 / 16u) * (g0.D / 2u) * cnt;  // a workgroup has a class pair
         float best = 1e30f;
         for (uint32_t per = 1; per <= pa::FWD_PER_MAX && rc == PA_OK; per *= 2) {
             if (per > 1u && wgs / per < (uint32_t)e->cus) break;
@@ -2294,7 +2294,7 @@ int st_unpack(pa_engine* e, Report& rp) {
             par = want & 1u;
             if (pre[i] != want) rp.fail("BinInt2float: n = 2^%u prefix word %u = %08x, want %08x", lg, i, pre[i], want);
         }
-        // tb[u N2 + t2] = E | O << 16: bit v of E / O = seed bit t2 + N2 (u + M v) / that + N
+        // tb[u N2 + t2]: seed bit t2 + N2 (u + M v) / that + N at mask_bit(D, 0 / 1, v)
         const uint64_t words = tb.size(), checks = std::min<uint64_t>(words, 65536);
         for (uint64_t c = 0; c < checks && rp.ok; ++c) {
             lcg = lcg * 6364136223846793005ull + 1442695040888963407ull;
@@ -2303,8 +2303,8 @@ int st_unpack(pa_engine* e, Report& rp) {
             uint32_t want = 0;
             for (uint32_t v = 0; v < g.D; ++v) {
                 const uint64_t p = t2 + (uint64_t)g.N2 * (u + (uint64_t)g.M * v);
-                want |= refbit(bin.data(), p) << v;
-                want |= refbit(bin.data(), p + g.N) << (16 + v);
+                want |= refbit(bin.data(), p) << pa::mask_bit(g.D, 0, v);
+                want |= refbit(bin.data(), p + g.N) << pa::mask_bit(g.D, 1, v);
             }
             if (tb[idx] != want) rp.fail("BinInt2float: n = 2^%u bit word %llu = %08x, want %08x", lg,
                                          (unsigned long long)idx, tb[idx], want);

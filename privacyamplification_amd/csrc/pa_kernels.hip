@@ -271,8 +271,8 @@ __device__ __forceinline__ void bit_transpose(uint32_t (&A)[32]) {
     bit_transpose_round<1>(A);
 }
 
-// tb[u*N2 + t2] = E | O << 16 with E bit v = x[t2 + N2(u + M v)], O bit v = x[N + t2 + N2(u + M v)]
-// (D = 32: E at tb[u*N2 + t2] and O at tb[(M + u) N2 + t2]).
+// tb[u*N2 + t2] has x[t2 + N2(u + M v)] and x[N + t2 + N2(u + M v)] at bits mask_bit(D, 0, v) and
+// mask_bit(D, 1, v) (D = 32: the second half's in the word tb[(M + u) N2 + t2]).
 // Workgroup (u, part): thread k covers t2 in [part*TB_SPAN + 32k, +32): for each class v it reads
 // the two words holding those bits (coalesced across the workgroup), transposes the 2 D x 32 bits
 // in registers, and the workgroup writes its TB_SPAN outputs through LDS.  The launch's first
@@ -318,49 +318,25 @@ __global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __rest
     }
     uint32_t* srow = stage + threadIdx.x * 33;
     uint32_t* out = tb + (size_t)u * g.N2 + (part << TB_SPAN_LOG);
-    auto write = [&] {
-        __syncthreads();
-        for (int e = threadIdx.x; e < (1 << TB_SPAN_LOG); e += TB_NT) out[e] = stage[(e >> 5) * 33 + (e & 31)];
-    };
-    if constexpr (D == 32) {  // a word per half: E in the first M N2 words, O in the next
+    // Row A[31 - i] = the words of bit i, transposed: A[c] then holds bit 31 - c (column t0 + c) of
+    // each at its place.
+    constexpr int NW = D == 32 ? 2 : 1;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            uint32_t A[32];
+    for (int k = 0; k < NW; ++k) {
+        uint32_t A[32] = {};
 #pragma unroll
-            for (int v = 0; v < 32; ++v) A[31 - v] = h ? w1[v] : w0[v];
-            bit_transpose(A);
-            if (h) __syncthreads();  // the first half has been written out
-#pragma unroll
-            for (int i = 0; i < 32; ++i) srow[i] = A[i];
-            write();
-            out += (size_t)g.M * g.N2;
-        }
-        return;
-    } else if constexpr (D >= 8) {
-        // Rows A[15 - v] = w1[v], A[31 - v] = w0[v] (zero for v >= D), transposed: A[c] then holds
-        // bit 31 - c (column t0 + c) of w0[v] at bit v and of w1[v] at bit v + 16: output c.
-        uint32_t A[32];
-#pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            A[15 - v] = v < D ? w1[v < D ? v : 0] : 0u;
-            A[31 - v] = v < D ? w0[v < D ? v : 0] : 0u;
+        for (int v = 0; v < D; ++v) {
+            A[31 - mask_bit(D, k, v)] = k ? w1[v] : w0[v];
+            if constexpr (NW == 1) A[31 - mask_bit(D, 1, v)] = w1[v];
         }
         bit_transpose(A);
+        if (k) __syncthreads();  // the first half has been written out
 #pragma unroll
         for (int i = 0; i < 32; ++i) srow[i] = A[i];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 32; ++i) {
-            uint32_t E = 0, O = 0;
-#pragma unroll
-            for (int v = 0; v < D; ++v) {
-                E |= ((w0[v] >> (31 - i)) & 1u) << v;
-                O |= ((w1[v] >> (31 - i)) & 1u) << v;
-            }
-            srow[i] = E | (O << 16);
-        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < (1 << TB_SPAN_LOG); e += TB_NT) out[e] = stage[(e >> 5) * 33 + (e & 31)];
+        out += (size_t)g.M * g.N2;
     }
-    write();
 }
 
 // ------------------------------------------------------------------ pass A ----
@@ -413,21 +389,23 @@ __device__ __forceinline__ uint32_t buf_load_u32(__amdgpu_buffer_rsrc_t rs, uint
     return __builtin_amdgcn_raw_buffer_load_b32(rs, (int)voff, (int)soff, 0);
 }
 
-// Pass A for L >= 2^25: a workgroup has 16 columns (group grp) and one class c of D, and computes
-// Y[k1][t2] for k1 = c + D k1', at the quarter-shifted frequencies k1 + 1/4 (c' = c + 1/4):
+// Pass A for L >= 2^25: a workgroup has 16 columns (group grp) and a pair of classes of the D, c = p
+// and p + D/2, and computes Y[k1][t2] for k1 = c + D k1', at the quarter-shifted frequencies k1 + 1/4
+// (c' = c + 1/4):
 //   Y = w_N^{t2 (k1 + 1/4)} * FFT_M( w_N1^{u c'} * sum_v z[t2 + N2(u + M v)] w_D^{v c'} ),
-// z[t] = a[t] - i a[t + N], a = bit - 1/2.  The class sum over v is one 256-entry table lookup per byte
-// of the bit masks, the -1/2 included in the tables.
+// z[t] = a[t] - i a[t + N], a = bit - 1/2.  The sums over the even and the odd v are table lookups by
+// the mask's bits (the -1/2 included) and serve both classes: their sum and their difference.
 // Plan R1 x 32 with M = 32 R1: M = 512 for N1 <= 2^13 (256 threads, two workgroups per compute unit),
 // M = 1024 for 2^14 and 2^15 (512 threads, one: its 16 columns take 135 KB of LDS).
 template <int LGM, int D>
 struct FwdPlan {
     static constexpr int M = 1 << LGM, R1 = M / 32, NT = fwd_cols_threads(LGM), JT = NT / 16, K1 = 32 / JT;
     static constexpr int NW = D == 32 ? 2 : 1;   // mask words per position (both halves in one up to D = 16)
-    static constexpr int BW = cls_bits(D), NB = cls_tables(D);  // bits per table, tables per half
+    static constexpr int BW = cls_bits(D), NB = cls_tables(D);  // index bits of a table, tables of a pair
     static constexpr int SEQS = seq_stride(M);
     static_assert(JT == R1, "one second-stage butterfly per thread");
     using Bits = uint32_t[K1][R1][NW];
+    using Sums = float2[K1][R1];
     using Tables = float2[NB][1 << BW];
 };
 // Pieces of the persistent walk.  Thread (col = t mod 16, jt = t / 16).
@@ -446,60 +424,80 @@ __device__ __forceinline__ void fwd_load_bits(typename FwdPlan<LGM, D>::Bits& tv
                 tv[i][r][h] = buf_load_u32(rtb, voff, (uint32_t)(32 * r + P::M * h) * N2 * 4u);
     }
 }
-// Table entries of the output twiddles w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + R1 r) = base step^r, with
-// anchors w_N^{t2 R1 D 8 (a+1)}: (lo, hi) pairs of base, step, anchor 0..2.  The products are
-// formed where they are used, so that gathering them never waits on other loads.
+// Class sums of p (a) and p + D/2 (d).
 template <int LGM, int D>
-__device__ __forceinline__ void fwd_load_tw(float2 (&tw)[10], const float2* __restrict__ lo,
-                                            const float2* __restrict__ hi, uint32_t L, uint32_t c, uint32_t t2, int jt) {
+__device__ __forceinline__ void fwd_sums(typename FwdPlan<LGM, D>::Sums& a, typename FwdPlan<LGM, D>::Sums& d,
+                                         const typename FwdPlan<LGM, D>::Bits& tv,
+                                         const typename FwdPlan<LGM, D>::Tables& TB) {
+    using P = FwdPlan<LGM, D>;
+    constexpr uint32_t MASK = (1u << P::BW) - 1u;
+#pragma unroll
+    for (int i = 0; i < P::K1; ++i)
+#pragma unroll
+        for (int r = 0; r < P::R1; ++r) {
+            const uint32_t w0 = tv[i][r][0], w1 = P::NW == 2 ? tv[i][r][P::NW - 1] : w0 >> 16;
+            float2 s[2];
+#pragma unroll
+            for (int o = 0; o < 2; ++o) {
+                if constexpr (D <= 8) {
+                    s[o] = TB[o][(w0 >> (D * o)) & MASK];
+                } else {
+                    constexpr int H = P::NB / 2;
+                    float2 e = TB[H * o][(w0 >> (8 * H * o)) & MASK], f = TB[H * o][(w1 >> (8 * H * o)) & MASK];
+#pragma unroll
+                    for (int q = 1; q < H; ++q) {
+                        e = cadd(e, TB[H * o + q][(w0 >> (8 * (H * o + q))) & MASK]);
+                        f = cadd(f, TB[H * o + q][(w1 >> (8 * (H * o + q))) & MASK]);
+                    }
+                    s[o] = make_float2(e.x + f.y, e.y - f.x);
+                }
+            }
+            a[i][r] = cadd(s[0], s[1]);
+            d[i][r] = csub(s[0], s[1]);
+        }
+}
+// Table entries of the output twiddles w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + R1 r) = base step^r, with
+// anchors w_N^{t2 R1 D 8 (a+1)}: (lo, hi) pairs of the base for c = p, step, anchor 0..2 and the base for
+// p + D/2.  The products are formed where they are used, so that gathering them never waits on other
+// loads.
+template <int LGM, int D>
+__device__ __forceinline__ void fwd_load_tw(float2 (&tw)[12], const float2* __restrict__ lo,
+                                            const float2* __restrict__ hi, uint32_t L, uint32_t p, uint32_t t2, int jt) {
     constexpr uint32_t R1 = FwdPlan<LGM, D>::R1;
     const uint32_t L2m = 2u * L - 1u;
-    uint32_t x[5];
-    x[0] = (t2 * (4u * (c + (uint32_t)D * (uint32_t)jt) + 1u)) & L2m;
+    uint32_t x[6];
+    x[0] = (t2 * (4u * (p + (uint32_t)D * (uint32_t)jt) + 1u)) & L2m;
     x[1] = (t2 * (4u * R1 * (uint32_t)D)) & L2m;
 #pragma unroll
     for (int a = 0; a < 3; ++a) x[2 + a] = (t2 * (4u * R1 * (uint32_t)D * 8u * (uint32_t)(a + 1))) & L2m;
+    x[5] = (x[0] + t2 * (2u * (uint32_t)D)) & L2m;
 #pragma unroll
-    for (int e = 0; e < 5; ++e) {
+    for (int e = 0; e < 6; ++e) {
         tw[2 * e] = lo[x[e] & (TW14 - 1)];
         tw[2 * e + 1] = hi[x[e] >> TW14_LOG];
     }
 }
-// tw1: the first stage's factors for w_N1^{32 c'} (one class per workgroup: uniform).
+// tw1: the first stage's factors for w_N1^{32 c'} (one class pair per workgroup: uniform).
 template <int LGM, int D>
-__device__ __forceinline__ void fwd_stage1(const typename FwdPlan<LGM, D>::Bits& tv, float2* seqbuf,
-                                           const typename FwdPlan<LGM, D>::Tables& TB,
+__device__ __forceinline__ void fwd_stage1(typename FwdPlan<LGM, D>::Sums& v, float2* seqbuf,
                                            const float2 (&tw1)[FwdPlan<LGM, D>::R1 / 2], int jt) {
     using P = FwdPlan<LGM, D>;
-    constexpr uint32_t MASK = (1u << P::BW) - 1u;
 #pragma unroll
     for (int i = 0; i < P::K1; ++i) {
-        const int j = jt + P::JT * i;
-        float2 v[P::R1];
+        dft_tw<P::R1>(v[i], tw1);
 #pragma unroll
-        for (int r = 0; r < P::R1; ++r) {
-            const uint32_t tE = tv[i][r][0], tO = P::NW == 2 ? tv[i][r][P::NW - 1] : tE >> 16;
-            float2 sE = TB[0][tE & MASK], sO = TB[0][tO & MASK];
-#pragma unroll
-            for (int q = 1; q < P::NB; ++q) {
-                sE = cadd(sE, TB[q][(tE >> (P::BW * q)) & MASK]);
-                sO = cadd(sO, TB[q][(tO >> (P::BW * q)) & MASK]);
-            }
-            v[r] = make_float2(sE.x + sO.y, sE.y - sO.x);
-        }
-        dft_tw<P::R1>(v, tw1);
-#pragma unroll
-        for (int r = 0; r < P::R1; ++r) seqbuf[padi(j * P::R1 + r)] = v[r];
+        for (int r = 0; r < P::R1; ++r) seqbuf[padi((jt + P::JT * i) * P::R1 + r)] = v[i][r];
     }
 }
 // tw2: the second stage's factors, row jt for w_M^jt w_N1^c' (the class twiddle of input j).
 template <int LGM, int D>
-__device__ __forceinline__ void fwd_stage2(const float2* seqbuf, const float2* tw2, const float2 (&tw)[10],
-                                           __amdgpu_buffer_rsrc_t ry, uint32_t N2, uint32_t c, uint32_t t2, int jt) {
+__device__ __forceinline__ void fwd_stage2(const float2* seqbuf, const float2* tw2, const float2 base,
+                                           const float2 (&tw)[12], __amdgpu_buffer_rsrc_t ry, uint32_t N2, uint32_t c,
+                                           uint32_t t2, int jt) {
     using P = FwdPlan<LGM, D>;
     float2 F[32];
     stage_last_from_lds_tab<32, P::M>(F, seqbuf, jt, tw2 + jt * stage_row<32>());
-    const float2 base = cmul(tw[0], tw[1]), step = cmul(tw[2], tw[3]);
+    const float2 step = cmul(tw[2], tw[3]);
     const uint32_t voff = ((c + (uint32_t)D * (uint32_t)jt) * N2 + t2) * 8u;
     float2 w = base;
 #pragma unroll
@@ -510,22 +508,25 @@ __device__ __forceinline__ void fwd_stage2(const float2* seqbuf, const float2* t
     }
 }
 
-// Persistent: workgroup L of G keeps one class c = L mod D and walks the column groups
-// [k per, k per + per), k = L / D, so its class tables are loaded once, and each group's stores drain
-// while the next group is transformed (its loads were issued before those stores).  The D workgroups
+// Persistent: workgroup L of G keeps one class pair p = L mod D/2 and walks the column groups
+// [k per, k per + per), k = L / (D/2), so its tables are loaded once, and each group's stores drain
+// while the next group is transformed (its loads were issued before those stores).  The workgroups
 // of one k sit on one XCD and walk the same groups in step, so each bit word is fetched into L2 once.
 // The class twiddles w_N1^{u c'}, u = j + 32 r, cost nothing: their r part is in the first stage's
 // factors, their j part in the second's.
+// Both operands at 2^27: 0.277 ms (one class per workgroup: 0.32), of which storing the 1.07 GB in this
+// order alone takes 0.237; at 2^29 1.54 ms (2.23), storing alone 0.84, the rest the lookups, 4 a value.
 template <int LGM, int D, bool BATCH>
 __global__ __launch_bounds__(fwd_cols_threads(LGM), LGM == 9 ? 2 : 1) void k_fwd_cols(
     FwdArgs a, Geom g, const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
     const float2* __restrict__ cls, uint32_t per, const BlockArgs* __restrict__ bt) {
     fwd_batch_args<BATCH, false>(a, g, bt);
     using P = FwdPlan<LGM, D>;
-    constexpr int NT = P::NT;
+    constexpr int NT = P::NT, TW2 = P::R1 * stage_row<32>(), R1H = P::R1 / 2;
     constexpr uint32_t MASK = (1u << P::BW) - 1u;
     __shared__ float2 buf[16 * P::SEQS];
-    __shared__ float2 tw2[P::R1 * stage_row<32>()];
+    __shared__ float2 tw2[2 * TW2];
+    __shared__ float2 tw1s[2 * R1H];
     __shared__ typename P::Tables TB;
     const uint32_t op = blockIdx.x / a.nA;
     const bool is_seed = a.first + op == 1u;
@@ -533,59 +534,80 @@ __global__ __launch_bounds__(fwd_cols_threads(LGM), LGM == 9 ? 2 : 1) void k_fwd
     float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
     if (BATCH && tb == nullptr) return;  // resident seed: nothing to transform
     const uint32_t logical = xcd_logical(blockIdx.x - op * a.nA, a.nA);
-    const uint32_t c = logical % D, grp0 = (logical / D) * per, N2 = g.N2;
+    const uint32_t p = logical % (D / 2), grp0 = (logical / (D / 2)) * per, N2 = g.N2;
     const __amdgpu_buffer_rsrc_t rtb = make_rsrc(tb, (uint32_t)(P::M * P::NW) * N2 * 4u);
     const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * N2 * 8u);
     {
-        const float2* src = cls + cls_table_offset(D) + (size_t)c * (P::NB << P::BW);
+        const float2* src = cls + cls_table_offset(D) + (size_t)p * (P::NB << P::BW);
         for (int e = threadIdx.x; e < P::NB << P::BW; e += NT) TB[e >> P::BW][e & (int)MASK] = src[e];
     }
-    const uint32_t m4 = 4u * g.N1 - 1u, f = 4u * c + 1u;  // exponents of w_4N1
+    const uint32_t m4 = 4u * g.N1 - 1u;  // exponents of w_4N1
     {
         static_assert(P::R1 * 16 == NT, "one factor per thread");
         const uint32_t q = threadIdx.x >> 4, i = threadIdx.x & 15u;
         uint32_t s = 2;  // the size of factor i and its index k at that size (dft_tw's order)
         while (s / 2u <= i && i > 0u) s *= 2u;
         const uint32_t k = i ? i - s / 4u : 0u;
-        tw2[q * stage_row<32>() + i] =
-            w_4n1(g, tw14, twlo, twhi, ((32u / s) * (4u * (uint32_t)D * q + f) + k * (4u * g.N1 / s)) & m4);
-    }
-    float2 tw1[P::R1 / 2];
 #pragma unroll
-    for (uint32_t i = 0; i < P::R1 / 2; ++i) {
-        const uint32_t s = i == 0 ? 2u : i == 1 ? 4u : i < 4 ? 8u : i < 8 ? 16u : 32u, k = i ? i - s / 4u : 0u;
-        tw1[i] = uniform_f2(w_4n1(g, tw14, twlo, twhi, ((P::R1 / s) * 32u * f + k * (4u * g.N1 / s)) & m4));
+        for (uint32_t o = 0; o < 2; ++o) {
+            const uint32_t f = 4u * (p + o * (D / 2)) + 1u;
+            tw2[o * TW2 + q * stage_row<32>() + i] =
+                w_4n1(g, tw14, twlo, twhi, ((32u / s) * (4u * (uint32_t)D * q + f) + k * (4u * g.N1 / s)) & m4);
+            if (q == 0 && i < (uint32_t)R1H)
+                tw1s[o * R1H + i] = w_4n1(g, tw14, twlo, twhi, ((P::R1 / s) * 32u * f + k * (4u * g.N1 / s)) & m4);
+        }
     }
     const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
     float2* seqbuf = buf + col * P::SEQS;
     typename P::Bits tv;
-    float2 tw[10], twn[10];
-    // group grp0, peeled: every entry into the loop below then has the same memory-operation
-    // history (next group's loads, then this group's stores), so the compiler's waits on the
-    // prefetched registers count past the stores instead of draining them
+    float2 tw[12], twn[12];
     uint32_t t2 = grp0 * 16u + (uint32_t)col;
     fwd_load_bits<LGM, D>(tv, rtb, N2, t2, jt);
-    fwd_load_tw<LGM, D>(tw, twlo, twhi, g.L, c, t2, jt);
+    fwd_load_tw<LGM, D>(tw, twlo, twhi, g.L, p, t2, jt);
     __syncthreads();  // tables
-    fwd_stage1<LGM, D>(tv, seqbuf, TB, tw1, jt);
-    __syncthreads();
-    if (per > 1) {
-        fwd_load_bits<LGM, D>(tv, rtb, N2, t2 + 16u, jt);
-        fwd_load_tw<LGM, D>(twn, twlo, twhi, g.L, c, t2 + 16u, jt);
+    // The first stage's factors: in scalar registers where they fit, else read again for each use.
+    float2 f0[R1H], f1[R1H];
+    auto factors = [&](float2 (&f)[R1H], int o) {
+#pragma unroll
+        for (int i = 0; i < R1H; ++i) f[i] = tw1s[o * R1H + i];
+    };
+    if constexpr (P::R1 <= 16) {
+        factors(f0, 0);
+        factors(f1, 1);
+#pragma unroll
+        for (int i = 0; i < R1H; ++i) {
+            f0[i] = uniform_f2(f0[i]);
+            f1[i] = uniform_f2(f1[i]);
+        }
     }
-    fwd_stage2<LGM, D>(seqbuf, tw2, tw, ry, N2, c, t2, jt);
+    typename P::Sums va, vd;
+    // One column group; more: the next one's loads are issued before its last stores.
+    auto group = [&](bool more) {
+        fwd_sums<LGM, D>(va, vd, tv, TB);
+        if constexpr (P::R1 > 16) factors(f0, 0);
+        fwd_stage1<LGM, D>(va, seqbuf, f0, jt);
+        __syncthreads();
+        fwd_stage2<LGM, D>(seqbuf, tw2, cmul(tw[0], tw[1]), tw, ry, N2, p, t2, jt);
+        __syncthreads();
+        if constexpr (P::R1 > 16) factors(f1, 1);
+        fwd_stage1<LGM, D>(vd, seqbuf, f1, jt);
+        __syncthreads();
+        if (more) {
+            fwd_load_bits<LGM, D>(tv, rtb, N2, t2 + 16u, jt);
+            fwd_load_tw<LGM, D>(twn, twlo, twhi, g.L, p, t2 + 16u, jt);
+        }
+        fwd_stage2<LGM, D>(seqbuf, tw2 + TW2, cmul(tw[10], tw[11]), tw, ry, N2, p + D / 2, t2, jt);
+    };
+    // The first group is peeled: every entry into the loop then has the same memory-operation
+    // history (next group's loads, then this group's stores), so the compiler's waits on the
+    // prefetched registers count past the stores instead of draining them.
+    group(per > 1);
     for (uint32_t it = 1; it < per; ++it) {
         t2 += 16u;
 #pragma unroll
-        for (int e = 0; e < 10; ++e) tw[e] = twn[e];
-        __syncthreads();  // stage-2 reads of the previous group are done
-        fwd_stage1<LGM, D>(tv, seqbuf, TB, tw1, jt);
-        __syncthreads();
-        if (it + 1 < per) {
-            fwd_load_bits<LGM, D>(tv, rtb, N2, t2 + 16u, jt);
-            fwd_load_tw<LGM, D>(twn, twlo, twhi, g.L, c, t2 + 16u, jt);
-        }
-        fwd_stage2<LGM, D>(seqbuf, tw2, tw, ry, N2, c, t2, jt);
+        for (int e = 0; e < 12; ++e) tw[e] = twn[e];
+        __syncthreads();  // second-stage reads of the previous group are done
+        group(it + 1 < per);
     }
 }
 
@@ -1476,7 +1498,7 @@ hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uin
         });
     return by_lg1(g.lg1, [&](auto lg) {
         constexpr int LG1 = decltype(lg)::value, LGM = LG1 <= 13 ? 9 : 10, D = 1 << (LG1 - LGM);
-        a.nA = g.N2 / 16u * (uint32_t)D / per;  // N2 / 16 = 512 groups and per divides it
+        a.nA = g.N2 / 16u * (uint32_t)(D / 2) / per;  // N2 / 16 = 512 groups and per divides it
         k_fwd_cols<LGM, D, BATCH><<<dim3(a.nA * a.ops, 1, count), fwd_cols_threads(LGM), 0, s>>>(a, g, t.tw14, t.lo, t.hi,
                                                                                                t.cls, per, bt);
         return hipGetLastError();
@@ -1570,17 +1592,19 @@ hipError_t launch_transpose(const uint32_t* key, const uint32_t* seed, uint32_t*
     return transpose<false>(key, seed, tbk, tbs, first, ops, g, scan, scan ? scan_chunks(g) : 0u, nullptr, 1, s);
 }
 
+// Column groups a workgroup of pass A walks: 8, fewer while that would leave under 512 workgroups per
+// operand (two per compute unit).  Fresh seed: 2^25 265 us with 2 and 4, 273 with 8, 325 with 16; 2^26
+// 475 with 4, 485 with 2 and 8; 2^27 891 with 8, 906 with 4, 895 with 16; 2^28 and 2^29 within 1%.
+static uint32_t default_walk(const Geom& g, uint32_t count) {
+    uint32_t per = 8u;
+    while (per > 1u && g.N2 / 16u * (g.D / 2u) / per * count < 512u) per >>= 1;
+    return per;
+}
+
 hipError_t launch_fwd_cols(const uint32_t* key_in, const uint32_t* seed_in, float2* Yk, float2* Ys, uint32_t first,
                            uint32_t ops, const Geom& g, const Tables& t, const ScanArgs* scan, hipStream_t s) {
-    // The persistent form: each workgroup holds one class of one operand and walks `per` column
-    // groups: 16 (8 for a single operand), fewer while that would leave under 256 (512) workgroups
-    // per operand.  1024 workgroups at 2^27, two waves of two per CU: as fast as one persistent
-    // wave, and a CU that cannot take its second workgroup at once delays a short walk, not a long one.
-    const uint32_t target = ops == 2u ? 256u : 512u;
-    uint32_t per = ops == 2u ? 16u : 8u;
-    while (per > 1u && g.N2 / 16u * g.D / per < target) per >>= 1;
     FwdArgs a{{key_in, seed_in}, {Yk, Ys}, first, ops, 0u, scan ? *scan : ScanArgs{}};
-    return fwd_cols<false>(a, g, t, per, scan ? scan_chunks(g) : 0u, nullptr, 1, s);
+    return fwd_cols<false>(a, g, t, default_walk(g, 1), scan ? scan_chunks(g) : 0u, nullptr, 1, s);
 }
 
 hipError_t launch_rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, uint32_t* info,
@@ -1642,10 +1666,7 @@ hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geo
 hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, uint32_t ops,
                                  uint32_t per, hipStream_t s) {
     const uint32_t groups = g0.N2 / 16u;
-    if (per == 0u) {
-        per = 16u;
-        while (per > 1u && groups * g0.D / per * count * ops < 512u) per >>= 1;
-    }
+    if (per == 0u) per = default_walk(g0, count);
     if (per > FWD_PER_MAX || (per & (per - 1u)) != 0u || (!mid_size(g0) && groups % per != 0u)) return hipErrorInvalidValue;
     FwdArgs a{};
     a.ops = ops;

@@ -22,9 +22,13 @@ constexpr int PACK_CW = 16;
 
 // Device twiddle tables: tw14[x] = exp(-2 pi i x / 2^14); lo/hi: exp(-2 pi i x / (2L)) split as
 // lo[x mod 2^14] * hi[x >> 14].
-// cls: pass A's class tables, cls_table_offset(D) onwards: entry [(c NB + q) 2^BW + byte] =
-// sum over the bits b of byte of (bit - 1/2) exp(-2 pi i (BW q + b)(c + 1/4) / D), BW = min(D, 8),
-// NB = D / BW; computed in double precision and rounded once.
+// cls: pass A's tables, cls_table_offset(D) onwards, of the class pairs (p, p + D/2), p < D/2.
+// The sum over v of z[v] w_D^{v (c + 1/4)} is S_even + S_odd for c = p and S_even - S_odd for
+// c = p + D/2, S_even over the even v.  Table q of pair p, entries [(p NB + q) 2^BW + index], BW index
+// bits: up to D = 8, q = 0 is S_even and q = 1 S_odd, and the index is the bits of a's D/2 values and
+// above them those of a[. + N] (z = a - i a[. + N]).  From D = 16 on the sums of one half's bits are
+// split into bytes, q < NB/2 even and the others odd.  a = bit - 1/2; computed in double precision
+// and rounded once.
 struct Tables {
     const float2* tw14;
     const float2* lo;
@@ -32,12 +36,16 @@ struct Tables {
     const float2* cls;
 };
 __host__ __device__ constexpr int cls_bits(int D) { return D < 8 ? D : 8; }
-__host__ __device__ constexpr int cls_tables(int D) { return D / cls_bits(D); }
-__host__ __device__ constexpr int cls_table_size(int D) { return D * cls_tables(D) * (1 << cls_bits(D)); }
+__host__ __device__ constexpr int cls_tables(int D) { return D <= 8 ? 2 : D / 8; }
+__host__ __device__ constexpr int cls_table_size(int D) { return D / 2 * cls_tables(D) * (1 << cls_bits(D)); }
 __host__ __device__ constexpr int cls_table_offset(int D) {
-    return D <= 1 ? 0 : cls_table_offset(D / 2) + cls_table_size(D / 2);
+    return D <= 4 ? 0 : cls_table_offset(D / 2) + cls_table_size(D / 2);
 }
-constexpr int CLS_TABLE_TOTAL = cls_table_offset(64);  // D = 1 .. 32
+constexpr int CLS_TABLE_TOTAL = cls_table_offset(64);  // D = 4 .. 32
+// Place in a mask word (D = 32: a word per half) of class bit v of half h, in the tables' order.
+__host__ __device__ constexpr int mask_bit(int D, int h, int v) {
+    return D <= 8 ? (v & 1) * D + h * (D / 2) + v / 2 : (D == 16 ? 16 * h : 0) + (v & 1) * (D / 2) + v / 2;
+}
 
 // Columns per workgroup in pass A' and its threads: N1 = 2^11, 2^12 take 8192 / N1 (about 68 KB of LDS)
 // and N1 = 8192 takes 2 columns one at a time, so that two workgroups share a compute unit.
@@ -95,8 +103,7 @@ hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2*
 uint32_t pack_halves(const Geom& g);  // halves of the conv positions (t, t + N) the window touches
 // ops: 1 (key) or 2 (key and seed).
 hipError_t launch_batch_transpose(const BlockArgs* bt, uint32_t count, const Geom& g0, uint32_t ops, hipStream_t s);
-// per: column groups each workgroup of the persistent pass A (N1 = 2^9 .. 2^13, N2 = 8192) walks, a
-// power of two up to 32; 0 picks 16, halved while the launch would have under 512 workgroups.
+// per: column groups each workgroup of pass A walks (L >= 2^25), a power of two up to 32; 0 picks one.
 hipError_t launch_batch_fwd_cols(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, uint32_t ops,
                                  uint32_t per, hipStream_t s);
 constexpr uint32_t FWD_PER_MAX = 32;
