@@ -216,7 +216,9 @@ struct Seed {
     uint32_t* ws = nullptr;    // device popcount (POP_SLOTS partials)
     uint32_t* sq = nullptr;    // prefix words (four-step path): L/8 bytes, 1/32 of the spectrum, not
                                // charged to the budget, so that it holds as many seeds as it says
-                               // (spec, ws and sq are one allocation at spec)
+    uint32_t* words = nullptr; // the seed itself up to 2^DIRECT_MAX_L_LOG bits, for the direct product;
+                               // at most L/8 bytes, not charged either
+                               // (spec, ws, sq and words are one allocation at spec)
     int32_t reuse = 0;
     uint64_t bytes = 0;
 };
@@ -571,10 +573,16 @@ hipError_t timed(pa_engine* e, int stage, hipStream_t s, F&& launch) {
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                     const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su);
 
+// A single block that takes the direct product: not with a margin, which is the transform's rounding
+// distance.
+bool direct_block(const Geom& g, const float* margin) { return !margin && pa::direct_size(g, pa::direct_work(g)); }
+
 // Orders the workspace's uses across streams (not while s is being captured into a graph: a
 // capture only records work, and the caller owns the ordering of its replays).
 int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su = nullptr) {
+    if (direct_block(g, margin))  // uses no scratch of the workspace
+        return run_device_body(e, g, w, key, seed, sd, out, s, margin, su);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     PA_HIP(hipStreamIsCapturing(s, &cap));
     const bool guard = cap == hipStreamCaptureStatusNone;
@@ -591,6 +599,10 @@ int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, c
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                     const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su) {
     const pa::Tables t = tables(e, g.L);
+    if (direct_block(g, margin)) {
+        PA_HIP(timed(e, ST_SMALL, s, [&] { return pa::launch_direct(key, sd ? sd->words : seed, out, g, s); }));
+        return PA_OK;
+    }
     if (g.N1 == 1) {
         PA_HIP(timed(e, ST_SMALL, s, [&] {
             return pa::launch_small(key, seed, sd ? sd->spec : nullptr, sd ? sd->ws : nullptr, out, g, t, margin, nullptr,
@@ -777,7 +789,9 @@ static int seed_alloc(pa_engine* e, Seed* sd) {
     sd->bytes = (uint64_t)(g.N + 1) * sizeof(float2) + pa::POP_SLOTS * sizeof(uint32_t);
     if (e->cfg.hbm_budget_bytes && e->used_bytes + sd->bytes > e->cfg.hbm_budget_bytes) return PA_ERR_NOMEM;
     uint8_t* p = nullptr;
-    const hipError_t r = hipMalloc((void**)&p, spec + ws + (g.N1 > 1 ? (uint64_t)g.L / 8 : 0));
+    const uint64_t sq = g.N1 > 1 ? (uint64_t)g.L / 8 : 0;
+    const bool words = g.L <= (1u << pa::DIRECT_MAX_L_LOG);
+    const hipError_t r = hipMalloc((void**)&p, spec + ws + sq + (words ? (uint64_t)g.n / 8 : 0));
     if (r != hipSuccess) {
         set_error(r, "hipMalloc", __FILE__, __LINE__);
         (void)hipGetLastError();
@@ -787,6 +801,7 @@ static int seed_alloc(pa_engine* e, Seed* sd) {
     sd->spec = reinterpret_cast<float2*>(p);
     sd->ws = reinterpret_cast<uint32_t*>(p + spec);
     if (g.N1 > 1) sd->sq = reinterpret_cast<uint32_t*>(p + spec + ws);
+    if (words) sd->words = reinterpret_cast<uint32_t*>(p + spec + ws + sq);
     return PA_OK;
 }
 static void seed_free(pa_engine* e, const Seed& sd) { dev_free(e, sd.spec, sd.bytes); }
@@ -805,17 +820,18 @@ int pa_seed_put(pa_engine* e, const uint32_t* seed, uint32_t n, uint32_t m, int3
         hipStream_t s = e->stream;
         // the workspace's masks and info words are scratch here: after a block on another stream
         if (w->last_stream && w->last_stream != s) PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
-        PA_HIP(hipMemcpyAsync(w->d_seed, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
+        uint32_t* src = sd.words ? sd.words : w->d_seed;
+        PA_HIP(hipMemcpyAsync(src, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
         const pa::Tables t = tables(e, g.L);
         if (g.N1 == 1) {
-            PA_HIP(pa::launch_small(nullptr, w->d_seed, nullptr, nullptr, nullptr, g, t, nullptr, sd.spec, sd.ws, s));
+            PA_HIP(pa::launch_small(nullptr, src, nullptr, nullptr, nullptr, g, t, nullptr, sd.spec, sd.ws, s));
         } else {
             Geom gs = g;  // every word's prefix, whatever window a block will read
             gs.out_off = 0;
             gs.out_bits = g.L;
-            const pa::ScanArgs scan{nullptr, w->d_seed, nullptr, sd.sq, w->info};
-            if (!mid_size(g)) PA_HIP(pa::launch_transpose(nullptr, w->d_seed, nullptr, w->tbs, 1, 1, gs, &scan, s));
-            PA_HIP(pa::launch_fwd_cols(nullptr, mid_size(g) ? w->d_seed : w->tbs, nullptr, sd.spec, 1, 1, gs, t, &scan, s));
+            const pa::ScanArgs scan{nullptr, src, nullptr, sd.sq, w->info};
+            if (!mid_size(g)) PA_HIP(pa::launch_transpose(nullptr, src, nullptr, w->tbs, 1, 1, gs, &scan, s));
+            PA_HIP(pa::launch_fwd_cols(nullptr, mid_size(g) ? src : w->tbs, nullptr, sd.spec, 1, 1, gs, t, &scan, s));
             PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, sd.spec, nullptr, g, t, w->info, nullptr, sd.ws, s));
             PA_HIP(pa::launch_prefix_apply(sd.sq, w->info, g, s));
         }
@@ -942,7 +958,7 @@ static int run_host(pa_engine* e, const uint32_t* key, const uint32_t* seed, pa_
     // a fresh seed of a multi-pass block goes up while the key's first passes run (the previous
     // call's kernels, the only other readers of d_seed, finished before it returned)
     const SeedUpload su{seed, w->d_seed, (size_t)(n / 32) * 4, e->upload, e->key_up, e->upload_done};
-    const bool overlap = seed && g.N1 > 1;
+    const bool overlap = seed && !direct_block(g, nullptr);
     if (overlap) PA_HIP(hipEventRecord(e->key_up, s));
     if (seed && !overlap) PA_HIP(hipMemcpyAsync(w->d_seed, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
     rc = run_device(e, g, w, w->d_key, seed ? w->d_seed : nullptr, sd, w->d_out, s, nullptr, overlap ? &su : nullptr);
@@ -1054,7 +1070,11 @@ struct BatchItem {
 
 struct BatchGroup {
     uint32_t L = 0;
-    bool dyn = true, small = false;
+    bool dyn = true;
+    bool small = false;         // no scratch: the one-workgroup sizes, and the direct product
+    bool direct = false, margin = false;
+    uint32_t words = 1, jpad = 16;  // direct product: the most output and padded key words of the group
+    uint64_t work = 0;
     std::vector<uint32_t> idx;  // blocks of the group (caller order)
     uint32_t tab0 = 0;          // first table row of the group
     uint32_t halves = 1;        // halves of the conv positions to pack: the most of the group
@@ -1110,10 +1130,18 @@ int batch_plan(pa_engine* e, const pa_block* blocks, uint32_t count, BatchPlan* 
         gr.idx.push_back(i);
         gr.cost += (double)it.g.L * (it.dyn ? 1.5 : 1.0);
         if (!gr.small) gr.halves = std::max(gr.halves, pa::pack_halves(it.g));
-        p->scratch_bytes += batch_scratch_bytes(it.g, it.dyn);
+        gr.margin = gr.margin || b.margin;
+        gr.words = std::max(gr.words, it.g.out_bits / 32u);
+        gr.jpad = std::max(gr.jpad, pa::direct_key_words(it.g));
+        gr.work += pa::direct_work(it.g);
     }
     uint32_t row = 0;
     for (auto& gr : p->groups) {
+        gr.direct = !gr.margin;
+        for (uint32_t i : gr.idx) gr.direct = gr.direct && pa::direct_size(p->items[i].g, gr.work);
+        gr.small = gr.small || gr.direct;
+        if (!gr.small)
+            for (uint32_t i : gr.idx) p->scratch_bytes += batch_scratch_bytes(p->items[i].g, p->items[i].dyn);
         gr.tab0 = row;
         row += (uint32_t)gr.idx.size();
     }
@@ -1153,6 +1181,10 @@ int batch_group_launch(pa_engine* e, const BatchPlan& p, const BatchGroup& gr, c
     const uint32_t cnt = (uint32_t)gr.idx.size();
     const Geom& g0 = p.items[gr.idx[0]].g;
     const pa::Tables t = tables(e, gr.L);
+    if (gr.direct) {
+        PA_HIP(pa::launch_batch_direct(bt, cnt, gr.words, gr.jpad, s));
+        return PA_OK;
+    }
     if (gr.small) {
         PA_HIP(pa::launch_batch_small(bt, cnt, g0, t, s));
         return PA_OK;
@@ -1281,7 +1313,7 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
             pa::BlockArgs a{};
             a.g = it.g;
             a.key = dev[i].key;
-            a.seed = it.dyn ? dev[i].seed : nullptr;
+            a.seed = it.dyn ? dev[i].seed : gr.direct ? it.sd->words : nullptr;
             a.sspec = it.sd ? it.sd->spec : nullptr;
             a.ws = it.sd ? it.sd->ws : nullptr;
             a.sq = it.sd ? it.sd->sq : nullptr;
@@ -1354,7 +1386,8 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
     auto replay = [&]() -> int {
         std::string key = std::to_string((uintptr_t)sl.arena) + ":";
         for (auto& gr : p.groups)
-            key += tune_key(gr) + "p" + std::to_string(gr.fwd_per) + "y" + std::to_string(gr.halves) + ";";
+            key += tune_key(gr) + (gr.direct ? "w" + std::to_string(gr.words) + "j" + std::to_string(gr.jpad)
+                                             : "p" + std::to_string(gr.fwd_per) + "y" + std::to_string(gr.halves)) + ";";
         auto f = sl.graphs.find(key);
         if (f == sl.graphs.end()) {
             hipGraph_t graph = nullptr;

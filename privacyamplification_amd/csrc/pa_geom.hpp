@@ -78,6 +78,23 @@ struct Geom {
 // A four-step transform of the mid sizes: no bit masks, no separate output stage.
 __host__ __device__ inline bool mid_size(const Geom& g) { return g.N1 > 1u && g.lgN <= (uint32_t)MID_MAX_LOG_N; }
 
+// The direct product (k_direct) serves what it finishes sooner than the transform: blocks of the one-
+// workgroup sizes, and up to L = 2^DIRECT_MAX_L_LOG one block, or all of a batch's group, of up to
+// DIRECT_WORK products of a key word and an output word.  One block: 2^17 bits (3.9 M) 10.3 against 18.0 us,
+// 2^18 (15.7 M) 21.8 against 20.8; batches of 128: 2^15 0.34 against 0.27 us a block beside the
+// call's fixed 27, 2^16 1.1 against 0.37.
+constexpr int DIRECT_MAX_L_LOG = 18;
+constexpr uint64_t DIRECT_WORK = 12u << 20;
+constexpr uint32_t DIRECT_NT_MAX = 1024;
+constexpr uint32_t DIRECT_JPAD_MAX = 8000;  // key and seed words in 64 KB of LDS
+// Key words of the direct product, padded to its chunks.
+__host__ __device__ inline uint32_t direct_key_words(const Geom& g) { return (g.key_hw + 16u) & ~15u; }
+inline uint64_t direct_work(const Geom& g) { return (uint64_t)(g.out_bits >> 5) * direct_key_words(g); }
+// work: of the block, or of the blocks that share a launch.
+inline bool direct_size(const Geom& g, uint64_t work) {
+    return g.N1 == 1u || (g.L <= (1u << DIRECT_MAX_L_LOG) && work <= DIRECT_WORK && direct_key_words(g) <= DIRECT_JPAD_MAX);
+}
+
 // Inputs and outputs of the input scan: conv words of the key and the fresh seed (or the resident
 // seed's finished prefix words sq); prefix words q, and the block's info words.
 struct ScanArgs {
@@ -109,7 +126,7 @@ inline uint64_t info_bytes(const Geom& g) {
 struct BlockArgs {
     Geom g;
     const uint32_t* key;
-    const uint32_t* seed;   // dynamic seed, or nullptr for a resident one
+    const uint32_t* seed;   // dynamic seed, or nullptr for a resident one (its words for the direct product)
     const float2* sspec;    // resident spectrum when seed == nullptr
     const uint32_t* ws;     // resident seed popcount partials when seed == nullptr
     const uint32_t* sq;     // resident seed prefix words when seed == nullptr (four-step path only)

@@ -22,6 +22,7 @@
 //   k_small           the whole block in one workgroup for L <= 2^14
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <type_traits>
 
@@ -1374,6 +1375,81 @@ __global__ __launch_bounds__(small_threads(LGN)) void k_small(
     if (margin) margin_publish(dist, margin);
 }
 
+// ------------------------------------------------------------------ direct product ----
+// The product itself for short blocks, 32 bit-products per two integer instructions: no transform and
+// no rounding.  Output position p = 32 W + s is the parity of the XOR over the key words j of
+//   key word j  AND  window(W - j, s),   window(k, s) bit t = S[32 k + s - 31 + t],
+// S the seed sequence (circular in n, rotated by seed_rot words), so that bit 31 - b of the window meets
+// key bit b = x[32 j + b].  U_k = the 32 bits from S[32 k - 31] on, staged in LDS; window(k, s) =
+// (U_{k+1} : U_k) >> s, one funnel shift per lane s, serves R output words.
+// A workgroup has R output words; its half-waves (lanes s) share out the key in chunks of 16 words.
+// Bound by the vector ALU from 2^17 bits on (1 T word products a second) and by the launch below: calls of
+// 2^10 to 2^16 bits take 6.8 to 7.5 us one after another, where the one-workgroup transform took 18 to 27
+// and the three launches of the mid-size one 17 to 18.
+template <int R, bool BATCH>
+__global__ __launch_bounds__(DIRECT_NT_MAX) void k_direct(const uint32_t* __restrict__ key,
+                                                          const uint32_t* __restrict__ seed, uint32_t* __restrict__ out,
+                                                          Geom g, const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) {
+        const BlockArgs& a = bt[blockIdx.z];
+        g = a.g;
+        key = a.key;
+        seed = a.seed;
+        out = a.out;
+    }
+    extern __shared__ __attribute__((aligned(16))) uint32_t lds[];
+    __shared__ uint32_t part[DIRECT_NT_MAX / 64][R];
+    const uint32_t words = g.out_bits >> 5, w0 = blockIdx.x * (uint32_t)R;
+    if (w0 >= words) return;
+    const uint32_t jpad = direct_key_words(g), NT = blockDim.x;
+    uint32_t* kx = lds;         // key words, zero from key_hw + 1 on
+    uint32_t* us = lds + jpad;  // U of words base .. base + jpad + R
+    const int W0 = (int)((g.out_off >> 5) + w0), base = W0 - (int)jpad + 1;
+    for (uint32_t i = threadIdx.x; i < jpad; i += NT) kx[i] = key_word(key, g, i);
+    const int nw = (int)g.seed_words;
+    auto at = [&](int k) {  // the words off the sequence's range only meet zero key words or unused outputs
+        int i = k + (int)g.seed_rot;
+        i = i < 0 ? i + nw : i >= nw ? i - nw : i;
+        return __brev(seed[min(max(i, 0), nw - 1)]);
+    };
+    for (uint32_t i = threadIdx.x; i < jpad + (uint32_t)R + 1u; i += NT)
+        us[i] = __builtin_amdgcn_alignbit(at(base + (int)i), at(base + (int)i - 1), 1u);
+    __syncthreads();
+    const uint32_t sh = threadIdx.x & 31u;
+    uint32_t acc[R] = {};
+    for (uint32_t j0 = 16u * (threadIdx.x >> 5); j0 < jpad; j0 += NT / 2u) {
+        constexpr int NU = (16 + R + 3) / 4 * 4;
+        uint32_t kw[16], u[NU];
+#pragma unroll
+        for (int i = 0; i < 16; i += 4) *reinterpret_cast<uint4*>(kw + i) = *reinterpret_cast<const uint4*>(kx + j0 + i);
+        const uint32_t* up = us + (jpad - 16u - j0);  // U of word W0 - j0 - 15 on
+#pragma unroll
+        for (int i = 0; i < NU; i += 4) *reinterpret_cast<uint4*>(u + i) = *reinterpret_cast<const uint4*>(up + i);
+#pragma unroll
+        for (int a = 0; a < 15 + R; ++a) {
+            const uint32_t win = __builtin_amdgcn_alignbit(u[a + 1], u[a], sh);
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int j = 15 - a + r;
+                if (j >= 0 && j < 16) acc[r] = __builtin_amdgcn_bitop3_b32(acc[r], kw[j], win, 0x78);  // acc ^ (kw & win)
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const uint64_t b = __ballot(__popc(acc[r]) & 1);
+        if ((threadIdx.x & 63u) == 0u) part[threadIdx.x >> 6][r] = (uint32_t)b ^ (uint32_t)(b >> 32);
+    }
+    __syncthreads();
+    const uint32_t wd = w0 + threadIdx.x;
+    if (threadIdx.x >= (uint32_t)R || wd >= words) return;
+    uint32_t c = 0;
+    for (uint32_t i = 0; i < NT / 64u; ++i) c ^= part[i][threadIdx.x];
+    c = __brev(c);  // position p at bit 31 - p mod 32
+    if (g.do_xor && 32u * wd < g.m) c ^= (key[g.key_hw + wd] << 1) | (key[g.key_hw + wd + 1] >> 31);
+    out[wd] = g.reverse_endian ? __builtin_bswap32(c) : c;
+}
+
 // ------------------------------------------------------------------ sub-block split ----
 // The m x (h+1) Toeplitz product cut into b x b tiles (the tiling of LargeBlocksizeExample,
 // LBS/main.cpp:104-124, 313-523): tile (band i, key column j) is the length-2b circular product of
@@ -1637,6 +1713,44 @@ hipError_t launch_mid_inv(const float2* R, const uint32_t* key, uint32_t* out, c
         k_mid_inv<LG1, false><<<g.N2 / 16u, mid_threads(LG1), 0, s>>>(R, key, out, g, info, q, t.tw14, margin, nullptr);
         return hipGetLastError();
     });
+}
+
+// R output words per workgroup: the fewest instruction slots on the busiest of 256 compute units, R + 1
+// per key word (R products and a window).  One block of 2^17 bits: 10.4 us with 6 (the rule's), 11.0 with
+// 8, 12.6 with 4, 18.5 with 1; of 2^16 7.4 with 3, 9.4 with 1.
+template <bool BATCH>
+hipError_t direct(const uint32_t* key, const uint32_t* seed, uint32_t* out, const Geom& g, uint32_t words, uint32_t jpad,
+                  const BlockArgs* bt, uint32_t count, hipStream_t s) {
+    const uint32_t NT = std::min(DIRECT_NT_MAX, (jpad * 2u + 63u) & ~63u);  // a half-wave per chunk of the key
+    uint32_t R = 1;
+    uint64_t best = ~0ull;
+    for (uint32_t r : {1u, 2u, 3u, 4u, 6u, 8u}) {
+        const uint64_t wgs = (uint64_t)(words + r - 1u) / r * count, cost = (wgs + 255u) / 256u * (r + 1u);
+        if (cost < best) {
+            best = cost;
+            R = r;
+        }
+    }
+    const size_t lds = (2u * jpad + 12u) * 4u;
+    auto go = [&](auto rc) {
+        constexpr int RR = decltype(rc)::value;
+        k_direct<RR, BATCH><<<dim3((words + RR - 1u) / RR, 1, count), NT, lds, s>>>(key, seed, out, g, bt);
+        return hipGetLastError();
+    };
+    switch (R) {
+    case 1: return go(std::integral_constant<int, 1>());
+    case 2: return go(std::integral_constant<int, 2>());
+    case 3: return go(std::integral_constant<int, 3>());
+    case 4: return go(std::integral_constant<int, 4>());
+    case 6: return go(std::integral_constant<int, 6>());
+    default: return go(std::integral_constant<int, 8>());
+    }
+}
+hipError_t launch_direct(const uint32_t* key, const uint32_t* seed, uint32_t* out, const Geom& g, hipStream_t s) {
+    return direct<false>(key, seed, out, g, g.out_bits >> 5, direct_key_words(g), nullptr, 1, s);
+}
+hipError_t launch_batch_direct(const BlockArgs* bt, uint32_t count, uint32_t words, uint32_t jpad, hipStream_t s) {
+    return direct<true>(nullptr, nullptr, nullptr, Geom{}, words, jpad, bt, count, s);
 }
 
 hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2* sspec,

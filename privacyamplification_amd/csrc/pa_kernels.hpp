@@ -94,6 +94,10 @@ hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, c
 // Pass A' and the output of a mid-size transform.
 hipError_t launch_mid_inv(const float2* R, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
                           const uint32_t* q, const Tables& t, float* margin, hipStream_t s);
+// A block by the direct product, and `count` of them: words, jpad: the most output words and key words
+// (direct_key_words) of a block of the launch.  BlockArgs: g, key, seed and out.
+hipError_t launch_direct(const uint32_t* key, const uint32_t* seed, uint32_t* out, const Geom& g, hipStream_t s);
+hipError_t launch_batch_direct(const BlockArgs* bt, uint32_t count, uint32_t words, uint32_t jpad, hipStream_t s);
 hipError_t launch_small(const uint32_t* key, const uint32_t* seed, const float2* sspec,
                         const uint32_t* ws_ptr, uint32_t* out, const Geom& g, const Tables& t,
                         float* margin, float2* sspec_out, uint32_t* ws_out, hipStream_t s);
