@@ -378,9 +378,13 @@ typedef unsigned int pa_u2v __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, (int)bytes, 0x00020000);
 }
-__device__ __forceinline__ void buf_store_nt(float2 v, __amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
+template <int AUX>
+__device__ __forceinline__ void buf_store(float2 v, __amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
     const pa_u2v x = {__float_as_uint(v.x), __float_as_uint(v.y)};
-    __builtin_amdgcn_raw_buffer_store_b64(x, rs, (int)voff, (int)soff, 2);  // aux 2: nt
+    __builtin_amdgcn_raw_buffer_store_b64(x, rs, (int)voff, (int)soff, AUX);  // aux 2: nt
+}
+__device__ __forceinline__ void buf_store_nt(float2 v, __amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
+    buf_store<2>(v, rs, voff, soff);
 }
 __device__ __forceinline__ float2 buf_load_f2(__amdgpu_buffer_rsrc_t rs, uint32_t voff, uint32_t soff) {
     const pa_u2v x = __builtin_amdgcn_raw_buffer_load_b64(rs, (int)voff, (int)soff, 0);
@@ -612,19 +616,31 @@ __global__ __launch_bounds__(fwd_cols_threads(LGM), LGM == 9 ? 2 : 1) void k_fwd
     }
 }
 
-// Pass A for L <= 2^24 (N1 = 2^6 .. 2^10), straight from the key's and the seed's words: 16 adjacent
-// columns of one row are half a word, so no bit transpose is needed.  Plan R1 x 16 (R1 x 32 from
+// Pass A for L <= 2^24 (N1 = 2^6 .. 2^10), straight from the key's and the seed's words: the 16 columns
+// of a group are half a word of every row, so no bit transpose is needed.  Plan R1 x 16 (R1 x 32 from
 // 512 on): the quarter shift sits in the stages' factors.
-template <int LG1, bool BATCH>
+// WALK: a workgroup takes `per` (even) consecutive groups, a pair of them from each word, and requests the
+// next pair's words and the next group's twiddles while it transforms; one group per workgroup
+// otherwise, for launches that leave compute units idle as it is.
+// Loading a group's bits (2 used bytes of each line) and its twiddles took 130 of the 387 us of 2^27
+// bits in blocks of 2^20 when every group was a workgroup of its own; now 328, of which storing the
+// 1.07 GB alone takes 202.  2^22: 440 to 380; 2^24: 490 to 334.
+template <int LG1>
+struct MidPlan {
+    static constexpr int N1 = 1 << LG1, NT = mid_threads(LG1), R1 = mid_r1(LG1), R2 = N1 / R1, S1 = N1 / R1;
+    static constexpr int K1 = 16 * S1 / NT, SEQS = seq_stride(N1), RPT = N1 / NT;
+    static_assert(16 * R1 == NT && K1 * R1 == R2, "one second-stage butterfly per thread");
+    static_assert(RPT * NT == N1, "a thread loads whole rows' words");
+};
+template <int LG1, bool BATCH, bool WALK>
 __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g, const float2* __restrict__ tw14,
                                                               const float2* __restrict__ twlo,
-                                                              const float2* __restrict__ twhi,
+                                                              const float2* __restrict__ twhi, uint32_t per,
                                                               const BlockArgs* __restrict__ bt) {
     fwd_batch_args<BATCH, true>(a, g, bt);
-    constexpr int N1 = 1 << LG1, NT = mid_threads(LG1), R1 = mid_r1(LG1), R2 = N1 / R1, S1 = N1 / R1;
-    constexpr int K1 = 16 * S1 / NT, SEQS = seq_stride(N1);
-    static_assert(16 * R1 == NT && K1 * R1 == R2, "one second-stage butterfly per thread");
-    __shared__ float2 buf[16 * SEQS];
+    using P = MidPlan<LG1>;
+    constexpr int N1 = P::N1, NT = P::NT, R1 = P::R1, R2 = P::R2, NA = R2 / 8;
+    __shared__ float2 buf[16 * P::SEQS];
     __shared__ float2 tab[R1 * stage_row<R2>()];
     __shared__ uint32_t bw[N1];  // the group's 16 bits of row u, and of row u + N1 above them
     const uint32_t op = blockIdx.x / a.nA;
@@ -636,13 +652,42 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g,
     const uint32_t* __restrict__ in = is_seed ? a.in[1] : a.in[0];
     float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
     if (BATCH && in == nullptr) return;
-    const uint32_t grp = blockIdx.x - op * a.nA, sh = (grp & 1u) ? 0u : 16u;
-    for (uint32_t u = threadIdx.x; u < (uint32_t)N1; u += NT) {
-        const uint32_t w = (16u * grp + g.N2 * u) >> 5, wh = w + (g.N >> 5);
-        const uint32_t lo = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
-        const uint32_t hi = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
-        bw[u] = ((lo >> sh) & 0xFFFFu) | ((hi >> sh) << 16);
-    }
+    const uint32_t grp0 = (blockIdx.x - op * a.nA) * (WALK ? per : 1u);
+    struct Words {
+        uint32_t lo[P::RPT], hi[P::RPT];
+    };
+    auto load_words = [&](Words& x, uint32_t wc) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < P::RPT; ++i) {
+            const uint32_t w = wc + (g.N2 >> 5) * (threadIdx.x + (uint32_t)(NT * i)), wh = w + (g.N >> 5);
+            x.lo[i] = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
+            x.hi[i] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
+        }
+    };
+    auto pack = [&](const Words& x, uint32_t grp) __attribute__((always_inline)) {
+        const uint32_t sh = (grp & 1u) ? 0u : 16u;
+#pragma unroll
+        for (int i = 0; i < P::RPT; ++i)
+            bw[threadIdx.x + NT * i] = ((x.lo[i] >> sh) & 0xFFFFu) | ((x.hi[i] >> sh) << 16);
+    };
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    const uint32_t L2m = 2u * g.L - 1u;
+    // (lo, hi) entries of w_2L^{t2 (4 k1 + 1)}, k1 = jt + R1 r = anchor step^(r mod 8): the anchors, then
+    // the step; their products are formed where they are used
+    using Tw = float2[2 * (NA + 1)];
+    auto load_tw = [&](Tw& x, uint32_t grp) __attribute__((always_inline)) {
+        const uint32_t t2 = 16u * grp + (uint32_t)col;
+#pragma unroll
+        for (int i = 0; i <= NA; ++i) {
+            const uint32_t e = (t2 * (i < NA ? 4u * ((uint32_t)jt + (uint32_t)(8 * R1 * i)) + 1u : 4u * R1)) & L2m;
+            x[2 * i] = twlo[e & (TW14 - 1)];
+            x[2 * i + 1] = twhi[e >> TW14_LOG];
+        }
+    };
+    Words cur, nxt;
+    Tw tw, twn;
+    load_words(cur, grp0 >> 1);
+    load_tw(tw, grp0);
     // second stage's factors: row q for w_N1^(q + 1/4)
     for (int e = threadIdx.x; e < R1 * (R2 / 2); e += NT) {
         const int q = e / (R2 / 2), i = e % (R2 / 2);
@@ -657,36 +702,70 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g,
         const int s = i == 0 ? 2 : i == 1 ? 4 : i < 4 ? 8 : i < 8 ? 16 : 32, k = i ? i - s / 4 : 0;
         tw1[i] = uniform_f2(tw14[(4 * k + 1) * (TW14 / (4 * s))]);
     }
-    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
-    const uint32_t t2 = 16u * grp + (uint32_t)col;
-    const uint32_t L2m = 2u * g.L - 1u;
-    const float2 step = tw_two_level(twlo, twhi, (t2 * 4u * R1) & L2m);
+    pack(cur, grp0);
     __syncthreads();
-    float2* seqbuf = buf + col * SEQS;
+    float2* seqbuf = buf + col * P::SEQS;
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * g.N2 * 8u);
+    auto stage1 = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < K1; ++i) {
-        const int j = jt + (NT / 16) * i;
-        float2 v[R1];
+        for (int i = 0; i < P::K1; ++i) {
+            const int j = jt + (NT / 16) * i;
+            float2 v[R1];
 #pragma unroll
-        for (int r = 0; r < R1; ++r) {  // z = (bit - 1/2) - i (bit' - 1/2)
-            const uint32_t b = bw[j + S1 * r] << (16 + col);
-            const uint32_t bh = bw[j + S1 * r] << col;
-            v[r] = make_float2((int)b < 0 ? 0.5f : -0.5f, (int)bh < 0 ? -0.5f : 0.5f);
+            for (int r = 0; r < R1; ++r) {  // z = (bit - 1/2) - i (bit' - 1/2)
+                const uint32_t b = bw[j + P::S1 * r] << (16 + col);
+                const uint32_t bh = bw[j + P::S1 * r] << col;
+                v[r] = make_float2((int)b < 0 ? 0.5f : -0.5f, (int)bh < 0 ? -0.5f : 0.5f);
+            }
+            dft_tw<R1>(v, tw1);
+#pragma unroll
+            for (int r = 0; r < R1; ++r) seqbuf[padi(j * R1 + r)] = v[r];
         }
-        dft_tw<R1>(v, tw1);
+        __syncthreads();
+    };
+    auto stage2 = [&](uint32_t grp) __attribute__((always_inline)) {
+        float2 F[R2];
+        stage_last_from_lds_tab<R2, N1>(F, seqbuf, jt, tab + jt * stage_row<R2>());
+        const float2 step = cmul(tw[2 * NA], tw[2 * NA + 1]);
+        const uint32_t vo = ((uint32_t)jt * g.N2 + 16u * grp + (uint32_t)col) * 8u;
+        float2 w = make_float2(0.f, 0.f);
 #pragma unroll
-        for (int r = 0; r < R1; ++r) seqbuf[padi(j * R1 + r)] = v[r];
-    }
-    __syncthreads();
-    float2 F[R2];
-    stage_last_from_lds_tab<R2, N1>(F, seqbuf, jt, tab + jt * stage_row<R2>());
-    // k1 = jt + R1 r: w_2L^{t2 (4 k1 + 1)} = base step^r, re-anchored from the table every 8 steps
-    float2 tw = make_float2(1.f, 0.f);
+        for (int r = 0; r < R2; ++r) {
+            w = (r & 7) == 0 ? cmul(tw[2 * (r / 8)], tw[2 * (r / 8) + 1]) : cmul(w, step);
+            buf_store<WALK ? 2 : 0>(cmul(F[r], w), ry, vo, (uint32_t)(R1 * r) * g.N2 * 8u);
+        }
+    };
+    auto advance = [&]() __attribute__((always_inline)) {  // to the next group: its bits are packed, its twiddles loaded
 #pragma unroll
-    for (int r = 0; r < R2; ++r) {
-        const uint32_t k1 = (uint32_t)jt + (uint32_t)(R1 * r);
-        tw = (r & 7) == 0 ? tw_two_level(twlo, twhi, (t2 * (4u * k1 + 1u)) & L2m) : cmul(tw, step);
-        Y[(size_t)k1 * g.N2 + t2] = cmul(F[r], tw);
+        for (int i = 0; i < 2 * (NA + 1); ++i) tw[i] = twn[i];
+        __syncthreads();  // packed bits; second-stage reads of the previous group are done
+    };
+    if constexpr (!WALK) {
+        stage1();
+        stage2(grp0);
+    } else {
+        // A pair of groups; more: another pair follows.
+        auto pair = [&](uint32_t grp, bool more) __attribute__((always_inline)) {
+            if (more) load_words(nxt, (grp >> 1) + 1u);
+            stage1();
+            pack(cur, grp + 1u);
+            load_tw(twn, grp + 1u);
+            stage2(grp);
+            advance();
+            stage1();
+            if (more) {
+                cur = nxt;
+                pack(cur, grp + 2u);
+                load_tw(twn, grp + 2u);
+            }
+            stage2(grp + 1u);
+        };
+        // the first pair is peeled: see k_fwd_cols
+        pair(grp0, per > 2u);
+        for (uint32_t it = 2; it < per; it += 2) {
+            advance();
+            pair(grp0 + it, it + 2u < per);
+        }
     }
 }
 
@@ -1560,6 +1639,17 @@ hipError_t by_lg1(uint32_t lg1, F&& f) {
     }
 }
 
+// Column groups a workgroup of k_mid_fwd walks: 4 at N1 = 2^10 (one workgroup per compute unit), else 2, and
+// 1 where that would leave compute units idle or, at N1 <= 2^8, where what the launch writes stays in the
+// 256 MB cache (64 blocks of 2^18 bits on a resident seed: 100 us with 1, 103 with 2).  Us a block, in batches of 2^27 bits together, with
+// 1 / 2 / 4: 2^19 3.24 / 2.95 / 3.03, 2^20 6.22 / 5.62 / 5.75, 2^22 26.7 / 23.9 / 24.5, 2^24 135 / 124 / 114;
+// one block: 2^20 26.0 / 26.5 / 29.0, 2^23 67.6 / 66.2 / 70.3, 2^24 133 / 136 / 127.
+static uint32_t mid_walk(const Geom& g, uint32_t operands) {
+    const uint64_t groups = (uint64_t)(g.N2 / 16u) * operands;
+    const uint32_t w = g.lg1 >= 10u ? 4u : 2u;
+    return groups / w >= (g.lg1 >= 10u ? 256u : g.lg1 == 9u ? 512u : 8192u) ? w : 1u;
+}
+
 // Pass A of `count` blocks (bt, BATCH) or one (a); per: see launch_batch_fwd_cols.
 template <bool BATCH>
 hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uint32_t scan_wgs, const BlockArgs* bt,
@@ -1567,9 +1657,11 @@ hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uin
     if (mid_size(g))
         return by_mid_lg1(g.lg1, [&](auto lg) {
             constexpr int LG1 = decltype(lg)::value;
-            a.nA = g.N2 / 16u;
-            k_mid_fwd<LG1, BATCH><<<dim3(a.nA * a.ops + scan_wgs, 1, count), mid_threads(LG1), 0, s>>>(
-                a, g, t.tw14, t.lo, t.hi, bt);
+            const uint32_t walk = mid_walk(g, a.ops * count);
+            a.nA = g.N2 / 16u / walk;
+            const dim3 grid(a.nA * a.ops + scan_wgs, 1, count);
+            if (walk > 1u) k_mid_fwd<LG1, BATCH, true><<<grid, mid_threads(LG1), 0, s>>>(a, g, t.tw14, t.lo, t.hi, walk, bt);
+            else k_mid_fwd<LG1, BATCH, false><<<grid, mid_threads(LG1), 0, s>>>(a, g, t.tw14, t.lo, t.hi, 1u, bt);
             return hipGetLastError();
         });
     return by_lg1(g.lg1, [&](auto lg) {
