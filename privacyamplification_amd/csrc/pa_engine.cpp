@@ -64,8 +64,10 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
     const bool pow2 = is_pow2(n);
     const bool compress = (flags & PA_COMPRESS) != 0;
     if (!pow2 && !compress) return PA_ERR_UNSUPPORTED;  // n/2-bit output is defined for 2^k only
-    const uint32_t L = pow2 ? n : (1u << log2u(n));
-    if (log2u(L) > pa::MAX_L_LOG || log2u(L) > max_n_log2) return PA_ERR_SIZE;
+    const uint32_t lgL = log2u(n);
+    if (lgL > pa::MAX_L_LOG || lgL > max_n_log2) return PA_ERR_SIZE;
+    const bool mix = lgL >= (uint32_t)pa::MIX_MIN_LOG_L && lgL <= (uint32_t)pa::MIX_MAX_LOG_L && n <= (3u << (lgL - 2));
+    const uint32_t L = mix ? 3u << (lgL - 2) : 1u << lgL;
     Geom x{};
     x.n = n;
     x.m = m;
@@ -81,6 +83,13 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
         x.lg2 = x.lgN;
         x.M = 1;
         x.D = 1;
+    } else if (mix) {
+        x.M = pa::MIX_M;
+        x.D = pa::mix_classes((int)lgL);
+        x.N1 = x.M * x.D;
+        x.lg1 = log2u(x.N1) - 1;
+        x.N2 = x.N / x.N1;
+        x.lg2 = log2u(x.N2);
     } else {
         x.lg1 = x.lgN <= (uint32_t)pa::MID_MAX_LOG_N ? (uint32_t)pa::mid_lg1((int)x.lgN) : x.lgN - pa::ROW_LOG;
         x.lg2 = x.lgN - x.lg1;
@@ -413,7 +422,7 @@ std::vector<float2> twiddles(uint64_t L, uint64_t count, uint64_t stride) {
 // Pass A's class tables (layout in pa_kernels.hpp): sums of the quarter-shifted D-th roots of unity
 // times the +-1/2-encoded bits of a byte, in double precision, rounded once.
 std::vector<float2> class_tables() {
-    std::vector<float2> t(pa::CLS_TABLE_TOTAL);
+    std::vector<float2> t(pa::CLS_TABLES_ALL);
     for (int D = 4; D <= 32; D *= 2) {
         const int BW = pa::cls_bits(D), NB = pa::cls_tables(D);
         for (int c = 0; c < D / 2; ++c)
@@ -433,6 +442,19 @@ std::vector<float2> class_tables() {
                     t[pa::cls_table_offset(D) + ((c * NB + q) << BW) + index] = make_float2((float)x, (float)y);
                 }
     }
+    for (int D = 3; D <= 6; D *= 2)
+        for (int c = 0; c < D; ++c)
+            for (int index = 0; index < 64; ++index) {
+                double x = 0.0, y = 0.0;
+                for (int b = 0; b < 6; ++b) {  // D = 3: bits 3 .. 5 are the second half's, a quarter turn on
+                    const int v = b % D, h = b / D;
+                    const double w = -2.0 * M_PI * ((v * (4 * c + 1) + h * D) % (4 * D)) / (4.0 * D);
+                    const double sign = ((index >> b) & 1) ? 0.5 : -0.5;
+                    x += sign * std::cos(w);
+                    y += sign * std::sin(w);
+                }
+                t[pa::mix_table_offset(D) + c * 64 + index] = make_float2((float)x, (float)y);
+            }
     return t;
 }
 
@@ -695,7 +717,7 @@ int pa_create(const pa_config* cfg, pa_engine** out) {
     if (rc != PA_OK) return rc;
     auto tw = twiddles(16384, 16384, 1);
     PA_HIP(hipMemcpy(e->tw14, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice));
-    rc = dev_alloc(e.get(), (void**)&e->cls, pa::CLS_TABLE_TOTAL * sizeof(float2));
+    rc = dev_alloc(e.get(), (void**)&e->cls, pa::CLS_TABLES_ALL * sizeof(float2));
     if (rc != PA_OK) return rc;
     auto cls = class_tables();
     PA_HIP(hipMemcpy(e->cls, cls.data(), cls.size() * sizeof(float2), hipMemcpyHostToDevice));
@@ -708,6 +730,7 @@ int pa_create(const pa_config* cfg, pa_engine** out) {
         for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= std::min(NOALLOC_MAX_L_LOG, e->cfg.max_n_log2); ++lg) {
             Twiddles* tw;
             rc = get_twiddles(e.get(), 1u << lg, &tw);
+            if (rc == PA_OK && lg >= (uint32_t)pa::MIX_MIN_LOG_L) rc = get_twiddles(e.get(), 3u << (lg - 2), &tw);
             if (rc != PA_OK) return rc;
         }
     }
@@ -775,7 +798,7 @@ int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform
     const int rc = make_geom(n, m, flags, 1, pa::MAX_L_LOG, &g);
     if (rc != PA_OK) return rc;
     const Extents x = block_extents(g);
-    if (transform_len) *transform_len = g.L;
+    if (transform_len) *transform_len = 1u << log2u(g.L);
     for (int i = 0; i < PA_BUF_COUNT; ++i) {
         if (touched) touched[i] = x.touched[i];
         if (alloc) alloc[i] = x.alloc[i];

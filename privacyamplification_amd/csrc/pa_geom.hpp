@@ -59,11 +59,22 @@ __host__ __device__ constexpr int mid_lg1(int lgN) {
 }
 constexpr int MID_MAX_LOG_N = 23;
 
+// Transforms of 3 * 2^k, for blocks of 2^(k+1) < n <= 3 * 2^k bits, which a power of two would pad by a third
+// and more: N1 = D * 256 columns points in D = 3 classes, or 6 where N2 = 8192 makes it necessary, whose
+// sums over the class bits come from a table (k_mix_fwd), so the factor 3 costs pass A nothing; pass B
+// is as ever.  Against the power of two, blocks of 0.7 * 2^k bits, us of one block / a block in a batch of 2^27
+// bits: k = 19 22.3 / 2.85 to 21.5 / 2.09, k = 22 43.3 / 22.8 to 42.5 / 16.9, k = 23 66 / 48 to 53 / 33, k = 24 123 /
+// 101 to 98 / 70, k = 25 266 / 214 to 174 / 155; on a resident seed k = 19 23.1 / 2.17 to 20 / 1.6, k = 22 32.7 / 16.7 to
+// 35.1 / 12.3 (the one loss), k = 25 215 / 171 to 140 / 121.  Below k = 19 the direct product takes single blocks.
+constexpr uint32_t MIX_M = 256;
+constexpr int MIX_MIN_LOG_L = 19, MIX_MAX_LOG_L = 25;  // ceil(log2 L) of the lengths served
+__host__ __device__ constexpr uint32_t mix_classes(int lgL) { return lgL == 25 ? 6u : 3u; }
+
 struct Geom {
     uint32_t n, m, h, kbits;           // block shape; kbits = h + 1
-    uint32_t L, N, lgN;                // transform length, half length, log2(N)
-    uint32_t N1, N2, lg1, lg2;         // four-step split (N1 = 1 on the small path)
-    uint32_t M, D;                     // pass A class length / classes
+    uint32_t L, N, lgN;                // transform length, half length, ceil(log2 N)
+    uint32_t N1, N2, lg1, lg2;         // four-step split (N1 = 1 on the small path); lg1: floor(log2 N1)
+    uint32_t M, D;                     // pass A class length / classes (3 or 6: a transform of 3 * 2^k)
     uint32_t out_bits, out_off;        // output window in conv indices
     uint32_t seed_words, seed_rot;     // n/32, rotation of the seed in words (m/32 when L > n); the
                                        // rotated seed repeats with period n up to L
@@ -76,7 +87,8 @@ struct Geom {
 };
 
 // A four-step transform of the mid sizes: no bit masks, no separate output stage.
-__host__ __device__ inline bool mid_size(const Geom& g) { return g.N1 > 1u && g.lgN <= (uint32_t)MID_MAX_LOG_N; }
+__host__ __device__ inline bool mixed(const Geom& g) { return g.D % 3u == 0u; }
+__host__ __device__ inline bool mid_size(const Geom& g) { return g.N1 > 1u && (g.lgN <= (uint32_t)MID_MAX_LOG_N || mixed(g)); }
 
 // The direct product (k_direct) serves what it finishes sooner than the transform: blocks of the one-
 // workgroup sizes, and up to L = 2^DIRECT_MAX_L_LOG one block, or all of a batch's group, of up to

@@ -769,6 +769,135 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g,
     }
 }
 
+// Transforms of 3 * 2^k: pass A and pass A' of N1 = D 256 points, D = 3 or 6 (pa_geom.hpp), 16 columns per
+// workgroup like the passes of the powers of two.
+// Stage factors of the 256-point transforms over u with inputs times w_N1^{u f / 4} (f / 4 = c + 1/4 in
+// pass A, the residue q in pass A'): tw2 row j for w_256^j w_N1^{f/4}, tw1 for w_N1^{16 f / 4}; exponents
+// in units of w_4N1.
+constexpr int MIX_TW2 = 16 * stage_row<16>(), MIX_TW1 = 8;
+template <int D, int NC, int NT>
+__device__ __forceinline__ void mix_factors(float2* tw2, float2* tw1, uint32_t f0, uint32_t fstep, const Geom& g,
+                                            const float2* __restrict__ twlo, const float2* __restrict__ twhi) {
+    for (uint32_t e = threadIdx.x; e < NC * 136u; e += NT) {
+        const uint32_t c = e / 136u, r = e % 136u, q = r >> 3, i = r & 7u, f = f0 + fstep * c;
+        uint32_t s = 2;  // the size of factor i and its index k at that size (dft_tw's order)
+        while (s / 2u <= i && i > 0u) s *= 2u;
+        const uint32_t k = i ? i - s / 4u : 0u, x = (16u / s) * (q < 16u ? 4u * D * q + f : 16u * f) + k * (4u * D * MIX_M / s);
+        const float2 w = tw_two_level(twlo, twhi, x * g.N2);
+        if (q < 16u) tw2[c * MIX_TW2 + q * stage_row<16>() + i] = w;
+        else tw1[c * MIX_TW1 + i] = w;
+    }
+}
+
+// Y[k1][t2], k1 = c + D k1', at the quarter-shifted frequencies: the sum over v < D of
+// z[t2 + N2 (u + 256 v)] w_D^{v (c + 1/4)} by the class bits, then 256 points over u (16 x 16).
+// A workgroup takes PER consecutive column groups (2: both of a word, streaming stores) and every class of
+// them, so bits, indexes and twiddles are fetched once per group; PER = 0: one group and one class, for
+// launches of few groups, which are bound by one workgroup's latency.  A batch's launch is bound by its
+// stores: 11 blocks of 11.7 M bits, key and seed, take 0.24 ms for 1.11 GB (4.6 TB/s; the 1.48 GB of the
+// power of two took 0.33).
+template <int D, int PER, bool BATCH>
+__global__ __launch_bounds__(256, PER == 0 ? 4 : 3) void k_mix_fwd(FwdArgs a, Geom g, const float2* __restrict__ twlo,
+                                                                   const float2* __restrict__ twhi,
+                                                                   const float2* __restrict__ cls,
+                                                                   const BlockArgs* __restrict__ bt) {
+    fwd_batch_args<BATCH, true>(a, g, bt);
+    constexpr bool SPLIT = PER == 0;
+    constexpr uint32_t per = SPLIT ? 1u : PER;
+    constexpr int NT = 256, M = (int)MIX_M, SEQS = seq_stride(M), NC = SPLIT ? 1 : D;
+    __shared__ float2 buf[16 * SEQS];
+    __shared__ float2 tw2[NC * MIX_TW2];
+    __shared__ float2 tw1s[NC * MIX_TW1];
+    __shared__ float2 TB[NC * 64];
+    __shared__ uint32_t bw[D * M];  // per row u + 256 v: 16 columns' bits, and those of a[. + N] above them
+    const uint32_t op = blockIdx.x / a.nA;
+    if (op >= a.ops) {
+        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, bw);
+        return;
+    }
+    const bool is_seed = a.first + op == 1u;
+    const uint32_t* __restrict__ in = is_seed ? a.in[1] : a.in[0];
+    float2* __restrict__ Y = is_seed ? a.Y[1] : a.Y[0];
+    if (BATCH && in == nullptr) return;
+    const uint32_t b = blockIdx.x - op * a.nA, grp0 = SPLIT ? b / D : b * per, c0 = SPLIT ? b % D : 0u;
+    uint32_t lo[D], hi[D];
+    auto load_words = [&](uint32_t wc) __attribute__((always_inline)) {
+#pragma unroll
+        for (int v = 0; v < D; ++v) {
+            const uint32_t w = wc + (g.N2 >> 5) * (threadIdx.x + (uint32_t)(M * v)), wh = w + (g.N >> 5);
+            lo[v] = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
+            hi[v] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
+        }
+    };
+    const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    // (lo, hi) entries of w_2L^{t2 (4 k1 + 1)}, k1 = c + D (jt + 16 r): of jt at c = 0, and the factors of r = 8,
+    // of r and of c
+    auto load_tw = [&](float2 (&x)[8], uint32_t grp) __attribute__((always_inline)) {
+        const uint32_t t2 = 16u * grp + (uint32_t)col;
+        const uint32_t f[4] = {4u * D * (uint32_t)jt + 1u, 4u * D * 128u, 4u * D * 16u, 4u};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            x[2 * i] = twlo[(t2 * f[i]) & (TW14 - 1)];
+            x[2 * i + 1] = twhi[(t2 * f[i]) >> TW14_LOG];
+        }
+    };
+    float2 tw[8];
+    load_words(grp0 >> 1);
+    load_tw(tw, grp0);
+    for (uint32_t e = threadIdx.x; e < NC * 64; e += NT) TB[e] = cls[mix_table_offset(D) + 64u * c0 + e];
+    mix_factors<D, NC, NT>(tw2, tw1s, 4u * c0 + 1u, 4u, g, twlo, twhi);
+    float2* seqbuf = buf + col * SEQS;
+    const __amdgpu_buffer_rsrc_t ry = make_rsrc(Y, g.N1 * g.N2 * 8u);
+    for (uint32_t it = 0; it < per; ++it) {
+        const uint32_t grp = grp0 + it, sh = (grp & 1u) ? 0u : 16u;
+#pragma unroll
+        for (int v = 0; v < D; ++v) bw[threadIdx.x + M * v] = ((lo[v] >> sh) & 0xFFFFu) | ((hi[v] >> sh) << 16);
+        __syncthreads();  // bits (and tables); second-stage reads of the last group are done
+        uint32_t idx[16];  // class bits of u = jt + 16 r: bit v, and v + 16 of a[. + N]
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            idx[r] = 0;
+#pragma unroll
+            for (int v = 0; v < D; ++v) idx[r] |= ((bw[jt + 16 * r + M * v] >> (15 - col)) & 0x10001u) << v;
+        }
+        const float2 a8 = cmul(tw[2], tw[3]), step = cmul(tw[4], tw[5]), cstep = cmul(tw[6], tw[7]);
+        float2 base = cmul(tw[0], tw[1]);
+        for (uint32_t c = 0; c < c0; ++c) base = cmul(base, cstep);
+        if (it + 1u < per) load_tw(tw, grp + 1u);
+        for (uint32_t i = 0; i < NC; ++i) {
+            const uint32_t c = c0 + i;
+            const float2* T = TB + 64u * i;
+            float2 z[16], f1[8];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if constexpr (D == 3) {
+                    z[r] = T[(idx[r] & 7u) | (idx[r] >> 13)];
+                } else {
+                    const float2 x = T[idx[r] & 63u], y = T[idx[r] >> 16];
+                    z[r] = make_float2(x.x + y.y, x.y - y.x);
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 8; ++k) f1[k] = uniform_f2(tw1s[i * MIX_TW1 + k]);
+            dft_tw<16>(z, f1);
+            if (i) __syncthreads();  // second-stage reads of the last class are done
+#pragma unroll
+            for (int r = 0; r < 16; ++r) seqbuf[padi(jt * 16 + r)] = z[r];
+            __syncthreads();
+            stage_last_from_lds_tab<16, M>(z, seqbuf, jt, tw2 + i * MIX_TW2 + jt * stage_row<16>());
+            const uint32_t vo = ((c + (uint32_t)(D * jt)) * g.N2 + 16u * grp + (uint32_t)col) * 8u;
+            float2 w = base;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                if (r == 8) w = cmul(base, a8);
+                buf_store<PER == 2 ? 2 : 0>(cmul(z[r], w), ry, vo, (uint32_t)(16 * D * r) * g.N2 * 8u);
+                w = cmul(w, step);
+            }
+            base = cmul(base, cstep);
+        }
+    }
+}
+
 // ------------------------------------------------------------------ pass B ----
 // Rows of N2 = 2^LG2 points.  The frequencies k1 + N1 k2 + 1/4 of a row have no partners in other
 // rows, so rows are independent:
@@ -889,13 +1018,13 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
     }
     // R'[row][t2] = F[t2] w_2L^{t2 (4 row + 1)}, t2 = j + NTR e: base step^e, re-anchored every 8
     // steps to bound the recurrence error
-    const uint32_t L2m = 2u * g.L - 1u, f = 4u * row + 1u;
-    const float2 base = tw_two_level(twlo, twhi, (f * (uint32_t)j) & L2m);
-    const float2 step = tw_two_level(twlo, twhi, (f * (uint32_t)NTR) & L2m);
+    const uint32_t f = 4u * row + 1u;  // f t2 < 2L
+    const float2 base = tw_two_level(twlo, twhi, f * (uint32_t)j);
+    const float2 step = tw_two_level(twlo, twhi, f * (uint32_t)NTR);
     float2 anchor[PPT / 8 - 1];
 #pragma unroll
     for (int a = 0; a < PPT / 8 - 1; ++a)
-        anchor[a] = tw_two_level(twlo, twhi, (f * (uint32_t)(NTR * 8 * (a + 1))) & L2m);
+        anchor[a] = tw_two_level(twlo, twhi, f * (uint32_t)(NTR * 8 * (a + 1)));
     // tiled (N2 = 8192): t2 = j + 256 e -> tile row t2 / RT_COLS = j / RT_COLS + (256 / RT_COLS) e, one
     // scalar offset per e; row-major: in place
     const bool tiled = LG2 == 13 && rt_tiled(g.lg1);
@@ -1312,6 +1441,153 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_inv(const float2* __re
     if (margin) margin_publish(dist, margin);
 }
 
+// The same for transforms of 3 * 2^k: rows t1 = q + D s are 256 points over i of
+// w_N1^{i q} sum_{r < D} R'[i + 256 r] w_D^{r q}.  D / NQ workgroups per column group, side by side on one XCD;
+// NQ = 3: workgroup h has the q of residue h mod D / 3 and forms their three sums of the D inputs in
+// registers, then their transforms in turn; NQ = 1 (launches of few groups): one q each.  The registers bound
+// it: at D = 6 the inputs of three sums and the second ones in flight take 212, two workgroups a compute unit
+// (with three, 90 spilled: 5 blocks of 23.5 M bits 0.30 ms, now 0.19).
+template <int D, int NQ, bool BATCH>
+__global__ __launch_bounds__(256, NQ == 1 ? 4 : D == 6 ? 2 : 3) void k_mix_inv(
+    const float2* __restrict__ Rp, const uint32_t* __restrict__ key, uint32_t* __restrict__ out, Geom g,
+    const uint32_t* __restrict__ info, const uint32_t* __restrict__ q, const float2* __restrict__ twlo,
+    const float2* __restrict__ twhi, float* __restrict__ margin, const BlockArgs* __restrict__ bt) {
+    if constexpr (BATCH) {
+        const BlockArgs& a = bt[blockIdx.z];
+        g = a.g;
+        Rp = a.Yk;
+        key = a.key;
+        out = a.out;
+        info = a.info;
+        q = a.q;
+        margin = a.margin;
+    }
+    constexpr int H = D / NQ, M = (int)MIX_M, SEQS = seq_stride(M);
+    static_assert(NQ == 3 || D == 3, "one q of three or three of D");
+    __shared__ float2 buf[16 * SEQS];
+    __shared__ float2 tw2[NQ * MIX_TW2];
+    __shared__ float2 tw1s[NQ * MIX_TW1];
+    const uint32_t logical = xcd_logical(blockIdx.x, gridDim.x);
+    const int h = (int)(logical % H), col = threadIdx.x & 15, jt = threadIdx.x >> 4;
+    const uint32_t grp = logical / H, t2 = 16u * grp + (uint32_t)col;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(Rp, g.N1 * g.N2 * 8u);
+    const uint32_t vo = ((uint32_t)jt * g.N2 + t2) * 8u;
+    float2 z[3][16];  // input r of i = jt + 16 e; D = 6: r plus or minus r + 3
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+#pragma unroll
+        for (int r = 0; r < 3; ++r) z[r][e] = buf_load_f2(rs, vo, (uint32_t)(16 * e + M * r) * g.N2 * 8u);
+    if constexpr (D == 6) {  // the others four e at a time, so that they never fill the registers
+        float2 y[2][12];
+        auto load_y = [&](int k) {
+#pragma unroll
+            for (int i = 0; i < 12; ++i) y[k & 1][i] = buf_load_f2(rs, vo, (uint32_t)(16 * (4 * k + i / 3) + M * (i % 3 + 3)) * g.N2 * 8u);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        const float sign = h ? -1.f : 1.f;
+        __builtin_amdgcn_sched_barrier(0);
+        load_y(0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (k < 3) load_y(k + 1);
+#pragma unroll
+            for (int i = 0; i < 12; ++i) {
+                float2& x = z[i % 3][4 * k + i / 3];
+                x = make_float2(fmaf(sign, y[k & 1][i].x, x.x), fmaf(sign, y[k & 1][i].y, x.y));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    mix_factors<D, NQ, 256>(tw2, tw1s, 4u * (uint32_t)h, 4u * (uint32_t)H, g, twlo, twhi);
+    const uint32_t pops = info[INFO_POPS], white = info[INFO_WHITE];
+    // sum b of NQ: q = h + H b
+    constexpr float S3 = 8.660254038e-01f;
+    const float cq = h ? -0.5f : 1.f, sq = h == 1 ? S3 : h ? -S3 : 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        if constexpr (NQ == 1) {  // w_3^q = cq - i sq
+            const float2 s = cadd(z[1][e], z[2][e]), d = csub(z[1][e], z[2][e]);
+            z[0][e] = make_float2(fmaf(sq, d.y, fmaf(cq, s.x, z[0][e].x)), fmaf(-sq, d.x, fmaf(cq, s.y, z[0][e].y)));
+            continue;
+        }
+        if constexpr (D == 6)
+            if (h) {  // odd q: input r times w_6^r
+                z[1][e] = cmul(z[1][e], make_float2(0.5f, -S3));
+                z[2][e] = cmul(z[2][e], make_float2(-0.5f, -S3));
+            }
+        const float2 s = cadd(z[1][e], z[2][e]), d = csub(z[1][e], z[2][e]);
+        const float2 m = make_float2(fmaf(-0.5f, s.x, z[0][e].x), fmaf(-0.5f, s.y, z[0][e].y));
+        z[0][e] = cadd(z[0][e], s);
+        z[1][e] = make_float2(fmaf(S3, d.y, m.x), fmaf(-S3, d.x, m.y));
+        z[2][e] = make_float2(fmaf(-S3, d.y, m.x), fmaf(S3, d.x, m.y));
+    }
+    const float mean = mean_half(pops, t2);
+    const uint32_t RW = g.N2 >> 5, w_lo = g.out_off >> 5, w_hi = (g.out_off + g.out_bits) >> 5;
+    const uint32_t lane = threadIdx.x & 63u, sh = (grp & 1u) ? 0u : 16u;
+    float dist = 0.f;
+    float2* seqbuf = buf + col * SEQS;
+    // w_4N1^{D jt + h} / N, and w_4N1^H for the next b
+    float2 K = cscale(tw_two_level(twlo, twhi, (uint32_t)(D * jt + h) * g.N2), g.inv_N);
+    const float2 kstep = tw_two_level(twlo, twhi, (uint32_t)H * g.N2);
+    __syncthreads();  // tables
+#pragma unroll
+    for (int b = 0; b < NQ; ++b) {
+        const int qr = h + H * b;
+        {
+            float2 f1[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) f1[i] = uniform_f2(tw1s[b * MIX_TW1 + i]);
+            dft_tw<16>(z[b], f1);
+        }
+        if (b) __syncthreads();  // second-stage reads of the last transform are done
+#pragma unroll
+        for (int r = 0; r < 16; ++r) seqbuf[padi(jt * 16 + r)] = z[b][r];
+        __syncthreads();
+        float2 G[16];
+        {
+            float2 tw[8];
+            const float2* trow = tw2 + b * MIX_TW2 + jt * stage_row<16>();
+            stage_last_read<16, M>(G, seqbuf, jt);
+#pragma unroll
+            for (int r = 0; r < 8; ++r) {
+                tw[r] = trow[r];
+                G[r] = cmul(G[r], K);
+            }
+            tw[0] = cmul(tw[0], K);
+            dft_tw<16>(G, tw);
+        }
+        K = cmul(K, kstep);
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            if (half == 0 ? g.out_off >= g.N : 32u * w_hi <= g.N) continue;
+            uint32_t mine = 0;  // the 16 bits of row qr + D (jt + 16 col)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t t1 = (uint32_t)(qr + D * (jt + 16 * e));
+                const float2 X = G[e], w = w64pow(make_float2(1.f, 0.f), e);
+                const float val = half == 0 ? fmaf(X.x, w.x, fmaf(-X.y, w.y, -mean)) : fmaf(X.x, w.y, fmaf(X.y, w.x, -mean));
+                float d = 0.f;
+                const uint64_t bits = __ballot(round_bit(val, d) != 0u);
+                const uint32_t pos = t2 + g.N2 * t1 + (half ? g.N : 0u) - g.out_off;
+                dist = fmaxf(dist, pos < g.out_bits ? d : 0.f);
+                const uint32_t word = (lane & 32u) ? (uint32_t)(bits >> 32) : (uint32_t)bits;
+                mine = col == e ? word >> (lane & 16u) : mine;
+            }
+            const uint32_t R = (uint32_t)half * g.N1 + (uint32_t)(qr + D * (jt + 16 * col));
+            const uint32_t w = R * RW + (grp >> 1);
+            if (w >= w_lo && w < w_hi) {
+                const uint32_t wo = w - w_lo;
+                // bit i of `mine` is column i: MSB first after the reversal
+                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, white, key) >> sh) & 0xFFFFu);
+                uint16_t* o = reinterpret_cast<uint16_t*>(out + wo);
+                if (g.reverse_endian) o[grp & 1u] = (uint16_t)((c16 >> 8) | (c16 << 8));
+                else o[(grp & 1u) ^ 1u] = (uint16_t)c16;
+            }
+        }
+    }
+    if (margin) margin_publish(dist, margin);
+}
+
 // ------------------------------------------------------------------ small path ----
 // The whole block in one workgroup: N = 2^LGN <= 8192 complex points per operand in LDS.
 // sspec != nullptr: static seed (precomputed split spectrum, N+1 values, popcount *ws_ptr).
@@ -1616,6 +1892,10 @@ hipError_t by_mid_lg1(uint32_t lg1, F&& f) {
     }
 }
 template <typename F>
+hipError_t by_classes(uint32_t D, F&& f) {
+    return D == 3u ? f(std::integral_constant<int, 3>()) : f(std::integral_constant<int, 6>());
+}
+template <typename F>
 hipError_t by_lg2(uint32_t lg2, F&& f) {
     switch (lg2) {
     case 8: return f(std::integral_constant<int, 8>());
@@ -1650,10 +1930,33 @@ static uint32_t mid_walk(const Geom& g, uint32_t operands) {
     return groups / w >= (g.lg1 >= 10u ? 256u : g.lg1 == 9u ? 512u : 8192u) ? w : 1u;
 }
 
+// Column groups of a launch below which the passes of 3 * 2^k give each class a workgroup of its own: fewer
+// than two a compute unit leave it idle.  One block of 3000032 bits (128 groups an operand): pass A 19.3 to
+// 18.4 us, pass A' 12.1 to 8.1.  From 2048 groups on pass A takes two a workgroup and streams its stores:
+// us a block in batches of 2^27 bits together with 1 / 2 / 2 streaming / 4, 2^20 bits 4.53 / 4.40 / 4.26 / 4.50,
+// 2^22 17.9 / 17.4 / 16.9 / 17.9, 2^24 75.8 / 72.4 / 70.5 / 75.3; one block of 2^25 bits 185 with 1, 185 streaming,
+// 181 with 2.
+static bool mix_split(uint64_t groups) { return groups < 512u; }
+
 // Pass A of `count` blocks (bt, BATCH) or one (a); per: see launch_batch_fwd_cols.
 template <bool BATCH>
 hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uint32_t scan_wgs, const BlockArgs* bt,
                     uint32_t count, hipStream_t s) {
+    if (mixed(g))
+        return by_classes(g.D, [&](auto d) {
+            constexpr int D = decltype(d)::value;
+            const uint64_t groups = (uint64_t)(g.N2 / 16u) * a.ops * count;
+            auto launch = [&](auto per, uint32_t wgs) {
+                a.nA = wgs;
+                k_mix_fwd<D, decltype(per)::value, BATCH><<<dim3(wgs * a.ops + scan_wgs, 1, count), 256, 0, s>>>(
+                    a, g, t.lo, t.hi, t.cls, bt);
+                return hipGetLastError();
+            };
+            if constexpr (D == 3)
+                if (mix_split(groups)) return launch(std::integral_constant<int, 0>(), g.N2 / 16u * D);
+            if (groups >= 2048u) return launch(std::integral_constant<int, 2>(), g.N2 / 32u);
+            return launch(std::integral_constant<int, 1>(), g.N2 / 16u);
+        });
     if (mid_size(g))
         return by_mid_lg1(g.lg1, [&](auto lg) {
             constexpr int LG1 = decltype(lg)::value;
@@ -1669,6 +1972,20 @@ hipError_t fwd_cols(FwdArgs a, const Geom& g, const Tables& t, uint32_t per, uin
         a.nA = g.N2 / 16u * (uint32_t)(D / 2) / per;  // N2 / 16 = 512 groups and per divides it
         k_fwd_cols<LGM, D, BATCH><<<dim3(a.nA * a.ops, 1, count), fwd_cols_threads(LGM), 0, s>>>(a, g, t.tw14, t.lo, t.hi,
                                                                                                t.cls, per, bt);
+        return hipGetLastError();
+    });
+}
+template <bool BATCH>
+hipError_t mix_inv(const float2* R, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
+                   const uint32_t* q, const Tables& t, float* margin, const BlockArgs* bt, uint32_t count, hipStream_t s) {
+    return by_classes(g.D, [&](auto d) {
+        constexpr int D = decltype(d)::value;
+        if constexpr (D == 3)
+            if (mix_split((uint64_t)(g.N2 / 16u) * count)) {
+                k_mix_inv<D, 1, BATCH><<<dim3(g.N2 / 16u * D, 1, count), 256, 0, s>>>(R, key, out, g, info, q, t.lo, t.hi, margin, bt);
+                return hipGetLastError();
+            }
+        k_mix_inv<D, 3, BATCH><<<dim3(g.N2 / 16u * (D / 3), 1, count), 256, 0, s>>>(R, key, out, g, info, q, t.lo, t.hi, margin, bt);
         return hipGetLastError();
     });
 }
@@ -1800,6 +2117,7 @@ hipError_t launch_pack(const uint8_t* nib, const uint32_t* key, uint32_t* out, c
 
 hipError_t launch_mid_inv(const float2* R, const uint32_t* key, uint32_t* out, const Geom& g, const uint32_t* info,
                           const uint32_t* q, const Tables& t, float* margin, hipStream_t s) {
+    if (mixed(g)) return mix_inv<false>(R, key, out, g, info, q, t, margin, nullptr, 1, s);
     return by_mid_lg1(g.lg1, [&](auto lg) {
         constexpr int LG1 = decltype(lg)::value;
         k_mid_inv<LG1, false><<<g.N2 / 16u, mid_threads(LG1), 0, s>>>(R, key, out, g, info, q, t.tw14, margin, nullptr);
@@ -1895,6 +2213,7 @@ hipError_t launch_batch_pack(const BlockArgs* bt, uint32_t count, const Geom& g0
 }
 
 hipError_t launch_batch_mid_inv(const BlockArgs* bt, uint32_t count, const Geom& g0, const Tables& t, hipStream_t s) {
+    if (mixed(g0)) return mix_inv<true>(nullptr, nullptr, nullptr, g0, nullptr, nullptr, t, nullptr, bt, count, s);
     return by_mid_lg1(g0.lg1, [&](auto lg) {
         constexpr int LG1 = decltype(lg)::value;
         k_mid_inv<LG1, true><<<dim3(g0.N2 / 16u, 1, count), mid_threads(LG1), 0, s>>>(nullptr, nullptr, nullptr, g0, nullptr,

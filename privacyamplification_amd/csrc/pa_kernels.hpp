@@ -42,6 +42,10 @@ __host__ __device__ constexpr int cls_table_offset(int D) {
     return D <= 4 ? 0 : cls_table_offset(D / 2) + cls_table_size(D / 2);
 }
 constexpr int CLS_TABLE_TOTAL = cls_table_offset(64);  // D = 4 .. 32
+// Tables of the transforms of 3 * 2^k, 64 entries a class, behind those: of D = 3 by the class bits of a
+// (bits 0 .. 2) and of a[. + N] (3 .. 5), of D = 6 by the bits of either, to be added with a factor -i.
+__host__ __device__ constexpr int mix_table_offset(int D) { return CLS_TABLE_TOTAL + (D == 6 ? 3 * 64 : 0); }
+constexpr int CLS_TABLES_ALL = CLS_TABLE_TOTAL + 9 * 64;
 // Place in a mask word (D = 32: a word per half) of class bit v of half h, in the tables' order.
 __host__ __device__ constexpr int mask_bit(int D, int h, int v) {
     return D <= 8 ? (v & 1) * D + h * (D / 2) + v / 2 : (D == 16 ? 16 * h : 0) + (v & 1) * (D / 2) + v / 2;

@@ -87,3 +87,45 @@ def test_direct_product_and_transform_agree(engine, oracle, n, m):
                                                          2048, 768, 3))
     finally:
         engine.seed_drop(sid)
+
+
+# transforms of 3 * 2^k: their shortest and longest blocks at every length, the next longer block (a power of
+# two's), one word out and one word of key, and as one batch with both kinds of transform in it
+MIXED = [(n, m) for e in range(18, 25) for n, m in
+         [((1 << e) + 32, 32), (3 << (e - 1), (3 << (e - 1)) - 32), ((3 << (e - 1)) - 32, 3 << (e - 3)), ((3 << (e - 1)) + 32, 1 << (e - 1))]]
+
+
+@pytest.mark.parametrize("n,m", MIXED)
+def test_mixed_radix_blocks(engine, oracle, n, m):
+    key, seed = oracle.synth_bits(0xE1 + n, n + 1), oracle.synth_bits(0xE2 + m, n)
+    sid = engine.seed_put(seed, n, m)
+    small_n, small_m = (1 << 18) + 64, 1 << 17
+    sk, ss = oracle.synth_bits(5, small_n + 1), oracle.synth_bits(6, small_n)
+    small_ref = oracle.amp_out(sk, ss, small_n, small_m, True, True, method=oracle.NTT)
+    try:
+        for flags in (P.XOR_KEY_REST | P.COMPRESS, P.COMPRESS):
+            say(f"mixed n={n} m={m} flags={flags}")
+            k = key if flags & P.XOR_KEY_REST else key[: (n - m) // 32 + 1].copy()
+            ref = oracle.amp_out(k, seed, n, m, bool(flags & P.XOR_KEY_REST), True, method=oracle.NTT)
+            d = _Device(key, seed, ref.size)
+            args = (n, m, flags, d.out.data_ptr(), 0, d.margin.data_ptr())
+            engine.block_device(d.key.data_ptr(), d.seed.data_ptr(), *args)
+            assert np.array_equal(d.take(), ref), (n, m, flags, "fresh")
+            engine.block_device_seeded(d.key.data_ptr(), sid, *args)
+            assert np.array_equal(d.take(), ref), (n, m, flags, "resident")
+            assert 0 < d.margin.item() < 0.25
+            other = _Device(sk, ss, small_ref.size)
+            for fresh in (True, False):
+                blk = (P.PaBlock * 3)()
+                for i, (b, bn, bm) in enumerate(((d, n, m), (other, small_n, small_m))):
+                    blk[i].key, blk[i].n, blk[i].m, blk[i].out = b.key.data_ptr(), bn, bm, b.out.data_ptr()
+                    blk[i].flags = flags if b is d else 3
+                    blk[i].seed = b.seed.data_ptr() if fresh or b is other else None
+                    blk[i].seed_id = 0 if fresh or b is other else sid
+                engine.batch_device((P.PaBlock * 2)(blk[0], blk[1]), P.BATCH_GRAPH, 0)
+                assert np.array_equal(d.take(), ref), (n, m, flags, "batch", fresh)
+                assert np.array_equal(other.take(), small_ref)
+        if n <= 1 << 22:
+            assert np.array_equal(engine.amplify(key, seed, n, m, False, True), ref), (n, m, "host")
+    finally:
+        engine.seed_drop(sid)
