@@ -909,12 +909,51 @@ __global__ __launch_bounds__(256, PER == 0 ? 4 : 3) void k_mix_fwd(FwdArgs a, Ge
 //   ROWS_STATIC:   key rows + resident S -> R'[k1][t2] = w_N^{t2 (k1 + 1/4)} FFT_N2(conj P)[t2], in
 //                  place, or into pass A''s tiles (Rt) when rt_tiled(lg1).
 //   ROWS_DYN:      key rows + seed rows; S is formed first and held in registers.
-// N2 = 8192 runs one row per 256-thread workgroup, 32 points per thread, 74 KB of LDS, so two share
-// a compute unit and one's memory requests overlap the other's transforms.  Shorter rows take 16
+// N2 = 8192 runs one row per 256-thread workgroup, 32 points per thread.  With a fresh seed it takes 74 KB of
+// LDS and 176 registers, so two share a compute unit and one's memory requests overlap the other's
+// transforms.  The other modes pass a row's real and imaginary parts through LDS one after the other
+// (row_exchange: half the LDS for twice the barriers), so three do: on a resident seed a block of 2^24 bits
+// takes 95 instead of 97.5 us, of 1.5 * 2^23 75 instead of 81 (its 768 rows are one round then), 2^25 208 instead
+// of 213, 2^27 710 instead of 715, 2^23 in a batch 35.5 instead of 36.8.  Not with a fresh seed, where the
+// seed row's 32 values more spill 23 registers and their reloads wait on the loads in flight: the pass
+// takes 0.437 ms instead of 0.397 at 2^27.  Shorter rows take 16
 // points per thread and at least one wave per workgroup (rows_per_wg rows).
 // The launch's first workgroup finishes the scan (scan_finish).
+// A row of 8192 points between two stages: value e of 32 goes to wi(e), comes back from ri(e), through LDS
+// of half the row: real parts, then imaginary parts.  Ends with a barrier.
+template <typename W, typename R>
+__device__ __forceinline__ void row_exchange(float2 (&x)[32], float* lds, W&& wi, R&& ri) {
+    float re[32];
+#pragma unroll
+    for (int e = 0; e < 32; ++e) lds[wi(e)] = x[e].x;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 32; ++e) re[e] = lds[ri(e)];
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 32; ++e) lds[wi(e)] = x[e].y;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 32; ++e) x[e] = make_float2(re[e], lds[ri(e)]);
+    __syncthreads();
+}
+// Two radix-16 butterflies with the factors of one table row.
+__device__ __forceinline__ void row_stage(float2 (&x)[32], const float2* trow) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        float2 y[16], tw[8];
+#pragma unroll
+        for (int r = 0; r < 8; ++r) tw[r] = trow[r];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) y[r] = x[16 * h + r];
+        dft_tw<16>(y, tw);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[16 * h + r] = y[r];
+        __builtin_amdgcn_sched_barrier(0);  // one butterfly's factors at a time
+    }
+}
 template <int LG2, int MODE, bool BATCH>
-__global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
+__global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? (MODE == ROWS_DYN ? 2 : 3) : 1) void k_rows(
     float2* __restrict__ Yk, float2* __restrict__ Sst, float2* __restrict__ Rt, Geom g,
     const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
     uint32_t* __restrict__ info, const uint32_t* __restrict__ ws, uint32_t* __restrict__ seed_ws,
@@ -932,7 +971,9 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
     constexpr int PPT = N2 / NTR, KL = PPT / 16;          // points and radix-16 butterflies per thread
     constexpr int R1 = LG2 == 8 ? 16 : N2 / 256, K1 = PPT / R1;
     constexpr int SEQS = seq_stride(N2);
-    __shared__ float2 buf[RPW * SEQS];
+    constexpr bool HALF = LG2 == 13 && MODE != ROWS_DYN;  // LDS holds one component of the row at a time
+    __shared__ float2 buf[HALF ? SEQS / 2 : RPW * SEQS];
+    float* fbuf = reinterpret_cast<float*>(buf);
     __shared__ float2 twl[TWL_SIZE];
     __shared__ float2 ttf[LG2 == 8 ? 1 : R1 * stage_row<16>()];  // forward middle stage (radix 16, span R1)
     __shared__ float2 tti[LG2 == 8 ? 1 : 16 * stage_row<16>()];  // inverse middle stage (radix 16, span 16)
@@ -960,7 +1001,29 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
     }
     __syncthreads();  // tables
     // forward stages 1 (inputs in v) .. 3; request() runs once stage 1 has consumed v
-    auto forward = [&](float2 (&z)[KL][16], auto&& request) {
+    auto forward = [&](float2 (&z)[KL][16], auto&& request) __attribute__((always_inline)) {
+        if constexpr (HALF) {
+            float2 x[32];
+#pragma unroll
+            for (int r = 0; r < 32; ++r) x[r] = v[r];
+            dft<32>(x);
+            request();
+            row_exchange(x, fbuf, [&](int e) { return 33 * j + e; }, [&](int e) { return padi(j + 256 * (e >> 4)) + 528 * (e & 15); });
+            row_stage(x, ttf + (j & 31) * stage_row<16>());
+            row_exchange(x, fbuf,
+                         [&](int e) { const int b = j + 256 * (e >> 4); return padi((b / 32) * 512 + b % 32) + 33 * (e & 15); },
+                         [&](int e) { return padi(j + 256 * (e >> 4)) + 528 * (e & 15); });
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                float2 tw[8];
+                twiddle_set_lds<16>(tw, twl, (j + 256 * h) * (TW14 / N2));
+#pragma unroll
+                for (int r = 0; r < 16; ++r) z[h][r] = x[16 * h + r];
+                dft_tw<16>(z[h], tw);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < K1; ++i) {
             float2 x[R1];
@@ -1000,21 +1063,45 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? 2 : 1) void k_rows(
                 for (int r = 0; r < 16; ++r) S[h][r] = buf_load_f2(rs, vrow, (uint32_t)(8 * NTR * h + (N2 / 2) * r));
         }
     });
-#pragma unroll
-    for (int h = 0; h < KL; ++h) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) z[h][r] = conjf2(cmul(z[h][r], S[h][r]));
-        stage_first_to_lds<16>(z[h], seqbuf, j + NTR * h);
-    }
-    __syncthreads();
-    if constexpr (LG2 != 8) stockham_stage<16, 16, LG2, RPW, SEQS, NT, true>(buf, tti);
     float2 F[PPT];
+    if constexpr (HALF) {
 #pragma unroll
-    for (int i = 0; i < K1; ++i) {
-        float2 x[R1];
-        stage_last_from_lds<R1, N2>(x, seqbuf, j + NTR * i, twl);
+        for (int h = 0; h < 2; ++h) {
 #pragma unroll
-        for (int r = 0; r < R1; ++r) F[i + K1 * r] = x[r];
+            for (int r = 0; r < 16; ++r) z[h][r] = conjf2(cmul(z[h][r], S[h][r]));
+            dft<16>(z[h]);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) F[16 * h + r] = z[h][r];
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        row_exchange(F, fbuf, [&](int e) { return padi(16 * (j + 256 * (e >> 4))) + (e & 15); },
+                     [&](int e) { return padi(j + 256 * (e >> 4)) + 528 * (e & 15); });
+        row_stage(F, tti + (j & 15) * stage_row<16>());
+        row_exchange(F, fbuf,
+                     [&](int e) {
+                         const int b = j + 256 * (e >> 4), r = e & 15;
+                         return padi((b / 16) * 256 + b % 16) + 16 * r + (r >> 1);
+                     },
+                     [&](int e) { return padi(j) + 264 * e; });
+        float2 tw[16];
+        twiddle_set_lds<32>(tw, twl, j * (TW14 / N2));
+        dft_tw<32>(F, tw);
+    } else {
+#pragma unroll
+        for (int h = 0; h < KL; ++h) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) z[h][r] = conjf2(cmul(z[h][r], S[h][r]));
+            stage_first_to_lds<16>(z[h], seqbuf, j + NTR * h);
+        }
+        __syncthreads();
+        if constexpr (LG2 != 8) stockham_stage<16, 16, LG2, RPW, SEQS, NT, true>(buf, tti);
+#pragma unroll
+        for (int i = 0; i < K1; ++i) {
+            float2 x[R1];
+            stage_last_from_lds<R1, N2>(x, seqbuf, j + NTR * i, twl);
+#pragma unroll
+            for (int r = 0; r < R1; ++r) F[i + K1 * r] = x[r];
+        }
     }
     // R'[row][t2] = F[t2] w_2L^{t2 (4 row + 1)}, t2 = j + NTR e: base step^e, re-anchored every 8
     // steps to bound the recurrence error
