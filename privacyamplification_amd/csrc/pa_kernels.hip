@@ -795,9 +795,11 @@ __device__ __forceinline__ void mix_factors(float2* tw2, float2* tw1, uint32_t f
 // them, so bits, indexes and twiddles are fetched once per group; PER = 0: one group and one class, for
 // launches of few groups, which are bound by one workgroup's latency.  A batch's launch is bound by its
 // stores: 11 blocks of 11.7 M bits, key and seed, take 0.24 ms for 1.11 GB (4.6 TB/s; the 1.48 GB of the
-// power of two took 0.33).
+// power of two took 0.33).  No kernel of the served lengths may spill: scratch memory is given to a stream's
+// queue at a launch's first use and stalls the streams in flight (17 registers spilled here at D = 6, with
+// three workgroups a unit, and 2 in k_rows: p99.9 of a served stream 1.2 to 8 ms).
 template <int D, int PER, bool BATCH>
-__global__ __launch_bounds__(256, PER == 0 ? 4 : 3) void k_mix_fwd(FwdArgs a, Geom g, const float2* __restrict__ twlo,
+__global__ __launch_bounds__(256, PER == 0 ? 4 : D == 6 ? 2 : 3) void k_mix_fwd(FwdArgs a, Geom g, const float2* __restrict__ twlo,
                                                                    const float2* __restrict__ twhi,
                                                                    const float2* __restrict__ cls,
                                                                    const BlockArgs* __restrict__ bt) {
@@ -924,6 +926,7 @@ __global__ __launch_bounds__(256, PER == 0 ? 4 : 3) void k_mix_fwd(FwdArgs a, Ge
 template <typename W, typename R>
 __device__ __forceinline__ void row_exchange(float2 (&x)[32], float* lds, W&& wi, R&& ri) {
     float re[32];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int e = 0; e < 32; ++e) lds[wi(e)] = x[e].x;
     __syncthreads();
@@ -1008,11 +1011,12 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? (MODE == ROWS_DYN ? 
             for (int r = 0; r < 32; ++r) x[r] = v[r];
             dft<32>(x);
             request();
+            const int o = opaque_int(j);  // per-exchange address arithmetic, never kept live
             row_exchange(x, fbuf, [&](int e) { return 33 * j + e; }, [&](int e) { return padi(j + 256 * (e >> 4)) + 528 * (e & 15); });
             row_stage(x, ttf + (j & 31) * stage_row<16>());
             row_exchange(x, fbuf,
-                         [&](int e) { const int b = j + 256 * (e >> 4); return padi((b / 32) * 512 + b % 32) + 33 * (e & 15); },
-                         [&](int e) { return padi(j + 256 * (e >> 4)) + 528 * (e & 15); });
+                         [&](int e) { const int b = o + 256 * (e >> 4); return padi((b / 32) * 512 + b % 32) + 33 * (e & 15); },
+                         [&](int e) { return padi(o + 256 * (e >> 4)) + 528 * (e & 15); });
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 float2 tw[8];
@@ -1083,9 +1087,12 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? (MODE == ROWS_DYN ? 
                          return padi((b / 16) * 256 + b % 16) + 16 * r + (r >> 1);
                      },
                      [&](int e) { return padi(j) + 264 * e; });
-        float2 tw[16];
-        twiddle_set_lds<32>(tw, twl, j * (TW14 / N2));
-        dft_tw<32>(F, tw);
+        {
+            float2 tw[16];
+            twiddle_set_lds<32>(tw, twl, opaque_int(j) * (TW14 / N2));
+            dft_tw<32>(F, tw);
+        }
+        __builtin_amdgcn_sched_barrier(0);
     } else {
 #pragma unroll
         for (int h = 0; h < KL; ++h) {
