@@ -117,7 +117,7 @@ int pa_block_device_seeded(pa_engine* eng, const uint32_t* d_key, pa_seed_id see
 
 /* pa_block_device that allocates nothing.  No counterpart in the reference: it is for callers that
  * cannot allocate device memory -- code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc.  The block's scratch (spectra, bit masks, nibbles, popcount partials)
+ * that forbid hipMalloc.  The block's scratch (spectra, rounded bits, scan results)
  * lives in one file-scope device array of 64 MiB per GPU, held until the process ends; the twiddle
  * tables it needs are made by pa_create.  Serves transform lengths up to 2^22 bits (n <= 2^22);
  * larger blocks return PA_ERR_SIZE (pa_strerror names the limit).  Same arguments and output as
@@ -140,7 +140,7 @@ typedef struct {
 
 /* Batch options: PA_BATCH_GRAPH replays a captured hipGraph for a batch of the same shape
  * (lengths classes, seed modes and counts); PA_BATCH_TUNE times the launch shapes of a shape not
- * seen before (pass A walk length, then row-pass grid) and keeps the fastest. */
+ * seen before (pass A's walk length) and keeps the fastest. */
 enum pa_batch_flags {
     PA_BATCH_GRAPH = 1u,
     PA_BATCH_TUNE = 2u
@@ -235,8 +235,8 @@ enum pa_buffer {
     PA_BUF_BITS_KEY,       /* key bit masks of pass A */
     PA_BUF_BITS_SEED,      /* seed bit masks */
     PA_BUF_NIB,            /* rounded output bits before packing */
-    PA_BUF_COUNTS,         /* popcount partials */
-    PA_BUF_TILES,          /* pass B's output in tiles for pass A' (transform lengths 2^24..2^27) */
+    PA_BUF_COUNTS,         /* input scan results */
+    PA_BUF_TILES,          /* pass B's output in tiles for pass A' (transform lengths 2^25..2^29) */
     PA_BUF_COUNT
 };
 /* Buffer extents of a block shape, a diagnostic with no counterpart in the reference: touched[b]
@@ -244,7 +244,8 @@ enum pa_buffer {
  * every allocation path gives it (the smallest over the per-size workspace, pa_submit, batch and
  * serving staging; for key, seed and out also the caller contract of the device entry points:
  * key_words * 4, n/8 and m/8 or n/16 bytes).  The engine refuses a shape with touched > alloc
- * (PA_ERR_UNSUPPORTED).  *transform_len receives L.  Runs on the host only. */
+ * (PA_ERR_UNSUPPORTED).  *transform_len receives the power of two that holds the block (the
+ * transform itself is 3/4 of it where that suffices, from 2^19 to 2^25).  Runs on the host only. */
 int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform_len,
                      uint64_t touched[PA_BUF_COUNT], uint64_t alloc[PA_BUF_COUNT]);
 

@@ -65,7 +65,7 @@ constexpr int MID_MAX_LOG_N = 23;
 // is as ever.  Against the power of two, blocks of 0.7 * 2^k bits, us of one block / a block in a batch of 2^27
 // bits: k = 19 22.3 / 2.85 to 21.5 / 2.09, k = 22 43.3 / 22.8 to 42.5 / 16.9, k = 23 66 / 48 to 53 / 33, k = 24 123 /
 // 101 to 98 / 70, k = 25 266 / 214 to 174 / 155; on a resident seed k = 19 23.1 / 2.17 to 20 / 1.6, k = 22 32.7 / 16.7 to
-// 35.1 / 12.3 (the one loss), k = 25 215 / 171 to 140 / 121.  Below k = 19 the direct product takes single blocks.
+// 35.1 / 12.3 (the one loss), k = 25 215 / 171 to 129 / 115.  Below k = 19 the direct product takes single blocks.
 constexpr uint32_t MIX_M = 256;
 constexpr int MIX_MIN_LOG_L = 19, MIX_MAX_LOG_L = 25;  // ceil(log2 L) of the lengths served
 __host__ __device__ constexpr uint32_t mix_classes(int lgL) { return lgL == 25 ? 6u : 3u; }

@@ -204,7 +204,7 @@ BUFFERS = ("key", "seed", "out", "spec_key", "spec_seed", "bits_key", "bits_seed
 
 
 def block_extents(n, m, flags=DEFAULT_FLAGS):
-    """pa_block_extents: (L, touched, alloc) for a block shape, touched / alloc as {buffer: bytes}
+    """pa_block_extents: (L, touched, alloc) for a block shape, L the power of two that holds it, touched / alloc as {buffer: bytes}
     (bytes its kernels index at most / bytes every allocation path gives it).  Host only."""
     L = load_library()
     tl = ctypes.c_uint32()
