@@ -919,7 +919,7 @@ __global__ __launch_bounds__(256, PER == 0 ? 4 : D == 6 ? 2 : 3) void k_mix_fwd(
 // of 213, 2^27 710 instead of 715, 2^23 in a batch 35.5 instead of 36.8.  Not with a fresh seed, where the
 // seed row's 32 values more spill 23 registers and their reloads wait on the loads in flight: the pass
 // takes 0.437 ms instead of 0.397 at 2^27.  Shorter rows take 16
-// points per thread and at least one wave per workgroup (rows_per_wg rows).
+// points per thread, rows_per_wg or rows_per_wg_many rows per workgroup.
 // The launch's first workgroup finishes the scan (scan_finish).
 // A row of 8192 points between two stages: value e of 32 goes to wi(e), comes back from ri(e), through LDS
 // of half the row: real parts, then imaginary parts.  Ends with a barrier.
@@ -955,8 +955,8 @@ __device__ __forceinline__ void row_stage(float2 (&x)[32], const float2* trow) {
         __builtin_amdgcn_sched_barrier(0);  // one butterfly's factors at a time
     }
 }
-template <int LG2, int MODE, bool BATCH>
-__global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? (MODE == ROWS_DYN ? 2 : 3) : 1) void k_rows(
+template <int LG2, int MODE, bool BATCH, int RPW>
+__global__ __launch_bounds__(rows_threads(LG2, RPW), LG2 == 13 ? (MODE == ROWS_DYN ? 2 : 3) : 1) void k_rows(
     float2* __restrict__ Yk, float2* __restrict__ Sst, float2* __restrict__ Rt, Geom g,
     const float2* __restrict__ tw14, const float2* __restrict__ twlo, const float2* __restrict__ twhi,
     uint32_t* __restrict__ info, const uint32_t* __restrict__ ws, uint32_t* __restrict__ seed_ws,
@@ -970,7 +970,7 @@ __global__ __launch_bounds__(rows_threads(LG2), LG2 == 13 ? (MODE == ROWS_DYN ? 
         info = a.info;
         ws = a.seed ? nullptr : a.ws;
     }
-    constexpr int N2 = 1 << LG2, NT = rows_threads(LG2), RPW = rows_per_wg(LG2), NTR = NT / RPW;
+    constexpr int N2 = 1 << LG2, NT = rows_threads(LG2, RPW), NTR = NT / RPW;
     constexpr int PPT = N2 / NTR, KL = PPT / 16;          // points and radix-16 butterflies per thread
     constexpr int R1 = LG2 == 8 ? 16 : N2 / 256, K1 = PPT / R1;
     constexpr int SEQS = seq_stride(N2);
@@ -2103,24 +2103,30 @@ template <bool BATCH>
 hipError_t rows(int mode, float2* Yk, float2* S, float2* Rt, const Geom& g, const Tables& t, uint32_t* info,
                 const uint32_t* ws, uint32_t* seed_ws, const BlockArgs* bt, uint32_t count, hipStream_t s) {
     return by_lg2(g.lg2, [&](auto lg) {
-        constexpr int LG2 = decltype(lg)::value, NT = rows_threads(LG2);
-        const dim3 grid(g.N1 / (uint32_t)rows_per_wg(LG2) + 1u, 1, count);  // + scan_finish
-        switch (mode) {
-        case ROWS_STATIC:
-            k_rows<LG2, ROWS_STATIC, BATCH><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
-            break;
-        case ROWS_DYN:
-            k_rows<LG2, ROWS_DYN, BATCH><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
-            break;
-        case ROWS_SEEDPREP:
-            if constexpr (!BATCH) {
-                k_rows<LG2, ROWS_SEEDPREP, false><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+        constexpr int LG2 = decltype(lg)::value;
+        auto launch = [&](auto rpw) {
+            constexpr int RPW = decltype(rpw)::value, NT = rows_threads(LG2, RPW);
+            const dim3 grid(g.N1 / (uint32_t)RPW + 1u, 1, count);  // + scan_finish
+            switch (mode) {
+            case ROWS_STATIC:
+                k_rows<LG2, ROWS_STATIC, BATCH, RPW><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
                 break;
+            case ROWS_DYN:
+                k_rows<LG2, ROWS_DYN, BATCH, RPW><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+                break;
+            case ROWS_SEEDPREP:
+                if constexpr (!BATCH) {
+                    k_rows<LG2, ROWS_SEEDPREP, false, RPW><<<grid, NT, 0, s>>>(Yk, S, Rt, g, t.tw14, t.lo, t.hi, info, ws, seed_ws, bt);
+                    break;
+                }
+                [[fallthrough]];
+            default: return hipErrorInvalidValue;
             }
-            [[fallthrough]];
-        default: return hipErrorInvalidValue;
-        }
-        return hipGetLastError();
+            return hipGetLastError();
+        };
+        if constexpr (BATCH && LG2 < 12)
+            if ((uint64_t)g.N1 * count >= 1024u * rows_per_wg_many(LG2)) return launch(std::integral_constant<int, rows_per_wg_many(LG2)>());
+        return launch(std::integral_constant<int, rows_per_wg(LG2)>());
     });
 }
 template <bool BATCH>

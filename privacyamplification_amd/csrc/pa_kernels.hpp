@@ -8,9 +8,14 @@
 namespace pa {
 
 enum { ROWS_DYN = 0, ROWS_STATIC = 1, ROWS_SEEDPREP = 2 };
-// Row pass: threads per workgroup and rows per workgroup (a row takes N2 / 16 threads, N2 / 32 at 8192).
+// Row pass: rows per workgroup (a row takes N2 / 16 threads, N2 / 32 at 8192), and those of batched launches
+// with at least 1024 such workgroups (four a compute unit), 256 threads each: the twiddle tables that a
+// workgroup loads first are 3 KB, as much as half a row of 2^9 points or less.  Us a block with few / many
+// rows: 2^18 bits, batch of 256, 1.52 / 1.47, resident 1.15 / 1.07; 2^19 2.95 / 2.84 and 2.25 / 2.12; 733984
+// bits, batch of 182, 4.35 / 4.19 and 3.29 / 3.09; 64 of 2^18 on a resident seed 98.8 / 95.0 us a call.
 __host__ __device__ constexpr int rows_per_wg(int lg2) { return lg2 == 8 ? 4 : lg2 == 9 ? 2 : 1; }
-__host__ __device__ constexpr int rows_threads(int lg2) { return lg2 == 13 ? 256 : rows_per_wg(lg2) * (1 << lg2) / 16; }
+__host__ __device__ constexpr int rows_per_wg_many(int lg2) { return lg2 >= 12 ? 1 : 4096 >> lg2; }
+__host__ __device__ constexpr int rows_threads(int lg2, int rpw) { return lg2 == 13 ? 256 : rpw * (1 << lg2) / 16; }
 // Column passes for L <= 2^22: threads and first radix (16 columns, one second-stage butterfly each).
 __host__ __device__ constexpr int mid_threads(int lg1) { return lg1 >= 10 ? 512 : lg1 >= 8 ? 256 : 1 << lg1; }
 __host__ __device__ constexpr int mid_r1(int lg1) { return lg1 >= 10 ? 32 : lg1 >= 8 ? 16 : 1 << (lg1 - 4); }

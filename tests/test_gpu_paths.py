@@ -129,3 +129,33 @@ def test_mixed_radix_blocks(engine, oracle, n, m):
             assert np.array_equal(engine.amplify(key, seed, n, m, False, True), ref), (n, m, "host")
     finally:
         engine.seed_drop(sid)
+
+
+# batches whose row passes take many rows a workgroup (from 1024 workgroups of 256 threads on) and one block
+# fewer; row lengths 2^8 .. 2^11, powers of two and 3 * 2^k.  Same inputs, so every output is the oracle's.
+@pytest.mark.parametrize("n,count", [(147456, 128), (147456, 127), (262144, 32), (262144, 31), (1 << 19, 16), (1 << 20, 8),
+                                     (1 << 20, 7), (393216, 22), (393216, 21), (786432, 11), (1572864, 3), (1572864, 2)])
+def test_batched_rows_per_workgroup(engine, oracle, n, count):
+    import torch
+    m = 3 * n // 8 // 32 * 32
+    key, seed = oracle.synth_bits(0xF1 + n, n + 1), oracle.synth_bits(0xF2, n)
+    ref = torch.from_numpy(oracle.amp_out(key, seed, n, m, True, True, method=oracle.NTT).copy()).cuda()
+    sid = engine.seed_put(seed, n, m)
+    try:
+        say(f"rows n={n} count={count}")
+        d = _Device(key, seed, count * (m // 8))
+        for fresh in (True, False):
+            blk = (P.PaBlock * count)()
+            for i in range(count):
+                blk[i].key, blk[i].n, blk[i].m, blk[i].flags = d.key.data_ptr(), n, m, 3
+                blk[i].out = d.out.data_ptr() + i * (m // 8)
+                if fresh:
+                    blk[i].seed = d.seed.data_ptr()
+                else:
+                    blk[i].seed_id = sid
+            engine.batch_device(blk, 0, 0)
+            torch.cuda.synchronize()
+            assert torch.equal(d.out[: count * (m // 8)].reshape(count, m // 8), ref.expand(count, -1)), (n, count, fresh)
+            d.take()
+    finally:
+        engine.seed_drop(sid)
