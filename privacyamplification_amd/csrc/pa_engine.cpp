@@ -11,6 +11,7 @@
 #include <cstdarg>
 #include <chrono>
 #include <cmath>
+#include <complex>
 #include <cstdio>
 #include <cstring>
 #include <map>
@@ -106,7 +107,7 @@ int make_geom(uint32_t n, uint32_t m, uint32_t flags, uint32_t reverse_endian, u
     x.do_xor = (flags & PA_XOR_KEY_REST) ? 1u : 0u;
     x.reverse_endian = reverse_endian ? 1u : 0u;
     if (x.N1 > 1) {
-        x.rho = pa::RHO;
+        x.white = mid_size(x) ? pa::WHITE_MID : pa::WHITE_BIG;
         x.scan = mid_size(x) ? 0 : 2;
         x.inv_N = 1.0f / (float)x.N;
     } else {
@@ -166,8 +167,8 @@ Extents block_extents(const Geom& g) {
     x.alloc[PA_BUF_OUT] = std::min({(uint64_t)out_bytes_of(g), stage_out_bytes(g), ws_out_bytes(g.L)});
     if (g.N1 == 1) return x;  // the one-workgroup path keeps everything else on chip
     x.alloc[PA_BUF_COUNTS] = pa::info_bytes(g);
-    // the last parity byte, scan_parities(info)[chunks - 1]
-    x.touched[PA_BUF_COUNTS] = pa::INFO_HEAD * 4 + pa::scan_chunks(g) * 9ull;
+    // the last word of the last fold slice
+    x.touched[PA_BUF_COUNTS] = ((uint64_t)pa::info_fold(g) + (uint64_t)pa::fold_slices(g) * g.white) * 4;
     if (!mid_size(g)) {
         // k_transpose_bits writes tb[u N2 + t2] for u < M, t2 < N2 (D = 32: u < 2 M)
         x.touched[PA_BUF_BITS_KEY] = x.touched[PA_BUF_BITS_SEED] = (uint64_t)g.M * g.N2 * (g.D == 32 ? 8 : 4);
@@ -222,7 +223,7 @@ struct Workspace {
 struct Seed {
     Geom g{};
     float2* spec = nullptr;    // spectrum: N complex (four-step path), N+1 split (small path)
-    uint32_t* ws = nullptr;    // device popcount (POP_SLOTS partials)
+    uint32_t* ws = nullptr;    // device popcount (POP_SLOTS partials), then conv(R, seed), g.white words
     uint32_t* sq = nullptr;    // prefix words (four-step path): L/8 bytes, 1/32 of the spectrum, not
                                // charged to the budget, so that it holds as many seeds as it says
     uint32_t* words = nullptr; // the seed itself up to 2^DIRECT_MAX_L_LOG bits, for the direct product;
@@ -808,7 +809,7 @@ int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform
 
 static int seed_alloc(pa_engine* e, Seed* sd) {
     const Geom& g = sd->g;
-    const uint64_t spec = align256((uint64_t)(g.N + 1) * sizeof(float2)), ws = align256(pa::POP_SLOTS * 4);
+    const uint64_t spec = align256((uint64_t)(g.N + 1) * sizeof(float2)), ws = align256((pa::POP_SLOTS + g.white) * 4ull);
     sd->bytes = (uint64_t)(g.N + 1) * sizeof(float2) + pa::POP_SLOTS * sizeof(uint32_t);
     if (e->cfg.hbm_budget_bytes && e->used_bytes + sd->bytes > e->cfg.hbm_budget_bytes) return PA_ERR_NOMEM;
     uint8_t* p = nullptr;
@@ -2193,25 +2194,28 @@ int st_correction(pa_engine* e, Report& rp) {
     return rp.done("CalculateCorrectionFloat");
 }
 
-// The seed's spectrum through the production pass A and row pass (pa_seed_put's launches), the seed
-// whitened by rho.
-int st_seed_spectrum(pa_engine* e, const uint32_t* h_seed, uint32_t n, uint32_t rho, std::vector<float2>& S, Geom& g,
-                     uint32_t& ws) {
+// The spectrum of L bits (n of them given) as the seed, or as a key that fills the whole sequence,
+// through the production pass A and row pass (pa_seed_put's launches); pops: the scan's popcount.
+int st_spectrum(pa_engine* e, const uint32_t* h_bits, uint32_t n, bool is_key, std::vector<float2>& S, Geom& g,
+                uint32_t& pops) {
     Workspace* w;
-    int rc = prepare(e, n, 3 * n / 8, PA_DEFAULT_FLAGS, &g, &w);
+    int rc = prepare(e, n, n / 2, PA_DEFAULT_FLAGS, &g, &w);
     if (rc != PA_OK) return rc;
-    g.rho = rho;
-    DevMem dS, dws, dseed;
+    g.key_hw = g.L / 32;  // every word is the key's
+    DevMem dS, dws, dbits;
     const bool mid = mid_size(g);
     ST_ALLOC(dS, (size_t)g.N * 8);
-    ST_ALLOC(dws, pa::POP_SLOTS * 4);
-    ST_ALLOC(dseed, (size_t)n / 8);
+    ST_ALLOC(dws, (pa::POP_SLOTS + g.white) * 4);
+    ST_ALLOC(dbits, (size_t)n / 8);
     hipStream_t s = e->stream;
-    PA_HIP(hipMemcpyAsync(dseed.p, h_seed, n / 8, hipMemcpyHostToDevice, s));
+    PA_HIP(hipMemcpyAsync(dbits.p, h_bits, n / 8, hipMemcpyHostToDevice, s));
     const pa::Tables t = tables(e, g.L);
-    const pa::ScanArgs scan{nullptr, dseed.as<uint32_t>(), nullptr, pa::prefix_words(w->nib, g.N), w->info};
-    if (!mid) PA_HIP(pa::launch_transpose(nullptr, dseed.as<uint32_t>(), nullptr, w->tbs, 1, 1, g, &scan, s));
-    PA_HIP(pa::launch_fwd_cols(nullptr, mid ? dseed.as<uint32_t>() : w->tbs, nullptr, dS.as<float2>(), 1, 1, g, t, &scan, s));
+    const uint32_t* bits = dbits.as<uint32_t>();
+    const uint32_t op = is_key ? 0u : 1u;
+    const pa::ScanArgs scan{is_key ? bits : nullptr, is_key ? nullptr : bits, nullptr, pa::prefix_words(w->nib, g.N), w->info};
+    if (!mid) PA_HIP(pa::launch_transpose(bits, bits, w->tbs, w->tbs, op, 1, g, &scan, s));
+    const uint32_t* in = mid ? bits : w->tbs;
+    PA_HIP(pa::launch_fwd_cols(in, in, dS.as<float2>(), dS.as<float2>(), op, 1, g, t, &scan, s));
     PA_HIP(pa::launch_rows(pa::ROWS_SEEDPREP, nullptr, dS.as<float2>(), nullptr, g, t, w->info, nullptr,
                            dws.as<uint32_t>(), s));
     S.resize(g.N);
@@ -2219,48 +2223,69 @@ int st_seed_spectrum(pa_engine* e, const uint32_t* h_seed, uint32_t n, uint32_t 
     PA_HIP(hipMemcpyAsync(S.data(), dS.p, (size_t)g.N * 8, hipMemcpyDeviceToHost, s));
     PA_HIP(hipMemcpyAsync(part.data(), dws.p, pa::POP_SLOTS * 4, hipMemcpyDeviceToHost, s));
     PA_HIP(hipStreamSynchronize(s));
-    ws = 0;
-    for (uint32_t v : part) ws += v;
+    pops = 0;
+    for (uint32_t v : part) pops += v;
     return PA_OK;
 }
 
+// Bin k of the whitened all-ones key: with theta = 2 pi (k + 1/4) / N and R = +-1 of period P bits, a product
+// of levels whose last one changes sign after half of it, the sum over t < N of (1 - i) R[t] / 2 e^{-i theta t} is
+//   (sum over 32 bits) (the other levels' sums) (half of the last one's) / (1 + e^{-i theta P / 2}).
+std::complex<double> st_white_bin(const Geom& g, double theta) {
+    const bool big = g.white == pa::WHITE_BIG;
+    const uint32_t levels = big ? 3 : 2;
+    std::complex<double> r = 1.0;
+    auto level = [&](double step, uint32_t count, auto&& sign) {
+        std::complex<double> x = 0.0;
+        for (uint32_t i = 0; i < count; ++i) x += std::polar(sign(i) ? -1.0 : 1.0, -theta * step * i);
+        r *= x;
+    };
+    level(1.0, 32, [](uint32_t) { return false; });
+    uint32_t b = 1;
+    for (uint32_t l = 0; l < levels; ++l, b *= 16) {
+        const uint32_t c = big || l == 0 ? 16 : 8;
+        level(32.0 * b, l + 1 == levels ? c / 2 : c, [&](uint32_t i) { return (pa::white_word(g, b * i) ^ pa::white_word(g, 0)) != 0; });
+    }
+    if (pa::white_word(g, 0)) r = -r;
+    return r / (1.0 + std::polar(1.0, -theta * 16.0 * g.white));
+}
+
 int st_dc_zero(pa_engine* e, Report& rp) {
-    // setFirstElementToZero (:377-418) removes the mean's contribution; here the +-1/2 encoding and
-    // the whitening do.  Unwhitened, an all-ones seed (a constant sequence) has the closed form
-    // S[k] = 1 / (1 - exp(-2 pi i (k + 1/4) / N)); whitened, nothing of its mean is left near k = 0;
-    // a random seed keeps a spectrum
-    const uint32_t n = 1u << 20;
-    std::vector<uint32_t> ones(n / 32, 0xFFFFFFFFu), rnd(n / 32);
-    pa_synth_bits(0x5E1F, 0.5, n, rnd.data());
-    for (int which = 0; which < 3 && rp.ok; ++which) {
-        std::vector<float2> S;
-        Geom g;
-        uint32_t ws = 0;
-        const uint32_t rho = which == 0 ? 0u : pa::RHO;
-        const std::vector<uint32_t>& seed = which == 2 ? rnd : ones;
-        int rc = st_seed_spectrum(e, seed.data(), n, rho, S, g, ws);
-        if (rc != PA_OK) return rc;
-        uint32_t want_ws = 0;
-        for (uint32_t v : seed) want_ws += (uint32_t)__builtin_popcount(v ^ rho);
-        if (ws != want_ws) rp.fail("SetFirstElementToZero: seed popcount %u, want %u", ws, want_ws);
-        auto at = [&](uint32_t k) { return S[(size_t)(k % g.N1) * g.N2 + k / g.N1]; };
-        double mx = 0.0;
-        for (uint32_t k = 0; k < g.N && rp.ok; ++k) {
-            const float2 v = at(k);
-            if (which == 0) {
-                const double a = 2.0 * M_PI * (k + 0.25) / g.N, d = 2.0 - 2.0 * std::cos(a);
-                const double re = (1.0 - std::cos(a)) / d, im = -std::sin(a) / d;
-                if (std::hypot(v.x - re, v.y - im) > 1e-6 * n)
-                    rp.fail("SetFirstElementToZero: constant seed, bin %u (%g, %g), want (%g, %g)", k, v.x, v.y, re, im);
-            } else {
-                mx = std::max(mx, k < g.N / 64 || which == 2 ? (double)std::hypot(v.x, v.y) : 0.0);
+    // setFirstElementToZero (:377-418) removes the mean's contribution; here the +-1/2 encoding and the
+    // key's whitening do.  An all-ones seed (a constant sequence) has the closed form
+    // S[k] = 1 / (1 - exp(-2 pi i (k + 1/4) / N)); of an all-ones key nothing is left near k = 0 and
+    // R's own lines elsewhere (st_white_bin); a random seed keeps a spectrum
+    for (uint32_t n : {1u << 15, 1u << 20, 3u << 18, 1u << 23, 3u << 22, 3u << 23, 1u << 25}) {
+        if (!rp.ok || log2u(n) > e->cfg.max_n_log2) break;
+        for (int which = 0; which < 3 && rp.ok; ++which) {  // constant seed, constant key, random seed
+            std::vector<uint32_t> bits(n / 32, 0xFFFFFFFFu);
+            if (which == 2) pa_synth_bits(0x5E1F, 0.5, n, bits.data());
+            std::vector<float2> S;
+            Geom g;
+            uint32_t pops = 0, want = 0;
+            int rc = st_spectrum(e, bits.data(), n, which == 1, S, g, pops);
+            if (rc != PA_OK) return rc;
+            for (uint32_t i = 0; i < n / 32; ++i) want += (uint32_t)__builtin_popcount(bits[i] ^ (which == 1 ? pa::white_word(g, i) : 0u));
+            if (pops != want) rp.fail("SetFirstElementToZero: n = %u popcount %u, want %u", n, pops, want);
+            auto at = [&](uint32_t k) { return S[(size_t)(k % g.N1) * g.N2 + k / g.N1]; };
+            double mx = 0.0;
+            // the bins around DC and, of the long transforms, a sample of the others
+            for (uint32_t k = 0; k < g.N && rp.ok; k += k < 4096 || k >= g.N - 4096 || g.N < (1u << 20) ? 1u : 61u) {
+                const float2 v = at(k);
+                if (which == 2) {
+                    mx = std::max(mx, (double)std::hypot(v.x, v.y));
+                    continue;
+                }
+                const double theta = 2.0 * M_PI * (k + 0.25) / g.N;
+                const std::complex<double> x = which == 0 ? 1.0 / (1.0 - std::polar(1.0, -theta)) : st_white_bin(g, theta);
+                if (std::hypot(v.x - x.real(), v.y - x.imag()) > 1e-6 * n)
+                    rp.fail("SetFirstElementToZero: n = %u constant %s, bin %u (%g, %g), want (%g, %g)", n,
+                            which ? "key" : "seed", k, v.x, v.y, x.real(), x.imag());
             }
+            if (rp.ok && which == 1 && std::hypot(at(0).x, at(0).y) > 1e-5 * n)
+                rp.fail("SetFirstElementToZero: n = %u constant key leaves |S| %.3g at DC", n, std::hypot(at(0).x, at(0).y));
+            if (rp.ok && which == 2 && mx < 1.0) rp.fail("SetFirstElementToZero: n = %u random seed spectrum vanished", n);
         }
-        // a 32-periodic balanced sequence sums to at most 16 ones; the bins below N / 64 lie far
-        // from the first line of its spectrum (N / 16)
-        if (rp.ok && which == 1 && mx > 64.0)
-            rp.fail("SetFirstElementToZero: whitened constant seed leaves |S| %.3g near DC", mx);
-        if (rp.ok && which == 2 && mx < 1.0) rp.fail("SetFirstElementToZero: random seed spectrum vanished");
     }
     return rp.done("SetFirstElementToZero");
 }
@@ -2312,7 +2337,7 @@ int st_unpack(pa_engine* e, Report& rp) {
     for (uint32_t i = 0; i < nmax / 32; ++i) bin[i] = i;
     DevMem dbin, dws;
     ST_ALLOC(dbin, nmax / 8);
-    ST_ALLOC(dws, pa::POP_SLOTS * 4);
+    ST_ALLOC(dws, (pa::POP_SLOTS + pa::WHITE_BIG) * 4);
     PA_HIP(hipMemcpy(dbin.p, bin.data(), nmax / 8, hipMemcpyHostToDevice));
     uint64_t lcg = 12345;
     for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
@@ -2321,7 +2346,6 @@ int st_unpack(pa_engine* e, Report& rp) {
         Workspace* w;
         int rc = prepare(e, n, 3 * n / 8, PA_DEFAULT_FLAGS, &g, &w);
         if (rc != PA_OK) return rc;
-        g.rho = 0;         // the plain bits
         g.out_bits = g.L;  // every word's prefix
         const bool mid = mid_size(g);
         uint32_t* bits = dbin.as<uint32_t>();

@@ -14,10 +14,15 @@
 // sequences up to q and W the sum of both popcounts, sum_j sgn x[j] t[(q-j) mod L] = c[q] + PX(q) +
 // PT(q) - (W + q + 1)/2 + L/4.  So round(c[q] - ((W + q + 1) mod 4)/2), plus the parities of PX and PT,
 // is the bit; the parities are a bit scan over the inputs (prefix_chunk).
-//   Whitening.  Where both means are far from 1/2 the values of c would grow like n/4, past FP32's
-// resolution for long blocks.  The seed is therefore XORed with a balanced word RHO of flat
-// spectrum, repeated; conv(x, RHO repeated) mod 2 has period 32 and follows from the XOR of the
-// key's words, one correction word for the whole output.
+//   Whitening.  The constant part of one operand (its mean, the key's zero pad) times a constant or
+// periodic part of the other would give values that grow like n/4, or spectral lines whose rounding errors
+// alone reach 1/2.  The key is therefore XORed with R, whole words of zeros and ones in a
+// pseudo-random order of long period (white_word): every simple key and its pad then have a flat spectrum, and
+// an operand with a flat spectrum multiplies any other to small values, as random keys do.
+//   The order is a sum mod 2 of levels: word w has sign s_l[(w / b_l) mod c_l], b = 1, 16, 256.  Each
+// level's second half is the complement of its first, so R is balanced and has no line at a frequency that
+// a sequence of half its period, or of any power of two below, has.  conv(R, t) mod 2 has R's period,
+// follows from the seed words folded to that period (white_table) and is added back by the output stage.
 //   N = N1 * N2 (t = t2 + N2*t1, k = k1 + N1*k2):
 //   pass A  column FFTs of length N1, 16 columns per workgroup.  L >= 2^23: decimated by D classes of
 //           k1 (M = N1/D per class), input from the bit-transposed key/seed; below, straight from
@@ -38,7 +43,17 @@ constexpr int ROW_LOG = 13;            // N2 = 8192 from L = 2^23 on
 constexpr int SMALL_MAX_LOG_N = 13;    // N <= 8192 -> single-workgroup path
 constexpr int MAX_L_LOG = 29;          // largest transform served (L = 2^29; the reference stops at 2^27)
 
-constexpr uint32_t RHO = 0x8F205B9Bu;   // 16 ones; |DFT_32| <= 3.57 away from DC, 0 there
+// The levels' signs: index i at bit i.  Periods of 16 * 8 words for the mid sizes, where the values are small
+// enough, and 16 * 16 * 16 for the others.  Chosen among 60 and 80 random ones by the rounding margin (max
+// |v - rint v|) of an all-ones key at 2^24 bits in an FP32 emulation of the passes, against constant seeds, square
+// waves and repeated random words: 0.05 and 0.011 at worst, for seeds of exactly R's period.  A constant seed
+// at 2^25 bits has 0.0017 with the long period, 0.028 with 128 words and 0.22 with alternating blocks of 256.
+// Largest margins measured over constant, 7/8 and random keys and seeds that repeat 1 to 64 words: 0.05 at 2^24,
+// 0.008 at 2^26, 0.014 at 2^27, 0.06 at 2^28, 0.13 at 2^29 bits (the seed alone whitened by a word of 32 bits: 0.5
+// from 2^26 on).
+constexpr uint32_t WHITE_MID = 128, WHITE_BIG = 4096;   // words
+constexpr uint32_t WHITE_S0 = 0x946Bu, WHITE_S1 = 0xD629u, WHITE_S2 = 0x15EAu;   // c = 16 each
+constexpr uint32_t WHITE_MID_S0 = 0x6699u, WHITE_MID_S1 = 0xC3u;                 // c = 16, 8
 
 // Pass B's output R'[k1][t2] when 2^RT_LG1_MIN <= N1 <= 2^RT_LG1_MAX (transforms of 2^25 to 2^29
 // bits) goes to its own buffer in tiles, Rt[((t2 / RT_COLS) N1 + k1) RT_COLS + t2 mod RT_COLS]: pass
@@ -80,7 +95,7 @@ struct Geom {
                                        // rotated seed repeats with period n up to L
     uint32_t key_hw;                   // h/32: index of the key word masked to its MSB
     uint32_t do_xor, reverse_endian;
-    uint32_t rho;                      // whitening word of the seed (0 on the small path)
+    uint32_t white;                    // period of the key's whitening in words (0 on the small path)
     uint32_t scan;                     // words per scan chunk: 1024 << scan
     float inv_N;                       // output normalisation: 1/N; on the small path 1/(8N), with the
                                        // factor of r2c_split / c2r_split
@@ -107,6 +122,14 @@ inline bool direct_size(const Geom& g, uint64_t work) {
     return g.N1 == 1u || (g.L <= (1u << DIRECT_MAX_L_LOG) && work <= DIRECT_WORK && direct_key_words(g) <= DIRECT_JPAD_MAX);
 }
 
+// Word w of the key's whitening R (zero on the small path).
+__host__ __device__ inline uint32_t white_word(const Geom& g, uint32_t w) {
+    const bool big = g.white == WHITE_BIG;
+    const uint32_t s0 = big ? WHITE_S0 : g.white ? WHITE_MID_S0 : 0u, s1 = big ? WHITE_S1 : g.white ? WHITE_MID_S1 : 0u;
+    const uint32_t s = (s0 >> (w & 15u)) ^ (s1 >> ((w >> 4) & (big ? 15u : 7u))) ^ (big ? WHITE_S2 >> ((w >> 8) & 15u) : 0u);
+    return 0u - (s & 1u);
+}
+
 // Inputs and outputs of the input scan: conv words of the key and the fresh seed (or the resident
 // seed's finished prefix words sq); prefix words q, and the block's info words.
 struct ScanArgs {
@@ -116,22 +139,20 @@ struct ScanArgs {
     uint32_t* q;
     uint32_t* info;
 };
-// A block's info buffer: what scan_finish writes, then per chunk its popcount and the XOR of its key
-// words (uint2), then per chunk one byte, its parity.
+// A block's info buffer: both popcounts; per chunk one byte, its parity; conv(R, t), g.white words; per
+// chunk its popcount; the fresh seed's words folded to the whitening's period, in fold_slices parts of
+// g.white words: one a chunk for the mid sizes (scan_chunk), else one per 16 values of the bit
+// transpose's u.
 constexpr int INFO_POPS = 0;    // both popcounts
-constexpr int INFO_WHITE = 1;   // the whitening's word
-constexpr int INFO_HEAD = 64;   // words before the chunk entries
+constexpr int INFO_HEAD = 64;   // words before the parities
 __host__ __device__ inline uint32_t scan_chunks(const Geom& g) { return g.L >> (15u + g.scan); }
-__host__ __device__ inline uint2* scan_entries(uint32_t* info) { return reinterpret_cast<uint2*>(info + INFO_HEAD); }
-__host__ __device__ inline uint8_t* scan_parities(uint32_t* info, const Geom& g) {
-    return reinterpret_cast<uint8_t*>(scan_entries(info) + scan_chunks(g));
-}
-__host__ __device__ inline const uint8_t* scan_parities(const uint32_t* info, const Geom& g) {
-    return scan_parities(const_cast<uint32_t*>(info), g);
-}
-inline uint64_t info_bytes(const Geom& g) {
-    return (uint64_t)INFO_HEAD * 4 + scan_chunks(g) * 8ull + (scan_chunks(g) + 255u) / 256u * 256u;
-}
+__host__ __device__ inline uint32_t fold_slices(const Geom& g) { return g.white == WHITE_BIG ? g.M / 16u : scan_chunks(g); }
+__host__ __device__ inline uint8_t* scan_parities(uint32_t* info) { return reinterpret_cast<uint8_t*>(info + INFO_HEAD); }
+__host__ __device__ inline const uint8_t* scan_parities(const uint32_t* info) { return reinterpret_cast<const uint8_t*>(info + INFO_HEAD); }
+__host__ __device__ inline uint32_t info_white(const Geom& g) { return (uint32_t)INFO_HEAD + (scan_chunks(g) + 255u) / 256u * 64u; }
+__host__ __device__ inline uint32_t info_pops(const Geom& g) { return info_white(g) + g.white; }
+__host__ __device__ inline uint32_t info_fold(const Geom& g) { return info_pops(g) + (scan_chunks(g) + 63u) / 64u * 64u; }
+inline uint64_t info_bytes(const Geom& g) { return ((uint64_t)info_fold(g) + (uint64_t)fold_slices(g) * g.white) * 4u; }
 
 // One block of a batched launch: its geometry and device buffers.  The blocks of one launch share
 // the transform length L (and so N1, N2, M, D, W); n, m, flags and the buffers are per block.
@@ -140,7 +161,7 @@ struct BlockArgs {
     const uint32_t* key;
     const uint32_t* seed;   // dynamic seed, or nullptr for a resident one (its words for the direct product)
     const float2* sspec;    // resident spectrum when seed == nullptr
-    const uint32_t* ws;     // resident seed popcount partials when seed == nullptr
+    const uint32_t* ws;     // resident seed popcount partials, and its conv(R, t), when seed == nullptr
     const uint32_t* sq;     // resident seed prefix words when seed == nullptr (four-step path only)
     float2* Yk;             // N values (four-step path only)
     float2* Ys;             // N+1 values (dynamic seed, four-step path only)

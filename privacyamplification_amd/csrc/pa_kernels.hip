@@ -41,7 +41,7 @@ __device__ __forceinline__ uint32_t key_word(const uint32_t* __restrict__ key, c
     return 0u;
 }
 // Word widx (< L/32) of the seed sequence t: the n seed bits rotated left by seed_rot words and
-// repeated with period n up to the transform length L, XORed with the whitening word g.rho.  The
+// repeated with period n up to the transform length L.  The
 // output window only reads t[0, n), where the repetition changes nothing; beyond n it keeps the
 // +-1/2-encoded sequence free of a constant block.  A zero pad there would become a -1/2 block
 // whose convolution with the key's pad swings by about h/4 across positions, far beyond FP32's
@@ -51,7 +51,7 @@ __device__ __forceinline__ uint32_t seed_word(const uint32_t* __restrict__ seed,
     uint32_t s = widx + g.seed_rot;  // < 3 seed_words: L < 2n when L > n
     if (s >= g.seed_words) s -= g.seed_words;
     if (s >= g.seed_words) s -= g.seed_words;
-    return seed[s] ^ g.rho;
+    return seed[s];
 }
 
 // A resident seed's popcount, kept as POP_SLOTS partials.
@@ -110,9 +110,10 @@ __global__ __launch_bounds__(COPY_NT) void k_copies(const CopyDesc* __restrict__
 // prefix sums of both bit sequences (see pa_geom.hpp); mod 2 only their parities matter.  A scan
 // workgroup takes one chunk of 1024 << g.scan words: inclusive prefix parities of x ^ t inside the
 // chunk go to q (bit p of word w: the parity of the chunk's bits up to there; only words up to the
-// end of the output window), the chunk's parity to its byte of cp, its popcount (key + seed) and
-// the XOR of its key words to its entry.  A resident seed brings its own finished prefix words sq;
-// x alone is scanned then.  The scan workgroups ride in the bit transpose's launch (in pass A's below
+// end of the output window), the chunk's parity to its byte of cp, its popcount (key + seed) to its
+// entry; for the mid sizes also the XOR of its seed words per word of the whitening's period (the bit
+// transpose has the others').  x is the whitened key.  A resident seed brings its own finished prefix
+// words sq; x alone is scanned then.  The scan workgroups ride in the bit transpose's launch (in pass A's below
 // L = 2^23); scan_finish, in pass B's, turns the entries into what pass A' and the output stage read.
 // (In pass A's launch at 2^27 they cost 15 us: with its 74 KB of LDS only two fit a compute unit.)
 __device__ __forceinline__ uint32_t prefix_bits(uint32_t w) {  // bit p: parity of bits 0..p, MSB first
@@ -122,7 +123,7 @@ __device__ __forceinline__ uint32_t prefix_bits(uint32_t w) {  // bit p: parity 
     w ^= w >> 8;
     return w ^ (w >> 16);
 }
-// NT threads; lds: 3 NT / 64 words.  key == nullptr scans the seed alone.  Per 1024 words a wave takes 64 PER
+// NT threads; lds: 2 NT (2 + 128) / 64 words at most.  key == nullptr scans the seed alone.  Per 1024 words a wave takes 64 PER
 // consecutive ones, 64 at a time: coalesced, the carry between lanes from a ballot.
 template <int NT>
 __device__ __forceinline__ void scan_chunk(uint32_t chunk, const ScanArgs& a, const Geom& g, uint32_t* lds) {
@@ -131,17 +132,24 @@ __device__ __forceinline__ void scan_chunk(uint32_t chunk, const ScanArgs& a, co
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
     const uint64_t before = (1ull << lane) - 1ull;
     const uint32_t w_end = (g.out_off + g.out_bits) >> 5;
-    uint32_t pops = 0, kx = 0, chunk_par = 0;
+    uint32_t pops = 0, chunk_par = 0, fold[2] = {0, 0};  // fold: words of lane and 64 + lane mod 128
     for (uint32_t sub = 0; sub < (1u << g.scan); ++sub) {
         const uint32_t w0 = ((chunk << g.scan) + sub) * 1024u + 64u * PER * wave + lane;
-        uint32_t w[PER], run = 0;
+        uint32_t w[PER], sw[PER], run = 0;
+        // no load is conditional on a lane, so that all are in flight together
 #pragma unroll
         for (uint32_t i = 0; i < PER; ++i) {
-            const uint32_t kw = a.key ? key_word(a.key, g, w0 + 64u * i) : 0u;
-            const uint32_t sw = a.seed ? seed_word(a.seed, g, w0 + 64u * i) : 0u;
-            pops += (uint32_t)(__popc(kw) + __popc(sw));
-            kx ^= kw;
-            w[i] = kw ^ sw;
+            const uint32_t wi = w0 + 64u * i;
+            w[i] = a.key ? a.key[wi < g.key_hw ? wi : g.key_hw] : 0u;
+            sw[i] = a.seed ? seed_word(a.seed, g, wi) : 0u;
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < PER; ++i) {
+            const uint32_t wi = w0 + 64u * i;
+            if (a.key) w[i] = (w[i] & (wi < g.key_hw ? ~0u : wi == g.key_hw ? 0x80000000u : 0u)) ^ white_word(g, wi);
+            pops += (uint32_t)(__popc(w[i]) + __popc(sw[i]));
+            fold[i & 1] ^= sw[i];
+            w[i] ^= sw[i];
         }
 #pragma unroll
         for (uint32_t i = 0; i < PER; ++i) {
@@ -167,54 +175,169 @@ __device__ __forceinline__ void scan_chunk(uint32_t chunk, const ScanArgs& a, co
             if (wi < w_end) a.q[wi] = w[i] ^ (0u - (carry & 1u)) ^ (a.sq ? a.sq[wi] : 0u);
         }
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        pops += __shfl_xor(pops, off);
-        kx ^= __shfl_xor(kx, off);
-    }
-    if (lane == 0) {
-        lds[NT / 64 + wave] = pops;
-        lds[2 * (NT / 64) + wave] = kx;
+    for (int off = 32; off > 0; off >>= 1) pops += __shfl_xor(pops, off);
+    if (lane == 0) lds[NT / 64 + wave] = pops;
+    const bool folds = a.seed && g.white == WHITE_MID;
+    uint32_t* lf = lds + 2 * (NT / 64);
+    if (folds) {
+        lf[128u * wave + lane] = fold[0];
+        lf[128u * wave + 64u + lane] = fold[1];
     }
     __syncthreads();
     if (threadIdx.x == 0) {
-        pops = kx = 0;
-        for (int k = 0; k < NT / 64; ++k) {
-            pops += lds[NT / 64 + k];
-            kx ^= lds[2 * (NT / 64) + k];
+        pops = 0;
+        for (int k = 0; k < NT / 64; ++k) pops += lds[NT / 64 + k];
+        a.info[info_pops(g) + chunk] = pops;
+        scan_parities(a.info)[chunk] = (uint8_t)chunk_par;
+    }
+    if (folds)
+        for (uint32_t c = threadIdx.x; c < WHITE_MID; c += NT) {
+            uint32_t x = 0;
+            for (int k = 0; k < NT / 64; ++k) x ^= lf[128u * k + c];
+            a.info[info_fold(g) + chunk * WHITE_MID + c] = x;
         }
-        scan_entries(a.info)[chunk] = make_uint2(pops, kx);
-        scan_parities(a.info, g)[chunk] = (uint8_t)chunk_par;
+}
+// In-place inclusive prefix parities of the `n` words at a (bit p of word w: of all bits up to there),
+// n / NT consecutive words a thread (one for the first n threads where n < NT); returns the parity of all.
+// part: NT / 64 words.  Ends with a barrier.
+template <int NT>
+__device__ __forceinline__ uint32_t prefix_words_lds(uint32_t* a, uint32_t n, uint32_t* part) {
+    const uint32_t per = n < (uint32_t)NT ? 1u : n / NT, i0 = threadIdx.x * per;
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const bool mine = i0 < n;
+    uint32_t par = 0;
+    if (mine)
+        for (uint32_t i = i0; i < i0 + per; ++i) {
+            const uint32_t w = prefix_bits(a[i]);
+            a[i] = w ^ (0u - par);
+            par ^= w & 1u;
+        }
+    const uint64_t b = __ballot(par != 0u);
+    if (lane == 0) part[wave] = (uint32_t)__popcll(b);
+    __syncthreads();
+    uint32_t carry = (uint32_t)__popcll(b & ((1ull << lane) - 1ull)), total = 0;
+    for (uint32_t k = 0; k < NT / 64; ++k) {
+        const uint32_t t = part[k];
+        if (k < wave) carry += t;
+        total += t;
+    }
+    if (mine && (carry & 1u))
+        for (uint32_t i = i0; i < i0 + per; ++i) a[i] = ~a[i];
+    __syncthreads();
+    return total & 1u;
+}
+// One level of conv(R, t): word w (< b c) of conv(s[(. / b) mod c], t) from the prefix words p of t folded to
+// that period, tau the parity of t.  The words of one sign are a window of t, the difference of two
+// prefixes b words apart, so that the sum has a prefix for each change of sign.
+template <uint32_t b, uint32_t c, uint32_t s>
+__device__ __forceinline__ uint32_t white_level(const uint32_t* p, uint32_t w, uint32_t tau) {
+    uint32_t x = 0u - ((s >> (w / b)) & tau & 1u);
+    uint32_t d = s ^ ((s << 1) | (s >> (c - 1u)));
+#pragma unroll
+    for (uint32_t i = 0; i < c; ++i, d >>= 1)
+        if (d & 1u) x ^= p[(w - b * i) & (b * c - 1u)];
+    return x;
+}
+// conv(R, t), g.white words, from the fold slices of t (pa_geom.hpp).  One workgroup; the slices (16 KB each
+// from 2^25 bits on, 512 bytes below) are 0.5 to 1 MB and 512 bytes a chunk, read while the other
+// workgroups of pass B transform.  lds: 16 + 4 NT + 144 words, or 16 + 4096 + 272 + 272.
+template <int NT>
+__device__ __forceinline__ void white_table(uint32_t* out, const uint4* fold, const Geom& g, uint32_t* lds) {
+    uint32_t* a2 = lds + 16;
+    const bool big = g.white == WHITE_BIG;
+    const uint32_t vecs = g.white / 4u, total = fold_slices(g) * vecs;  // 16-byte entries
+    const uint32_t runs = big ? vecs / NT : 1u;  // a thread's entries are of one class, of `runs` in turn
+    for (uint32_t c = 0; c < runs; ++c) {
+        uint4 x = make_uint4(0u, 0u, 0u, 0u);
+        const uint32_t step = big ? vecs : (uint32_t)NT;
+        for (uint32_t e0 = threadIdx.x + NT * c; e0 < total; e0 += 16u * step) {
+            uint4 y[16];  // requested together
+#pragma unroll
+            for (uint32_t k = 0; k < 16; ++k) {
+                const uint32_t e = e0 + k * step;
+                y[k] = fold[e < total ? e : e0];
+                if (e >= total) y[k] = make_uint4(0u, 0u, 0u, 0u);
+            }
+#pragma unroll
+            for (uint32_t k = 0; k < 16; ++k) {
+                x.x ^= y[k].x;
+                x.y ^= y[k].y;
+                x.z ^= y[k].z;
+                x.w ^= y[k].w;
+            }
+        }
+        uint32_t* v = a2 + 4u * (threadIdx.x + NT * c);
+        v[0] = x.x;
+        v[1] = x.y;
+        v[2] = x.z;
+        v[3] = x.w;
+    }
+    __syncthreads();
+    if (big) {
+        uint32_t *a1 = a2 + 4096, *a0 = a1 + 256, *o1 = a0 + 16, *o0 = o1 + 256;
+        for (uint32_t w = threadIdx.x; w < 256u; w += NT) {
+            uint32_t x = 0;
+            for (uint32_t i = 0; i < 16u; ++i) x ^= a2[w + 256u * i];
+            a1[w] = x;
+        }
+        __syncthreads();
+        if (threadIdx.x < 16u) {
+            uint32_t x = 0;
+            for (uint32_t i = 0; i < 16u; ++i) x ^= a1[threadIdx.x + 16u * i];
+            a0[threadIdx.x] = x;
+        }
+        __syncthreads();
+        prefix_words_lds<NT>(a0, 16u, lds);
+        prefix_words_lds<NT>(a1, 256u, lds);
+        const uint32_t tau = prefix_words_lds<NT>(a2, 4096u, lds);
+        if (threadIdx.x < 16u) o0[threadIdx.x] = white_level<1, 16, WHITE_S0>(a0, threadIdx.x, tau);
+        for (uint32_t w = threadIdx.x; w < 256u; w += NT) o1[w] = white_level<16, 16, WHITE_S1>(a1, w, tau);
+        __syncthreads();
+        for (uint32_t w = threadIdx.x; w < 4096u; w += NT)
+            out[w] = o0[w & 15u] ^ o1[w & 255u] ^ white_level<256, 16, WHITE_S2>(a2, w, tau);
+    } else {
+        // thread t has the words 4 t mod 128 on, so thread t + 32 k those of thread t too
+        uint32_t *a1 = a2 + 4 * NT, *a0 = a1 + 128;
+        for (uint32_t w = threadIdx.x; w < 128u; w += NT) {
+            uint32_t x = 0;
+            for (uint32_t k = 0; k < NT / 32u; ++k) x ^= a2[128u * k + w];
+            a1[w] = x;
+        }
+        __syncthreads();
+        if (threadIdx.x < 16u) {
+            uint32_t x = 0;
+            for (uint32_t i = 0; i < 8u; ++i) x ^= a1[threadIdx.x + 16u * i];
+            a0[threadIdx.x] = x;
+        }
+        __syncthreads();
+        prefix_words_lds<NT>(a0, 16u, lds);
+        const uint32_t tau = prefix_words_lds<NT>(a1, 128u, lds);
+        for (uint32_t w = threadIdx.x; w < 128u; w += NT)
+            out[w] = white_level<1, 16, WHITE_MID_S0>(a0, w & 15u, tau) ^ white_level<16, 8, WHITE_MID_S1>(a1, w, tau);
     }
 }
-// One workgroup of NT threads: info[INFO_POPS] = both popcounts (ws: a resident seed's partials),
-// info[INFO_WHITE] = conv(x, rho) mod 2 at conv bits 32 w .. 32 w + 31, the same word for every w
-// (the seed was whitened by rho, period 32, so that product depends on x only through K, the XOR of
-// its words), and the chunks' parities become their exclusive prefix.  lds: 3 NT / 64 words.
-// seed_ws != nullptr (resident seed being prepared): it receives the popcount as partials.
-template <int NT>
+// One workgroup of NT threads: info[INFO_POPS] = both popcounts, conv(R, t) (RESIDENT: from ws, a resident
+// seed's popcount partials and behind them its conv(R, t)), and the chunks' parities become their exclusive prefix.
+// lds: as white_table.
+// seed_ws != nullptr (resident seed being prepared): it receives what ws holds.
+template <int NT, bool RESIDENT>
 __device__ __forceinline__ void scan_finish(uint32_t* info, const Geom& g, const uint32_t* ws, uint32_t* seed_ws,
                                             uint32_t* lds) {
     const uint32_t count = scan_chunks(g), per = (count + NT - 1) / NT, i0 = threadIdx.x * per;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint8_t* cp = scan_parities(info, g);
-    uint32_t par = 0, pops = 0, k = 0;
+    uint8_t* cp = scan_parities(info);
+    uint32_t par = 0, pops = 0;
 #pragma unroll 4
     for (uint32_t i = i0; i < i0 + per && i < count; ++i) {
         par ^= cp[i];
-        const uint2 e = scan_entries(info)[i];
-        pops += e.x;
-        k ^= e.y;
+        pops += info[info_pops(g) + i];
     }
-    for (int off = 32; off > 0; off >>= 1) {
-        pops += __shfl_xor(pops, off);
-        k ^= __shfl_xor(k, off);
-    }
+    for (int off = 32; off > 0; off >>= 1) pops += __shfl_xor(pops, off);
     const uint64_t b = __ballot(par != 0u);
     uint32_t carry = (uint32_t)__popcll(b & ((1ull << lane) - 1ull));
     if (lane == 0) {
         lds[wave] = (uint32_t)__popcll(b);
         lds[NT / 64 + wave] = pops;
-        lds[2 * (NT / 64) + wave] = k;
     }
     __syncthreads();
     for (uint32_t i = 0; i < wave; ++i) carry += lds[i];
@@ -225,26 +348,25 @@ __device__ __forceinline__ void scan_finish(uint32_t* info, const Geom& g, const
         carry ^= c;
     }
     if (wave == 0) {
-        pops = k = 0;
-        for (int i = 0; i < NT / 64; ++i) {
-            pops += lds[NT / 64 + i];
-            k ^= lds[2 * (NT / 64) + i];
-        }
-        const uint32_t sh = lane & 31u;  // bit sh of K moves rho sh places on
-        uint32_t e = (lane < 32u && ((k >> (31u - sh)) & 1u)) ? ((g.rho >> sh) | (g.rho << ((32u - sh) & 31u))) : 0u;
-        for (int off = 32; off > 0; off >>= 1) e ^= __shfl_xor(e, off);
-        if (lane == 0) {
-            info[INFO_POPS] = pops + (ws ? pop_total(ws) : 0u);
-            info[INFO_WHITE] = e;
-        }
+        pops = 0;
+        for (int i = 0; i < NT / 64; ++i) pops += lds[NT / 64 + i];
+        if (lane == 0) info[INFO_POPS] = pops + (ws ? pop_total(ws) : 0u);
         if (seed_ws) seed_ws[lane] = lane == 0 ? pops : 0u;
+    }
+    uint32_t* white = info + info_white(g);
+    if constexpr (RESIDENT) {
+        const uint4* src = reinterpret_cast<const uint4*>(ws + POP_SLOTS);
+        for (uint32_t i = threadIdx.x; i < g.white / 4u; i += NT) reinterpret_cast<uint4*>(white)[i] = src[i];
+    } else {
+        __syncthreads();  // lds
+        white_table<NT>(seed_ws ? seed_ws + POP_SLOTS : white, reinterpret_cast<const uint4*>(info + info_fold(g)), g, lds);
     }
 }
 // A resident seed's prefix words once their chunks' exclusive parities are known (pa_seed_put).
 __global__ __launch_bounds__(256) void k_prefix_apply(uint32_t* __restrict__ q, const uint32_t* __restrict__ info,
                                                       Geom g) {
     const uint32_t w = blockIdx.x * 256u + threadIdx.x;
-    if (scan_parities(info, g)[w >> (10u + g.scan)]) q[w] = ~q[w];
+    if (scan_parities(info)[w >> (10u + g.scan)]) q[w] = ~q[w];
 }
 
 // ------------------------------------------------------------------ bit transpose ----
@@ -311,12 +433,17 @@ __global__ __launch_bounds__(TB_NT) void k_transpose_bits(const uint32_t* __rest
     const uint32_t u = b >> PARTS_LOG, part = b & ((1u << PARTS_LOG) - 1u);
     const uint32_t t0 = (part << TB_SPAN_LOG) + 32u * threadIdx.x;
     uint32_t w0[D], w1[D];
+    // M rows and N positions are whole periods of the whitening: one word of it for all
+    const uint32_t white = is_seed ? 0u : white_word(g, (t0 + g.N2 * u) >> 5);
+    uint32_t fold = 0;
 #pragma unroll
     for (int v = 0; v < D; ++v) {
         const uint32_t widx = (t0 + g.N2 * (u + g.M * (uint32_t)v)) >> 5;
-        w0[v] = is_seed ? seed_word(bits, g, widx) : key_word(bits, g, widx);
-        w1[v] = is_seed ? seed_word(bits, g, widx + (g.N >> 5)) : key_word(bits, g, widx + (g.N >> 5));
+        w0[v] = is_seed ? seed_word(bits, g, widx) : key_word(bits, g, widx) ^ white;
+        w1[v] = is_seed ? seed_word(bits, g, widx + (g.N >> 5)) : key_word(bits, g, widx + (g.N >> 5)) ^ white;
+        fold ^= w0[v] ^ w1[v];
     }
+    if (is_seed) scan.info[info_fold(g) + ((t0 + g.N2 * u) >> 5)] = fold;
     uint32_t* srow = stage + threadIdx.x * 33;
     uint32_t* out = tb + (size_t)u * g.N2 + (part << TB_SPAN_LOG);
     // Row A[31 - i] = the words of bit i, transposed: A[c] then holds bit 31 - c (column t0 + c) of
@@ -645,7 +772,7 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g,
     __shared__ uint32_t bw[N1];  // the group's 16 bits of row u, and of row u + N1 above them
     const uint32_t op = blockIdx.x / a.nA;
     if (op >= a.ops) {
-        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, bw);
+        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, reinterpret_cast<uint32_t*>(buf));
         return;
     }
     const bool is_seed = a.first + op == 1u;
@@ -660,8 +787,9 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_fwd(FwdArgs a, Geom g,
 #pragma unroll
         for (int i = 0; i < P::RPT; ++i) {
             const uint32_t w = wc + (g.N2 >> 5) * (threadIdx.x + (uint32_t)(NT * i)), wh = w + (g.N >> 5);
-            x.lo[i] = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
-            x.hi[i] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
+            const uint32_t white = is_seed ? 0u : white_word(g, w);  // N positions are whole periods
+            x.lo[i] = is_seed ? seed_word(in, g, w) : key_word(in, g, w) ^ white;
+            x.hi[i] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh) ^ white;
         }
     };
     auto pack = [&](const Words& x, uint32_t grp) __attribute__((always_inline)) {
@@ -814,7 +942,7 @@ __global__ __launch_bounds__(256, PER == 0 ? 4 : D == 6 ? 2 : 3) void k_mix_fwd(
     __shared__ uint32_t bw[D * M];  // per row u + 256 v: 16 columns' bits, and those of a[. + N] above them
     const uint32_t op = blockIdx.x / a.nA;
     if (op >= a.ops) {
-        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, bw);
+        scan_chunk<NT>(blockIdx.x - a.ops * a.nA, a.scan, g, reinterpret_cast<uint32_t*>(buf));
         return;
     }
     const bool is_seed = a.first + op == 1u;
@@ -824,11 +952,13 @@ __global__ __launch_bounds__(256, PER == 0 ? 4 : D == 6 ? 2 : 3) void k_mix_fwd(
     const uint32_t b = blockIdx.x - op * a.nA, grp0 = SPLIT ? b / D : b * per, c0 = SPLIT ? b % D : 0u;
     uint32_t lo[D], hi[D];
     auto load_words = [&](uint32_t wc) __attribute__((always_inline)) {
+        // M rows and N positions are whole periods of the whitening
+        const uint32_t white = is_seed ? 0u : white_word(g, wc + (g.N2 >> 5) * threadIdx.x);
 #pragma unroll
         for (int v = 0; v < D; ++v) {
             const uint32_t w = wc + (g.N2 >> 5) * (threadIdx.x + (uint32_t)(M * v)), wh = w + (g.N >> 5);
-            lo[v] = is_seed ? seed_word(in, g, w) : key_word(in, g, w);
-            hi[v] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh);
+            lo[v] = is_seed ? seed_word(in, g, w) : key_word(in, g, w) ^ white;
+            hi[v] = is_seed ? seed_word(in, g, wh) : key_word(in, g, wh) ^ white;
         }
     };
     const int col = threadIdx.x & 15, jt = threadIdx.x >> 4;
@@ -982,7 +1112,7 @@ __global__ __launch_bounds__(rows_threads(LG2, RPW), LG2 == 13 ? (MODE == ROWS_D
     __shared__ float2 tti[LG2 == 8 ? 1 : 16 * stage_row<16>()];  // inverse middle stage (radix 16, span 16)
     const uint32_t N1 = g.N1;
     if (blockIdx.x == 0) {
-        scan_finish<NT>(info, g, ws, seed_ws, reinterpret_cast<uint32_t*>(buf));
+        scan_finish<NT, MODE == ROWS_STATIC>(info, g, ws, seed_ws, reinterpret_cast<uint32_t*>(buf));
         return;
     }
     const uint32_t row = (blockIdx.x - 1u) * RPW + threadIdx.x / NTR;
@@ -1372,14 +1502,14 @@ __global__ __launch_bounds__(256) void k_inv_big2(const float2* __restrict__ Rp,
 }
 
 // ------------------------------------------------------------------ output ----
-// The correction of conv word w, MSB first: the prefix parities (q and its chunk's cp), the
-// whitening's word and key_rest word wo = w - out_off / 32 ((key[h/32+wo] << 1) | (key[h/32+wo+1] >> 31),
+// The correction of conv word w, MSB first: the prefix parities (q and its chunk's cp), conv(R, t)
+// and key_rest word wo = w - out_off / 32 ((key[h/32+wo] << 1) | (key[h/32+wo+1] >> 31),
 // key2StartRest PrivacyAmplification.cu:873-878).  No load is conditional on a lane, so that a thread
 // with several words has all their operands in flight.
 __device__ __forceinline__ uint32_t out_correction(uint32_t w, uint32_t wo, const Geom& g, const uint32_t* __restrict__ q,
-                                                   const uint32_t* __restrict__ info, uint32_t white,
+                                                   const uint32_t* __restrict__ info,
                                                    const uint32_t* __restrict__ key) {
-    uint32_t c = q[w] ^ (0u - (uint32_t)scan_parities(info, g)[w >> (10u + g.scan)]) ^ white;
+    uint32_t c = q[w] ^ (0u - (uint32_t)scan_parities(info)[w >> (10u + g.scan)]) ^ info[info_white(g) + (w & (g.white - 1u))];
     if (g.do_xor) {
         const bool in = 32u * wo < g.m;
         const uint32_t k = g.key_hw + (in ? wo : 0u);
@@ -1424,20 +1554,21 @@ __global__ __launch_bounds__(PACK_NT) void k_pack(const uint8_t* __restrict__ ni
 #pragma unroll
         for (int b = 0; b < 32; ++b) tile[(b * 8 + jl) * (PACK_CW + 1) + cl] = A[31 - b];
     }
-    const uint32_t white = info[INFO_WHITE];
     __syncthreads();
     const uint32_t lane = threadIdx.x % PACK_CW;
-    const uint8_t* cp = scan_parities(info, g);
+    const uint8_t* cp = scan_parities(info);
+    const uint32_t* white = info + info_white(g);
     for (uint32_t r0 = threadIdx.x / PACK_CW; r0 < 256u; r0 += 64u) {
         // the operands of out_correction for eight words, requested together
-        uint32_t w[8], c[8], flip[8], k0[8], k1[8];
+        uint32_t w[8], c[8], flip[8], r[8], k0[8], k1[8];
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
-            const uint32_t r = r0 + 8u * k, b = r >> 3, t1 = 2u * (jp0 + (r & 7u)) + (b >> 4) + S * (b & 15u);
+            const uint32_t row = r0 + 8u * k, b = row >> 3, t1 = 2u * (jp0 + (row & 7u)) + (b >> 4) + S * (b & 15u);
             w[k] = (half * g.N1 + t1) * (g.N2 >> 5) + c0 + lane;  // conv word
             const uint32_t wc = w[k] >= w_lo && w[k] < w_hi ? w[k] : w_lo;
             c[k] = q[wc];
             flip[k] = cp[wc >> (10u + g.scan)];
+            r[k] = white[w[k] & (WHITE_BIG - 1u)];
         }
         if (g.do_xor) {
 #pragma unroll
@@ -1450,7 +1581,7 @@ __global__ __launch_bounds__(PACK_NT) void k_pack(const uint8_t* __restrict__ ni
 #pragma unroll
         for (uint32_t k = 0; k < 8; ++k) {
             const uint32_t wo = w[k] - w_lo;
-            uint32_t cw = tile[(r0 + 8u * k) * (PACK_CW + 1) + lane] ^ c[k] ^ (0u - flip[k]) ^ white;
+            uint32_t cw = tile[(r0 + 8u * k) * (PACK_CW + 1) + lane] ^ c[k] ^ (0u - flip[k]) ^ r[k];
             if (g.do_xor && 32u * wo < g.m) cw ^= (k0[k] << 1) | (k1[k] >> 31);
             if (w[k] >= w_lo && w[k] < w_hi) out[wo] = g.reverse_endian ? __builtin_bswap32(cw) : cw;
         }
@@ -1492,7 +1623,7 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_inv(const float2* __re
         for (int r = 0; r < R1; ++r) v[i][r] = Rp[(size_t)(jt + (NT / 16) * i + S1 * r) * g.N2 + t2];
     fill_stage_table<R2, R1>(tab, tw14, NT);
     for (int e = threadIdx.x; e < N1; e += NT) tq[e] = cscale(tw14[e * (TW14 / (4 * N1))], g.inv_N);
-    const uint32_t pops = info[INFO_POPS], white = info[INFO_WHITE];
+    const uint32_t pops = info[INFO_POPS];
 #pragma unroll
     for (int i = 0; i < K1; ++i) stage_first_to_lds<R1>(v[i], buf + col * SEQS, jt + (NT / 16) * i);
     __syncthreads();
@@ -1525,7 +1656,7 @@ __global__ __launch_bounds__(mid_threads(LG1)) void k_mid_inv(const float2* __re
             if (w >= w_lo && w < w_hi) {
                 const uint32_t wo = w - w_lo;
                 // bit i of `mine` is column i: MSB first after the reversal
-                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, white, key) >> sh) & 0xFFFFu);
+                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, key) >> sh) & 0xFFFFu);
                 uint16_t* o = reinterpret_cast<uint16_t*>(out + wo);
                 if (g.reverse_endian) o[grp & 1u] = (uint16_t)((c16 >> 8) | (c16 << 8));
                 else o[(grp & 1u) ^ 1u] = (uint16_t)c16;
@@ -1593,7 +1724,7 @@ __global__ __launch_bounds__(256, NQ == 1 ? 4 : D == 6 ? 2 : 3) void k_mix_inv(
         }
     }
     mix_factors<D, NQ, 256>(tw2, tw1s, 4u * (uint32_t)h, 4u * (uint32_t)H, g, twlo, twhi);
-    const uint32_t pops = info[INFO_POPS], white = info[INFO_WHITE];
+    const uint32_t pops = info[INFO_POPS];
     // sum b of NQ: q = h + H b
     constexpr float S3 = 8.660254038e-01f;
     const float cq = h ? -0.5f : 1.f, sq = h == 1 ? S3 : h ? -S3 : 0.f;
@@ -1672,7 +1803,7 @@ __global__ __launch_bounds__(256, NQ == 1 ? 4 : D == 6 ? 2 : 3) void k_mix_inv(
             if (w >= w_lo && w < w_hi) {
                 const uint32_t wo = w - w_lo;
                 // bit i of `mine` is column i: MSB first after the reversal
-                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, white, key) >> sh) & 0xFFFFu);
+                const uint32_t c16 = (__brev(mine) >> 16) ^ ((out_correction(w, wo, g, q, info, key) >> sh) & 0xFFFFu);
                 uint16_t* o = reinterpret_cast<uint16_t*>(out + wo);
                 if (g.reverse_endian) o[grp & 1u] = (uint16_t)((c16 >> 8) | (c16 << 8));
                 else o[(grp & 1u) ^ 1u] = (uint16_t)c16;
