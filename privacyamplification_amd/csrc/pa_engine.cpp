@@ -596,15 +596,46 @@ hipError_t timed(pa_engine* e, int stage, hipStream_t s, F&& launch) {
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                     const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su);
 
+// The direct product's workgroups write output words while others still read the key and the seed; the
+// transforms read both to the end first, so a block whose output lies over them takes a transform.
+struct Span {
+    uintptr_t lo, hi;
+    bool out;
+};
+void block_spans(const Geom& g, const void* key, const void* seed, const void* out, std::vector<Span>& v) {
+    auto add = [&](const void* p, uint64_t bytes, bool is_out) {
+        if (p) v.push_back({(uintptr_t)p, (uintptr_t)p + bytes, is_out});
+    };
+    add(key, (uint64_t)key_words_for(g) * 4, false);
+    add(seed, (uint64_t)g.seed_words * 4, false);
+    add(out, out_bytes_of(g), true);
+}
+bool in_place(std::vector<Span>& v) {
+    std::sort(v.begin(), v.end(), [](const Span& a, const Span& b) { return a.lo < b.lo; });
+    uintptr_t in_hi = 0, out_hi = 0;
+    for (const Span& x : v) {
+        if (x.lo < (x.out ? in_hi : out_hi)) return true;
+        uintptr_t& hi = x.out ? out_hi : in_hi;
+        hi = std::max(hi, x.hi);
+    }
+    return false;
+}
+
 // A single block that takes the direct product: not with a margin, which is the transform's rounding
 // distance.
 bool direct_block(const Geom& g, const float* margin) { return !margin && pa::direct_size(g, pa::direct_work(g)); }
+bool direct_block(const Geom& g, const float* margin, const uint32_t* key, const uint32_t* seed, const uint32_t* out) {
+    if (!direct_block(g, margin)) return false;
+    const uintptr_t o = (uintptr_t)out, oe = o + out_bytes_of(g);
+    auto apart = [&](const uint32_t* p, uint64_t words) { return !p || (uintptr_t)p >= oe || (uintptr_t)(p + words) <= o; };
+    return apart(key, key_words_for(g)) && apart(seed, g.seed_words);
+}
 
 // Orders the workspace's uses across streams (not while s is being captured into a graph: a
 // capture only records work, and the caller owns the ordering of its replays).
 int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su = nullptr) {
-    if (direct_block(g, margin))  // uses no scratch of the workspace
+    if (direct_block(g, margin, key, seed, out))  // uses no scratch of the workspace
         return run_device_body(e, g, w, key, seed, sd, out, s, margin, su);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     PA_HIP(hipStreamIsCapturing(s, &cap));
@@ -622,7 +653,7 @@ int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, c
 int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                     const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su) {
     const pa::Tables t = tables(e, g.L);
-    if (direct_block(g, margin)) {
+    if (direct_block(g, margin, key, seed, out)) {
         PA_HIP(timed(e, ST_SMALL, s, [&] { return pa::launch_direct(key, sd ? sd->words : seed, out, g, s); }));
         return PA_OK;
     }
@@ -1163,6 +1194,12 @@ int batch_plan(pa_engine* e, const pa_block* blocks, uint32_t count, BatchPlan* 
     for (auto& gr : p->groups) {
         gr.direct = !gr.margin;
         for (uint32_t i : gr.idx) gr.direct = gr.direct && pa::direct_size(p->items[i].g, gr.work);
+        if (gr.direct) {
+            std::vector<Span> spans;
+            spans.reserve(3 * gr.idx.size());
+            for (uint32_t i : gr.idx) block_spans(p->items[i].g, blocks[i].key, blocks[i].seed, blocks[i].out, spans);
+            gr.direct = !in_place(spans);
+        }
         gr.small = gr.small || gr.direct;
         if (!gr.small)
             for (uint32_t i : gr.idx) p->scratch_bytes += batch_scratch_bytes(p->items[i].g, p->items[i].dyn);
