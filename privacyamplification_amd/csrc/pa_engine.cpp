@@ -199,9 +199,9 @@ struct Twiddles {
     float2* hi = nullptr;      // max(1, 2L / 2^14) entries
 };
 
-// Per transform length: the device scratch of one (unbatched) block.
+// Per octave of transform lengths: the device scratch of one (unbatched) block.
 struct Workspace {
-    uint32_t L = 0;
+    uint32_t octave = 0;
     float2* Yk = nullptr;      // N complex (key rows / R')
     float2* Ys = nullptr;      // N+1 complex (seed rows)
     float2* Rt = nullptr;      // N complex: pass B's output tiles (rt_tiled(lg1) only)
@@ -459,26 +459,49 @@ std::vector<float2> class_tables() {
     return t;
 }
 
-uint64_t workspace_bytes(const Geom& g) {
-    const uint64_t N = g.N;
-    uint64_t b = (16384 + (N > 8192 ? g.L / 8192 : 1)) * sizeof(float2);
-    if (g.N1 > 1) {
-        b += N * sizeof(float2) + (N + 1) * sizeof(float2);
-        b += 2 * mask_bytes(g) + pa::nib_bytes(g.N) + pa::info_bytes(g);
-        if (pa::rt_tiled(g.lg1)) b += N * sizeof(float2);
+// The transform lengths of one octave, (2^(k-1), 2^k]: 2^k, and 3 * 2^(k-2) where it is served.  They
+// share a workspace, and their twiddle tables are made together, so that whichever comes first, the
+// other's blocks need no memory more (under a budget, or while a stream is being captured).
+uint32_t octave_of(uint32_t L) { return 1u << log2u(L); }
+std::vector<uint32_t> octave_lengths(uint32_t octave) {
+    const int lg = (int)log2u(octave);
+    if (lg < pa::MIX_MIN_LOG_L || lg > pa::MIX_MAX_LOG_L) return {octave};
+    return {octave, octave / 4 * 3};
+}
+// Bytes of each of a workspace's buffers: the larger of its octave's lengths.
+struct WorkspaceSizes {
+    uint64_t Yk = 0, Ys = 0, masks = 0, nib = 0, info = 0, Rt = 0, key = 0, out = 0;
+};
+WorkspaceSizes workspace_sizes(uint32_t octave) {
+    WorkspaceSizes z;
+    z.key = ws_key_bytes(octave);
+    z.out = ws_out_bytes(octave);
+    for (uint32_t L : octave_lengths(octave)) {
+        Geom g;  // a block that fills the transform
+        if (make_geom(L, 32, PA_COMPRESS, 1, pa::MAX_L_LOG, &g) != PA_OK || g.N1 == 1) continue;
+        const uint64_t N = g.N;
+        z.Yk = std::max(z.Yk, N * sizeof(float2));
+        z.Ys = std::max(z.Ys, (N + 1) * sizeof(float2));
+        z.masks = std::max(z.masks, mask_bytes(g));
+        z.nib = std::max(z.nib, pa::nib_bytes(g.N));
+        z.info = std::max(z.info, pa::info_bytes(g));
+        if (pa::rt_tiled(g.lg1)) z.Rt = std::max(z.Rt, N * sizeof(float2));
     }
-    b += ws_key_bytes(g.L) * 2 + ws_out_bytes(g.L);  // key/seed and output staging
+    return z;
+}
+uint64_t twiddle_hi_count(uint32_t L) { return L > 8192 ? L / 8192 : 1; }
+uint64_t workspace_bytes(const Geom& g) {
+    const uint32_t octave = octave_of(g.L);
+    const WorkspaceSizes z = workspace_sizes(octave);
+    uint64_t b = z.Yk + z.Ys + 2 * z.masks + z.nib + z.info + z.Rt + 2 * z.key + z.out;  // key and seed staging: 2 key
+    for (uint32_t L : octave_lengths(octave)) b += (16384 + twiddle_hi_count(L)) * sizeof(float2);
     return b;
 }
 
-int get_twiddles(pa_engine* e, uint32_t L, Twiddles** out) {
-    auto it = e->tw.find(L);
-    if (it != e->tw.end()) {
-        *out = &it->second;
-        return PA_OK;
-    }
+int make_twiddles(pa_engine* e, uint32_t L) {
+    if (e->tw.find(L) != e->tw.end()) return PA_OK;
     Twiddles t;
-    const uint64_t hi_n = L > 8192 ? L / 8192 : 1;
+    const uint64_t hi_n = twiddle_hi_count(L);
     int rc = dev_alloc(e, (void**)&t.lo, 16384 * sizeof(float2));
     if (rc != PA_OK) return rc;
     rc = dev_alloc(e, (void**)&t.hi, hi_n * sizeof(float2));
@@ -490,39 +513,46 @@ int get_twiddles(pa_engine* e, uint32_t L, Twiddles** out) {
     auto hi = twiddles(2ull * L, hi_n, 16384);
     PA_HIP(hipMemcpy(t.lo, lo.data(), lo.size() * sizeof(float2), hipMemcpyHostToDevice));
     PA_HIP(hipMemcpy(t.hi, hi.data(), hi.size() * sizeof(float2), hipMemcpyHostToDevice));
-    *out = &e->tw.emplace(L, t).first->second;
+    e->tw.emplace(L, t);
+    return PA_OK;
+}
+// The tables of L and of the other length of its octave.
+int get_twiddles(pa_engine* e, uint32_t L) {
+    if (e->tw.find(L) != e->tw.end()) return PA_OK;
+    for (uint32_t l : octave_lengths(octave_of(L))) {
+        const int rc = make_twiddles(e, l);
+        if (rc != PA_OK) return rc;
+    }
     return PA_OK;
 }
 
 int get_workspace(pa_engine* e, const Geom& g, Workspace** out) {
-    auto it = e->ws.find(g.L);
+    const uint32_t octave = octave_of(g.L);
+    int rc = get_twiddles(e, g.L);
+    if (rc != PA_OK) return rc;
+    auto it = e->ws.find(octave);
     if (it != e->ws.end()) {
         *out = it->second.get();
         return PA_OK;
     }
-    Twiddles* tw;
-    int rc = get_twiddles(e, g.L, &tw);
-    if (rc != PA_OK) return rc;
     auto w = std::make_unique<Workspace>();
-    w->L = g.L;
-    const size_t key_bytes = ws_key_bytes(g.L), out_bytes = ws_out_bytes(g.L);
+    w->octave = octave;
+    const WorkspaceSizes z = workspace_sizes(octave);
     struct A { void** p; size_t b; };
-    std::vector<A> allocs = {
-        {(void**)&w->d_key, key_bytes},
-        {(void**)&w->d_seed, key_bytes},
-        {(void**)&w->d_out, out_bytes},
+    std::vector<A> allocs;
+    auto want = [&](auto& p, uint64_t bytes) {
+        if (bytes) allocs.push_back({(void**)&p, (size_t)bytes});
     };
-    if (g.N1 > 1) {
-        allocs.push_back({(void**)&w->Yk, (size_t)g.N * sizeof(float2)});
-        allocs.push_back({(void**)&w->Ys, (size_t)(g.N + 1) * sizeof(float2)});
-        if (!mid_size(g)) {
-            allocs.push_back({(void**)&w->tbk, (size_t)mask_bytes(g)});
-            allocs.push_back({(void**)&w->tbs, (size_t)mask_bytes(g)});
-        }
-        allocs.push_back({(void**)&w->nib, (size_t)pa::nib_bytes(g.N)});
-        allocs.push_back({(void**)&w->info, (size_t)pa::info_bytes(g)});
-        if (pa::rt_tiled(g.lg1)) allocs.push_back({(void**)&w->Rt, (size_t)g.N * sizeof(float2)});
-    }
+    want(w->d_key, z.key);
+    want(w->d_seed, z.key);
+    want(w->d_out, z.out);
+    want(w->Yk, z.Yk);
+    want(w->Ys, z.Ys);
+    want(w->tbk, z.masks);
+    want(w->tbs, z.masks);
+    want(w->nib, z.nib);
+    want(w->info, z.info);
+    want(w->Rt, z.Rt);
     for (auto& a : allocs) {
         rc = dev_alloc(e, a.p, a.b);
         if (rc != PA_OK) {
@@ -534,7 +564,7 @@ int get_workspace(pa_engine* e, const Geom& g, Workspace** out) {
     }
     PA_HIP(hipEventCreateWithFlags(&w->last_done, hipEventDisableTiming));
     *out = w.get();
-    e->ws.emplace(g.L, std::move(w));
+    e->ws.emplace(octave, std::move(w));
     return PA_OK;
 }
 
@@ -760,9 +790,7 @@ int pa_create(const pa_config* cfg, pa_engine** out) {
         PA_HIP(scratch_address(e->cfg.device, &sp));
         e->noalloc = static_cast<uint8_t*>(sp);
         for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= std::min(NOALLOC_MAX_L_LOG, e->cfg.max_n_log2); ++lg) {
-            Twiddles* tw;
-            rc = get_twiddles(e.get(), 1u << lg, &tw);
-            if (rc == PA_OK && lg >= (uint32_t)pa::MIX_MIN_LOG_L) rc = get_twiddles(e.get(), 3u << (lg - 2), &tw);
+            rc = get_twiddles(e.get(), 1u << lg);
             if (rc != PA_OK) return rc;
         }
     }
@@ -967,7 +995,7 @@ int pa_block_device_noalloc(pa_engine* e, const uint32_t* d_key, const uint32_t*
     if (!e->noalloc || e->tw.find(g.L) == e->tw.end()) return PA_ERR_UNSUPPORTED;
     // the workspace of this block, carved from the scratch array (no allocation)
     Workspace w;
-    w.L = g.L;
+    w.octave = octave_of(g.L);
     if (g.N1 > 1) {
         uint64_t off = 0;
         auto take = [&](uint64_t bytes) {
@@ -1168,8 +1196,7 @@ int batch_plan(pa_engine* e, const pa_block* blocks, uint32_t count, BatchPlan* 
             rc = seed_lookup(e, b.seed_id, it.g, &it.sd);
             if (rc != PA_OK) return rc;
         }
-        Twiddles* tw;
-        rc = get_twiddles(e, it.g.L, &tw);
+        rc = get_twiddles(e, it.g.L);
         if (rc != PA_OK) return rc;
         const auto key = std::make_pair(it.g.L, it.dyn);
         auto f = gid.find(key);
