@@ -224,13 +224,10 @@ struct Seed {
     Geom g{};
     float2* spec = nullptr;    // spectrum: N complex (four-step path), N+1 split (small path)
     uint32_t* ws = nullptr;    // device popcount (POP_SLOTS partials), then conv(R, seed), g.white words
-    uint32_t* sq = nullptr;    // prefix words (four-step path): L/8 bytes, 1/32 of the spectrum, not
-                               // charged to the budget, so that it holds as many seeds as it says
-    uint32_t* words = nullptr; // the seed itself up to 2^DIRECT_MAX_L_LOG bits, for the direct product;
-                               // at most L/8 bytes, not charged either
-                               // (spec, ws, sq and words are one allocation at spec)
+    uint32_t* sq = nullptr;    // prefix words (four-step path): L/8 bytes, 1/32 of the spectrum
+    uint32_t* words = nullptr; // the seed itself up to 2^DIRECT_MAX_L_LOG bits, for the direct product
     int32_t reuse = 0;
-    uint64_t bytes = 0;
+    uint64_t bytes = 0;        // of the one allocation at spec that holds all four
 };
 
 struct Ticket {
@@ -869,18 +866,12 @@ int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform
 static int seed_alloc(pa_engine* e, Seed* sd) {
     const Geom& g = sd->g;
     const uint64_t spec = align256((uint64_t)(g.N + 1) * sizeof(float2)), ws = align256((pa::POP_SLOTS + g.white) * 4ull);
-    sd->bytes = (uint64_t)(g.N + 1) * sizeof(float2) + pa::POP_SLOTS * sizeof(uint32_t);
-    if (e->cfg.hbm_budget_bytes && e->used_bytes + sd->bytes > e->cfg.hbm_budget_bytes) return PA_ERR_NOMEM;
-    uint8_t* p = nullptr;
     const uint64_t sq = g.N1 > 1 ? (uint64_t)g.L / 8 : 0;
     const bool words = g.L <= (1u << pa::DIRECT_MAX_L_LOG);
-    const hipError_t r = hipMalloc((void**)&p, spec + ws + sq + (words ? (uint64_t)g.n / 8 : 0));
-    if (r != hipSuccess) {
-        set_error(r, "hipMalloc", __FILE__, __LINE__);
-        (void)hipGetLastError();
-        return PA_ERR_NOMEM;
-    }
-    e->used_bytes += sd->bytes;
+    sd->bytes = spec + ws + sq + (words ? (uint64_t)g.n / 8 : 0);
+    uint8_t* p = nullptr;
+    const int rc = dev_alloc(e, (void**)&p, sd->bytes);
+    if (rc != PA_OK) return rc;
     sd->spec = reinterpret_cast<float2*>(p);
     sd->ws = reinterpret_cast<uint32_t*>(p + spec);
     if (g.N1 > 1) sd->sq = reinterpret_cast<uint32_t*>(p + spec + ws);
