@@ -139,7 +139,8 @@ typedef struct {
 } pa_block;
 
 /* Batch options: PA_BATCH_GRAPH replays a captured hipGraph for a batch of the same shape
- * (lengths classes, seed modes and counts); PA_BATCH_TUNE times the launch shapes of a shape not
+ * (lengths classes, seed modes and counts, and for short blocks the quarters of their class that the longest
+ * output and key reach), of the last 64 shapes; PA_BATCH_TUNE times the launch shapes of a shape not
  * seen before (pass A's walk length) and keeps the fastest. */
 enum pa_batch_flags {
     PA_BATCH_GRAPH = 1u,
@@ -156,6 +157,10 @@ int pa_batch_device(pa_engine* eng, const pa_block* blocks, uint32_t count, uint
                     void* stream);
 /* Same with host buffers; returns when every output has been written. */
 int pa_run_batch(pa_engine* eng, const pa_block* blocks, uint32_t count, uint32_t batch_flags);
+
+/* Graphs that PA_BATCH_GRAPH has captured in pa_batch_device and pa_run_batch so far, and those kept: a
+ * diagnostic with no counterpart in the reference.  Either pointer may be NULL. */
+int pa_batch_graphs(pa_engine* eng, uint64_t* captured, uint32_t* kept);
 
 /* Sub-block (tiled) evaluation of one block, the device form of LargeBlocksizeExample's tiling
  * (LBS/main.cpp:104-124, 313-523) used as the precision fallback: the m x (h+1) Toeplitz product is

@@ -257,7 +257,15 @@ struct BatchSlot {
     uint32_t hdesc_cap = 0;
     hipEvent_t htab_free = nullptr;            // recorded after the last read of htab / hdesc
     bool htab_pending = false;
-    std::map<std::string, hipGraphExec_t> graphs;
+    // At most MAX_GRAPHS, the least recently replayed one dropped for a new one: a server's batches take
+    // ever new mixes of lengths and counts.
+    static constexpr size_t MAX_GRAPHS = 64;
+    struct Graph {
+        hipGraphExec_t exec;
+        uint64_t used;
+    };
+    std::map<std::string, Graph> graphs;
+    uint64_t replays = 0, captures = 0;
 };
 
 // ------------------------------------------------------------------ allocation-free scratch ----
@@ -389,7 +397,7 @@ int slot_init(BatchSlot* sl, bool own_stream) {
 
 void slot_release(pa_engine* e, BatchSlot* sl) {
     if (sl->stream) (void)hipStreamSynchronize(sl->stream);
-    for (auto& kv : sl->graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto& kv : sl->graphs) (void)hipGraphExecDestroy(kv.second.exec);
     sl->graphs.clear();
     for (int i = 0; i < BatchSlot::FORKS; ++i) {
         if (sl->fork[i]) {
@@ -1235,7 +1243,7 @@ int ensure_arena(pa_engine* e, BatchSlot& sl, uint64_t bytes, uint64_t limit = 0
     if (limit && bytes > limit) return PA_ERR_NOMEM;
     if (sl.stream) PA_HIP(hipStreamSynchronize(sl.stream));
     else PA_HIP(hipDeviceSynchronize());
-    for (auto& kv : sl.graphs) (void)hipGraphExecDestroy(kv.second);
+    for (auto& kv : sl.graphs) (void)hipGraphExecDestroy(kv.second.exec);
     sl.graphs.clear();
     if (sl.arena) dev_free(e, sl.arena, sl.arena_cap);
     sl.arena = nullptr;
@@ -1463,6 +1471,15 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
             }
     if (!(bflags & PA_BATCH_GRAPH)) return finish(batch_launch_all(e, sl, p, dtab, s));
     auto replay = [&]() -> int {
+        // The direct product's launch shape is that of the longest output and key of the group; in quarters of
+        // the length's most, or ragged short blocks would hardly ever have one in common.  A
+        // workgroup beyond its block's output returns, and loops run to the block's own key words.
+        for (auto& gr : p.groups)
+            if (gr.direct) {
+                auto quarters = [](uint32_t x, uint32_t step) { return (x + step - 1u) / step * step; };
+                gr.words = std::min(gr.L / 32u, quarters(gr.words, std::max(1u, gr.L / 128u)));
+                gr.jpad = std::min(pa::DIRECT_JPAD_MAX, quarters(gr.jpad, std::max(16u, gr.L / 128u)));
+            }
         std::string key = std::to_string((uintptr_t)sl.arena) + ":";
         for (auto& gr : p.groups)
             key += tune_key(gr) + (gr.direct ? "w" + std::to_string(gr.words) + "j" + std::to_string(gr.jpad)
@@ -1482,9 +1499,18 @@ int batch_execute(pa_engine* e, BatchSlot& sl, BatchPlan& p, const pa_block* dev
             hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
             (void)hipGraphDestroy(graph);
             PA_HIP(ei);
-            f = sl.graphs.emplace(key, exec).first;
+            if (sl.graphs.size() >= BatchSlot::MAX_GRAPHS) {
+                // its last launch is over: the table that it read was waited for above
+                auto old = std::min_element(sl.graphs.begin(), sl.graphs.end(),
+                                            [](const auto& a, const auto& b) { return a.second.used < b.second.used; });
+                (void)hipGraphExecDestroy(old->second.exec);
+                sl.graphs.erase(old);
+            }
+            f = sl.graphs.emplace(key, BatchSlot::Graph{exec, 0}).first;
+            ++sl.captures;
         }
-        PA_HIP(hipGraphLaunch(f->second, s));
+        f->second.used = ++sl.replays;
+        PA_HIP(hipGraphLaunch(f->second.exec, s));
         return PA_OK;
     };
     return finish(replay());
@@ -1503,6 +1529,14 @@ int pa_batch_device(pa_engine* e, const pa_block* blocks, uint32_t count, uint32
     rc = ensure_arena(e, e->batch, p.table_bytes + p.scratch_bytes);
     if (rc != PA_OK) return rc;
     return batch_execute(e, e->batch, p, blocks, batch_flags, stream_of(e, stream));
+}
+
+int pa_batch_graphs(pa_engine* e, uint64_t* captured, uint32_t* kept) {
+    if (!e) return PA_ERR_ARG;
+    std::lock_guard<std::mutex> lk(e->mu);
+    if (captured) *captured = e->batch.captures;
+    if (kept) *kept = (uint32_t)e->batch.graphs.size();
+    return PA_OK;
 }
 
 int pa_run_batch(pa_engine* e, const pa_block* blocks, uint32_t count, uint32_t batch_flags) {

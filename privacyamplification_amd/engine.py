@@ -135,6 +135,7 @@ def load_library():
                                           vp, vp]
     L.pa_batch_device.argtypes = [eng, ctypes.POINTER(PaBlock), ctypes.c_uint32, ctypes.c_uint32, vp]
     L.pa_run_batch.argtypes = [eng, ctypes.POINTER(PaBlock), ctypes.c_uint32, ctypes.c_uint32]
+    L.pa_batch_graphs.argtypes = [eng, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint32)]
     L.pa_block_device_split.argtypes = [eng, vp, vp, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32,
                                         ctypes.c_uint32, vp, vp, vp]
     L.pa_run_block_split.argtypes = [eng, u32p, u32p, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32,
@@ -166,7 +167,7 @@ def load_library():
                  "pa_batch_device", "pa_run_batch", "pa_serve_start", "pa_serve_submit",
                  "pa_serve_submit_many",
                  "pa_serve_wait", "pa_serve_stop", "pa_host_alloc", "pa_host_free",
-                 "pa_block_device_split", "pa_run_block_split", "pa_block_extents", "pa_selftest",
+                 "pa_batch_graphs", "pa_block_device_split", "pa_run_block_split", "pa_block_extents", "pa_selftest",
                  "pa_block_device_noalloc"):
         getattr(L, name).restype = ctypes.c_int
     _lib = L
@@ -342,6 +343,12 @@ class Engine:
         else:
             arr = blocks
         _check(self._L.pa_batch_device(self._h, arr, len(arr), batch_flags, stream), "pa_batch_device")
+
+    def batch_graphs(self):
+        """Graphs captured by BATCH_GRAPH batches so far, and those kept (pa_batch_graphs)."""
+        captured, kept = ctypes.c_uint64(), ctypes.c_uint32()
+        _check(self._L.pa_batch_graphs(self._h, ctypes.byref(captured), ctypes.byref(kept)), "pa_batch_graphs")
+        return captured.value, kept.value
 
     def amplify_split(self, key, seed, n, m, sub_log2, do_xor_key_rest=True):
         """Sub-block (tiled, b = 2^sub_log2) evaluation of one block (pa_run_block_split)."""
