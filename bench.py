@@ -49,17 +49,20 @@ def kernel_bytes(n, m):
     """Algorithmic bytes per launch of each kernel as built: the compulsory HBM reads and writes of
     its inputs and outputs. A complex FP32 spectrum of an n-bit operand is 4n bytes, its packed
     bits n/8 bytes, the output nibbles m/4 bytes."""
-    return {
+    kb = {
         "k_transpose_bits(key)": n / 8 + n / 8,
         "k_transpose_bits(key+seed)": 2 * (n / 8 + n / 8),
-        "k_fwd_cols(key)": n / 8 + 4 * n,
-        "k_fwd_cols(key+seed)": 2 * (n / 8 + 4 * n),
-        "k_rows(seedprep)": 8 * n,
         "k_rows": 12 * n,
         "k_inv_cols": 4 * n + m / 4,
+        "k_inv_big1+k_inv_big2": 12 * n + m / 4,
         "k_pack": m / 4 + m / 8 + m / 8,
-        "k_zero_u32": 8,
     }
+    for fwd in ("k_fwd_cols", "k_mid_fwd", "k_mix_fwd"):
+        kb[fwd + "(key)"] = n / 8 + 4 * n
+        kb[fwd + "(key+seed)"] = 2 * (n / 8 + 4 * n)
+    for inv in ("k_mid_inv", "k_mix_inv"):  # with the output words
+        kb[inv] = 4 * n + m / 8 + m / 8
+    return kb
 
 
 def read_traffic(kernel, log2n, mode):

@@ -296,6 +296,8 @@ hipError_t scratch_address(int dev, void** out) {
 
 }  // namespace
 
+constexpr int MAX_STAGES = 24;
+
 struct pa_engine {
     pa_config cfg{};
     hipStream_t stream = nullptr;
@@ -317,8 +319,8 @@ struct pa_engine {
     struct Pending { int stage; hipEvent_t a, b; };
     std::vector<Pending> pending;
     std::vector<hipEvent_t> event_pool;
-    double stage_ms[16] = {};
-    uint32_t stage_count[16] = {};
+    double stage_ms[MAX_STAGES] = {};
+    uint32_t stage_count[MAX_STAGES] = {};
     // batched launches
     BatchSlot batch;                         // pa_batch_device / pa_run_batch
     std::map<std::string, uint32_t> tuned;   // pass A walk length per (L, seed mode, count)
@@ -581,13 +583,22 @@ pa::Tables tables(pa_engine* e, uint32_t L) {
 
 hipStream_t stream_of(pa_engine* e, void* s) { return s ? (hipStream_t)s : e->stream; }
 
-enum Stage { ST_SMALL, ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, ST_TRANSPOSE_BOTH, ST_FWD_COLS_BOTH,
-             ST_ROWS_SEEDPREP, ST_ROWS, ST_INV_COLS, ST_PACK, ST_TRANSPOSE_SEED, ST_FWD_COLS_SEED, ST_COUNT };
+// Timed stages, named by the kernel that runs them; pass A and its bit transpose once more per operands.
+enum Operands { OP_KEY, OP_BOTH, OP_SEED, OP_COUNT };
+enum Stage { ST_SMALL, ST_DIRECT, ST_TRANSPOSE, ST_FWD_COLS = ST_TRANSPOSE + OP_COUNT, ST_MID_FWD = ST_FWD_COLS + OP_COUNT,
+             ST_MIX_FWD = ST_MID_FWD + OP_COUNT, ST_ROWS = ST_MIX_FWD + OP_COUNT, ST_INV_COLS, ST_INV_BIG, ST_MID_INV,
+             ST_MIX_INV, ST_PACK, ST_COUNT };
 const char* const kStageNames[ST_COUNT] = {
-    "k_small", "k_transpose_bits(key)", "k_fwd_cols(key)", "k_transpose_bits(key+seed)",
-    "k_fwd_cols(key+seed)", "k_rows(seedprep)", "k_rows", "k_inv_cols", "k_pack", "k_transpose_bits(seed)",
-    "k_fwd_cols(seed)"};
-static_assert(ST_COUNT <= 16, "stage tables hold 16 entries");
+    "k_small", "k_direct", "k_transpose_bits(key)", "k_transpose_bits(key+seed)", "k_transpose_bits(seed)",
+    "k_fwd_cols(key)", "k_fwd_cols(key+seed)", "k_fwd_cols(seed)", "k_mid_fwd(key)", "k_mid_fwd(key+seed)",
+    "k_mid_fwd(seed)", "k_mix_fwd(key)", "k_mix_fwd(key+seed)", "k_mix_fwd(seed)", "k_rows", "k_inv_cols",
+    "k_inv_big1+k_inv_big2", "k_mid_inv", "k_mix_inv", "k_pack"};
+static_assert(ST_COUNT <= MAX_STAGES, "stage tables");
+int fwd_stage(const Geom& g) { return pa::mixed(g) ? ST_MIX_FWD : mid_size(g) ? ST_MID_FWD : ST_FWD_COLS; }
+int inv_stage(const Geom& g) {
+    if (mid_size(g)) return pa::mixed(g) ? ST_MIX_INV : ST_MID_INV;
+    return g.lg1 > (uint32_t)pa::RT_LG1 ? ST_INV_BIG : ST_INV_COLS;
+}
 
 // A fresh seed still in host memory (pa_run_block): it is copied to dev on the upload stream
 // after the key's copy (event key_up; both share the bus, so running them together would only
@@ -689,7 +700,7 @@ int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* k
                     const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su) {
     const pa::Tables t = tables(e, g.L);
     if (direct_block(g, margin, key, seed, out)) {
-        PA_HIP(timed(e, ST_SMALL, s, [&] { return pa::launch_direct(key, sd ? sd->words : seed, out, g, s); }));
+        PA_HIP(timed(e, ST_DIRECT, s, [&] { return pa::launch_direct(key, sd ? sd->words : seed, out, g, s); }));
         return PA_OK;
     }
     if (g.N1 == 1) {
@@ -707,39 +718,39 @@ int run_device_body(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* k
     const uint32_t* kin = mid ? key : w->tbk;
     const uint32_t* sin = mid ? scan.seed : w->tbs;
     // `ops` operands from `first` on through the bit transpose and pass A; sc: with the input scan
-    auto fwd = [&](int tstage, int fstage, uint32_t first, uint32_t ops, const pa::ScanArgs* sc) {
+    auto fwd = [&](int op, uint32_t first, uint32_t ops, const pa::ScanArgs* sc) {
         hipError_t r = hipSuccess;
         if (!mid)
-            r = timed(e, tstage, s, [&] {
+            r = timed(e, ST_TRANSPOSE + op, s, [&] {
                 return pa::launch_transpose(key, scan.seed, w->tbk, w->tbs, first, ops, g, sc, s);
             });
         if (r != hipSuccess) return r;
-        return timed(e, fstage, s, [&] { return pa::launch_fwd_cols(kin, sin, w->Yk, w->Ys, first, ops, g, t, sc, s); });
+        return timed(e, fwd_stage(g) + op, s, [&] { return pa::launch_fwd_cols(kin, sin, w->Yk, w->Ys, first, ops, g, t, sc, s); });
     };
     if (!sd && su) {  // key passes first, the seed's (and the scan of both) after its upload
-        PA_HIP(fwd(ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, 0, 1, nullptr));
+        PA_HIP(fwd(OP_KEY, 0, 1, nullptr));
         PA_HIP(hipStreamWaitEvent(su->up, su->key_up, 0));
         PA_HIP(hipMemcpyAsync(su->dev, su->host, su->bytes, hipMemcpyHostToDevice, su->up));
         PA_HIP(hipEventRecord(su->done, su->up));
         PA_HIP(hipStreamWaitEvent(s, su->done, 0));
-        PA_HIP(fwd(ST_TRANSPOSE_SEED, ST_FWD_COLS_SEED, 1, 1, &scan));
+        PA_HIP(fwd(OP_SEED, 1, 1, &scan));
     } else if (!sd) {  // key and seed share each launch of the bit transpose and of pass A
-        PA_HIP(fwd(ST_TRANSPOSE_BOTH, ST_FWD_COLS_BOTH, 0, 2, &scan));
+        PA_HIP(fwd(OP_BOTH, 0, 2, &scan));
     } else {
         S = sd->spec;
         scan.seed = nullptr;
         scan.sq = sd->sq;
-        PA_HIP(fwd(ST_TRANSPOSE_KEY, ST_FWD_COLS_KEY, 0, 1, &scan));
+        PA_HIP(fwd(OP_KEY, 0, 1, &scan));
     }
     PA_HIP(timed(e, ST_ROWS, s, [&] {
         return pa::launch_rows(sd ? pa::ROWS_STATIC : pa::ROWS_DYN, w->Yk, S, w->Rt, g, t, w->info, sd ? sd->ws : nullptr,
                                nullptr, s);
     }));
     if (mid) {
-        PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_mid_inv(w->Yk, key, out, g, w->info, q, t, margin, s); }));
+        PA_HIP(timed(e, inv_stage(g), s, [&] { return pa::launch_mid_inv(w->Yk, key, out, g, w->info, q, t, margin, s); }));
         return PA_OK;
     }
-    PA_HIP(timed(e, ST_INV_COLS, s, [&] { return pa::launch_inv_cols(w->Rt, w->nib, g, w->info, t, margin, s); }));
+    PA_HIP(timed(e, inv_stage(g), s, [&] { return pa::launch_inv_cols(w->Rt, w->nib, g, w->info, t, margin, s); }));
     PA_HIP(timed(e, ST_PACK, s, [&] { return pa::launch_pack(w->nib, key, out, g, w->info, q, s); }));
     return PA_OK;
 }
