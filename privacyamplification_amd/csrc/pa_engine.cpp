@@ -2430,8 +2430,9 @@ inline uint32_t refbit(const uint32_t* w, uint64_t p) { return (w[p >> 5] >> (31
 
 int st_unpack(pa_engine* e, Report& rp) {
     // binInt2float (:484-602): binIn[i] = i; the popcount of n bits is A000788(n/32 - 1).  The
-    // production input scan counts them here; its prefix parities, and from 2^23 bits on the layout
-    // that the bit transpose gives pass A's class tables, are checked too
+    // production input scan counts them here; its prefix parities, from 2^25 bits on the layout
+    // that the bit transpose gives pass A's class tables, and up to 2^20 bits a sample of the spectrum (what
+    // the passes that read words have made of the bits) are checked too
     const uint32_t nmax = 1u << 27;
     std::vector<uint32_t> bin(nmax / 32);
     for (uint32_t i = 0; i < nmax / 32; ++i) bin[i] = i;
@@ -2440,12 +2441,17 @@ int st_unpack(pa_engine* e, Report& rp) {
     ST_ALLOC(dws, (pa::POP_SLOTS + pa::WHITE_BIG) * 4);
     PA_HIP(hipMemcpy(dbin.p, bin.data(), nmax / 8, hipMemcpyHostToDevice));
     uint64_t lcg = 12345;
-    for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
-        const uint32_t n = 1u << lg;
+    std::vector<uint32_t> sizes;
+    for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= 27; ++lg) sizes.push_back(1u << lg);
+    for (uint32_t k : {17u, 18u, 20u, 23u}) sizes.push_back(3u << k);
+    for (uint32_t n : sizes) {
+        if (!rp.ok) break;
         Geom g;
         Workspace* w;
         int rc = prepare(e, n, 3 * n / 8, PA_DEFAULT_FLAGS, &g, &w);
         if (rc != PA_OK) return rc;
+        g.seed_rot = 0;
+        g.out_off = 0;
         g.out_bits = g.L;  // every word's prefix
         const bool mid = mid_size(g);
         uint32_t* bits = dbin.as<uint32_t>();
@@ -2463,7 +2469,7 @@ int st_unpack(pa_engine* e, Report& rp) {
         if (!mid) PA_HIP(hipMemcpyAsync(tb.data(), w->tbs, tb.size() * 4, hipMemcpyDeviceToHost, e->stream));
         PA_HIP(hipStreamSynchronize(e->stream));
         if (info[0] != (uint32_t)ones_upto(n / 32 - 1)) {
-            rp.fail("BinInt2float: n = 2^%u popcount %u, want %llu", lg, info[0], (unsigned long long)ones_upto(n / 32 - 1));
+            rp.fail("BinInt2float: n = %u popcount %u, want %llu", n, info[0], (unsigned long long)ones_upto(n / 32 - 1));
             break;
         }
         uint32_t par = 0;
@@ -2472,7 +2478,23 @@ int st_unpack(pa_engine* e, Report& rp) {
             for (int sh = 1; sh < 32; sh *= 2) want ^= want >> sh;
             if (par) want = ~want;
             par = want & 1u;
-            if (pre[i] != want) rp.fail("BinInt2float: n = 2^%u prefix word %u = %08x, want %08x", lg, i, pre[i], want);
+            if (pre[i] != want) rp.fail("BinInt2float: n = %u prefix word %u = %08x, want %08x", n, i, pre[i], want);
+        }
+        if (n <= 1u << 20) {
+            std::vector<float2> S(g.N);
+            PA_HIP(hipMemcpy(S.data(), w->Ys, (size_t)g.N * 8, hipMemcpyDeviceToHost));
+            for (uint32_t c = 0; c < 24 && rp.ok; ++c) {
+                lcg = lcg * 6364136223846793005ull + 1442695040888963407ull;
+                const uint32_t k = (uint32_t)((lcg >> 20) % g.N);
+                std::complex<double> x = 0.0, z = 1.0;  // z[t] = a[t] - i a[t + N], times exp(-i theta t)
+                const std::complex<double> step = std::polar(1.0, -2.0 * M_PI * (k + 0.25) / g.N);
+                for (uint32_t p = 0; p < g.N; ++p, z *= step)
+                    x += z * std::complex<double>(refbit(bin.data(), p) - 0.5, 0.5 - refbit(bin.data(), p + g.N));
+                const float2 v = S[(size_t)(k % g.N1) * g.N2 + k / g.N1];
+                // 2^15 .. 2^20 values of rms sqrt(L) / 2 each, up to 0.5 L near the lines of the low bins
+                if (std::hypot(v.x - x.real(), v.y - x.imag()) > 1e-6 * n)
+                    rp.fail("BinInt2float: n = %u bin %u (%g, %g), want (%g, %g)", n, k, v.x, v.y, x.real(), x.imag());
+            }
         }
         // tb[u N2 + t2]: seed bit t2 + N2 (u + M v) / that + N at mask_bit(D, 0 / 1, v)
         const uint64_t words = tb.size(), checks = std::min<uint64_t>(words, 65536);
@@ -2486,59 +2508,130 @@ int st_unpack(pa_engine* e, Report& rp) {
                 want |= refbit(bin.data(), p) << pa::mask_bit(g.D, 0, v);
                 want |= refbit(bin.data(), p + g.N) << pa::mask_bit(g.D, 1, v);
             }
-            if (tb[idx] != want) rp.fail("BinInt2float: n = 2^%u bit word %llu = %08x, want %08x", lg,
+            if (tb[idx] != want) rp.fail("BinInt2float: n = %u bit word %llu = %08x, want %08x", n,
                                          (unsigned long long)idx, tb[idx], want);
         }
     }
     return rp.done("BinInt2float");
 }
 
+// out[k] = sum over j of in[j step] roots[j k (count / n)], roots[x] = exp(2 pi i x / count), n = 2^a or 3 * 2^a.
+void st_dft(std::complex<double>* out, const std::complex<double>* in, uint32_t n, uint32_t step,
+            const std::vector<std::complex<double>>& roots) {
+    if (n == 1) {
+        out[0] = in[0];
+        return;
+    }
+    const uint32_t r = n % 3 == 0 ? 3 : 2, q = n / r, rs = (uint32_t)roots.size() / n;
+    for (uint32_t i = 0; i < r; ++i) st_dft(out + i * q, in + (size_t)i * step, q, step * r, roots);
+    for (uint32_t k = 0; k < q; ++k) {
+        std::complex<double> x[3];
+        for (uint32_t i = 0; i < r; ++i) x[i] = out[i * q + k];
+        for (uint32_t b = 0; b < r; ++b) {
+            std::complex<double> y = 0.0;
+            for (uint32_t i = 0; i < r; ++i) y += x[i] * roots[(uint64_t)i * (k + b * q) * rs % roots.size()];
+            out[b * q + k] = y;
+        }
+    }
+}
+
 int st_epilogue(pa_engine* e, Report& rp) {
     // ToBinaryArray (:605-737): v[p] = bit 31 - p % 32 of p / 32, corr = 1.9, norm = 1, key rest
-    // 0xAAAAAAAA words; output bit p = v[p] ^ key-rest bit p (NoXOR: v[p]), m = n/4 + n/8, for the
-    // lengths whose output stage is a kernel of its own, n = 2^23 .. 2^27 (shorter ones round and
-    // write in pass A').  round_bit writes the pieces, the production pack stage assembles, XORs and
-    // orders the words.
-    const uint32_t nmax = 1u << 27;
-    DevMem dkey, dnib, dout, dinfo, dq;  // zero prefix parities: the rounded bits come out as they are
-    const size_t info_cap = 1u << 20;
-    ST_ALLOC(dinfo, info_cap);
-    ST_ALLOC(dq, nmax / 8);
-    PA_HIP(hipMemset(dinfo.p, 0, info_cap));
-    PA_HIP(hipMemset(dq.p, 0, nmax / 8));
-    ST_ALLOC(dkey, (nmax / 32 + 2) * 4);
-    ST_ALLOC(dout, nmax / 8 + 64);
-    ST_ALLOC(dnib, (size_t)nmax / 2 + 64);
-    {
-        // key words 0x55555555: key rest word w = (key[h/32+w] << 1) | (key[h/32+w+1] >> 31) = 0xAAAAAAAA
-        std::vector<uint32_t> key(nmax / 32 + 2, 0x55555555u);
-        PA_HIP(hipMemcpy(dkey.p, key.data(), key.size() * 4, hipMemcpyHostToDevice));
-    }
-    for (uint32_t lg = pa::MID_MAX_LOG_N + 2; lg <= 27 && rp.ok; ++lg) {
-        const uint32_t n = 1u << lg, m = n / 4 + n / 8;
-        for (int do_xor = 1; do_xor >= 0 && rp.ok; --do_xor) {
-            Geom g;
-            int rc = make_geom(n, m, PA_COMPRESS | (do_xor ? PA_XOR_KEY_REST : 0u), e->cfg.out_reverse_endian,
-                               e->cfg.max_n_log2, &g);
+    // 0xAAAAAAAA words; output bit p = v[p] ^ key-rest bit p (NoXOR: v[p]), m = n/4 + n/8 and 7n/8, n
+    // = 2^15 .. 2^27 (to the engine's largest) and 3 * 2^k.  The values enter as the pass B output they
+    // stand for and go through the production pass A' with its rounding, and the output
+    // stage.  A part of the columns has the pattern, the others v = 0.  corr: 1.9 - 2 on every conv value,
+    // which is also the rounding margin to be found.
+    const double corr = 1.9 - 2.0;
+    std::vector<uint32_t> sizes;
+    const uint32_t top = std::min(std::max(27u, e->cfg.max_n_log2), (uint32_t)pa::MAX_L_LOG);
+    for (uint32_t lg = pa::SMALL_MAX_LOG_N + 2; lg <= top; ++lg) sizes.push_back(1u << lg);
+    for (uint32_t k : {17u, 19u, 21u, 23u}) sizes.push_back(3u << k);
+    for (uint32_t n : sizes) {
+        if (!rp.ok) break;
+        Geom g;
+        int rc = make_geom(n, n / 2, PA_DEFAULT_FLAGS, e->cfg.out_reverse_endian, e->cfg.max_n_log2, &g);
+        if (rc != PA_OK) return rc;
+        const uint32_t nc = std::min(g.N2, std::max(64u, (1u << 18) / g.N1 & ~31u)), c0 = g.N2 - nc, pops = 12345;
+        using cplx = std::complex<double>;
+        std::vector<cplx> roots(g.N1), x(g.N1), y(g.N1);
+        std::vector<float2> base(g.N1), cols((size_t)nc * g.N1);
+        auto f2 = [](cplx z) { return make_float2((float)z.real(), (float)z.imag()); };
+        for (uint32_t k = 0; k < g.N1; ++k) {
+            roots[k] = std::polar(1.0, 2.0 * M_PI * k / g.N1);
+            // R' of the value 1 at every position of the column
+            base[k] = f2(2.0 * g.N2 / (1.0 - std::polar(1.0, 2.0 * M_PI * (k + 0.25) / g.N1)));
+        }
+        auto mean = [&](uint32_t t2) { return 0.5 * ((pops + t2 + 1u) & 3u); };
+        for (uint32_t c = 0; c < nc; ++c) {
+            const uint32_t t2 = c0 + c;
+            auto conv = [&](uint32_t q) { return (double)(((q >> 5) >> (31u - (q & 31u))) & 1u) + mean(t2) + corr; };
+            for (uint32_t t1 = 0; t1 < g.N1; ++t1) {
+                const uint32_t t = t2 + g.N2 * t1;
+                x[t1] = cplx(conv(t), conv(t + g.N)) * std::polar((double)g.N2, 0.5 * M_PI * t1 / g.N1);
+            }
+            st_dft(y.data(), x.data(), g.N1, 1, roots);
+            for (uint32_t k = 0; k < g.N1; ++k) cols[(size_t)c * g.N1 + k] = f2(y[k]);
+        }
+        const float4 cm = make_float4((float)(mean(0) + corr), (float)(mean(1) + corr), (float)(mean(2) + corr),
+                                      (float)(mean(3) + corr));
+        DevMem dR, dbase, dcols, dkey, dnib, dout, dinfo, dq, dmargin;  // zero prefix parities and conv(R, t)
+        ST_ALLOC(dR, (size_t)g.N * 8);
+        ST_ALLOC(dbase, base.size() * 8);
+        ST_ALLOC(dcols, cols.size() * 8);
+        ST_ALLOC(dkey, ((size_t)n / 32 + 2) * 4);
+        ST_ALLOC(dnib, pa::nib_bytes(g.N));
+        ST_ALLOC(dout, (size_t)n / 8 + 64);
+        ST_ALLOC(dinfo, pa::info_bytes(g));
+        ST_ALLOC(dq, (size_t)g.L / 8);
+        ST_ALLOC(dmargin, 4);
+        PA_HIP(hipMemcpy(dbase.p, base.data(), base.size() * 8, hipMemcpyHostToDevice));
+        PA_HIP(hipMemcpy(dcols.p, cols.data(), cols.size() * 8, hipMemcpyHostToDevice));
+        // key rest word w = (key[h/32+w] << 1) | (key[h/32+w+1] >> 31) = 0xAAAAAAAA
+        PA_HIP(hipMemset(dkey.p, 0x55, ((size_t)n / 32 + 2) * 4));
+        PA_HIP(hipMemset(dq.p, 0, (size_t)g.L / 8));
+        PA_HIP(hipMemset(dinfo.p, 0, pa::info_bytes(g)));
+        PA_HIP(hipMemcpy(dinfo.as<uint32_t>() + pa::INFO_POPS, &pops, 4, hipMemcpyHostToDevice));
+        rc = get_twiddles(e, g.L);
+        if (rc != PA_OK) return rc;
+        const pa::Tables t = tables(e, g.L);
+        std::vector<uint32_t> out;
+        for (uint32_t run = 0; run < 8 && rp.ok; ++run) {
+            const bool do_xor = !(run & 1), with_margin = run & 2;
+            uint32_t flags = do_xor ? PA_XOR_KEY_REST : 0u;
+            if (!is_pow2(n) || run < 6) flags |= PA_COMPRESS;
+            const uint32_t m = run & 4 ? n / 8 * 7 : n / 4 + n / 8;
+            rc = make_geom(n, m, flags, e->cfg.out_reverse_endian, e->cfg.max_n_log2, &g);
             if (rc != PA_OK) return rc;
-            if (pa::info_bytes(g) > info_cap) return PA_ERR_UNSUPPORTED;
-            PA_HIP(pa::launch_st_pieces(dnib.as<uint8_t>(), g, 1.9f, 1.0f, e->stream));
-            PA_HIP(pa::launch_pack(dnib.as<uint8_t>(), dkey.as<uint32_t>(), dout.as<uint32_t>(), g, dinfo.as<uint32_t>(),
-                                   dq.as<uint32_t>(), e->stream));
-            std::vector<uint8_t> out(m / 8);
-            PA_HIP(hipMemcpyAsync(out.data(), dout.p, m / 8, hipMemcpyDeviceToHost, e->stream));
+            float* mg = with_margin ? dmargin.as<float>() : nullptr;
+            PA_HIP(hipMemsetAsync(dmargin.p, 0, 4, e->stream));
+            PA_HIP(pa::launch_st_rows(dR.as<float2>(), g, dbase.as<float2>(), cm, dcols.as<float2>(), c0, nc, e->stream));
+            if (mid_size(g)) {
+                PA_HIP(pa::launch_mid_inv(dR.as<float2>(), dkey.as<uint32_t>(), dout.as<uint32_t>(), g,
+                                          dinfo.as<uint32_t>(), dq.as<uint32_t>(), t, mg, e->stream));
+            } else {
+                PA_HIP(pa::launch_inv_cols(dR.as<float2>(), dnib.as<uint8_t>(), g, dinfo.as<uint32_t>(), t, mg, e->stream));
+                PA_HIP(pa::launch_pack(dnib.as<uint8_t>(), dkey.as<uint32_t>(), dout.as<uint32_t>(), g,
+                                       dinfo.as<uint32_t>(), dq.as<uint32_t>(), e->stream));
+            }
+            out.resize(g.out_bits / 32);
+            float margin = 0.f;
+            PA_HIP(hipMemcpyAsync(out.data(), dout.p, out.size() * 4, hipMemcpyDeviceToHost, e->stream));
+            PA_HIP(hipMemcpyAsync(&margin, dmargin.p, 4, hipMemcpyDeviceToHost, e->stream));
             PA_HIP(hipStreamSynchronize(e->stream));
-            for (uint32_t p = 0; p < m; ++p) {
-                const uint32_t v = ((p >> 5) >> (31u - (p & 31u))) & 1u;
-                const uint32_t want = v ^ (do_xor ? (0xAAAAAAAAu >> (31u - (p & 31u))) & 1u : 0u);
-                uint32_t got;
-                if (g.reverse_endian) got = (out[p >> 3] >> (7u - (p & 7u))) & 1u;
-                else got = refbit(reinterpret_cast<const uint32_t*>(out.data()), p);
+            for (uint32_t w = 0; w < out.size(); ++w) {
+                const uint32_t qw = w + g.out_off / 32;  // conv word
+                const uint32_t v = 32u * qw % g.N2 >= c0 ? qw : 0u;
+                const uint32_t want = v ^ (do_xor && 32u * w < m ? 0xAAAAAAAAu : 0u);
+                const uint32_t got = g.reverse_endian ? __builtin_bswap32(out[w]) : out[w];
                 if (got != want) {
-                    rp.fail("ToBinaryArray%s: n = 2^%u output bit %u = %u, want %u", do_xor ? "" : "NoXOR", lg, p, got, want);
+                    rp.fail("ToBinaryArray%s: n = %u m = %u output word %u = %08x, want %08x", do_xor ? "" : "NoXOR", n, m, w,
+                            got, want);
                     break;
                 }
             }
+            if (with_margin && std::fabs(margin + corr) > 0.01)
+                rp.fail("ToBinaryArray: n = %u m = %u margin %.4f, want %.4f", n, m, margin, -corr);
         }
     }
     return rp.done("ToBinaryArray");

@@ -142,6 +142,7 @@ hipError_t launch_st_correction(const uint32_t* wk, const uint32_t* ws, uint32_t
                                 hipStream_t s);
 hipError_t launch_st_product(const float2* a, const float2* b, float r, float2* prod, const float2* z, float2* zz,
                              uint32_t N, hipStream_t s);
-hipError_t launch_st_pieces(uint8_t* nib, const Geom& g, float corr, float invN, hipStream_t s);
+hipError_t launch_st_rows(float2* R, const Geom& g, const float2* base, float4 c, const float2* cols, uint32_t c0,
+                          uint32_t nc, hipStream_t s);
 
 }  // namespace pa

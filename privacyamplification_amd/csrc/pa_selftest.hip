@@ -40,20 +40,17 @@ __global__ __launch_bounds__(256) void k_st_product(const float2* __restrict__ a
     }
 }
 
-// Pass A' output for the ToBinaryArray closed form (PrivacyAmplification.cu:669-737): the
-// pre-rounding value of conv index p is v[p] = bit 31 - (p mod 32) of the integer p / 32 (0 or 1);
-// the pieces hold round_bit(v * invN + corr) of their positions, in pass A''s layout: bit e of
-// piece[(half N2 + t2) N1/16 + j] is position half N + t2 + N2 (j + (N1/16) e).
-__device__ __forceinline__ float st_pattern(uint32_t p) { return (float)(((p >> 5) >> (31u - (p & 31u))) & 1u); }
-__global__ __launch_bounds__(256) void k_st_pieces(uint16_t* __restrict__ piece, Geom g, float corr, float invN) {
-    const uint64_t e = (uint64_t)blockIdx.x * 256u + threadIdx.x;
-    if (e >= (uint64_t)g.L / 16) return;
-    const uint32_t S = g.N1 / 16u, j = (uint32_t)(e % S), ht = (uint32_t)(e / S);  // ht = half N2 + t2
-    const uint32_t p0 = (ht / g.N2) * g.N + ht % g.N2 + g.N2 * j;
-    float dist = 0.f;
-    uint32_t bits = 0;
-    for (uint32_t k = 0; k < 16; ++k) bits |= round_bit(st_pattern(p0 + g.N2 * S * k) * invN + corr, dist) << k;
-    piece[e] = (uint16_t)bits;
+// Pass B's output R' for the ToBinaryArray closed form (PrivacyAmplification.cu:669-737): column t2 is
+// cols[(t2 - c0) N1 + k1] for c0 <= t2 < c0 + nc, else base[k1] times c's component t2 mod 4; in pass A''s
+// tiles where they are used.
+__global__ __launch_bounds__(256) void k_st_rows(float2* __restrict__ R, Geom g, const float2* __restrict__ base, float4 c,
+                                                 const float2* __restrict__ cols, uint32_t c0, uint32_t nc) {
+    const uint32_t e = blockIdx.x * 256u + threadIdx.x;
+    if (e >= g.N) return;
+    const uint32_t k1 = e / g.N2, t2 = e % g.N2, r = t2 & 3u;
+    const float2 v = t2 >= c0 && t2 - c0 < nc ? cols[(size_t)(t2 - c0) * g.N1 + k1]
+                                              : cscale(base[k1], r == 0u ? c.x : r == 1u ? c.y : r == 2u ? c.z : c.w);
+    R[rt_tiled(g.lg1) ? ((size_t)(t2 / RT_COLS) * g.N1 + k1) * RT_COLS + t2 % RT_COLS : (size_t)e] = v;
 }
 
 hipError_t launch_st_correction(const uint32_t* wk, const uint32_t* ws, uint32_t L, float* out, uint32_t count,
@@ -66,8 +63,9 @@ hipError_t launch_st_product(const float2* a, const float2* b, float r, float2* 
     k_st_product<<<(N + 255u) / 256u, 256, 0, s>>>(a, b, r, prod, z, zz, N);
     return hipGetLastError();
 }
-hipError_t launch_st_pieces(uint8_t* nib, const Geom& g, float corr, float invN, hipStream_t s) {
-    k_st_pieces<<<g.L / 16u / 256u, 256, 0, s>>>(reinterpret_cast<uint16_t*>(nib), g, corr, invN);
+hipError_t launch_st_rows(float2* R, const Geom& g, const float2* base, float4 c, const float2* cols, uint32_t c0,
+                          uint32_t nc, hipStream_t s) {
+    k_st_rows<<<(g.N + 255u) / 256u, 256, 0, s>>>(R, g, base, c, cols, c0, nc);
     return hipGetLastError();
 }
 
