@@ -261,10 +261,7 @@ def run_batched(ctx, steps, warmup, man):
         arr[i].key, arr[i].seed = keys[i].data_ptr(), seeds[i].data_ptr()
         arr[i].n, arr[i].m, arr[i].flags, arr[i].out = n, m, P.DEFAULT_FLAGS, outb[i].data_ptr()
     total_bits = sum(n for n, _, _, _ in spec)
-    def transform_bits(n, m):  # from the key spectrum's buffer, 4 bytes a bit
-        L, touched, _ = P.block_extents(n, m)
-        return touched["spec_key"] // 4 or L
-    padded_bits = sum(transform_bits(n, m) for n, m, _, _ in spec)
+    padded_bits = sum(P.transform_len(n, m) for n, m, _, _ in spec)
 
     def one_per_block():
         for i, (n, m, _, _) in enumerate(spec):

@@ -227,6 +227,11 @@ int pa_stage_timing(pa_engine* eng, int enable);
 int pa_stage_times(pa_engine* eng, const char** names, double* ms, uint32_t* counts,
                    uint32_t* n_stages);
 
+/* Length of the transform that serves a block of this shape, in bits (0 for an unsupported shape): the power of
+ * two that holds it, or three quarters of that.  Short blocks take the direct product instead of it
+ * unless a margin is asked for. */
+uint32_t pa_transform_len(uint32_t n, uint32_t m, uint32_t flags);
+
 /* Bytes of device workspace a block of this shape uses (0 for an unsupported shape). */
 uint64_t pa_workspace_bytes(uint32_t n, uint32_t m, uint32_t flags);
 
@@ -249,8 +254,8 @@ enum pa_buffer {
  * every allocation path gives it (the smallest over the per-size workspace, pa_submit, batch and
  * serving staging; for key, seed and out also the caller contract of the device entry points:
  * key_words * 4, n/8 and m/8 or n/16 bytes).  The engine refuses a shape with touched > alloc
- * (PA_ERR_UNSUPPORTED).  *transform_len receives the power of two that holds the block (the
- * transform itself is 3/4 of it where that suffices, from 2^19 to 2^25).  Runs on the host only. */
+ * (PA_ERR_UNSUPPORTED).  *transform_len receives the power of two that holds the block;
+ * the transform can be shorter (pa_transform_len).  Runs on the host only. */
 int pa_block_extents(uint32_t n, uint32_t m, uint32_t flags, uint32_t* transform_len,
                      uint64_t touched[PA_BUF_COUNT], uint64_t alloc[PA_BUF_COUNT]);
 

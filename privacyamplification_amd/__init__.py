@@ -22,5 +22,6 @@ from .engine import (  # noqa: F401
     load_library,
     out_bytes,
     synth_bits,
+    transform_len,
     workspace_bytes,
 )

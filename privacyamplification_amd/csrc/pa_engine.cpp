@@ -862,6 +862,11 @@ int pa_destroy(pa_engine* e) {
     return PA_OK;
 }
 
+uint32_t pa_transform_len(uint32_t n, uint32_t m, uint32_t flags) {
+    Geom g;
+    return make_geom(n, m, flags, 1, pa::MAX_L_LOG, &g) == PA_OK ? g.L : 0u;
+}
+
 uint64_t pa_workspace_bytes(uint32_t n, uint32_t m, uint32_t flags) {
     Geom g;
     if (make_geom(n, m, flags, 1, 31, &g) != PA_OK) return 0;

@@ -151,6 +151,8 @@ def load_library():
     L.pa_stage_timing.argtypes = [eng, ctypes.c_int]
     L.pa_stage_times.argtypes = [eng, ctypes.POINTER(ctypes.c_char_p), ctypes.POINTER(ctypes.c_double),
                                  ctypes.POINTER(ctypes.c_uint32), ctypes.POINTER(ctypes.c_uint32)]
+    L.pa_transform_len.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32]
+    L.pa_transform_len.restype = ctypes.c_uint32
     L.pa_workspace_bytes.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32]
     L.pa_workspace_bytes.restype = ctypes.c_uint64
     L.pa_block_extents.argtypes = [ctypes.c_uint32, ctypes.c_uint32, ctypes.c_uint32,
@@ -195,6 +197,11 @@ def synth_bits(seed, nbits, p=0.5):
 
 def workspace_bytes(n, m, flags=DEFAULT_FLAGS):
     return int(load_library().pa_workspace_bytes(n, m, flags))
+
+
+def transform_len(n, m, flags=DEFAULT_FLAGS):
+    """Length in bits of the transform that serves a block of this shape (pa_transform_len)."""
+    return int(load_library().pa_transform_len(n, m, flags))
 
 
 def out_bytes(n, m, do_compress=True):

@@ -13,7 +13,7 @@ def test_resident_seeds_stay_in_the_budget(oracle, n):
     fixed = P.workspace_bytes(n, m) + (8 << 20)  # the workspace and the tables of pa_create
     budget = fixed + 4 * n * max(100, (1 << 27) // n)  # room for 100 spectra and more, so that a few percent show
     seed = oracle.synth_bits(0xB0, n)
-    L = P.block_extents(n, m)[1]["spec_key"] // 4 or n
+    L = P.transform_len(n, m)
     kept = 4 * L + (L // 8 if L > 1 << 14 else 0) + (n // 8 if L <= 1 << 18 else 0)  # spectrum, prefix words, seed words
     print(f"[case] n={n} budget {budget}, {kept} bytes a seed", flush=True)
     with P.Engine(max_n_log2=22, hbm_budget_bytes=budget) as eng:
