@@ -137,7 +137,7 @@ uint64_t stage_out_bytes(const Geom& g) { return out_bytes_of(g) + 16; }
 uint64_t ws_key_bytes(uint32_t L) { return (uint64_t)(L / 32 + 2) * 4; }
 uint64_t ws_out_bytes(uint32_t L) { return (uint64_t)L / 8 + 16; }
 
-// one operand's bit masks (none below L = 2^23)
+// one operand's bit masks (none for the mid sizes)
 uint64_t mask_bytes(const Geom& g) {
     return g.N1 == 1 || mid_size(g) ? 0 : (uint64_t)(g.N / g.D) * (g.D == 32 ? 8 : 4);
 }
@@ -155,11 +155,11 @@ struct Extents {
 Extents block_extents(const Geom& g) {
     Extents x;
     const uint64_t N = g.N;
-    // key: pass A, the scan and k_small read words [0, h/32] through key_word(); with the key-rest
+    // key: pass A, the scan, k_direct and k_small read words [0, h/32]; with the key-rest
     // XOR, the output stages read key[h/32 + w + 1] for 32 w < m, i.e. up to word n/32
     x.touched[PA_BUF_KEY] = (uint64_t)(g.do_xor ? g.n / 32 + 1 : g.key_hw + 1) * 4;
     x.touched[PA_BUF_SEED] = (uint64_t)g.seed_words * 4;  // seed_word(): words [0, n/32)
-    // k_pack, k_mid_inv and k_small write output words [0, out_bits / 32)
+    // k_pack, k_mid_inv, k_mix_inv, k_direct and k_small write output words [0, out_bits / 32)
     x.touched[PA_BUF_OUT] = (uint64_t)g.out_bits / 8;
     x.alloc[PA_BUF_KEY] = std::min(stage_key_bytes(g), ws_key_bytes(g.L));
     x.alloc[PA_BUF_SEED] = std::min(stage_seed_bytes(g), ws_key_bytes(g.L));
@@ -205,7 +205,7 @@ struct Workspace {
     float2* Yk = nullptr;      // N complex (key rows / R')
     float2* Ys = nullptr;      // N+1 complex (seed rows)
     float2* Rt = nullptr;      // N complex: pass B's output tiles (rt_tiled(lg1) only)
-    uint32_t* tbk = nullptr;   // N/D words (not below L = 2^23)
+    uint32_t* tbk = nullptr;   // N/D words (not for the mid sizes)
     uint32_t* tbs = nullptr;
     uint8_t* nib = nullptr;    // rounded bits, then prefix words
     uint32_t* info = nullptr;  // scan results (pa_geom.hpp)
@@ -304,8 +304,8 @@ struct pa_engine {
     hipStream_t upload = nullptr;        // pa_run_block: a fresh seed's host-to-device copy
     hipEvent_t upload_done = nullptr, key_up = nullptr;
     float2* tw14 = nullptr;
-    float2* cls = nullptr;  // pass-A class tables (pa::CLS_TABLE_TOTAL entries)
-    int cus = 256;  // compute units of the device (persistent kernels launch one workgroup each)
+    float2* cls = nullptr;  // pass-A class tables (pa::CLS_TABLES_ALL entries)
+    int cus = 256;  // compute units of the device
     std::map<uint32_t, Twiddles> tw;
     std::map<uint32_t, std::unique_ptr<Workspace>> ws;
     std::map<pa_seed_id, Seed> seeds;
@@ -1341,7 +1341,7 @@ std::string tune_key(const BatchGroup& gr) {
 }
 
 // The autotuner: times a group's whole launch sequence (the outputs are rewritten by the real run
-// that follows) over the pass A walk length (column groups per persistent workgroup, for L = 2^23 ..
+// that follows) over the pass A walk length (column groups per persistent workgroup, for L = 2^25 ..
 // 2^27) and records the fastest per (L, seed mode, count).
 int batch_tune_group(pa_engine* e, const BatchPlan& p, BatchGroup& gr, const pa::BlockArgs* tab, hipStream_t s) {
     const Geom& g0 = p.items[gr.idx[0]].g;

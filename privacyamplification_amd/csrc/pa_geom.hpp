@@ -24,14 +24,14 @@
 // a sequence of half its period, or of any power of two below, has.  conv(R, t) mod 2 has R's period,
 // follows from the seed words folded to that period (white_table) and is added back by the output stage.
 //   N = N1 * N2 (t = t2 + N2*t1, k = k1 + N1*k2):
-//   pass A  column FFTs of length N1, 16 columns per workgroup.  L >= 2^23: decimated by D classes of
-//           k1 (M = N1/D per class), input from the bit-transposed key/seed; below, straight from
-//           the words (k_mid_fwd);
+//   pass A  column FFTs of length N1, 16 columns per workgroup.  L >= 2^25: decimated by D classes of
+//           k1 (M = N1/D per class), input from the bit-transposed key/seed; the mid sizes (mid_size:
+//           up to 2^24 and every 3 * 2^k), straight from the words (k_mid_fwd, k_mix_fwd);
 //   pass B  row FFTs of length N2, complex product, inverse row FFTs;
-//   pass A' inverse column FFTs of length N1, rounding; below L = 2^23 the output words too.
-// L >= 2^23 has N2 = 8192.  Below, N1 is 2^6 .. 2^9 and N2 = N / N1 is 2^8 .. 2^12 (mid_lg1): as many row
-// and column workgroups as the length allows, because there the time is one workgroup's latency --
-// at N2 = 8192 a row's three transforms alone take 20 us on one compute unit.
+//   pass A' inverse column FFTs of length N1, rounding; for the mid sizes the output words too.
+// L >= 2^23 has N2 = 8192.  Below, N1 is 2^6 .. 2^9 and N2 = N / N1 is 2^8 .. 2^12 (mid_lg1; N1 is 2^9 and 2^10
+// at 2^23 and 2^24): as many row and column workgroups as the length allows, because there the time is one
+// workgroup's latency -- at N2 = 8192 a row's three transforms alone take 20 us on one compute unit.
 // N <= 8192 (L <= 2^14) runs fully on chip in one workgroup (small path).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -155,7 +155,7 @@ __host__ __device__ inline uint32_t info_fold(const Geom& g) { return info_pops(
 inline uint64_t info_bytes(const Geom& g) { return ((uint64_t)info_fold(g) + (uint64_t)fold_slices(g) * g.white) * 4u; }
 
 // One block of a batched launch: its geometry and device buffers.  The blocks of one launch share
-// the transform length L (and so N1, N2, M, D, W); n, m, flags and the buffers are per block.
+// the transform length L (and so N1, N2, M, D); n, m, flags and the buffers are per block.
 struct BlockArgs {
     Geom g;
     const uint32_t* key;
@@ -165,7 +165,7 @@ struct BlockArgs {
     const uint32_t* sq;     // resident seed prefix words when seed == nullptr (four-step path only)
     float2* Yk;             // N values (four-step path only)
     float2* Ys;             // N+1 values (dynamic seed, four-step path only)
-    uint32_t* tbk;          // bit masks (N1 > 2^9 or N2 = 8192 only)
+    uint32_t* tbk;          // bit masks (not for mid_size)
     uint32_t* tbs;
     float2* Rt;             // R' tiles (rt_tiled(lg1)), else nullptr
     uint8_t* nib;

@@ -8,8 +8,8 @@
 //
 //   k_transpose_bits  key/seed RefBits -> per-(class,column) bit masks for pass A
 //   k_fwd_cols        pass A: decimated column FFTs of the +-1/2-encoded bits (R2C forward part);
-//   k_mid_fwd         its form for L <= 2^24, straight from the key's and the seed's words.
-//                     Their launches also scan the inputs' popcounts (binInt2float's popcount,
+//   k_mid_fwd         its form for L <= 2^24, straight from the key's and the seed's words, and
+//   k_mix_fwd         for L = 3 * 2^k.  Their launches (the bit transpose's from 2^25 on) also scan the inputs' popcounts (binInt2float's popcount,
 //                     PrivacyAmplification.cu:570-602) and prefix parities
 //   k_rows            pass B: row FFTs, complex product (ElementWiseProduct, :465-481), inverse row FFTs
 //   k_inv_cols        pass A': inverse column FFTs + round-mod-2 (ToBinaryArray :739-783)
@@ -18,7 +18,9 @@
 //                     XOR and byte order (key2StartRest's key_rest :873-878, ToBinaryArray's bswap
 //                     XOR :757-762)
 //   k_inv_big1, 2     pass A' for L >= 2^28
-//   k_mid_inv         pass A' and the output in one for L <= 2^24
+//   k_mid_inv         pass A' and the output in one for L <= 2^24, and
+//   k_mix_inv         for L = 3 * 2^k
+//   k_direct          short blocks without a transform
 //   k_small           the whole block in one workgroup for L <= 2^14
 #include <hip/hip_runtime.h>
 
@@ -113,8 +115,8 @@ __global__ __launch_bounds__(COPY_NT) void k_copies(const CopyDesc* __restrict__
 // end of the output window), the chunk's parity to its byte of cp, its popcount (key + seed) to its
 // entry; for the mid sizes also the XOR of its seed words per word of the whitening's period (the bit
 // transpose has the others').  x is the whitened key.  A resident seed brings its own finished prefix
-// words sq; x alone is scanned then.  The scan workgroups ride in the bit transpose's launch (in pass A's below
-// L = 2^23); scan_finish, in pass B's, turns the entries into what pass A' and the output stage read.
+// words sq; x alone is scanned then.  The scan workgroups ride in the bit transpose's launch (in pass A's for the
+// mid sizes); scan_finish, in pass B's, turns the entries into what pass A' and the output stage read.
 // (In pass A's launch at 2^27 they cost 15 us: with its 74 KB of LDS only two fit a compute unit.)
 __device__ __forceinline__ uint32_t prefix_bits(uint32_t w) {  // bit p: parity of bits 0..p, MSB first
     w ^= w >> 1;
@@ -1588,7 +1590,7 @@ __global__ __launch_bounds__(PACK_NT) void k_pack(const uint8_t* __restrict__ ni
     }
 }
 
-// Pass A' and the output in one for L <= 2^22: 16 columns per workgroup, plan R1 x 16 (R1 x 32 at 512).
+// Pass A' and the output in one for L <= 2^24: 16 columns per workgroup, plan R1 x 16 (R1 x 32 at 512).
 // A wave's 64 lanes are 16 columns x 4 rows, so a ballot is 4 rows' 16 bits: half an output word
 // each, corrected and written as 16 bits.
 template <int LG1, bool BATCH>
@@ -1964,8 +1966,8 @@ __global__ __launch_bounds__(small_threads(LGN)) void k_small(
 // (U_{k+1} : U_k) >> s, one funnel shift per lane s, serves R output words.
 // A workgroup has R output words; its half-waves (lanes s) share out the key in chunks of 16 words.
 // Bound by the vector ALU from 2^17 bits on (1 T word products a second) and by the launch below: calls of
-// 2^10 to 2^16 bits take 6.8 to 7.5 us one after another, where the one-workgroup transform took 18 to 27
-// and the three launches of the mid-size one 17 to 18.
+// 2^10 to 2^16 bits take 4.5 to 5.8 us one after another, where the one-workgroup transform took 18 to 27
+// and the three launches of the mid-size one 17 to 18; 3.2 of it is the kernel at 2^12.
 template <int R, bool BATCH>
 __global__ __launch_bounds__(DIRECT_NT_MAX) void k_direct(const uint32_t* __restrict__ key,
                                                           const uint32_t* __restrict__ seed, uint32_t* __restrict__ out,

@@ -16,7 +16,7 @@ enum { ROWS_DYN = 0, ROWS_STATIC = 1, ROWS_SEEDPREP = 2 };
 __host__ __device__ constexpr int rows_per_wg(int lg2) { return lg2 == 8 ? 4 : lg2 == 9 ? 2 : 1; }
 __host__ __device__ constexpr int rows_per_wg_many(int lg2) { return lg2 >= 12 ? 1 : 4096 >> lg2; }
 __host__ __device__ constexpr int rows_threads(int lg2, int rpw) { return lg2 == 13 ? 256 : rpw * (1 << lg2) / 16; }
-// Column passes for L <= 2^22: threads and first radix (16 columns, one second-stage butterfly each).
+// Column passes of the mid sizes, powers of two: threads and first radix (16 columns, one second-stage butterfly each).
 __host__ __device__ constexpr int mid_threads(int lg1) { return lg1 >= 10 ? 512 : lg1 >= 8 ? 256 : 1 << lg1; }
 __host__ __device__ constexpr int mid_r1(int lg1) { return lg1 >= 10 ? 32 : lg1 >= 8 ? 16 : 1 << (lg1 - 4); }
 constexpr int TB_NT = 128;        // bit-transpose threads: 32 outputs each
