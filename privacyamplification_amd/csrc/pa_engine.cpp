@@ -215,9 +215,11 @@ struct Workspace {
     uint64_t bytes = 0;
     // The last stream that used this workspace and an event recorded after its last kernel: a
     // block on another stream waits for it, so calls on two streams serialise instead of
-    // overwriting each other's spectra.
+    // overwriting each other's spectra.  A direct product records none (the event takes as long as its
+    // kernel); the next call on another stream does.
     hipStream_t last_stream = nullptr;
     hipEvent_t last_done = nullptr;
+    bool recorded = false;
 };
 
 struct Seed {
@@ -677,20 +679,44 @@ bool direct_block(const Geom& g, const float* margin, const uint32_t* key, const
     return apart(key, key_words_for(g)) && apart(seed, g.seed_words);
 }
 
+// Makes s wait for the workspace's last use, if that was on another stream.
+int wait_for_last(Workspace* w, hipStream_t s) {
+    if (!w->last_stream || w->last_stream == s) return PA_OK;
+    if (!w->recorded) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        // a destroyed stream has finished; into one that is being captured nothing can be recorded
+        if (hipStreamIsCapturing(w->last_stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+            hipEventRecord(w->last_done, w->last_stream) != hipSuccess) {
+            (void)hipGetLastError();
+            return PA_OK;
+        }
+        w->recorded = true;
+    }
+    PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
+    return PA_OK;
+}
+
 // Orders the workspace's uses across streams (not while s is being captured into a graph: a
 // capture only records work, and the caller owns the ordering of its replays).
 int run_device(pa_engine* e, const Geom& g, Workspace* w, const uint32_t* key, const uint32_t* seed,
                const Seed* sd, uint32_t* out, hipStream_t s, float* margin, const SeedUpload* su = nullptr) {
-    if (direct_block(g, margin, key, seed, out))  // uses no scratch of the workspace
+    const bool direct = direct_block(g, margin, key, seed, out);
+    if (direct && w->last_stream == s) {
+        w->recorded = false;
         return run_device_body(e, g, w, key, seed, sd, out, s, margin, su);
+    }
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     PA_HIP(hipStreamIsCapturing(s, &cap));
     const bool guard = cap == hipStreamCaptureStatusNone;
-    if (guard && w->last_stream && w->last_stream != s) PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
+    if (guard) {
+        const int rc = wait_for_last(w, s);
+        if (rc != PA_OK) return rc;
+    }
     const int rc = run_device_body(e, g, w, key, seed, sd, out, s, margin, su);
     if (rc != PA_OK) return rc;
     if (guard) {
-        PA_HIP(hipEventRecord(w->last_done, s));
+        if (!direct) PA_HIP(hipEventRecord(w->last_done, s));
+        w->recorded = !direct;
         w->last_stream = s;
     }
     return PA_OK;
@@ -917,7 +943,8 @@ int pa_seed_put(pa_engine* e, const uint32_t* seed, uint32_t n, uint32_t m, int3
     auto launch = [&]() -> int {
         hipStream_t s = e->stream;
         // the workspace's masks and info words are scratch here: after a block on another stream
-        if (w->last_stream && w->last_stream != s) PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
+        const int order = wait_for_last(w, s);
+        if (order != PA_OK) return order;
         uint32_t* src = sd.words ? sd.words : w->d_seed;
         PA_HIP(hipMemcpyAsync(src, seed, (size_t)(n / 32) * 4, hipMemcpyHostToDevice, s));
         const pa::Tables t = tables(e, g.L);

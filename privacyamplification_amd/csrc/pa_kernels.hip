@@ -9,7 +9,8 @@
 //   k_transpose_bits  key/seed RefBits -> per-(class,column) bit masks for pass A
 //   k_fwd_cols        pass A: decimated column FFTs of the +-1/2-encoded bits (R2C forward part);
 //   k_mid_fwd         its form for L <= 2^24, straight from the key's and the seed's words, and
-//   k_mix_fwd         for L = 3 * 2^k.  Their launches (the bit transpose's from 2^25 on) also scan the inputs' popcounts (binInt2float's popcount,
+//   k_mix_fwd         for L = 3 * 2^k.  Their launches (the bit transpose's from 2^25 on) also scan
+//                     the inputs' popcounts (binInt2float's popcount,
 //                     PrivacyAmplification.cu:570-602) and prefix parities
 //   k_rows            pass B: row FFTs, complex product (ElementWiseProduct, :465-481), inverse row FFTs
 //   k_inv_cols        pass A': inverse column FFTs + round-mod-2 (ToBinaryArray :739-783)
