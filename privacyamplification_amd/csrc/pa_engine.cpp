@@ -684,13 +684,13 @@ int wait_for_last(Workspace* w, hipStream_t s) {
     if (!w->last_stream || w->last_stream == s) return PA_OK;
     if (!w->recorded) {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        // a destroyed stream has finished; into one that is being captured nothing can be recorded
-        if (hipStreamIsCapturing(w->last_stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
-            hipEventRecord(w->last_done, w->last_stream) != hipSuccess) {
+        // a destroyed stream has finished; into one that is being captured nothing can be recorded, and
+        // what the event has from before is waited for
+        if (hipStreamIsCapturing(w->last_stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone &&
+            hipEventRecord(w->last_done, w->last_stream) == hipSuccess)
+            w->recorded = true;
+        else
             (void)hipGetLastError();
-            return PA_OK;
-        }
-        w->recorded = true;
     }
     PA_HIP(hipStreamWaitEvent(s, w->last_done, 0));
     return PA_OK;

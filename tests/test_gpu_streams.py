@@ -42,3 +42,33 @@ def test_second_stream_comes_second(oracle, n, routes):
             run(1)
             torch.cuda.synchronize()
             assert np.array_equal(out.cpu().numpy(), ref), (n, routes)
+
+
+def test_first_stream_being_captured(oracle):
+    """A short block on a stream that is then captured, and one on another stream meanwhile: neither call fails."""
+    import torch
+    n, m = 4096, 1536
+    up = lambda a: torch.from_numpy(a.view(np.int32).copy()).cuda()
+    key, seed = oracle.synth_bits(0x67, n + 1), oracle.synth_bits(0x68, n)
+    ref = oracle.amp_out(key, seed, n, m, True, True, method=oracle.DIRECT)
+    print("[case] n=4096, capture on the stream of the last block", flush=True)
+    with P.Engine(max_n_log2=20) as eng:
+        dk, ds = up(key), up(seed)
+        outs = [torch.zeros(m // 8, dtype=torch.uint8, device="cuda") for _ in range(2)]
+        streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+        run = lambda o, s: eng.block_device(dk.data_ptr(), ds.data_ptr(), n, m, 3, outs[o].data_ptr(), s.cuda_stream)
+        run(0, streams[1])
+        run(0, streams[0])
+        torch.cuda.synchronize()
+        outs[0].zero_()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=streams[0], capture_error_mode="relaxed"):
+            run(0, streams[0])
+            run(1, streams[1])
+        for _ in range(3):
+            outs[0].zero_()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert np.array_equal(outs[0].cpu().numpy(), ref)
+        assert np.array_equal(outs[1].cpu().numpy(), ref)
